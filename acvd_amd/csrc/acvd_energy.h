@@ -26,18 +26,42 @@ struct EnergyArgs {
   const EnergyMesh* meshes;
   const int32_t* item_mesh;  // null for one mesh
   const int32_t* clus_mesh;  // null for one mesh
-  const int32_t* tri;        // 3 global vertex ids per face
-  const int32_t* vfptr;      // vertex -> incident faces (mesh-local face ids)
+  const int32_t* tri;        // 3 global vertex ids per face (contexts with QEM meshes; else null)
+  const int32_t* vfptr;      // vertex -> incident faces, one entry per corner
   const int32_t* vfcol;
+  // rings (faces around each QEM vertex as chains of neighbour ids): group g of
+  // 64 items holds slots [ring_slot[g], ring_slot[g + 1]) of 64 ids
+  const int32_t* ring_slot;
+  const int32_t* ring;
   // inputs of one call
   const float* xyz;          // 3 per item
   const float* w;            // 1 per item
   const int32_t* labels;     // mesh-local cluster ids, K or out of range = none
   // state kept from the forward for the backward
-  double* acc;               // 13 per cluster: W, S[3], Q[9]
-  double* pts;               // 6 per cluster: centroid, point
-  double* adj;               // 12 per cluster: dE/dQ[9], (dE/dc)/W
+  int32_t acc_stride;        // 13 with QEM meshes, else 4
+  double* acc;               // per cluster: W, S[3] and (QEM) Q[9]
+  double* pts;               // 4 per cluster: point, unused
+  double* adj;               // kAdjStride per cluster (null without QEM meshes): for a unit gradient
+                             // dE/dQ[9], (dE/dc)/W [3]; centroid [3]
 };
+
+constexpr int kAdjStride = 16;
+// Ring entries: a neighbour id; with the sign bit set the first id of a chain;
+// kRingEnd past the end; kRingLong (first entry alone) for a vertex of more than
+// kRingFaces faces, whose faces are read from its vertex -> face row.
+constexpr int32_t kRingEnd = -1;
+constexpr int32_t kRingLong = -2;
+constexpr int32_t kRingId = 0x7fffffff;
+constexpr int kRingFaces = 16;
+constexpr int kRingChunk = 8;  // ids read at once
+
+// Device build of the vertex -> face rows and rings.
+hipError_t energy_offset_tri(hipStream_t s, int64_t n3, int32_t off, int32_t* tri);
+hipError_t energy_vf_count(hipStream_t s, int64_t n3, const int32_t* tri, int32_t* deg);
+hipError_t energy_vf_fill(hipStream_t s, int64_t n, int64_t n3, const int32_t* tri, const int32_t* vfptr,
+                          int32_t* fill, int32_t* vfcol);
+hipError_t energy_ring_slots(hipStream_t s, const EnergyArgs& a, int32_t* slots);
+hipError_t energy_ring_fill(hipStream_t s, const EnergyArgs& a, const int32_t* slot, int32_t* ring);
 
 hipError_t energy_forward(hipStream_t s, const EnergyArgs& a, double* energy, int n_meshes);
 // Largest cluster count of energy_forward_cvt_noalloc (its static scratch).

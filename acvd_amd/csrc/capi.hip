@@ -1844,9 +1844,10 @@ struct acvd_energy {
   bool built = false;
   int64_t N = 0, K = 0, F = 0;
   DBuf<EnergyMesh> d_meshes;
-  DBuf<int32_t> d_item_mesh, d_clus_mesh, d_tri, d_vfptr, d_vfcol;
+  DBuf<int32_t> d_item_mesh, d_clus_mesh, d_topo, d_ring;  // d_topo: tri, vfptr, vfcol, ring_slot
   DBuf<double> d_acc, d_pts, d_adj;
   bool have_forward = false;
+  bool any_qem = false;
   EnergyArgs args() const {
     EnergyArgs a{};
     a.n_items = N;
@@ -1854,12 +1855,17 @@ struct acvd_energy {
     a.meshes = d_meshes.p;
     a.item_mesh = meshes.size() > 1 ? d_item_mesh.p : nullptr;
     a.clus_mesh = meshes.size() > 1 ? d_clus_mesh.p : nullptr;
-    a.tri = d_tri.p;
-    a.vfptr = d_vfptr.p;
-    a.vfcol = d_vfcol.p;
+    if (any_qem) {
+      a.tri = d_topo.p;
+      a.vfptr = d_topo.p + 3 * F;
+      a.vfcol = d_topo.p + 3 * F + N + 1;
+      a.ring_slot = d_topo.p + 6 * F + N + 1;
+      a.ring = d_ring.p;
+    }
+    a.acc_stride = any_qem ? 13 : 4;
     a.acc = d_acc.p;
     a.pts = d_pts.p;
-    a.adj = d_adj.p;
+    a.adj = any_qem ? d_adj.p : nullptr;
     return a;
   }
 };
@@ -1880,18 +1886,17 @@ int energy_build(acvd_energy* e) {
   if (N >= (int64_t(1) << 31) - 1 || K >= (int64_t(1) << 31) - 1 || 3 * F >= (int64_t(1) << 31))
     return fail(ACVD_ERR_LIMIT, "energy context exceeds 2^31 items, clusters or face corners");
   std::vector<EnergyMesh> hm(M);
-  std::vector<int32_t> tri(3 * F), item_mesh, clus_mesh, vfptr(N + 1, 0), vfcol(3 * F);
+  std::vector<int32_t> item_mesh, clus_mesh;
   if (M > 1) {
     item_mesh.resize(N);
     clus_mesh.resize(K);
   }
+  e->any_qem = false;
   int64_t io = 0, co = 0, fo = 0;
   for (int m = 0; m < M; ++m) {
     const auto& h = e->meshes[m];
     hm[m] = EnergyMesh{io, h.nv, co, fo, h.K, h.metric, h.level, 0};
-    for (int64_t k = 0; k < 3 * h.nf; ++k) tri[3 * fo + k] = int32_t(h.tri[k] + io);
-    // vertex -> faces (mesh-local face ids), faces by increasing id
-    for (int64_t k = 0; k < 3 * h.nf; ++k) vfptr[io + h.tri[k] + 1]++;
+    e->any_qem |= h.metric == ACVD_METRIC_QEM;
     if (M > 1) {
       std::fill(item_mesh.begin() + io, item_mesh.begin() + io + h.nv, m);
       std::fill(clus_mesh.begin() + co, clus_mesh.begin() + co + h.K, m);
@@ -1899,15 +1904,6 @@ int energy_build(acvd_energy* e) {
     io += h.nv;
     co += h.K;
     fo += h.nf;
-  }
-  for (int64_t i = 0; i < N; ++i) vfptr[i + 1] += vfptr[i];
-  {
-    std::vector<int32_t> fill(vfptr.begin(), vfptr.end() - 1);
-    for (int m = 0; m < M; ++m) {
-      const auto& h = e->meshes[m];
-      for (int64_t f = 0; f < h.nf; ++f)
-        for (int j = 0; j < 3; ++j) vfcol[fill[hm[m].item_off + h.tri[3 * f + j]]++] = int32_t(f);
-    }
   }
   HIP_TRY(e->d_meshes.alloc(M));
   HIP_TRY(hipMemcpy(e->d_meshes.p, hm.data(), M * sizeof(EnergyMesh), hipMemcpyHostToDevice));
@@ -1917,18 +1913,51 @@ int energy_build(acvd_energy* e) {
     HIP_TRY(hipMemcpy(e->d_item_mesh.p, item_mesh.data(), N * sizeof(int32_t), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(e->d_clus_mesh.p, clus_mesh.data(), K * sizeof(int32_t), hipMemcpyHostToDevice));
   }
-  HIP_TRY(e->d_tri.alloc(3 * F));
-  HIP_TRY(hipMemcpy(e->d_tri.p, tri.data(), 3 * F * sizeof(int32_t), hipMemcpyHostToDevice));
-  HIP_TRY(e->d_vfptr.alloc(N + 1));
-  HIP_TRY(hipMemcpy(e->d_vfptr.p, vfptr.data(), (N + 1) * sizeof(int32_t), hipMemcpyHostToDevice));
-  HIP_TRY(e->d_vfcol.alloc(3 * F));
-  HIP_TRY(hipMemcpy(e->d_vfcol.p, vfcol.data(), 3 * F * sizeof(int32_t), hipMemcpyHostToDevice));
-  HIP_TRY(e->d_acc.alloc(13 * K));
-  HIP_TRY(e->d_pts.alloc(6 * K));
-  HIP_TRY(e->d_adj.alloc(12 * K));
+  HIP_TRY(e->d_acc.alloc((e->any_qem ? 13 : 4) * K));
+  HIP_TRY(e->d_pts.alloc(4 * K));
+  e->d_topo.release();
+  e->d_ring.release();
+  e->d_adj.release();
   e->N = N;
   e->K = K;
   e->F = F;
+  if (e->any_qem) {  // the isotropic energy needs no faces
+    const hipStream_t s = nullptr;  // as the copies above: the default stream
+    const int64_t G = (N + 63) / 64;
+    HIP_TRY(e->d_adj.alloc(kAdjStride * K));
+    HIP_TRY(e->d_topo.alloc(6 * F + (N + 1) + (G + 1)));
+    int32_t* tri = e->d_topo.p;
+    int32_t* vfptr = tri + 3 * F;
+    int32_t* vfcol = vfptr + N + 1;
+    int32_t* ring_slot = vfcol + 3 * F;
+    DBuf<int32_t> tmp;  // face counts, fill counts, ring slots
+    struct Tmp {  // scan workspace
+      void* p = nullptr;
+      size_t n = 0;
+      ~Tmp() {
+        if (p) (void)hipFree(p);
+      }
+    } scan;
+    HIP_TRY(tmp.alloc((N + 1) + N + (G + 1)));
+    int32_t *deg = tmp.p, *fill = deg + N + 1, *slots = fill + N;
+    HIP_TRY(hipMemsetAsync(tmp.p, 0, tmp.n * sizeof(int32_t), s));
+    for (int m = 0; m < M; ++m) {
+      const auto& h = e->meshes[m];
+      int32_t* t = tri + 3 * hm[m].face_off;
+      HIP_TRY(hipMemcpy(t, h.tri.data(), 3 * h.nf * sizeof(int32_t), hipMemcpyHostToDevice));
+      HIP_TRY(energy_offset_tri(s, 3 * h.nf, int32_t(hm[m].item_off), t));
+    }
+    HIP_TRY(energy_vf_count(s, 3 * F, tri, deg));
+    HIP_TRY(exclusive_scan_i32(s, deg, vfptr, N + 1, &scan.p, &scan.n));
+    HIP_TRY(energy_vf_fill(s, N, 3 * F, tri, vfptr, fill, vfcol));
+    HIP_TRY(energy_ring_slots(s, e->args(), slots));
+    HIP_TRY(exclusive_scan_i32(s, slots, ring_slot, G + 1, &scan.p, &scan.n));
+    int32_t total = 0;
+    HIP_TRY(hipMemcpy(&total, ring_slot + G, sizeof(int32_t), hipMemcpyDeviceToHost));
+    HIP_TRY(e->d_ring.alloc(64 * size_t(total)));
+    HIP_TRY(energy_ring_fill(s, e->args(), ring_slot, e->d_ring.p));
+    HIP_TRY(hipStreamSynchronize(s));  // a caller's stream need not wait for the default one
+  }
   e->built = true;
   return ACVD_OK;
 }

@@ -14,17 +14,26 @@
 // quadrics are recomputed from the positions (so that they are differentiable),
 // unlike the sweep, which uses FP32 vertex quadrics.
 //
-// Forward: cluster sums (W, S, Q) with block-level LDS aggregation and FP64
-// atomics, cluster points, per-mesh energy.  Backward (adjoint): per cluster,
-// dE/dq = -2 gE (S - W q) is pulled back through q(c, A, b) -- the truncated
-// pseudo-inverse's derivative includes the coupling of kept and dropped
-// eigen-directions -- into dE/dQ (9 entries) and dE/dc; then per vertex the
-// direct terms, the centroid path and the face-quadric path (over the faces
-// around the vertex, recomputed, no per-item partials stored) give dE/dx and
-// dE/dw.
+// Forward: cluster sums (W, S, Q), cluster points, per-mesh energy.  The
+// points kernel also computes the adjoint of each QEM cluster for a unit
+// upstream gradient (dE/dq = -2 (S - W q) pulled back through q(c, A, b); the
+// truncated pseudo-inverse's derivative includes the coupling of kept and
+// dropped eigen-directions) into dE/dQ (9 entries) and dE/dc: the adjoint is
+// linear in the gradient, and the eigen-decomposition is at hand.  Backward:
+// per vertex the direct terms, the centroid path and the face-quadric path
+// (over the faces around the vertex, recomputed, no per-item partials stored)
+// give dE/dx and dE/dw.
+//
+// The faces around a vertex v are read as a chain of neighbour ids (the ring):
+// two ids in a row are the other two vertices of a face, in its orientation, so
+// an interior vertex of valence d takes d + 1 ids and one position gather per
+// neighbour, instead of d face ids, 3 d vertex ids and 3 d positions.  The rings
+// of 64 consecutive vertices are stored slot by slot (slot s of all 64, then
+// slot s + 1): one 256-byte load per slot and wave.
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "acvd_energy.h"
@@ -34,49 +43,87 @@ namespace acvd {
 namespace {
 
 constexpr int kEBlock = 256;
-constexpr int kAcc = 13;  // W, Sx, Sy, Sz, Q0..Q8
+constexpr int kAccBlock = 512;          // threads of ke_accumulate and ke_energy
+constexpr int kAccMaxBlocks = 512;      // 2 blocks of ke_accumulate per CU (its registers)
 constexpr double kThreshold = 1e-3;
 
 inline unsigned egrid(int64_t n) { return unsigned((n + kEBlock - 1) / kEBlock); }
 
 __device__ inline int mesh_of(const EnergyArgs& a, int64_t i) { return a.item_mesh ? a.item_mesh[i] : 0; }
 
-// global cluster of item i, or -1
-__device__ inline int64_t cluster_of(const EnergyArgs& a, int64_t i, int m) {
-  const EnergyMesh& em = a.meshes[m];
-  const int32_t l = a.labels[i];
-  if (l < 0 || l >= em.K) return -1;
-  return em.clus_off + l;
+// global cluster of an item labelled l, or -1
+__device__ inline int32_t cluster_of(const EnergyMesh& em, int32_t l) {
+  return (l < 0 || l >= em.K) ? -1 : int32_t(em.clus_off) + l;
 }
 
-// plane quadric entries 0..8 of face f ([n;d][n;d]^T upper part, without d^2)
-__device__ inline void face_plane(const EnergyArgs& a, int64_t f, double p[4], double x1[3], double u[3],
-                                  double v[3]) {
-  const int32_t i0 = a.tri[3 * f], i1 = a.tri[3 * f + 1], i2 = a.tri[3 * f + 2];
-  double x2[3], x3[3];
-  for (int k = 0; k < 3; ++k) {
-    x1[k] = double(a.xyz[3 * int64_t(i0) + k]);
-    x2[k] = double(a.xyz[3 * int64_t(i1) + k]);
-    x3[k] = double(a.xyz[3 * int64_t(i2) + k]);
-    u[k] = x2[k] - x1[k];
-    v[k] = x3[k] - x1[k];
+struct Vec3 {
+  double x, y, z;
+};
+
+__device__ inline Vec3 load_point(const float* __restrict__ xyz, int64_t i) {
+  return Vec3{double(xyz[3 * i]), double(xyz[3 * i + 1]), double(xyz[3 * i + 2])};
+}
+
+__device__ inline Vec3 sub(const Vec3& a, const Vec3& b) { return Vec3{a.x - b.x, a.y - b.y, a.z - b.z}; }
+
+// Normal of the face (v, v + u, v + w) (plain products, so that a degenerate
+// face gives an exact zero).
+__device__ inline Vec3 cross(const Vec3& u, const Vec3& w) {
+  return Vec3{u.y * w.z - u.z * w.y, u.z * w.x - u.x * w.z, u.x * w.y - u.y * w.x};
+}
+
+struct RingPoint {
+  float x, y, z;
+};
+
+__device__ inline Vec3 ring_point(const EnergyArgs& a, int32_t e) {
+  return load_point(a.xyz, int64_t(e & kRingId));
+}
+
+// The first kRingChunk ring entries of item i (64 consecutive items per wave:
+// i = 64 g + lane), loaded together; returns the group's slots.
+__device__ inline int32_t load_ring(const EnergyArgs& a, int64_t i, int32_t e[kRingChunk]) {
+  const int64_t g = __builtin_amdgcn_readfirstlane(int32_t(i >> 6));
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int k = 0; k < kRingChunk; ++k) e[k] = kRingEnd;
+  if (64 * g >= a.n_items) return 0;  // a wave past the last group
+  const int32_t s0 = a.ring_slot[g], n = a.ring_slot[g + 1] - s0;  // scalar loads
+#pragma unroll
+  for (int k = 0; k < kRingChunk; ++k)
+    if (k < n) e[k] = a.ring[int64_t(s0 + k) * 64 + lane];
+  return n;
+}
+
+// Faces around item i past its first `from` ring entries (u: the previous ring
+// vertex less the item's position, cu: its tag), and those of a vertex with more
+// faces than a ring holds: the paths of rare vertices, an entry at a time.
+// tag(id) labels a ring vertex; face(u, cu, s, cs) takes a face.
+template <class Tag, class Face>
+__device__ inline void walk_rest(const EnergyArgs& a, int64_t i, const Vec3& x, int32_t first, int from, Vec3 u,
+                                 int32_t cu, Tag&& tag, Face&& face) {
+  if (first == kRingLong) {
+    for (int32_t k = a.vfptr[i]; k < a.vfptr[i + 1]; ++k) {
+      const int64_t f = a.vfcol[k];
+      // the corner of this entry: a face listed more than once for the vertex
+      // (a degenerate face, whose normal is zero) takes its first corner
+      int j = 0;
+      while (j < 2 && a.tri[3 * f + j] != int32_t(i)) ++j;
+      const int32_t v1 = a.tri[3 * f + (j + 1) % 3], v2 = a.tri[3 * f + (j + 2) % 3];
+      face(sub(load_point(a.xyz, v1), x), tag(v1), sub(load_point(a.xyz, v2), x), tag(v2));
+    }
+    return;
   }
-  p[0] = u[1] * v[2] - u[2] * v[1];
-  p[1] = u[2] * v[0] - u[0] * v[2];
-  p[2] = u[0] * v[1] - u[1] * v[0];
-  p[3] = -(p[0] * x1[0] + p[1] * x1[1] + p[2] * x1[2]);
-}
-
-__device__ inline void plane_to_q9(const double p[4], double q[9]) {
-  q[0] = p[0] * p[0];
-  q[1] = p[0] * p[1];
-  q[2] = p[0] * p[2];
-  q[3] = p[0] * p[3];
-  q[4] = p[1] * p[1];
-  q[5] = p[1] * p[2];
-  q[6] = p[1] * p[3];
-  q[7] = p[2] * p[2];
-  q[8] = p[2] * p[3];
+  const int32_t s0 = a.ring_slot[i >> 6], s1 = a.ring_slot[(i >> 6) + 1];
+  for (int32_t s = s0 + from; s < s1; ++s) {
+    const int32_t e = a.ring[int64_t(s) * 64 + (i & 63)];
+    if (e == kRingEnd) break;
+    const Vec3 t = sub(ring_point(a, e), x);
+    const int32_t ct = tag(e & kRingId);
+    if (e >= 0) face(u, cu, t, ct);
+    u = t;
+    cu = ct;
+  }
 }
 
 // Symmetric 3x3 eigen-decomposition by cyclic Jacobi to convergence.
@@ -149,83 +196,329 @@ __device__ inline void kept_set(const double lam[3], int level, bool keep[3]) {
 
 __device__ inline double dot3(const double* a, const double* b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; }
 
-// ------------------------------------------------------------------ forward
-__global__ __launch_bounds__(kEBlock) void ke_zero(int64_t n, double* p) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0.0;
+// ---------------------------------------------------------------- ring build
+__global__ void ke_offset_tri(int64_t n, int32_t off, int32_t* tri) {
+  const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (k < n) tri[k] += off;
 }
 
-// Cluster sums with a per-block LDS table keyed by cluster (256 slots for 256
-// items: every insertion finds a slot), flushed with one FP64 atomic per
-// (cluster, value) per block.
-__global__ __launch_bounds__(kEBlock) void ke_accumulate(EnergyArgs a) {
-  __shared__ int32_t keys[kEBlock];
-  __shared__ double vals[kEBlock * kAcc];
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  keys[threadIdx.x] = -1;
-  for (int k = 0; k < kAcc; ++k) vals[threadIdx.x * kAcc + k] = 0.0;
-  __syncthreads();
-  int64_t c = -1;
-  int m = 0;
-  if (i < a.n_items) {
-    m = mesh_of(a, i);
-    c = cluster_of(a, i, m);
-  }
-  if (c >= 0) {
-    const double w = double(a.w[i]);
-    double v[kAcc];
-    v[0] = w;
-    for (int k = 0; k < 3; ++k) v[1 + k] = w * double(a.xyz[3 * i + k]);
-    for (int k = 0; k < 9; ++k) v[4 + k] = 0.0;
-    if (a.meshes[m].metric == 1) {
-      const EnergyMesh& em = a.meshes[m];
-      for (int32_t k = a.vfptr[i]; k < a.vfptr[i + 1]; ++k) {
-        double p[4], x1[3], u[3], vv[3], q9[9];
-        face_plane(a, em.face_off + a.vfcol[k], p, x1, u, vv);
-        plane_to_q9(p, q9);
-        for (int e = 0; e < 9; ++e) v[4 + e] += q9[e];
-      }
-    }
-    const int32_t key = int32_t(c);
-    uint32_t h = (uint32_t(key) * 2654435761u) >> 24;
-    int slot = -1;
-    for (int probe = 0; probe < kEBlock; ++probe) {
-      const int32_t old = atomicCAS(&keys[h], -1, key);
-      if (old == -1 || old == key) {
-        slot = int(h);
-        break;
-      }
-      h = (h + 1) & (kEBlock - 1);
-    }
-    for (int k = 0; k < kAcc; ++k) atomicAdd(&vals[slot * kAcc + k], v[k]);
-  }
-  __syncthreads();
-  const int32_t key = keys[threadIdx.x];
-  if (key >= 0) {
-    double* dst = a.acc + int64_t(key) * kAcc;
-    for (int k = 0; k < kAcc; ++k) {
-      const double x = vals[threadIdx.x * kAcc + k];
-      if (x != 0.0) atomicAdd(&dst[k], x);
-    }
-  }
+__global__ void ke_vf_count(int64_t n3, const int32_t* __restrict__ tri, int32_t* deg) {
+  const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (k < n3) atomicAdd(&deg[tri[k]], 1);
 }
 
-// Cluster points: centroid c and (QEM) the representative point q.
-__global__ __launch_bounds__(kEBlock) void ke_points(EnergyArgs a) {
-  const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (c >= a.n_clusters) return;
-  const int m = a.clus_mesh ? a.clus_mesh[c] : 0;
-  const EnergyMesh& em = a.meshes[m];
-  const double* s = a.acc + c * kAcc;
-  double* out = a.pts + c * 6;  // c[3], q[3]
-  if (!(s[0] > 0.0)) {
-    for (int k = 0; k < 6; ++k) out[k] = 0.0;
+__global__ void ke_vf_fill(int64_t n3, const int32_t* __restrict__ tri, const int32_t* __restrict__ vfptr,
+                           int32_t* fill, int32_t* vfcol) {
+  const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (k >= n3) return;
+  const int32_t v = tri[k];
+  vfcol[vfptr[v] + atomicAdd(&fill[v], 1)] = int32_t(k / 3);
+}
+
+// Sorts the vertex -> face rows by face id (heap sort: a row of any length in
+// n log n steps), so that a ring does not depend on the order of the atomics.
+__global__ void ke_vf_sort(int64_t n, const int32_t* __restrict__ vfptr, int32_t* vfcol) {
+  const int64_t v = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (v >= n) return;
+  int32_t* r = vfcol + vfptr[v];
+  const int32_t len = vfptr[v + 1] - vfptr[v];
+  if (len <= 32) {
+    for (int32_t i = 1; i < len; ++i) {
+      const int32_t x = r[i];
+      int32_t j = i - 1;
+      for (; j >= 0 && r[j] > x; --j) r[j + 1] = r[j];
+      r[j + 1] = x;
+    }
     return;
   }
-  double cc[3] = {s[1] / s[0], s[2] / s[0], s[3] / s[0]};
-  double q[3] = {cc[0], cc[1], cc[2]};
-  if (em.metric == 1) {
-    const double* Q = s + 4;
+  for (int32_t half = len / 2, end = len; end > 1;) {
+    int32_t x;
+    if (half > 0) {
+      x = r[--half];
+    } else {
+      x = r[--end];
+      r[end] = r[0];
+    }
+    int32_t p = half;
+    for (int32_t c = 2 * p + 1; c < end; c = 2 * p + 1) {
+      if (c + 1 < end && r[c + 1] > r[c]) ++c;
+      if (r[c] <= x) break;
+      r[p] = r[c];
+      p = c;
+    }
+    r[p] = x;
+  }
+}
+
+// Ring of vertex v (at most kRingFaces faces): the links a -> b of its faces
+// (v, a, b) strung into chains.  A chain starts at a link no unused link leads
+// to (a boundary vertex, a bowtie), else at the first unused one (a closed fan).
+// emit(k, entry) is called for every entry; returns their number.
+template <class Emit>
+__device__ int ring_chains(const EnergyArgs& a, int64_t v, Emit&& emit) {
+  const int32_t k0 = a.vfptr[v], d = a.vfptr[v + 1] - k0;
+  int32_t la[kRingFaces], lb[kRingFaces];
+  for (int k = 0; k < d; ++k) {
+    const int64_t f = a.vfcol[k0 + k];
+    int j = 0;
+    while (j < 2 && a.tri[3 * f + j] != int32_t(v)) ++j;
+    la[k] = a.tri[3 * f + (j + 1) % 3];
+    lb[k] = a.tri[3 * f + (j + 2) % 3];
+  }
+  uint32_t left = d == 32 ? ~0u : (1u << d) - 1u;
+  int n = 0;
+  while (left) {
+    int s = -1;
+    for (int k = 0; k < d && s < 0; ++k) {
+      if (!(left >> k & 1u)) continue;
+      bool led = false;
+      for (int t = 0; t < d; ++t) led = led || (t != k && (left >> t & 1u) && lb[t] == la[k]);
+      if (!led) s = k;
+    }
+    if (s < 0) s = __builtin_ctz(left);
+    emit(n++, int32_t(uint32_t(la[s]) | 0x80000000u));
+    while (s >= 0) {
+      left &= ~(1u << s);
+      const int32_t cur = lb[s];
+      emit(n++, cur);
+      s = -1;
+      for (int t = 0; t < d && s < 0; ++t)
+        if ((left >> t & 1u) && la[t] == cur) s = t;
+    }
+  }
+  return n;
+}
+
+// Slots of each group of 64 vertices: the longest ring of its QEM vertices.
+__global__ __launch_bounds__(64) void ke_ring_slots(EnergyArgs a, int32_t* slots) {
+  const int64_t v = int64_t(blockIdx.x) * 64 + threadIdx.x;
+  int n = 0;
+  if (v < a.n_items && a.meshes[mesh_of(a, v)].metric == 1) {
+    if (a.vfptr[v + 1] - a.vfptr[v] > kRingFaces) n = 1;
+    else n = ring_chains(a, v, [](int, int32_t) {});
+  }
+  for (int off = 32; off > 0; off >>= 1) n = max(n, __shfl_xor(n, off));
+  if (threadIdx.x == 0) slots[blockIdx.x] = n;
+}
+
+__global__ __launch_bounds__(64) void ke_ring_fill(EnergyArgs a, const int32_t* __restrict__ slot, int32_t* ring) {
+  const int64_t v = int64_t(blockIdx.x) * 64 + threadIdx.x;
+  const int32_t s0 = slot[blockIdx.x], s1 = slot[blockIdx.x + 1];
+  int32_t* r = ring + int64_t(s0) * 64 + threadIdx.x;
+  int n = 0;
+  if (v < a.n_items && a.meshes[mesh_of(a, v)].metric == 1) {
+    if (a.vfptr[v + 1] - a.vfptr[v] > kRingFaces) {
+      r[0] = kRingLong;
+      n = 1;
+    } else {
+      n = ring_chains(a, v, [&](int k, int32_t e) { r[int64_t(k) * 64] = e; });
+    }
+  }
+  for (; n < s1 - s0; ++n) r[int64_t(n) * 64] = kRingEnd;
+}
+
+// ------------------------------------------------------------------ forward
+// Clears the cluster sums and the energies (one launch; stores of 16 bytes).
+__global__ __launch_bounds__(kEBlock) void ke_zero(int64_t n_acc, double* acc, int64_t n_meshes, double* energy) {
+  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (2 * i + 1 < n_acc) reinterpret_cast<double2*>(acc)[i] = make_double2(0.0, 0.0);
+  else if (2 * i < n_acc) acc[2 * i] = 0.0;
+  if (i < n_meshes) energy[i] = 0.0;
+}
+
+template <int CTRL>
+__device__ inline double dpp_f64(double x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+// One doubling step of the segmented sum over runs of equal keys: lane l adds
+// lane l + D when that lane belongs to its run (rem = lanes left in the run).
+template <int D, int V>
+__device__ inline void merge_step(double (&v)[V], int rem) {
+  const bool take = rem >= D;
+  if (__ballot(take) == 0ull) return;
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    const double t = dpp_f64<0x100 | D>(v[k]);  // row_shl:D
+    v[k] += take ? t : 0.0;
+  }
+}
+
+// Cluster sums.  Block b takes a contiguous range of items, 512 at a time: the
+// lanes of a wave first merge runs of equal clusters in registers (aligned runs
+// of at most 8 lanes), each run then adds once into the block's LDS table keyed
+// by cluster, and the table goes to the global sums when it is three quarters
+// full and at the end, consecutive threads to consecutive words.
+// A table of 256 items (one mesh row's worth) flushed every cluster about 7
+// times, 34 M f64 atomics for 16.8 M QEM vertices and most of the kernel's time;
+// kept over a block's range it flushes each 1 to 2 times.  Now bound by the f64
+// work (580 instructions a step of 64 items, 60 % of the time) and the gathers'
+// latency at 4 waves per SIMD: 16.8 M QEM vertices 2328 -> 372 us (a copy of the
+// bytes takes 168 us), 1 M isotropic ones 45.7 -> 16.7 us.
+template <bool kQem>
+__global__ __launch_bounds__(kAccBlock) void ke_accumulate(EnergyArgs a, int64_t chunk) {
+  constexpr int V = kQem ? 13 : 4;  // W, S[3], Q[9]
+  constexpr int kSlots = kQem ? 512 : 1024;
+  constexpr int kSlotBits = kQem ? 9 : 10;
+  constexpr int kFlushAt = kSlots * 3 / 4;
+  constexpr int kProbes = 32;
+  constexpr int kRun = 8;         // lanes merged at most (16 M QEM vertices: 1 592 us, 2 467, 4 429, 8 432, 16 425)
+  constexpr int kCheckSteps = 4;  // steps between looks at the table's fill (1: 432 us, 4: 407)
+  __shared__ int32_t keys[kSlots];
+  __shared__ double vals[kSlots * V];
+  __shared__ int32_t n_keys;
+  for (int k = threadIdx.x; k < kSlots; k += kAccBlock) keys[k] = -1;
+  for (int k = threadIdx.x; k < kSlots * V; k += kAccBlock) vals[k] = 0.0;
+  if (threadIdx.x == 0) n_keys = 0;
+  __syncthreads();
+  const int64_t begin = int64_t(blockIdx.x) * chunk;
+  const int64_t end = min(begin + chunk, a.n_items);
+  const int lane = threadIdx.x & 63;
+  auto flush = [&]() {  // every thread of the block; the table is complete
+    for (int k = threadIdx.x; k < kSlots * V; k += kAccBlock) {
+      const int32_t key = keys[k / V];
+      const double x = vals[k];
+      vals[k] = 0.0;
+      if (key >= 0 && x != 0.0) atomicAdd(&a.acc[int64_t(key) * a.acc_stride + k % V], x);
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < kSlots; k += kAccBlock) keys[k] = -1;
+    if (threadIdx.x == 0) n_keys = 0;
+    __syncthreads();
+  };
+  const int m0 = mesh_of(a, begin), m1 = mesh_of(a, end - 1);
+  int step = 0;
+  for (int m = m0; m <= m1; ++m) {
+    const EnergyMesh em = a.meshes[m];
+    const int64_t first = max(begin, em.item_off), last = min(end, em.item_off + em.n_items);
+    const bool qem = kQem && em.metric == 1;  // block-uniform
+    // steps stay aligned to the chunk (and so to the ring groups)
+    const int64_t base0 = begin + (first - begin) / kAccBlock * kAccBlock;
+    int32_t e[kRingChunk];
+    int32_t slots = 0, lab = -1;
+    // the ring entries and labels of a step are read during the step before it
+    if (qem && base0 < last) slots = load_ring(a, base0 + threadIdx.x, e);
+    if (base0 + int64_t(threadIdx.x) >= first && base0 + int64_t(threadIdx.x) < last) lab = a.labels[base0 + threadIdx.x];
+    for (int64_t base = base0; base < last; base += kAccBlock) {
+      const int64_t i = base + threadIdx.x;
+      const bool active = i >= first && i < last;
+      const int32_t c = active ? cluster_of(em, lab) : -1;
+      double v[V];
+#pragma unroll
+      for (int k = 0; k < V; ++k) v[k] = 0.0;
+      Vec3 x{0.0, 0.0, 0.0};
+      RingPoint q[kRingChunk];
+      const int32_t e0 = e[0], cur_slots = slots;
+      uint32_t faces = 0;  // entries that close a face
+      if (qem && c >= 0) {
+#pragma unroll
+        for (int k = 0; k < kRingChunk; ++k) {
+          const int64_t j = (e[k] == kRingEnd || e0 == kRingLong) ? i : int64_t(e[k] & kRingId);
+          q[k] = RingPoint{a.xyz[3 * j], a.xyz[3 * j + 1], a.xyz[3 * j + 2]};
+          if (e[k] >= 0) faces |= 1u << k;
+        }
+      }
+      const bool more = qem && c >= 0 && (e0 == kRingLong || (cur_slots > kRingChunk && e[kRingChunk - 1] != kRingEnd));
+      if (c >= 0) {
+        const double w = double(a.w[i]);
+        x = load_point(a.xyz, i);
+        v[0] = w;
+        v[1] = w * x.x;
+        v[2] = w * x.y;
+        v[3] = w * x.z;
+      }
+      if (base + kAccBlock < last) {
+        if (qem) slots = load_ring(a, i + kAccBlock, e);
+        lab = i + kAccBlock < last ? a.labels[i + kAccBlock] : -1;
+      }
+      if constexpr (kQem) {
+        if (qem && c >= 0) {
+          auto add = [&](const Vec3& n) {
+            v[4] = __builtin_fma(n.x, n.x, v[4]);
+            v[5] = __builtin_fma(n.x, n.y, v[5]);
+            v[6] = __builtin_fma(n.x, n.z, v[6]);
+            v[8] = __builtin_fma(n.y, n.y, v[8]);
+            v[9] = __builtin_fma(n.y, n.z, v[9]);
+            v[11] = __builtin_fma(n.z, n.z, v[11]);
+          };
+          Vec3 u{0.0, 0.0, 0.0};
+#pragma unroll
+          for (int k = 0; k < kRingChunk; ++k) {
+            const Vec3 t = sub(Vec3{double(q[k].x), double(q[k].y), double(q[k].z)}, x);
+            if (faces >> k & 1u) add(cross(u, t));
+            u = t;
+          }
+          if (more)
+            walk_rest(
+                a, i, x, e0, kRingChunk, u, 0, [](int32_t) { return 0; },
+                [&](const Vec3& r, int32_t, const Vec3& t, int32_t) { add(cross(r, t)); });
+          // every plane passes through the vertex (d = -n . x): sum n d = -(sum n n^T) x
+          v[7] = -(v[4] * x.x + v[5] * x.y + v[6] * x.z);
+          v[10] = -(v[5] * x.x + v[8] * x.y + v[9] * x.z);
+          v[12] = -(v[6] * x.x + v[9] * x.y + v[11] * x.z);
+        }
+      }
+      // runs of equal clusters
+      const int32_t prev = __builtin_amdgcn_update_dpp(-2, c, 0x111, 0xf, 0xf, false);  // row_shr:1
+      const bool head = prev != c || (lane & (kRun - 1)) == 0;
+      const unsigned long long heads = __ballot(head);
+      const unsigned long long after = lane == 63 ? 0ull : heads >> (lane + 1);
+      const int rem = after ? __builtin_ctzll(after) : 63 - lane;
+      static_assert(kRun == 8, "three doubling steps");
+      merge_step<1>(v, rem);
+      merge_step<2>(v, rem);
+      merge_step<4>(v, rem);
+      if (head && c >= 0) {
+        uint32_t h = (uint32_t(c) * 2654435761u) >> (32 - kSlotBits);
+        int slot = -1;
+        for (int probe = 0; probe < kProbes; ++probe) {
+          const int32_t old = atomicCAS(&keys[h], -1, c);
+          if (old == -1) atomicAdd(&n_keys, 1);
+          if (old == -1 || old == c) {
+            slot = int(h);
+            break;
+          }
+          h = (h + 1) & (kSlots - 1);
+        }
+        if (slot >= 0) {
+#pragma unroll
+          for (int k = 0; k < V; ++k) atomicAdd(&vals[slot * V + k], v[k]);
+        } else {  // no free slot near by: straight to the global sums
+#pragma unroll
+          for (int k = 0; k < V; ++k)
+            if (v[k] != 0.0) atomicAdd(&a.acc[int64_t(c) * a.acc_stride + k], v[k]);
+        }
+      }
+      if (++step % kCheckSteps == 0) {  // block-uniform
+        __syncthreads();
+        const bool full = n_keys > kFlushAt;
+        __syncthreads();
+        if (full) flush();
+      }
+    }
+  }
+  __syncthreads();
+  flush();
+}
+
+// Cluster points: q, and for QEM meshes the unit adjoint (adj: dE/dQ at 0..8,
+// (dE/dc) / W at 9..11, the centroid at 12..14).
+__global__ __launch_bounds__(64) void ke_points(EnergyArgs a) {
+  const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (c >= a.n_clusters) return;
+  const EnergyMesh& em = a.meshes[a.clus_mesh ? a.clus_mesh[c] : 0];
+  const double* s = a.acc + c * a.acc_stride;
+  const double W = s[0];
+  double cc[3] = {0.0, 0.0, 0.0}, q[3] = {0.0, 0.0, 0.0};
+  double adj[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  const bool some = W > 0.0;
+  if (some)
+    for (int k = 0; k < 3; ++k) q[k] = cc[k] = s[1 + k] / W;
+  if (some && em.metric == 1) {
+    double Q[9];
+    for (int k = 0; k < 9; ++k) Q[k] = s[4 + k];
     const double A[6] = {Q[0], Q[1], Q[2], Q[4], Q[5], Q[7]};
     double lam[3], V[9];
     bool keep[3];
@@ -234,193 +527,337 @@ __global__ __launch_bounds__(kEBlock) void ke_points(EnergyArgs a) {
     const double r[3] = {-Q[3] - (Q[0] * cc[0] + Q[1] * cc[1] + Q[2] * cc[2]),
                          -Q[6] - (Q[1] * cc[0] + Q[4] * cc[1] + Q[5] * cc[2]),
                          -Q[8] - (Q[2] * cc[0] + Q[5] * cc[1] + Q[7] * cc[2])};
+    double vr[3];
     for (int k = 0; k < 3; ++k) {
-      if (!keep[k]) continue;
       const double vk[3] = {V[k], V[3 + k], V[6 + k]};
-      const double f = dot3(vk, r) / lam[k];
+      vr[k] = dot3(vk, r);
+      if (!keep[k]) continue;
+      const double f = vr[k] / lam[k];
       for (int e = 0; e < 3; ++e) q[e] += f * vk[e];
     }
+    // dE/dq = -2 (S - W q)
+    const double gq[3] = {-2.0 * (s[1] - W * q[0]), -2.0 * (s[2] - W * q[1]), -2.0 * (s[3] - W * q[2])};
+    double vg[3];
+    // y = A+ r = q - c; h = A+ gq; P gq = gq - sum_kept v_k (v_k . gq)
+    double h[3] = {0, 0, 0}, pg[3] = {gq[0], gq[1], gq[2]};
+    for (int k = 0; k < 3; ++k) {
+      const double vk[3] = {V[k], V[3 + k], V[6 + k]};
+      vg[k] = dot3(vk, gq);
+      if (!keep[k]) continue;
+      for (int e = 0; e < 3; ++e) {
+        h[e] += V[3 * e + k] * vg[k] / lam[k];
+        pg[e] -= V[3 * e + k] * vg[k];
+      }
+    }
+    // G = -h (y + c)^T + sum_{k kept, j dropped} coef_kj v_j v_k^T, y + c = q
+    double G[3][3];
+    for (int r0 = 0; r0 < 3; ++r0)
+      for (int c0 = 0; c0 < 3; ++c0) G[r0][c0] = -h[r0] * q[c0];
+    for (int k = 0; k < 3; ++k) {
+      if (!keep[k]) continue;
+      for (int j = 0; j < 3; ++j) {
+        if (keep[j]) continue;
+        const double gap = lam[k] - lam[j];
+        if (gap == 0.0) continue;
+        const double coef = (vg[j] * vr[k] + vg[k] * vr[j]) / (lam[k] * gap);
+        for (int r0 = 0; r0 < 3; ++r0)
+          for (int c0 = 0; c0 < 3; ++c0) G[r0][c0] += coef * V[3 * r0 + j] * V[3 * c0 + k];
+      }
+    }
+    // dE/dA as the symmetric matrix B with dE = n^T B dn for a plane normal n
+    // (00, 01, 02, 11, 12, 22), then dE/d(n d) = -A+ gq
+    adj[0] = 2.0 * G[0][0];
+    adj[1] = G[0][1] + G[1][0];
+    adj[2] = G[0][2] + G[2][0];
+    adj[3] = 2.0 * G[1][1];
+    adj[4] = G[1][2] + G[2][1];
+    adj[5] = 2.0 * G[2][2];
+    for (int e = 0; e < 3; ++e) adj[6 + e] = -h[e];
+    for (int e = 0; e < 3; ++e) adj[9 + e] = pg[e] / W;
   }
-  for (int k = 0; k < 3; ++k) {
-    out[k] = cc[k];
-    out[3 + k] = q[k];
+  double* out = a.pts + 4 * c;
+  for (int k = 0; k < 3; ++k) out[k] = q[k];
+  if (a.adj) {
+    double* o = a.adj + kAdjStride * c;
+    for (int k = 0; k < 12; ++k) o[k] = adj[k];
+    for (int k = 0; k < 3; ++k) o[12 + k] = cc[k];
   }
 }
 
-// Per-mesh energy: block sum when the block lies in one mesh, else per item.
-__global__ __launch_bounds__(kEBlock) void ke_energy(EnergyArgs a, double* energy) {
-  __shared__ double red[kEBlock];
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  double e = 0.0;
-  int m = 0;
-  if (i < a.n_items) {
-    m = mesh_of(a, i);
-    const int64_t c = cluster_of(a, i, m);
-    if (c >= 0) {
-      const double* q = a.pts + c * 6 + 3;
-      double d2 = 0.0;
-      for (int k = 0; k < 3; ++k) {
-        const double d = double(a.xyz[3 * i + k]) - q[k];
-        d2 += d * d;
+// Per-mesh energy.  Few blocks, each over a contiguous range of items, add
+// their sums to the mesh's energy: one atomic per block and mesh (atomics on one
+// address take 12.7 ns each; with one per 256 items they were this kernel's
+// time: 1 M vertices 52 -> 8 us, 16 x 1 M 694 -> 92 us, 3.6 TB/s).
+__global__ __launch_bounds__(kAccBlock) void ke_energy(EnergyArgs a, int64_t chunk, double* energy) {
+  __shared__ double red[kAccBlock / 64];
+  const int64_t begin = int64_t(blockIdx.x) * chunk;
+  const int64_t end = min(begin + chunk, a.n_items);
+  const int m0 = mesh_of(a, begin), m1 = mesh_of(a, end - 1);
+  for (int m = m0; m <= m1; ++m) {
+    const EnergyMesh em = a.meshes[m];
+    const int64_t first = max(begin, em.item_off), last = min(end, em.item_off + em.n_items);
+    double e = 0.0;
+#pragma unroll 4
+    for (int64_t i = first + threadIdx.x; i < last; i += kAccBlock) {
+      const int32_t c = cluster_of(em, a.labels[i]);
+      const Vec3 x = load_point(a.xyz, i);
+      const double w = double(a.w[i]);
+      if (c >= 0) {
+        const double* q = a.pts + 4 * int64_t(c);
+        const double dx = x.x - q[0], dy = x.y - q[1], dz = x.z - q[2];
+        e += w * (dx * dx + dy * dy + dz * dz);
       }
-      e = double(a.w[i]) * d2;
+    }
+    for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off);
+    __syncthreads();  // red of the previous mesh has been read
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = e;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int k = 1; k < kAccBlock / 64; ++k) e += red[k];
+      atomicAdd(&energy[m], e);
     }
   }
-  const int64_t first = int64_t(blockIdx.x) * blockDim.x;
-  const int64_t last = min(first + kEBlock, a.n_items) - 1;
-  const bool one_mesh = mesh_of(a, first) == mesh_of(a, last);
-  if (!one_mesh) {
-    if (e != 0.0) atomicAdd(&energy[m], e);
-    return;
-  }
-  red[threadIdx.x] = e;
-  __syncthreads();
-  for (int s = kEBlock / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) atomicAdd(&energy[mesh_of(a, first)], red[0]);
 }
 
 // ----------------------------------------------------------------- backward
-// Per cluster: adj[0..8] = dE/dQ (entries 0..8), adj[9..11] = (dE/dc) / W.
-__global__ __launch_bounds__(kEBlock) void ke_cluster_adjoint(EnergyArgs a, const double* __restrict__ gE) {
-  const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (c >= a.n_clusters) return;
-  const int m = a.clus_mesh ? a.clus_mesh[c] : 0;
-  const EnergyMesh& em = a.meshes[m];
-  double* adj = a.adj + c * 12;
-  for (int k = 0; k < 12; ++k) adj[k] = 0.0;
-  const double* s = a.acc + c * kAcc;
-  if (em.metric != 1 || !(s[0] > 0.0)) return;  // isotropic: dE/dc = 0 at the centroid
-  const double g = gE[m];
-  const double W = s[0];
-  const double* cc = a.pts + c * 6;
-  const double* q = cc + 3;
-  // dE/dq = -2 g (S - W q)
-  const double gq[3] = {-2.0 * g * (s[1] - W * q[0]), -2.0 * g * (s[2] - W * q[1]), -2.0 * g * (s[3] - W * q[2])};
-  const double* Q = s + 4;
-  const double A[6] = {Q[0], Q[1], Q[2], Q[4], Q[5], Q[7]};
-  double lam[3], V[9];
-  bool keep[3];
-  eig_sym3(A, lam, V);
-  kept_set(lam, em.level, keep);
-  const double r[3] = {-Q[3] - (Q[0] * cc[0] + Q[1] * cc[1] + Q[2] * cc[2]),
-                       -Q[6] - (Q[1] * cc[0] + Q[4] * cc[1] + Q[5] * cc[2]),
-                       -Q[8] - (Q[2] * cc[0] + Q[5] * cc[1] + Q[7] * cc[2])};
-  double vg[3], vr[3];
-  for (int k = 0; k < 3; ++k) {
-    const double vk[3] = {V[k], V[3 + k], V[6 + k]};
-    vg[k] = dot3(vk, gq);
-    vr[k] = dot3(vk, r);
-  }
-  // y = A+ r = q - c; h = A+ gq; P gq = gq - sum_kept v_k (v_k . gq)
-  double h[3] = {0, 0, 0}, pg[3] = {gq[0], gq[1], gq[2]};
-  for (int k = 0; k < 3; ++k) {
-    if (!keep[k]) continue;
-    for (int e = 0; e < 3; ++e) {
-      h[e] += V[3 * e + k] * vg[k] / lam[k];
-      pg[e] -= V[3 * e + k] * vg[k];
-    }
-  }
-  // G = -h (y + c)^T + sum_{k kept, j dropped} coef_kj v_j v_k^T
-  const double yc[3] = {q[0], q[1], q[2]};  // y + c = q
-  double G[3][3];
-  for (int r0 = 0; r0 < 3; ++r0)
-    for (int c0 = 0; c0 < 3; ++c0) G[r0][c0] = -h[r0] * yc[c0];
-  for (int k = 0; k < 3; ++k) {
-    if (!keep[k]) continue;
-    for (int j = 0; j < 3; ++j) {
-      if (keep[j]) continue;
-      const double gap = lam[k] - lam[j];
-      if (gap == 0.0) continue;
-      const double coef = (vg[j] * vr[k] + vg[k] * vr[j]) / (lam[k] * gap);
-      for (int r0 = 0; r0 < 3; ++r0)
-        for (int c0 = 0; c0 < 3; ++c0) G[r0][c0] += coef * V[3 * r0 + j] * V[3 * c0 + k];
-    }
-  }
-  // symmetric part onto the quadric entries; b = -(Q3, Q6, Q8) gets A+ gq
-  adj[0] = G[0][0];
-  adj[1] = G[0][1] + G[1][0];
-  adj[2] = G[0][2] + G[2][0];
-  adj[4] = G[1][1];
-  adj[5] = G[1][2] + G[2][1];
-  adj[7] = G[2][2];
-  adj[3] = -h[0];
-  adj[6] = -h[1];
-  adj[8] = -h[2];
-  for (int e = 0; e < 3; ++e) adj[9 + e] = pg[e] / W;
+// Adjoint of one cluster's quadric as the planes through a vertex x see it.  With
+// d = -n . x, dE = n^T B dn + g . d(n d) pulls back to dE/dn = M n with
+// M = B - g x^T - x g^T, and x receives -(g . n) n: both depend on the vertex,
+// not on the face.
+struct PlaneAdjoint {
+  double m[6];  // M: 00, 01, 02, 11, 12, 22
+  double g[3];
+};
+
+__device__ inline PlaneAdjoint plane_adjoint(const double* __restrict__ adj, const Vec3& x) {
+  PlaneAdjoint r;
+  for (int k = 0; k < 3; ++k) r.g[k] = adj[6 + k];
+  r.m[0] = adj[0] - 2.0 * (r.g[0] * x.x);
+  r.m[1] = adj[1] - (r.g[0] * x.y + r.g[1] * x.x);
+  r.m[2] = adj[2] - (r.g[0] * x.z + r.g[2] * x.x);
+  r.m[3] = adj[3] - 2.0 * (r.g[1] * x.y);
+  r.m[4] = adj[4] - (r.g[1] * x.z + r.g[2] * x.y);
+  r.m[5] = adj[5] - 2.0 * (r.g[2] * x.z);
+  return r;
 }
 
-// Per vertex: dE/dx (3) and dE/dw.
-__global__ __launch_bounds__(kEBlock) void ke_item_grad(EnergyArgs a, const double* __restrict__ gE, float* dxyz,
-                                                        float* dw) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= a.n_items) return;
-  const int m = mesh_of(a, i);
-  const EnergyMesh& em = a.meshes[m];
-  const double g = gE[m];
-  double gx[3] = {0, 0, 0}, gw = 0.0;
-  const double x[3] = {double(a.xyz[3 * i]), double(a.xyz[3 * i + 1]), double(a.xyz[3 * i + 2])};
-  const int64_t c = cluster_of(a, i, m);
-  if (c >= 0) {
-    const double w = double(a.w[i]);
-    const double* cc = a.pts + c * 6;
-    const double* q = cc + 3;
-    const double* adj = a.adj + c * 12;
-    double d2 = 0.0;
-    for (int k = 0; k < 3; ++k) {
-      const double d = x[k] - q[k];
-      gx[k] = 2.0 * g * w * d + w * adj[9 + k];
-      d2 += d * d;
-    }
-    gw = g * d2 + adj[9] * (x[0] - cc[0]) + adj[10] * (x[1] - cc[1]) + adj[11] * (x[2] - cc[2]);
-  }
-  if (em.metric == 1) {
-    // faces around i: their quadrics feed the clusters of their three vertices
-    for (int32_t k = a.vfptr[i]; k < a.vfptr[i + 1]; ++k) {
-      const int64_t f = em.face_off + a.vfcol[k];
-      double gq9[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-      int role = 0;
-      for (int j = 0; j < 3; ++j) {
-        const int32_t vj = a.tri[3 * f + j];
-        if (vj == i) role = j;
-        const int64_t cj = cluster_of(a, vj, m);
-        if (cj < 0) continue;
-        const double* aj = a.adj + cj * 12;
-        for (int e = 0; e < 9; ++e) gq9[e] += aj[e];
+__device__ inline PlaneAdjoint no_adjoint() {
+  PlaneAdjoint r;
+  for (int k = 0; k < 6; ++k) r.m[k] = 0.0;
+  for (int k = 0; k < 3; ++k) r.g[k] = 0.0;
+  return r;
+}
+
+// Per vertex: dE/dx (3) and dE/dw.  QEM: the faces around the vertex v, each as
+// (v, v + u, v + s), feed the clusters of their three vertices.  The adjoints of
+// the vertex's cluster and of the first two others its ring meets are read
+// before the faces are visited (a third one, rare, in a second walk): read face
+// by face, behind the labels, they were most of this kernel's waits.  Consecutive
+// blocks run on one XCD, whose L2 then holds the rows a block shares with its
+// neighbours (HBM reads 1.27 -> 0.87 GB).  Bound by the f64 work (950
+// instructions per 64 vertices, half of the time) and by gather latency at 3
+// waves per SIMD (158 registers; held to 128 the spills cost more: 1359 us;
+// a loop over the faces that keeps one position in flight: 831 us).
+// 16.8 M QEM vertices 2050 -> 765 us, 1 M isotropic ones 10.5 -> 8.6 us.
+template <bool kQem>
+__global__ __launch_bounds__(kEBlock) void ke_item_grad(EnergyArgs a, const double* __restrict__ gE,
+                                                        float* __restrict__ dxyz, float* __restrict__ dw) {
+  constexpr int kXcd = 8;
+  const int64_t nb = gridDim.x, xcd = blockIdx.x % kXcd;
+  const int64_t block = xcd * (nb / kXcd) + min(xcd, nb % kXcd) + blockIdx.x / kXcd;
+  const int64_t begin = block * kEBlock;
+  const int64_t end = min(begin + kEBlock, a.n_items);
+  const int64_t i = begin + threadIdx.x;
+  // what does not depend on the mesh is read with the mesh's number
+  const int64_t ic = min(i, a.n_items - 1);
+  const int32_t lab = a.labels[ic];
+  const float wf = a.w[ic];
+  const Vec3 x = load_point(a.xyz, ic);
+  int32_t e[kRingChunk];
+  int32_t slots = 0;
+  if constexpr (kQem) slots = load_ring(a, i, e);
+  const int m0 = mesh_of(a, begin), m1 = mesh_of(a, end - 1);
+  for (int m = m0; m <= m1; ++m) {
+    const EnergyMesh em = a.meshes[m];
+    const bool active = i < end && i >= em.item_off && i < em.item_off + em.n_items;
+    const double g = gE[m];
+    double gx[3] = {0, 0, 0}, gw = 0.0;
+    const int32_t c = active ? cluster_of(em, lab) : -1;
+    const bool qem = kQem && em.metric == 1;  // block-uniform
+    if (c >= 0) {
+      const double w = double(wf);
+      const double* q = a.pts + 4 * int64_t(c);
+      const double d[3] = {x.x - q[0], x.y - q[1], x.z - q[2]};
+      for (int k = 0; k < 3; ++k) gx[k] = 2.0 * w * d[k];
+      gw = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+      if (qem) {
+        const double* adj = a.adj + kAdjStride * int64_t(c);
+        for (int k = 0; k < 3; ++k) gx[k] += w * adj[9 + k];
+        gw += adj[9] * (x.x - adj[12]) + adj[10] * (x.y - adj[13]) + adj[11] * (x.z - adj[14]);
       }
-      double p[4], x1[3], u[3], v[3];
-      face_plane(a, f, p, x1, u, v);
-      const double dp[4] = {2.0 * gq9[0] * p[0] + gq9[1] * p[1] + gq9[2] * p[2] + gq9[3] * p[3],
-                            gq9[1] * p[0] + 2.0 * gq9[4] * p[1] + gq9[5] * p[2] + gq9[6] * p[3],
-                            gq9[2] * p[0] + gq9[5] * p[1] + 2.0 * gq9[7] * p[2] + gq9[8] * p[3],
-                            gq9[3] * p[0] + gq9[6] * p[1] + gq9[8] * p[2]};
-      // d = -n.x1: n receives -dp3 x1, x1 receives -dp3 n
-      const double gn[3] = {dp[0] - dp[3] * x1[0], dp[1] - dp[3] * x1[1], dp[2] - dp[3] * x1[2]};
-      // n = u x v: gu = v x gn, gv = gn x u
-      const double gu[3] = {v[1] * gn[2] - v[2] * gn[1], v[2] * gn[0] - v[0] * gn[2], v[0] * gn[1] - v[1] * gn[0]};
-      const double gv[3] = {gn[1] * u[2] - gn[2] * u[1], gn[2] * u[0] - gn[0] * u[2], gn[0] * u[1] - gn[1] * u[0]};
-      for (int e = 0; e < 3; ++e) {
-        if (role == 0) gx[e] += -gu[e] - gv[e] - dp[3] * p[e];
-        else if (role == 1) gx[e] += gu[e];
-        else gx[e] += gv[e];
+    }
+    if (qem && active) {
+      // clusters of the ring: code 0 the vertex's own, 1 and 2 the first two
+      // others, 3 none or a further one (more = true)
+      int32_t c1 = -1, c2 = -1;
+      uint32_t code = 0;
+      const bool is_long = e[0] == kRingLong;
+      bool more = is_long || (slots > kRingChunk && e[kRingChunk - 1] != kRingEnd);
+      {
+        int32_t l[kRingChunk];
+#pragma unroll
+        for (int k = 0; k < kRingChunk; ++k) {
+          if (k >= slots) break;  // wave-uniform
+          if (e[k] == kRingEnd || is_long) e[k] = int32_t(uint32_t(i) | 0x80000000u);  // no face
+          l[k] = a.labels[e[k] & kRingId];
+        }
+#pragma unroll
+        for (int k = 0; k < kRingChunk; ++k) {
+          if (k >= slots) break;
+          const int32_t cj = cluster_of(em, l[k]);
+          uint32_t t = 3;
+          if (cj == c) t = c >= 0 ? 0 : 3;
+          else if (cj >= 0) {
+            if (c1 < 0) c1 = cj;
+            if (cj == c1) t = 1;
+            else {
+              if (c2 < 0) c2 = cj;
+              if (cj == c2) t = 2;
+              else more = true;
+            }
+          }
+          code |= t << (2 * k);
+        }
+      }
+      const PlaneAdjoint A0 = c >= 0 ? plane_adjoint(a.adj + kAdjStride * int64_t(c), x) : no_adjoint();
+      const PlaneAdjoint A1 = c1 >= 0 ? plane_adjoint(a.adj + kAdjStride * int64_t(c1), x) : no_adjoint();
+      const PlaneAdjoint A2 = c2 >= 0 ? plane_adjoint(a.adj + kAdjStride * int64_t(c2), x) : no_adjoint();
+      // the face (v, v + u, v + s) with adjoint F: n = u x s; u receives s x dn,
+      // s receives dn x u, and v minus both (dn x (u - s)) and minus (g . n) n
+      auto pull = [&](const PlaneAdjoint& F, const Vec3& u, const Vec3& s) {
+        const Vec3 n = cross(u, s), t = sub(u, s);
+        const double n0 = __builtin_fma(F.m[2], n.z, __builtin_fma(F.m[1], n.y, F.m[0] * n.x));
+        const double n1 = __builtin_fma(F.m[4], n.z, __builtin_fma(F.m[3], n.y, F.m[1] * n.x));
+        const double n2 = __builtin_fma(F.m[5], n.z, __builtin_fma(F.m[4], n.y, F.m[2] * n.x));
+        const double gn = __builtin_fma(F.g[2], n.z, __builtin_fma(F.g[1], n.y, F.g[0] * n.x));
+        gx[0] -= __builtin_fma(gn, n.x, __builtin_fma(n1, t.z, -(n2 * t.y)));
+        gx[1] -= __builtin_fma(gn, n.y, __builtin_fma(n2, t.x, -(n0 * t.z)));
+        gx[2] -= __builtin_fma(gn, n.z, __builtin_fma(n0, t.y, -(n1 * t.x)));
+      };
+      Vec3 u{0.0, 0.0, 0.0};
+      const double own = c >= 0 ? 1.0 : 0.0;
+#pragma unroll
+      for (int k = 0; k < kRingChunk; ++k) {
+        if (k >= slots) break;
+        const Vec3 s = sub(ring_point(a, e[k]), x);
+        if (k > 0 && e[k] >= 0) {
+          const uint32_t tu = code >> (2 * (k - 1)) & 3u, ts = code >> (2 * k) & 3u;
+          const double w0 = own + (tu == 0 ? 1.0 : 0.0) + (ts == 0 ? 1.0 : 0.0);
+          const double w1 = (tu == 1 ? 1.0 : 0.0) + (ts == 1 ? 1.0 : 0.0);
+          const double w2 = (tu == 2 ? 1.0 : 0.0) + (ts == 2 ? 1.0 : 0.0);
+          PlaneAdjoint F;
+          for (int j = 0; j < 6; ++j) F.m[j] = __builtin_fma(w2, A2.m[j], __builtin_fma(w1, A1.m[j], w0 * A0.m[j]));
+          for (int j = 0; j < 3; ++j) F.g[j] = __builtin_fma(w2, A2.g[j], __builtin_fma(w1, A1.g[j], w0 * A0.g[j]));
+          pull(F, u, s);
+        }
+        u = s;
+      }
+      if (more) {
+        // faces past the first entries in full; of the others the part of the
+        // clusters the codes leave out
+        auto tag = [&](int32_t j) { return cluster_of(em, a.labels[j]); };
+        auto pull_of = [&](int32_t cj, const Vec3& r, const Vec3& s) {
+          if (cj >= 0) pull(plane_adjoint(a.adj + kAdjStride * int64_t(cj), x), r, s);
+        };
+        int32_t cu = -1;
+        u = Vec3{0.0, 0.0, 0.0};
+        if (!is_long)
+          for (int k = 0; k < kRingChunk; ++k) {
+            const int32_t ek = k < slots ? a.ring[int64_t(a.ring_slot[i >> 6] + k) * 64 + (i & 63)] : kRingEnd;
+            if (ek == kRingEnd) break;
+            const Vec3 s = sub(ring_point(a, ek), x);
+            const int32_t cs = tag(ek & kRingId);
+            if (ek >= 0) {
+              if (cu != c && cu != c1 && cu != c2) pull_of(cu, u, s);
+              if (cs != c && cs != c1 && cs != c2) pull_of(cs, u, s);
+            }
+            u = s;
+            cu = cs;
+          }
+        walk_rest(a, i, x, is_long ? kRingLong : 0, kRingChunk, u, cu, tag,
+                  [&](const Vec3& r, int32_t cr, const Vec3& s, int32_t cs) {
+                    pull_of(c, r, s);
+                    pull_of(cr, r, s);
+                    pull_of(cs, r, s);
+                  });
       }
     }
+    if (active) {
+      for (int k = 0; k < 3; ++k) dxyz[3 * i + k] = float(g * gx[k]);
+      dw[i] = float(g * gw);
+    }
   }
-  for (int k = 0; k < 3; ++k) dxyz[3 * i + k] = float(gx[k]);
-  dw[i] = float(gw);
 }
 
 }  // namespace
 
+// Items per block of ke_accumulate and ke_energy: a multiple of the block, at
+// least 4,096 where that still leaves a block per CU, so that a block's table
+// sees several mesh rows; at most `max_blocks` blocks.
+static int64_t item_chunk(int64_t n, int64_t max_blocks) {
+  int64_t blocks = (n + kAccBlock - 1) / kAccBlock;
+  blocks = std::min(blocks, std::max<int64_t>(256, std::min(max_blocks, n / 4096)));
+  const int64_t per = (n + blocks - 1) / blocks;
+  return (per + kAccBlock - 1) / kAccBlock * kAccBlock;
+}
+
 hipError_t energy_forward(hipStream_t s, const EnergyArgs& a, double* energy, int n_meshes) {
-  const int64_t nacc = a.n_clusters * kAcc;
-  hipLaunchKernelGGL(ke_zero, dim3(egrid(nacc)), dim3(kEBlock), 0, s, nacc, a.acc);
-  hipLaunchKernelGGL(ke_zero, dim3(egrid(n_meshes)), dim3(kEBlock), 0, s, int64_t(n_meshes), energy);
-  if (a.n_items > 0) hipLaunchKernelGGL(ke_accumulate, dim3(egrid(a.n_items)), dim3(kEBlock), 0, s, a);
-  if (a.n_clusters > 0) hipLaunchKernelGGL(ke_points, dim3(egrid(a.n_clusters)), dim3(kEBlock), 0, s, a);
-  if (a.n_items > 0) hipLaunchKernelGGL(ke_energy, dim3(egrid(a.n_items)), dim3(kEBlock), 0, s, a, energy);
+  const int64_t nacc = a.n_clusters * a.acc_stride;
+  hipLaunchKernelGGL(ke_zero, dim3(egrid(std::max<int64_t>((nacc + 1) / 2, n_meshes))), dim3(kEBlock), 0, s, nacc,
+                     a.acc, int64_t(n_meshes), energy);
+  if (a.n_items > 0) {
+    const int64_t chunk = item_chunk(a.n_items, kAccMaxBlocks);
+    const dim3 grid(unsigned((a.n_items + chunk - 1) / chunk));
+    if (a.adj) hipLaunchKernelGGL(ke_accumulate<true>, grid, dim3(kAccBlock), 0, s, a, chunk);
+    else hipLaunchKernelGGL(ke_accumulate<false>, grid, dim3(kAccBlock), 0, s, a, chunk);
+  }
+  if (a.n_clusters > 0)
+    hipLaunchKernelGGL(ke_points, dim3(unsigned((a.n_clusters + 63) / 64)), dim3(64), 0, s, a);
+  if (a.n_items > 0) {
+    const int64_t chunk = item_chunk(a.n_items, 512);
+    hipLaunchKernelGGL(ke_energy, dim3(unsigned((a.n_items + chunk - 1) / chunk)), dim3(kAccBlock), 0, s, a, chunk,
+                       energy);
+  }
+  return hipGetLastError();
+}
+
+hipError_t energy_offset_tri(hipStream_t s, int64_t n3, int32_t off, int32_t* tri) {
+  if (n3 == 0 || off == 0) return hipSuccess;
+  hipLaunchKernelGGL(ke_offset_tri, dim3(egrid(n3)), dim3(kEBlock), 0, s, n3, off, tri);
+  return hipGetLastError();
+}
+
+hipError_t energy_vf_count(hipStream_t s, int64_t n3, const int32_t* tri, int32_t* deg) {
+  if (n3 == 0) return hipSuccess;
+  hipLaunchKernelGGL(ke_vf_count, dim3(egrid(n3)), dim3(kEBlock), 0, s, n3, tri, deg);
+  return hipGetLastError();
+}
+
+hipError_t energy_vf_fill(hipStream_t s, int64_t n, int64_t n3, const int32_t* tri, const int32_t* vfptr,
+                          int32_t* fill, int32_t* vfcol) {
+  if (n3 == 0) return hipSuccess;
+  hipLaunchKernelGGL(ke_vf_fill, dim3(egrid(n3)), dim3(kEBlock), 0, s, n3, tri, vfptr, fill, vfcol);
+  hipLaunchKernelGGL(ke_vf_sort, dim3(egrid(n)), dim3(kEBlock), 0, s, n, vfptr, vfcol);
+  return hipGetLastError();
+}
+
+hipError_t energy_ring_slots(hipStream_t s, const EnergyArgs& a, int32_t* slots) {
+  hipLaunchKernelGGL(ke_ring_slots, dim3(unsigned((a.n_items + 63) / 64)), dim3(64), 0, s, a, slots);
+  return hipGetLastError();
+}
+
+hipError_t energy_ring_fill(hipStream_t s, const EnergyArgs& a, const int32_t* slot, int32_t* ring) {
+  hipLaunchKernelGGL(ke_ring_fill, dim3(unsigned((a.n_items + 63) / 64)), dim3(64), 0, s, a, slot, ring);
   return hipGetLastError();
 }
 
@@ -428,14 +865,14 @@ hipError_t energy_forward(hipStream_t s, const EnergyArgs& a, double* energy, in
 namespace {
 
 // Scratch of energy_forward_cvt_noalloc: the mesh descriptor, then the
-// per-cluster sums (kAcc doubles) and points (6 doubles) of at most
+// per-cluster sums (4 doubles) and points (4 doubles) of at most
 // kNoAllocMaxClusters clusters; one copy per device, held until the process
 // ends.  Host code never passes `scratch` itself to a kernel (in host code the
 // name is only a stand-in): it uses the device address found once per device
 // by hipGetSymbolAddress.
 constexpr size_t kNoAllocMeshBytes = 256;
 constexpr size_t kNoAllocBytes =
-    kNoAllocMeshBytes + size_t(kNoAllocMaxClusters) * size_t(kAcc + 6) * sizeof(double);
+    kNoAllocMeshBytes + size_t(kNoAllocMaxClusters) * size_t(4 + 4) * sizeof(double);
 static_assert(sizeof(EnergyMesh) <= kNoAllocMeshBytes, "mesh descriptor slot");
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
@@ -479,17 +916,18 @@ hipError_t energy_forward_cvt_noalloc(hipStream_t s, int64_t n, int32_t K, const
   a.w = w;
   a.labels = labels;
   a.acc = acc;
-  a.pts = acc + size_t(kNoAllocMaxClusters) * kAcc;
+  a.acc_stride = 4;
+  a.pts = acc + size_t(kNoAllocMaxClusters) * 4;
   // the descriptor is written by a kernel (no host copy: the call may be captured)
   hipLaunchKernelGGL(ke_set_mesh, dim3(1), dim3(1), 0, s, EnergyMesh{0, n, 0, 0, K, 0, 0, 0}, mesh);
   return energy_forward(s, a, energy, 1);
 }
 
 hipError_t energy_backward(hipStream_t s, const EnergyArgs& a, const double* grad_energy, float* dxyz, float* dw) {
-  if (a.n_clusters > 0)
-    hipLaunchKernelGGL(ke_cluster_adjoint, dim3(egrid(a.n_clusters)), dim3(kEBlock), 0, s, a, grad_energy);
-  if (a.n_items > 0)
-    hipLaunchKernelGGL(ke_item_grad, dim3(egrid(a.n_items)), dim3(kEBlock), 0, s, a, grad_energy, dxyz, dw);
+  if (a.n_items > 0 && a.adj)
+    hipLaunchKernelGGL(ke_item_grad<true>, dim3(egrid(a.n_items)), dim3(kEBlock), 0, s, a, grad_energy, dxyz, dw);
+  else if (a.n_items > 0)
+    hipLaunchKernelGGL(ke_item_grad<false>, dim3(egrid(a.n_items)), dim3(kEBlock), 0, s, a, grad_energy, dxyz, dw);
   return hipGetLastError();
 }
 

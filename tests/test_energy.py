@@ -184,6 +184,74 @@ def test_gpu_energy_batch_equals_separate(gpu_ready):
         np.testing.assert_allclose(dw[sl].cpu().numpy(), dw1.cpu().numpy(), rtol=1e-6, atol=1e-7)
 
 
+def ring_problem(shape):
+    """Meshes whose rings of faces are not one closed fan of at most 7 neighbours:
+    a hub of 9 / 16 / 17 / 70 faces, an open grid (boundary vertices), two cones
+    joined at their tip (a bowtie, with a degenerate face and a vertex without
+    faces), and scattered labels (every ring meets many clusters; more clusters
+    than a block's table holds)."""
+    rng = np.random.default_rng(7)
+    if shape.startswith("hub"):
+        n = int(shape[3:])
+        t = 2 * np.pi * np.arange(n) / n
+        x = np.concatenate([[[0, 0, 0.4]], np.stack([np.cos(t), np.sin(t), 0.1 * np.cos(3 * t)], 1), [[0, 0, -0.6]]])
+        i = np.arange(n)
+        tri = np.concatenate([np.stack([np.zeros(n, int), 1 + i, 1 + (i + 1) % n], 1),
+                              np.stack([np.full(n, n + 1), 1 + (i + 1) % n, 1 + i], 1)])
+        lab, K = rng.integers(0, 4, len(x)), 4
+    elif shape == "grid":
+        n = 19
+        u, v = np.meshgrid(np.arange(n), np.arange(n), indexing="ij")
+        x = np.stack([u / n, v / n, 0.05 * rng.standard_normal((n, n))], -1).reshape(-1, 3)
+        i = (u * n + v)[:-1, :-1].reshape(-1)
+        tri = np.concatenate([np.stack([i, i + n, i + n + 1], 1), np.stack([i, i + n + 1, i + 1], 1)])
+        lab, K = (u // 5 * 4 + v // 5).reshape(-1), 18  # two clusters stay empty
+        lab[rng.random(len(lab)) < 0.1] = 18
+    elif shape == "bowtie":
+        x0, _, t0, _, _ = ring_problem("hub6")
+        x1 = x0[1:] * [1, 1, -1] + [0, 0, 0.8]
+        x = np.concatenate([x0, x1, [[3, 3, 3]]])
+        t1 = np.where(t0 == 0, 0, t0 + len(x0) - 1)[:, ::-1]
+        tri = np.concatenate([t0, t1, [[1, 1, 2]]])
+        lab, K = rng.integers(0, 3, len(x)), 3
+    else:
+        xyz, tri = meshgen.icosphere(4 if shape == "scattered4" else 5, 3, 0.05)
+        x, K = np.asarray(xyz), 60 if shape == "scattered4" else 5000
+        lab = rng.integers(0, K, len(x))
+    x = np.asarray(x, np.float32).astype(np.float64)
+    w = rng.uniform(0.5, 2.0, len(x)).astype(np.float32).astype(np.float64)
+    return x, w, np.ascontiguousarray(tri, np.int32), lab.astype(np.int32), K
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", ["hub9", "hub16", "hub17", "hub70", "grid", "bowtie", "scattered4", "scattered5"])
+@pytest.mark.parametrize("metric", [ISO, QEM])
+def test_gpu_energy_rings_match_oracle(gpu_ready, metric, shape):
+    """Against the oracle on meshes with every form of ring, alone and behind
+    another mesh of 37 vertices (rings and blocks not aligned to the mesh).
+    Tolerances: the energy sums FP64 terms in another order (1e-9), the gradients
+    are rounded to FP32 (1e-5 of the largest component, as above)."""
+    import torch
+    from acvd_amd.energy import ClusterEnergy
+    x, w, tri, lab, K = ring_problem(shape)
+    ref = po.EnergyRef(len(x), tri, np.where(lab < K, lab, K), K, metric, 2)
+    e_ref, d = ref.total(x, w), ref.derivatives(x, w, np.arange(4 * len(x)))
+    pad = ring_problem("hub35")
+    for lead in (False, True):
+        meshes = ([(pad, QEM)] if lead else []) + [((x, w, tri, lab, K), metric)]
+        ce = ClusterEnergy(0)
+        for (mx, _, mt, _, mk), mm in meshes:
+            ce.add_mesh(len(mx), mt, mk, mm, 2)
+        parts = [gpu_inputs(mx, mw, ml, mk) for (mx, mw, _, ml, mk), _ in meshes]
+        tx, tw, tl = (torch.cat(t).contiguous() for t in zip(*parts))
+        e = ce.forward_raw(tx, tw, tl).cpu().numpy()
+        assert np.isclose(e[-1], e_ref, rtol=1e-9), (e[-1], e_ref)
+        g = torch.full((len(meshes),), 1.5, dtype=torch.float64, device=tx.device)
+        dx, dw = (t[-len(x):].cpu().numpy() / 1.5 for t in ce.backward_raw(tx, tw, tl, g))
+        got = np.concatenate([dx.reshape(-1), dw]).astype(np.float64)
+        assert np.abs(got - d).max() < 1e-5 * np.abs(d).max(), np.abs(got - d).max() / np.abs(d).max()
+
+
 @pytest.mark.gpu
 def test_gpu_energy_errors(gpu_ready):
     import torch

@@ -49,6 +49,18 @@ constexpr int kTilesPerScanBlock = kBlock / 64;  // k_scan: one wavefront per ti
 // (QEM torus of 8.39M vertices, K = 100k: K/32 263.0 ms, K/16 260.7 ms,
 // K/8 260.9 ms to convergence).
 constexpr int kTileOnDivisor = 16;
+// Contexts of at most kFusedItems items scan and evaluate in one launch (768
+// blocks of 256 items, the 3 per CU that the QEM evaluate's registers allow, so
+// that every block has at most one step).  To convergence, two launches / one:
+// icosphere of 2,562 items 1.51 / 1.34 ms, 40,962 4.69 / 4.29, 163,842 10.45 /
+// 9.86; QEM torus of 260,533 37.5 / 37.9, of 503,503 44.7 / 47.3.
+constexpr int64_t kFusedItems = 768 * kBlock;
+// Contexts of at most kTileMinItems items keep no tile sets: a scan of all their
+// items costs less than the sets' upkeep.  To convergence, with / without:
+// icosphere of 40,962 items 5.46 / 4.69 ms, 163,842 12.4 / 10.5; QEM torus of
+// 260,533 39.3 / 37.5, of 503,503 47.1 / 44.7; torus of 883,300 22.59 / 22.88;
+// QEM cube of 960,002 25.6 / 25.9.
+constexpr int64_t kTileMinItems = 700000;
 
 struct DevMesh {
   int64_t item_off;
@@ -208,6 +220,7 @@ hipError_t launch_tile_sets(hipStream_t s, const SweepArgs& a, const int32_t* me
 hipError_t launch_tile_order(hipStream_t s, const SweepArgs& a, const float* bbox, int32_t* tile_items,
                              int32_t* item_tile, void** tmp, size_t* tmp_bytes);
 hipError_t launch_eval(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained);
+hipError_t launch_scan_eval(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained);
 hipError_t launch_apply(hipStream_t s, const SweepArgs& a, int round, bool constrained);
 hipError_t launch_tile_update(hipStream_t s, const SweepArgs& a);
 hipError_t launch_reeval(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained,

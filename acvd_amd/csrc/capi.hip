@@ -616,9 +616,14 @@ int recompute_statistics(acvd_ctx* c, const int32_t* mask, int set_stamp, unsign
 int enqueue_chunk(acvd_ctx* c, bool qem_unc, bool tiles, int n_pass, int n_rounds) {
   hipStream_t s = c->stream;
   SweepArgs a = c->args();
+  const bool fused = !tiles && c->N <= kFusedItems;
   for (int p = 0; p < n_pass; ++p) {
-    HIP_TRY(launch_scan(s, a, tiles));
-    HIP_TRY(launch_eval(s, a, c->any_iso, c->any_qem, qem_unc));
+    if (fused) {
+      HIP_TRY(launch_scan_eval(s, a, c->any_iso, c->any_qem, qem_unc));
+    } else {
+      HIP_TRY(launch_scan(s, a, tiles));
+      HIP_TRY(launch_eval(s, a, c->any_iso, c->any_qem, qem_unc));
+    }
     HIP_TRY(launch_apply(s, a, 0, !qem_unc));
     for (int r = 1; r < n_rounds; ++r) {
       HIP_TRY(launch_reeval(s, a, c->any_iso, c->any_qem, qem_unc, r));
@@ -636,13 +641,15 @@ int enqueue_chunk(acvd_ctx* c, bool qem_unc, bool tiles, int n_pass, int n_round
 int run_chunk_timed(acvd_ctx* c, bool qem_unc, bool tiles, int n_pass, int n_rounds) {
   hipStream_t s = c->stream;
   SweepArgs a = c->args();
+  const bool fused = !tiles && c->N <= kFusedItems;
   std::vector<hipEvent_t> ev(5 * n_pass);
   for (auto& e : ev) HIP_TRY(hipEventCreate(&e));
   for (int p = 0; p < n_pass; ++p) {
     HIP_TRY(hipEventRecord(ev[5 * p], s));
-    HIP_TRY(launch_scan(s, a, tiles));
+    if (!fused) HIP_TRY(launch_scan(s, a, tiles));
     HIP_TRY(hipEventRecord(ev[5 * p + 1], s));
-    HIP_TRY(launch_eval(s, a, c->any_iso, c->any_qem, qem_unc));
+    if (fused) HIP_TRY(launch_scan_eval(s, a, c->any_iso, c->any_qem, qem_unc));  // counted with the evaluate
+    else HIP_TRY(launch_eval(s, a, c->any_iso, c->any_qem, qem_unc));
     HIP_TRY(hipEventRecord(ev[5 * p + 2], s));
     HIP_TRY(launch_apply(s, a, 0, !qem_unc));
     for (int r = 1; r < n_rounds; ++r) {
@@ -936,7 +943,7 @@ int minimize_energy(acvd_ctx* c) {
       near_end = 2 * int64_t(c->h_ctrl->pass_log[(c->h_ctrl->passes - 1) % kPassLogCap][2]) <= 3 * stop_props;
     // tile sets on once the last pass moved at most K / kTileOnDivisor items:
     // most tiles then hold no changed cluster and the scan skips them
-    if (!tiles && c->h_ctrl->passes > 0 &&
+    if (!tiles && c->N > kTileMinItems && c->h_ctrl->passes > 0 &&
         int64_t(c->h_ctrl->pass_log[(c->h_ctrl->passes - 1) % kPassLogCap][3]) * c->tuning.tile_on_divisor <= c->K) {
       HIP_TRY(launch_tile_sets(s, a, nullptr));
       tiles = true;

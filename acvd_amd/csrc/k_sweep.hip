@@ -745,12 +745,77 @@ __device__ bool qem_pool_choose(const SweepArgs& a, const SweepView& v, QemPool*
   return target != kNull && qem_accept(best_d, best_m);
 }
 
-// Evaluate (round 0): best move of each work item (shared rule of
+// Adds one to counter(m) for every lane of the wave with `want`: one atomic per
+// distinct mesh of the wave (its lanes mostly lie in one).  Every lane calls it.
+template <class Counter>
+__device__ inline void count_per_mesh(bool want, int32_t m, Counter&& counter) {
+  unsigned long long todo = __ballot(want);
+  while (todo) {
+    const int leader = __ffsll((long long)todo) - 1;
+    const int32_t m0 = __shfl(m, leader);
+    const unsigned long long same = __ballot(want && m == m0);
+    if (int(__lane_id()) == leader) atomicAdd(counter(m0), __popcll(same));
+    todo &= ~same;
+  }
+}
+
+// Evaluate (round 0) of item i (when valid): its best move (shared rule of
 // acvd_math.h) against the state at the pass start; a proposal registers its
-// round-0 accept key at both clusters and joins the block's candidate
-// segment.  Block b owns segment b (capacity cand_cap, count seg_cand[b]);
-// the second launch of a mixed batch (append = 1) continues the segments of
-// the first.
+// round-0 accept key at both clusters and joins the block's candidate segment.
+// Every lane of the block calls it (the QEM solve pool is shared by the wave).
+template <int METRIC, bool kExtras>
+__device__ inline void eval_item(const SweepArgs& a, const SweepView& v, QemPool* pool, KeyAgg* agg, int64_t seg,
+                                 int32_t* s_n, bool valid, int32_t i) {
+  bool want = false;
+  int32_t lab = kNull, target = kNull, L = 0, m = 0;
+  int32_t nb[kRingCache];
+  QemItem s;
+  uint32_t open = 0;
+  int kind = kPoolNone, ntask = 0;
+  if (valid) {
+    m = mesh_of_item(a, i);
+    const DevMesh& dm = a.meshes[m];
+    if (dm.metric == mesh_metric(METRIC)) {
+      const MeshState* st = &a.state[m];
+      L = st->loops;
+      lab = a.labels[i];
+      if (METRIC == 1 && lab != kNull && qem_mode(*st))
+        kind = pool_screen(v, i, lab, st->connexity, nb, &s, &open, &ntask);
+      else  // no FP64 solve: the null-item rule or the isotropic one
+        want = propose_item<METRIC == 1 ? 2 : METRIC>(v, i, lab, st->connexity, st->constrained, dm.level, dm.scales,
+                                                      &target);
+    }
+  }
+  if constexpr (METRIC == 1) {
+    int32_t pt = kNull;
+    const bool r = qem_pool_choose<kExtras>(a, v, pool, kind, ntask, i, lab, m, nb, s, open, &pt);
+    if (kind != kPoolNone) {
+      want = r;
+      target = pt;
+    }
+  }
+  if (want) {
+    const DevMesh& dm = a.meshes[m];
+    const unsigned long long key = accept_key(dm.seed, L, 0, uint32_t(i - dm.item_off));
+    if (lab != kNull) keyagg_min(agg, lab, key);
+    keyagg_min(agg, target, key);
+    a.cand_pass[i] = L;
+    a.tile_prop[a.item_tile[i]] = L;
+  }
+  if (a.item_mesh) count_per_mesh(want, m, [&](int32_t mm) { return &a.state[mm].pass_props; });
+  const int64_t e = seg_append(seg, s_n, want);
+  if (want) {
+    a.cand[e] = i;
+    a.cand_lab[e] = lab;
+    a.cand_tgt[e] = target;
+    a.cand_since[e] = L * kMatchRounds;
+  }
+  keyagg_flush(agg, a.prio);
+}
+
+// Evaluate the work list of the scan.  Block b owns segment b (capacity
+// cand_cap, count seg_cand[b]); the second launch of a mixed batch (append = 1)
+// continues the segments of the first.
 template <int METRIC, bool kExtras>
 __global__ __launch_bounds__(kBlock) void k_eval(SweepArgs a, int append) {
   __shared__ WorkIndex wi;
@@ -763,63 +828,61 @@ __global__ __launch_bounds__(kBlock) void k_eval(SweepArgs a, int append) {
   const int32_t n = wi.start[kWorkSlices];
   const SweepView v = make_view<kExtras>(a);
   const int64_t seg = int64_t(blockIdx.x) * a.cand_cap;
+  QemPool* pool = &pools[METRIC == 1 ? threadIdx.x >> 6 : 0];
   for (int32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {
     const int32_t t = base + int32_t(threadIdx.x);
-    bool want = false;
-    int32_t i = 0, lab = kNull, target = kNull, L = 0, m = 0;
-    int32_t nb[kRingCache];
-    QemItem s;
-    uint32_t open = 0;
-    int kind = kPoolNone, ntask = 0;
-    if (t < n) {
-      i = work_entry(a, &wi, t);
-      m = mesh_of_item(a, i);
-      const DevMesh& dm = a.meshes[m];
-      if (dm.metric == mesh_metric(METRIC)) {
-        const MeshState* st = &a.state[m];
-        L = st->loops;
-        lab = a.labels[i];
-        if (METRIC == 1 && lab != kNull && qem_mode(*st))
-          kind = pool_screen(v, i, lab, st->connexity, nb, &s, &open, &ntask);
-        else  // no FP64 solve: the null-item rule or the isotropic one
-          want = propose_item<METRIC == 1 ? 2 : METRIC>(v, i, lab, st->connexity, st->constrained, dm.level,
-                                                        dm.scales, &target);
-      }
-    }
-    if constexpr (METRIC == 1) {
-      int32_t pt = kNull;
-      const bool r =
-          qem_pool_choose<kExtras>(a, v, &pools[threadIdx.x >> 6], kind, ntask, i, lab, m, nb, s, open, &pt);
-      if (kind != kPoolNone) {
-        want = r;
-        target = pt;
-      }
-    }
-    if (want) {
-      const DevMesh& dm = a.meshes[m];
-      const unsigned long long key = accept_key(dm.seed, L, 0, uint32_t(i - dm.item_off));
-      if (lab != kNull) keyagg_min(&agg, lab, key);
-      keyagg_min(&agg, target, key);
-      a.cand_pass[i] = L;
-      a.tile_prop[a.item_tile[i]] = L;
-      if (a.item_mesh) atomicAdd(&a.state[m].pass_props, 1);
-    }
-    const int64_t e = seg_append(seg, &s_n, want);
-    if (want) {
-      a.cand[e] = i;
-      a.cand_lab[e] = lab;
-      a.cand_tgt[e] = target;
-      a.cand_since[e] = L * kMatchRounds;
-    }
-    keyagg_flush(&agg, a.prio);
+    const int32_t i = t < n ? work_entry(a, &wi, t) : 0;
+    eval_item<METRIC, kExtras>(a, v, pool, &agg, seg, &s_n, t < n, i);
   }
   __syncthreads();
   if (threadIdx.x == 0) a.seg_cand[blockIdx.x] = s_n;
 }
 
-// Re-evaluation of candidate entry e (when valid) for round `round`; every
-// lane of the wave calls it (the QEM solve pool is shared by the wave).
-// reg(c, key) registers an accept key at cluster c.
+// Scan and evaluate in one launch, on contexts of at most kFusedItems items:
+// block b takes the item blocks b, b + n_seg, ... , compacts the items to
+// evaluate in LDS and evaluates them.  The work list, its index of slice starts
+// and a launch go; what they give, an even share of the work items for every
+// block, counts only where the blocks have more than a step or two of them.
+template <int METRIC, bool kExtras>
+__global__ __launch_bounds__(kBlock) void k_scan_eval(SweepArgs a, int append) {
+  __shared__ KeyAgg agg;
+  __shared__ QemPool pools[METRIC == 1 ? kBlock / 64 : 1];
+  __shared__ int32_t s_n, s_cnt[kBlock / 64], s_item[kBlock];
+  if (threadIdx.x == 0) s_n = append ? a.seg_cand[blockIdx.x] : 0;
+  keyagg_clear(&agg);
+  const SweepView v = make_view<kExtras>(a);
+  const int64_t seg = int64_t(blockIdx.x) * a.cand_cap;
+  QemPool* pool = &pools[METRIC == 1 ? threadIdx.x >> 6 : 0];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  for (int64_t base = int64_t(blockIdx.x) * kBlock; base < a.n_items; base += int64_t(gridDim.x) * kBlock) {
+    const int64_t i = base + threadIdx.x;
+    bool want = false;
+    if (i < a.n_items) {
+      const int m = mesh_of_item(a, i);
+      const MeshState& st = a.state[m];
+      if (st.phase == kPhaseSweep && a.meshes[m].metric == mesh_metric(METRIC))
+        want = needs_eval_fast(a, i, a.labels[i], st.loops);
+    }
+    const unsigned long long bal = __ballot(want);
+    if (lane == 0) s_cnt[w] = __popcll(bal);
+    __syncthreads();
+    int32_t before = 0, n = 0;
+    for (int k = 0; k < kBlock / 64; ++k) {
+      if (k < w) before += s_cnt[k];
+      n += s_cnt[k];
+    }
+    if (want) s_item[before + __popcll(bal & ((1ull << lane) - 1ull))] = int32_t(i);
+    if (n && threadIdx.x == 0) atomicAdd(&a.work_count[blockIdx.x % kWorkSlices], n);  // items evaluated
+    __syncthreads();
+    if (n) {  // block-uniform
+      const bool valid = int32_t(threadIdx.x) < n;
+      eval_item<METRIC, kExtras>(a, v, pool, &agg, seg, &s_n, valid, valid ? s_item[threadIdx.x] : 0);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) a.seg_cand[blockIdx.x] = s_n;
+}
+
 // Block sum of v (the result is valid in thread 0; synchronises the block).
 __device__ inline int block_sum(int v) {
   __shared__ int s_red[kBlock / 64];
@@ -833,6 +896,9 @@ __device__ inline int block_sum(int v) {
   return tot;  // valid in thread 0
 }
 
+// Re-evaluation of candidate entry e (when valid) for round `round`; every
+// lane of the wave calls it (the QEM solve pool is shared by the wave).
+// reg(c, key) registers an accept key at cluster c.
 template <int METRIC, bool kExtras, bool kCount, class Reg>
 __device__ inline void reeval_entry(const SweepArgs& a, const SweepView& v, QemPool* pool, bool valid, int64_t e,
                                     int round, Reg&& reg, int* n_live, int* n_stale, int* n_recheck) {
@@ -987,11 +1053,12 @@ __device__ inline bool apply_entry(const SweepArgs& a, DeriveList* dl, bool vali
   const int32_t b = valid ? a.cand_tgt[e] : -1;
   const int32_t i_e = valid ? a.cand[e] : 0;
   const int32_t lab_e = valid ? a.cand_lab[e] : kNull;
+  int32_t mesh = 0;
   if (b >= 0) {
     i = i_e;
     lab = lab_e;
-    const int m = mesh_of_item(a, i);
-    MeshState* st = &a.state[m];
+    const int m = mesh = mesh_of_item(a, i);
+    const MeshState* st = &a.state[m];
     const int32_t L = st->loops;
     const DevMesh& dm = a.meshes[m];
     const unsigned long long key = accept_key(dm.seed, L, round, uint32_t(i - dm.item_off));
@@ -1034,13 +1101,13 @@ __device__ inline bool apply_entry(const SweepArgs& a, DeriveList* dl, bool vali
       a.sizes[b] += 1;
       a.stamp[b] = L;
       a.cl_round[b] = rtag;
-      if (a.item_mesh) atomicAdd(&st->pass_mods, 1);
       if (!kSolve) {
         if (lab != kNull) derive_cluster<kExtras>(a, lab, dm, 0, false);
         derive_cluster<kExtras>(a, b, dm, 0, false);
       }
     }
   }
+  if (a.item_mesh) count_per_mesh(win, mesh, [&](int32_t mm) { return &a.state[mm].pass_mods; });
   if constexpr (kSolve) {
     const int cnt = win ? (lab != kNull ? 2 : 1) : 0;
     const int inc = wave_prefix(cnt);
@@ -1574,6 +1641,20 @@ void launch_eval_x(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem
 hipError_t launch_eval(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained) {
   if (a.anchor || a.frozen) launch_eval_x<true>(s, a, any_iso, any_qem, qem_unconstrained);
   else launch_eval_x<false>(s, a, any_iso, any_qem, qem_unconstrained);
+  return hipGetLastError();
+}
+
+template <bool kX>
+void launch_scan_eval_x(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained) {
+  const dim3 g(unsigned(a.n_seg)), b(kBlock);
+  if (any_iso) hipLaunchKernelGGL((k_scan_eval<0, kX>), g, b, 0, s, a, 0);
+  if (any_qem && qem_unconstrained) hipLaunchKernelGGL((k_scan_eval<2, kX>), g, b, 0, s, a, any_iso ? 1 : 0);
+  else if (any_qem) hipLaunchKernelGGL((k_scan_eval<1, kX>), g, b, 0, s, a, any_iso ? 1 : 0);
+}
+
+hipError_t launch_scan_eval(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained) {
+  if (a.anchor || a.frozen) launch_scan_eval_x<true>(s, a, any_iso, any_qem, qem_unconstrained);
+  else launch_scan_eval_x<false>(s, a, any_iso, any_qem, qem_unconstrained);
   return hipGetLastError();
 }
 

@@ -112,6 +112,24 @@ def test_labels_bit_exact_against_replay(gpu_ready, name):
     np.testing.assert_array_equal(ctx.cluster_sizes(0), np.bincount(lab, minlength=K)[:K])
 
 
+@pytest.mark.parametrize("nu,nv,metric", [(512, 384, QEM), (512, 385, QEM), (1024, 683, ISO), (1024, 684, ISO)])
+def test_labels_bit_exact_where_the_scan_changes(gpu_ready, nu, nv, metric):
+    """Either side of the sizes where the scan and the evaluate part (196,608
+    items) and where the tile sets are kept (700,000)."""
+    xyz, tri = meshgen.torus(nu, nv, 11)
+    K = len(xyz) // 128
+    init = meshgen.seed_labels(len(xyz), K, 3)
+    ctx = run_gpu(xyz, tri, metric, K, int(metric == QEM), init)
+    rp, col = ctx.adjacency(0)
+    xw, q = ctx.items(0)
+    rlab, rst = po.replay_run(rp, col, xw, q, ctx.scales(0), K, metric, init, seed=7, unconstrained=int(metric == QEM),
+                              max_loops=200000)
+    st = ctx.stats(0)
+    print(nu * nv, st["loops"], st["total_moves"], flush=True)
+    assert st["loops"] == rst["loops"] and st["total_moves"] == rst["total_moves"]
+    np.testing.assert_array_equal(ctx.labels(0), rlab)
+
+
 @pytest.mark.parametrize("name", ["C1-iso", "ico5-qem", "cube40-qem", "torus-graded-qem"])
 def test_energy_against_serial_reference(gpu_ready, name):
     """Final unshifted FP64 energy of the GPU labels against oracle A run from

@@ -62,6 +62,11 @@ constexpr int64_t kFusedItems = 768 * kBlock;
 // QEM cube of 960,002 25.6 / 25.9.
 constexpr int64_t kTileMinItems = 700000;
 
+// Short rows: the CSR row of an item in eight words at a fixed place, so that its
+// ids are read without its bounds.
+constexpr int32_t kRowPad = -1;
+constexpr int32_t kRowLong = -2;
+
 struct DevMesh {
   int64_t item_off;
   int64_t n_items;
@@ -127,6 +132,7 @@ struct SweepArgs {
   const int32_t* clus_mesh;  // null when n_meshes == 1
   const int32_t* row_ptr;    // n_items + 1
   const int32_t* col;        // global item ids
+  const int4* row8;          // 2 per item: the row's ids if at most 8 (kRowPad past it), else kRowLong first
   const unsigned long long* ring_adj;  // ring adjacency per item (ring_adjacency of acvd_math.h)
   const int32_t* anchor;     // per cluster: global id of its fixed item or -1; null when no mesh has any
   const int32_t* frozen;     // per cluster: nonzero when frozen (ForceManifold restarts); null when none is
@@ -183,7 +189,7 @@ hipError_t launch_csr_compact(hipStream_t s, int64_t n, const int32_t* tptr, con
 hipError_t exclusive_scan_i32(hipStream_t s, const int32_t* in, int32_t* out, int64_t n, void** tmp,
                               size_t* tmp_bytes);
 hipError_t launch_ring_adj(hipStream_t s, int64_t n, const int32_t* row_ptr, const int32_t* col,
-                            unsigned long long* ring_adj);
+                            unsigned long long* ring_adj, int4* row8);
 hipError_t launch_curvature(hipStream_t s, int64_t off, int64_t n, const double* pos, const int32_t* tri,
                             const int32_t* row_ptr, const int32_t* col, const int32_t* vfptr, const int32_t* vfcol,
                             double* out);

@@ -513,6 +513,7 @@ ACVD_HD bool ring_problem_rows(const int32_t* rp, const int32_t* col, const int3
 // i) share a mesh edge.  A property of the mesh alone, built once; with it
 // the ring check needs only the labels of the ring neighbours.
 constexpr int kRingAdjMax = 8;
+static_assert(kRingAdjMax == kRingCache, "a short row has a ring adjacency");
 ACVD_HD uint64_t ring_adjacency(const int32_t* rp, const int32_t* col, int32_t i) {
   const int32_t r0 = rp[i], deg = rp[i + 1] - r0;
   if (deg > kRingAdjMax) return 0;
@@ -760,43 +761,107 @@ ACVD_HD int32_t ring_label(const int32_t* nb, int p) {
   return b;
 }
 
-// Screen of the QEM rule for rows of at most kRingCache neighbours: the
-// neighbour labels are read once into nb (independent loads, no chains
-// through the row), then the guards of qem_screen (size, ring check, leave
-// condition) and the exact prune of each neighbouring cluster at its first
-// CSR position.  Bit p of *open marks an open target nb[p]; returns *open != 0.
+// What the rules for short rows (at most kRingCache neighbours) read of an item
+// and of its cluster, none of it dependent on another: the callers load it at
+// once, the device before it knows whether the item is evaluated at all.
+struct ShortItem {
+  float px, py, pz, pw;
+  int32_t deg;       // neighbours
+  int32_t size_a;    // of the item's cluster
+  uint64_t adj;      // ring adjacency
+  ClusterGeom ga;
+};
+
+// Guards of a labelled short-row item leaving its cluster lab: size, frozen
+// cluster, ring check on the neighbour labels nb, leave condition.
+ACVD_HD bool short_can_move(const SweepView& v, const ShortItem& t, int32_t lab, int connexity, const int32_t* nb) {
+  if (t.size_a <= 1 || is_frozen(v, lab)) return false;
+  if (connexity && ring_problem_mask(t.adj, nb, t.deg, lab)) return false;
+  return can_leave(t.pw, t.ga);
+}
+
+// nb[p] is a neighbouring cluster other than lab, at its first position in nb.
+ACVD_HD bool first_target(const int32_t* nb, int p, int32_t lab) {
+  bool first = nb[p] != kNull && nb[p] != lab;
+  ACVD_UNROLL
+  for (int t = 0; t < p; ++t) first = first && nb[t] != nb[p];
+  return first;
+}
+
+// Isotropic rule of a labelled short-row item (propose_item): the neighbouring
+// cluster of the smallest join term (ties: lowest id).  The records of the
+// distinct neighbours are read side by side.
+ACVD_HD bool iso_propose_short(const SweepView& v, const ShortItem& t, int32_t lab, int connexity, const int32_t* nb,
+                               int32_t* target_out) {
+  if (!short_can_move(v, t, lab, connexity, nb)) return false;
+  float tb[kRingCache];
+  ACVD_UNROLL
+  for (int p = 0; p < kRingCache; ++p) {
+    tb[p] = 3.0e38f;
+    if (first_target(nb, p, lab) && !is_frozen(v, nb[p])) tb[p] = join_term(t.px, t.py, t.pz, t.pw, v.geom[nb[p]]);
+  }
+  float best = 3.0e38f;
+  int32_t target = kNull;
+  ACVD_UNROLL
+  for (int p = 0; p < kRingCache; ++p)
+    if (tb[p] < best || (tb[p] == best && nb[p] < target)) {
+      best = tb[p];
+      target = nb[p];
+    }
+  *target_out = target;
+  return target != kNull && iso_accept(leave_term(t.px, t.py, t.pz, t.pw, t.ga), best);
+}
+
+// iso_recheck of a short-row item, gb the target's record.
+ACVD_HD bool iso_recheck_short(const SweepView& v, const ShortItem& t, int32_t lab, int32_t b, int connexity,
+                               const int32_t* nb, const ClusterGeom& gb) {
+  bool adjacent = false;
+  ACVD_UNROLL
+  for (int p = 0; p < kRingCache; ++p) adjacent = adjacent || (p < t.deg && nb[p] == b);
+  if (!adjacent || is_frozen(v, b) || !short_can_move(v, t, lab, connexity, nb)) return false;
+  return iso_accept(leave_term(t.px, t.py, t.pz, t.pw, t.ga), join_term(t.px, t.py, t.pz, t.pw, gb));
+}
+
+// Screen of the QEM rule for a short-row item (no anchor item): the guards of
+// qem_screen and the exact prune of each neighbouring cluster at its first CSR
+// position.  Bit p of *open marks an open target nb[p]; returns *open != 0.
+ACVD_HD bool qem_screen_short(const SweepView& v, const ShortItem& t, int32_t lab, int connexity, double Ta,
+                              int constrained, const int32_t* nb, QemItem* s, uint32_t* open_out) {
+  *open_out = 0;
+  if (!short_can_move(v, t, lab, connexity, nb)) return false;
+  s->px = t.px;
+  s->py = t.py;
+  s->pz = t.pz;
+  s->pw = t.pw;
+  s->r0 = s->r1 = 0;  // the open targets are in nb
+  s->ta = leave_term(t.px, t.py, t.pz, t.pw, t.ga);
+  s->Ta = constrained ? Ta : 0.0;
+  uint32_t open = 0;
+  ACVD_UNROLL
+  for (int p = 0; p < kRingCache; ++p)
+    if (first_target(nb, p, lab) && qem_open(v, *s, nb[p], constrained)) open |= 1u << p;
+  *open_out = open;
+  return open != 0;
+}
+
+// The screen with its loads, for callers that hold nothing of the item yet.
 ACVD_HD bool qem_screen_short_row(const SweepView& v, int64_t i, int32_t lab, int connexity, int constrained,
                                   int32_t* nb, QemItem* s, uint32_t* open_out) {
   const int32_t r0 = v.row_ptr[i], deg = v.row_ptr[i + 1] - r0;
-  // the words of the item and of its cluster, read with the row bounds (they
-  // do not depend on the row), so that the guards below wait on one round trip
-  const int32_t size_a = v.sizes[lab];
-  const unsigned long long adj = v.ring_adj ? v.ring_adj[i] : 0ull;
-  const float w_i = v.xw[4 * i + 3];
-  const ClusterGeom ga = v.geom[lab];
+  ShortItem t;
+  t.px = v.xw[4 * i];
+  t.py = v.xw[4 * i + 1];
+  t.pz = v.xw[4 * i + 2];
+  t.pw = v.xw[4 * i + 3];
+  t.deg = deg;
+  t.size_a = v.sizes[lab];
+  t.adj = v.ring_adj ? v.ring_adj[i] : ring_adjacency(v.row_ptr, v.col, int32_t(i));
+  t.ga = v.geom[lab];
   ACVD_UNROLL
   for (int p = 0; p < kRingCache; ++p) nb[p] = p < deg ? v.labels[v.col[r0 + p]] : kNull;
   *open_out = 0;
-  if (size_a <= 1) return false;
-  if (is_anchor(v, i, lab) || is_frozen(v, lab)) return false;
-  if (connexity) {
-    const bool split = (v.ring_adj && deg <= kRingAdjMax)
-                           ? ring_problem_mask(adj, nb, deg, lab)
-                           : ring_problem(v.row_ptr, v.col, v.labels, int32_t(i), lab);
-    if (split) return false;
-  }
-  if (!can_leave(w_i, ga)) return false;
-  qem_item_terms(v, i, lab, constrained, s);
-  uint32_t open = 0;
-  ACVD_UNROLL
-  for (int p = 0; p < kRingCache; ++p) {
-    bool first = nb[p] != kNull && nb[p] != lab;
-    ACVD_UNROLL
-    for (int t = 0; t < p; ++t) first = first && nb[t] != nb[p];
-    if (first && qem_open(v, *s, nb[p], constrained)) open |= 1u << p;
-  }
-  *open_out = open;
-  return open != 0;
+  if (is_anchor(v, i, lab)) return false;
+  return qem_screen_short(v, t, lab, connexity, constrained ? v.T[lab] : 0.0, constrained, nb, s, open_out);
 }
 
 // The QEM rule for rows of at most kRingCache neighbours: the same tests in

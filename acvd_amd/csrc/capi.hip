@@ -115,6 +115,7 @@ struct acvd_ctx {
   DBuf<double> d_pos;
   DBuf<int32_t> d_vfptr, d_vfcol;
   DBuf<float4> d_xw;
+  DBuf<int4> d_row8;
   DBuf<float> d_q;
   DBuf<int32_t> d_labels, d_sizes, d_stamp, d_cand_pass, d_pending;
   DBuf<unsigned long long> d_acc_ws, d_acc_q, d_prio, d_ring_adj;
@@ -184,6 +185,7 @@ struct acvd_ctx {
     a.clus_mesh = meshes.size() > 1 ? d_clus_mesh.p : nullptr;
     a.row_ptr = d_row_ptr.p;
     a.col = d_col.p;
+    a.row8 = d_row8.p;
     a.ring_adj = d_ring_adj.p;
     a.xw = d_xw.p;
     a.q = d_q.p;
@@ -455,7 +457,8 @@ int build(acvd_ctx* c) {
     HIP_TRY(c->d_col.alloc(e2));
     HIP_TRY(launch_csr_compact(s, N, tptr.p, tcol.p, c->d_row_ptr.p, c->d_col.p));
     HIP_TRY(c->d_ring_adj.alloc(N));
-    HIP_TRY(launch_ring_adj(s, N, c->d_row_ptr.p, c->d_col.p, c->d_ring_adj.p));
+    HIP_TRY(c->d_row8.alloc(2 * N));
+    HIP_TRY(launch_ring_adj(s, N, c->d_row_ptr.p, c->d_col.p, c->d_ring_adj.p, c->d_row8.p));
     // ---- curvature indicators (before the weights that use them)
     for (int m = 0; m < M; ++m) {
       HostMesh& h = c->meshes[m];

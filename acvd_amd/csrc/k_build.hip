@@ -235,12 +235,20 @@ __global__ void k_clamp(SweepArgs a, const double* __restrict__ raw_w, const dou
   xw[v].w = float(w);
 }
 
-// Ring adjacency of every item (bits of neighbour pairs sharing an edge).
+// Ring adjacency of every item (bits of neighbour pairs sharing an edge) and
+// its short row.
 __global__ void k_ring_adj(int64_t n, const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col,
-                           unsigned long long* ring_adj) {
+                           unsigned long long* ring_adj, int4* row8) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
   ring_adj[i] = ring_adjacency(row_ptr, col, int32_t(i));
+  const int32_t r0 = row_ptr[i], deg = row_ptr[i + 1] - r0;
+  int32_t c[kRingCache];
+  ACVD_UNROLL
+  for (int k = 0; k < kRingCache; ++k) c[k] = deg <= kRingCache && k < deg ? col[r0 + k] : kRowPad;
+  if (deg > kRingCache) c[0] = kRowLong;
+  row8[2 * i] = make_int4(c[0], c[1], c[2], c[3]);
+  row8[2 * i + 1] = make_int4(c[4], c[5], c[6], c[7]);
 }
 
 }  // namespace
@@ -267,9 +275,9 @@ hipError_t launch_csr_sort_unique(hipStream_t s, int64_t n, const int32_t* tptr,
 }
 
 hipError_t launch_ring_adj(hipStream_t s, int64_t n, const int32_t* row_ptr, const int32_t* col,
-                           unsigned long long* ring_adj) {
+                           unsigned long long* ring_adj, int4* row8) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_ring_adj, dim3(grid_for(n)), dim3(kBlock), 0, s, n, row_ptr, col, ring_adj);
+  hipLaunchKernelGGL(k_ring_adj, dim3(grid_for(n)), dim3(kBlock), 0, s, n, row_ptr, col, ring_adj, row8);
   return hipGetLastError();
 }
 

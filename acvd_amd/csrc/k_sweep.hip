@@ -169,36 +169,89 @@ __device__ inline SweepView make_view(const SweepArgs& a) {
   return v;
 }
 
-// needs_eval of acvd_math.h with the neighbour loads issued together (up to 8
-// neighbours in registers) so that the label and stamp gathers overlap.
+// Neighbours of item i from the short rows (kRowPad past the row); false for a
+// row of more than kRingCache neighbours, which is in the CSR alone.
+__device__ inline bool load_row8(const SweepArgs& a, int64_t i, int32_t* nbr) {
+  const int4 u = a.row8[2 * i], v = a.row8[2 * i + 1];
+  nbr[0] = u.x;
+  nbr[1] = u.y;
+  nbr[2] = u.z;
+  nbr[3] = u.w;
+  nbr[4] = v.x;
+  nbr[5] = v.y;
+  nbr[6] = v.z;
+  nbr[7] = v.w;
+  return nbr[0] != kRowLong;
+}
+
+// Labels of the neighbours of a short row (kNull past it); returns their number.
+__device__ inline int32_t load_labels8(const SweepArgs& a, const int32_t* nbr, int32_t* nb) {
+  int32_t deg = 0;
+#pragma unroll
+  for (int p = 0; p < kRingCache; ++p) {
+    nb[p] = nbr[p] >= 0 ? a.labels[nbr[p]] : kNull;
+    deg += nbr[p] >= 0;
+  }
+  return deg;
+}
+
+// needs_eval of acvd_math.h with the neighbour loads issued together so that the
+// label and stamp gathers overlap.
 __device__ inline bool needs_eval_fast(const SweepArgs& a, int64_t i, int32_t lab, int32_t L) {
-  const int32_t r0 = a.row_ptr[i], r1 = a.row_ptr[i + 1];
+  int32_t nbr[kRingCache], lb[kRingCache];
+  const bool is_short = load_row8(a, i, nbr);
   bool dirty = (a.cand_pass[i] == L - 1);
   if (lab != kNull) dirty |= (a.stamp[lab] + 1 >= L);
   bool boundary = false;
-  const int32_t deg = r1 - r0;
-  int32_t nb[8], lb[8];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) nb[k] = k < deg ? a.col[r0 + k] : 0;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) lb[k] = k < deg ? a.labels[nb[k]] : lab;
+  for (int k = 0; k < kRingCache; ++k) lb[k] = nbr[k] >= 0 ? a.labels[nbr[k]] : lab;
   // neighbour stamps are read only while the item is not already dirty
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
+  for (int k = 0; k < kRingCache; ++k) {
     if (lb[k] != lab) {
       boundary = true;
       if (!dirty && lb[k] != kNull && a.stamp[lb[k]] + 1 >= L) dirty = true;
     }
   }
-  for (int32_t k = r0 + 8; k < r1; ++k) {
-    const int32_t b = a.labels[a.col[k]];
-    if (b != lab) {
-      boundary = true;
-      if (!dirty && b != kNull && a.stamp[b] + 1 >= L) dirty = true;
+  if (!is_short)
+    for (int32_t k = a.row_ptr[i]; k < a.row_ptr[i + 1]; ++k) {
+      const int32_t b = a.labels[a.col[k]];
+      if (b != lab) {
+        boundary = true;
+        if (!dirty && b != kNull && a.stamp[b] + 1 >= L) dirty = true;
+      }
     }
-  }
   return boundary && dirty;
 }
+
+// Control values of a mesh that the sweep kernels read per item.  In a context of
+// one mesh (kB = false) they are read once, at the kernel's start, with its
+// other first loads.
+struct MeshCtl {
+  int64_t item_off;
+  uint32_t seed;
+  int32_t metric, level;
+  int32_t loops, connexity, constrained, mode, rounds;
+};
+__device__ inline MeshCtl load_mesh(const SweepArgs& a, int32_t m) {
+  const DevMesh& dm = a.meshes[m];
+  const MeshState& st = a.state[m];
+  return MeshCtl{dm.item_off, dm.seed, dm.metric, dm.level, st.loops, st.connexity, st.constrained, qem_mode(st),
+                 pass_rounds(st)};
+}
+template <bool kB>
+struct MeshReader {
+  const SweepArgs& a;
+  MeshCtl one;
+  __device__ explicit MeshReader(const SweepArgs& args) : a(args) {
+    if constexpr (!kB) one = load_mesh(a, 0);
+  }
+  __device__ int32_t of_item(int64_t i) const { return kB ? mesh_of_item(a, i) : 0; }
+  __device__ MeshCtl operator()(int32_t m) const {
+    if constexpr (kB) return load_mesh(a, m);
+    else return one;
+  }
+};
 
 // Scan while the tile sets are off (nearly every tile holds a changed
 // cluster): every item in id order, so that the item words and CSR rows are
@@ -440,23 +493,12 @@ __device__ inline int64_t seg_pos(const SegIndex* si, int32_t cap, int32_t p) {
   return int64_t(lo) * cap + (p - si->start[lo]);
 }
 
-// True (in every thread of the block) when round r applied no move: the
-// later rounds of the pass then apply nothing either and are skipped.
+// True (in every lane) when round r applied no move: the later rounds of the
+// pass then apply nothing either and are skipped.  Every wave reads the counters
+// itself, with its first loads: no barrier stands before the candidates.
 __device__ inline bool round_was_empty(const SweepArgs& a, int r) {
-  __shared__ int s_empty;
-  if (threadIdx.x < 64) {
-    int m = a.ctrl->mods[r][threadIdx.x];
-    for (int off = 32; off > 0; off >>= 1) m += __shfl_xor(m, off);
-    if (threadIdx.x == 0) s_empty = m == 0;
-  }
-  __syncthreads();
-  return s_empty != 0;
-}
-
-// True when round r lies past the pass's last round for the only mesh of the
-// context (a batch checks each candidate's mesh instead).
-__device__ inline bool past_last_round(const SweepArgs& a, int r) {
-  return !a.item_mesh && r >= pass_rounds(a.state[0]);
+  static_assert(kSlices == 64, "one slice per lane");
+  return __ballot(a.ctrl->mods[r][__lane_id()] != 0) == 0ull;
 }
 
 // Metric of the meshes a kernel instantiation sweeps: 0 isotropic, 1 QEM,
@@ -482,25 +524,43 @@ __device__ inline WalkCtl load_walk_ctl(const SweepArgs& a) {
   return w;
 }
 
+// A candidate entry: item, its label (a live candidate has not moved), its live
+// target (< 0: none) and the loop and round of its last evaluation.
+struct CandRec {
+  int32_t b, i, lab, since;
+};
+__device__ inline CandRec load_cand(const SweepArgs& a, int64_t e) {
+  return CandRec{a.cand_tgt[e], a.cand[e], a.cand_lab[e], a.cand_since[e]};
+}
+
+// f(valid, entry, record); first: this thread's record of its block's segment,
+// read by the kernel with its first loads (any value past the fill count).
 template <class F>
-__device__ inline void walk_candidates(const SweepArgs& a, const WalkCtl& w, SegIndex* si, F&& f) {
-  int32_t n, first, stride;
+__device__ inline void walk_candidates(const SweepArgs& a, const WalkCtl& w, SegIndex* si, const CandRec& first_rec,
+                                       F&& f) {
   if (w.by_seg) {  // block-uniform
-    n = w.n_own;
-    first = 0;
-    stride = kBlock;
-  } else {
-    load_seg_index(a.seg_cand, a.n_seg, si);
-    n = si->start[kMaxSeg];
-    first = blockIdx.x * kBlock;
-    stride = gridDim.x * kBlock;
+    const int64_t seg = int64_t(blockIdx.x) * a.cand_cap;
+    for (int32_t base = 0; base < w.n_own; base += kBlock) {
+      const int32_t k = base + int32_t(threadIdx.x);
+      const bool valid = k < w.n_own;
+      CandRec c = first_rec;
+      if (base > 0 && valid) c = load_cand(a, seg + k);
+      f(valid, seg + k, c);
+    }
+    return;
   }
-  const int64_t seg = int64_t(blockIdx.x) * a.cand_cap;
-  for (int32_t base = first; base < n; base += stride) {
+  load_seg_index(a.seg_cand, a.n_seg, si);
+  const int32_t n = si->start[kMaxSeg];
+  for (int32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {
     const int32_t k = base + int32_t(threadIdx.x);
+    const bool valid = k < n;
     int64_t e = 0;
-    if (k < n) e = w.by_seg ? seg + k : seg_pos(si, a.cand_cap, k);
-    f(k < n, e);
+    CandRec c{-1, 0, kNull, 0};
+    if (valid) {
+      e = seg_pos(si, a.cand_cap, k);
+      c = load_cand(a, e);
+    }
+    f(valid, e, c);
   }
 }
 
@@ -609,16 +669,11 @@ __device__ inline int wave_prefix(int v) {
 // nb / open) or a longer one (open targets found again by walking the row).
 enum PoolKind : int { kPoolNone = 0, kPoolShort = 1, kPoolLong = 2 };
 
-// Screen of a labelled item of a constrained QEM mesh for the pool: its kind
-// (kPoolNone when no target is open) and its number of solves.
-__device__ inline int pool_screen(const SweepView& v, int64_t i, int32_t lab, int connexity, int32_t* nb,
-                                  QemItem* s, uint32_t* open, int* ntask) {
+// Screen of a labelled item with a long row for the pool: its kind (kPoolNone
+// when no target is open) and its number of solves.
+__device__ inline int pool_screen_long(const SweepView& v, int64_t i, int32_t lab, int connexity, QemItem* s,
+                                       int* ntask) {
   *ntask = 0;
-  if (v.row_ptr[i + 1] - v.row_ptr[i] <= kRingCache) {
-    if (!qem_screen_short_row(v, i, lab, connexity, 1, nb, s, open)) return kPoolNone;
-    *ntask = 1 + __popc(*open);
-    return kPoolShort;
-  }
   if (!qem_screen(v, i, lab, connexity, 1, s)) return kPoolNone;
   int n = 1;
   for (int32_t k = qem_next_open(v, lab, *s, 1, s->r0 - 1); k < s->r1; k = qem_next_open(v, lab, *s, 1, k)) ++n;
@@ -651,7 +706,7 @@ __device__ inline void pool_post_long(const SweepView& v, QemPool* pool, int64_t
 // solves first (a wave posts at most kPoolTasks of them), so that the lanes
 // keep only the choice state across the solve steps; long-row owners post
 // after them what fits and the rest in later fills.
-template <bool kExtras>
+template <bool kExtras, bool kB>
 __device__ bool qem_pool_choose(const SweepArgs& a, const SweepView& v, QemPool* pool, int kind, int ntask,
                                 int64_t i, int32_t lab, int32_t m, const int32_t* nb, const QemItem& s,
                                 uint32_t open, int32_t* target_out) {
@@ -688,7 +743,7 @@ __device__ bool qem_pool_choose(const SweepArgs& a, const SweepView& v, QemPool*
       const bool solve = lane < total - base;
       const int ow = solve ? pool->owner[base + lane] : lane;
       const int64_t ti = __shfl(int32_t(i), ow);
-      const int32_t tm = __shfl(m, ow);
+      const int32_t tm = kB ? __shfl(m, ow) : 0;
       if (solve) {
         const int32_t tc = pool->cl[base + lane];
         const int32_t c = tc < 0 ? ~tc : tc;
@@ -759,56 +814,72 @@ __device__ inline void count_per_mesh(bool want, int32_t m, Counter&& counter) {
   }
 }
 
-// Evaluate (round 0) of item i (when valid): its best move (shared rule of
+// Evaluate (round 0) of item i (when valid): its best move (shared rules of
 // acvd_math.h) against the state at the pass start; a proposal registers its
 // round-0 accept key at both clusters and joins the block's candidate segment.
 // Every lane of the block calls it (the QEM solve pool is shared by the wave).
-template <int METRIC, bool kExtras>
-__device__ inline void eval_item(const SweepArgs& a, const SweepView& v, QemPool* pool, KeyAgg* agg, int64_t seg,
-                                 int32_t* s_n, bool valid, int32_t i) {
+// Bound by its chain of dependent loads: a short row's chain is item -> neighbour
+// ids, label -> neighbour labels, own cluster -> neighbour clusters, each step's
+// loads side by side (walked neighbour by neighbour it was three per neighbour).
+template <int METRIC, bool kExtras, bool kB>
+__device__ inline void eval_item(const SweepArgs& a, const SweepView& v, const MeshReader<kB>& mesh, QemPool* pool,
+                                 KeyAgg* agg, int64_t seg, int32_t* s_n, bool valid, int32_t i) {
   bool want = false;
-  int32_t lab = kNull, target = kNull, L = 0, m = 0;
+  int32_t lab = kNull, target = kNull, m = 0;
   int32_t nb[kRingCache];
+  MeshCtl mc{};
   QemItem s;
   uint32_t open = 0;
   int kind = kPoolNone, ntask = 0;
   if (valid) {
-    m = mesh_of_item(a, i);
-    const DevMesh& dm = a.meshes[m];
-    if (dm.metric == mesh_metric(METRIC)) {
-      const MeshState* st = &a.state[m];
-      L = st->loops;
+    m = mesh.of_item(i);
+    mc = mesh(m);
+    if (mc.metric == mesh_metric(METRIC)) {
+      int32_t nbr[kRingCache];
       lab = a.labels[i];
-      if (METRIC == 1 && lab != kNull && qem_mode(*st))
-        kind = pool_screen(v, i, lab, st->connexity, nb, &s, &open, &ntask);
-      else  // no FP64 solve: the null-item rule or the isotropic one
-        want = propose_item<METRIC == 1 ? 2 : METRIC>(v, i, lab, st->connexity, st->constrained, dm.level, dm.scales,
-                                                      &target);
+      const bool is_short = load_row8(a, i, nbr);
+      const float4 p = a.xw[i];
+      const bool qem = METRIC == 1 && mc.mode != 0;
+      if (lab != kNull && is_short) {
+        ShortItem t{p.x, p.y, p.z, p.w, 0, a.sizes[lab], a.ring_adj[i], a.geom[lab]};
+        const double Ta = qem ? a.T[lab] : 0.0;
+        t.deg = load_labels8(a, nbr, nb);
+        if (!qem) {  // no FP64 solve: the isotropic rule
+          want = iso_propose_short(v, t, lab, mc.connexity, nb, &target);
+        } else if (!is_anchor(v, i, lab) && qem_screen_short(v, t, lab, mc.connexity, Ta, 1, nb, &s, &open)) {
+          kind = kPoolShort;
+          ntask = 1 + __popc(open);
+        }
+      } else if (lab != kNull && qem) {
+        kind = pool_screen_long(v, i, lab, mc.connexity, &s, &ntask);
+      } else {  // the null-item rule, or the isotropic one over a long row
+        want = propose_item<METRIC == 1 ? 2 : METRIC>(v, i, lab, mc.connexity, mc.constrained, mc.level,
+                                                      a.meshes[m].scales, &target);
+      }
     }
   }
   if constexpr (METRIC == 1) {
     int32_t pt = kNull;
-    const bool r = qem_pool_choose<kExtras>(a, v, pool, kind, ntask, i, lab, m, nb, s, open, &pt);
+    const bool r = qem_pool_choose<kExtras, kB>(a, v, pool, kind, ntask, i, lab, m, nb, s, open, &pt);
     if (kind != kPoolNone) {
       want = r;
       target = pt;
     }
   }
   if (want) {
-    const DevMesh& dm = a.meshes[m];
-    const unsigned long long key = accept_key(dm.seed, L, 0, uint32_t(i - dm.item_off));
+    const unsigned long long key = accept_key(mc.seed, mc.loops, 0, uint32_t(i - mc.item_off));
     if (lab != kNull) keyagg_min(agg, lab, key);
     keyagg_min(agg, target, key);
-    a.cand_pass[i] = L;
-    a.tile_prop[a.item_tile[i]] = L;
+    a.cand_pass[i] = mc.loops;
+    a.tile_prop[a.item_tile[i]] = mc.loops;
   }
-  if (a.item_mesh) count_per_mesh(want, m, [&](int32_t mm) { return &a.state[mm].pass_props; });
+  if constexpr (kB) count_per_mesh(want, m, [&](int32_t mm) { return &a.state[mm].pass_props; });
   const int64_t e = seg_append(seg, s_n, want);
   if (want) {
     a.cand[e] = i;
     a.cand_lab[e] = lab;
     a.cand_tgt[e] = target;
-    a.cand_since[e] = L * kMatchRounds;
+    a.cand_since[e] = mc.loops * kMatchRounds;
   }
   keyagg_flush(agg, a.prio);
 }
@@ -816,12 +887,13 @@ __device__ inline void eval_item(const SweepArgs& a, const SweepView& v, QemPool
 // Evaluate the work list of the scan.  Block b owns segment b (capacity
 // cand_cap, count seg_cand[b]); the second launch of a mixed batch (append = 1)
 // continues the segments of the first.
-template <int METRIC, bool kExtras>
-__global__ __launch_bounds__(kBlock) void k_eval(SweepArgs a, int append) {
+template <int METRIC, bool kExtras, bool kB>
+__global__ __launch_bounds__(kBlock, METRIC == 1 ? 3 : 4) void k_eval(SweepArgs a, int append) {
   __shared__ WorkIndex wi;
   __shared__ KeyAgg agg;
   __shared__ QemPool pools[METRIC == 1 ? kBlock / 64 : 1];
   __shared__ int32_t s_n;
+  const MeshReader<kB> mesh(a);
   if (threadIdx.x == 0) s_n = append ? a.seg_cand[blockIdx.x] : 0;
   keyagg_clear(&agg);
   load_work_index(a.work_count, &wi);
@@ -832,7 +904,7 @@ __global__ __launch_bounds__(kBlock) void k_eval(SweepArgs a, int append) {
   for (int32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {
     const int32_t t = base + int32_t(threadIdx.x);
     const int32_t i = t < n ? work_entry(a, &wi, t) : 0;
-    eval_item<METRIC, kExtras>(a, v, pool, &agg, seg, &s_n, t < n, i);
+    eval_item<METRIC, kExtras, kB>(a, v, mesh, pool, &agg, seg, &s_n, t < n, i);
   }
   __syncthreads();
   if (threadIdx.x == 0) a.seg_cand[blockIdx.x] = s_n;
@@ -843,11 +915,12 @@ __global__ __launch_bounds__(kBlock) void k_eval(SweepArgs a, int append) {
 // evaluate in LDS and evaluates them.  The work list, its index of slice starts
 // and a launch go; what they give, an even share of the work items for every
 // block, counts only where the blocks have more than a step or two of them.
-template <int METRIC, bool kExtras>
-__global__ __launch_bounds__(kBlock) void k_scan_eval(SweepArgs a, int append) {
+template <int METRIC, bool kExtras, bool kB>
+__global__ __launch_bounds__(kBlock, METRIC == 1 ? 3 : 4) void k_scan_eval(SweepArgs a, int append) {
   __shared__ KeyAgg agg;
   __shared__ QemPool pools[METRIC == 1 ? kBlock / 64 : 1];
   __shared__ int32_t s_n, s_cnt[kBlock / 64], s_item[kBlock];
+  const MeshReader<kB> mesh(a);
   if (threadIdx.x == 0) s_n = append ? a.seg_cand[blockIdx.x] : 0;
   keyagg_clear(&agg);
   const SweepView v = make_view<kExtras>(a);
@@ -876,7 +949,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_eval(SweepArgs a, int append) {
     __syncthreads();
     if (n) {  // block-uniform
       const bool valid = int32_t(threadIdx.x) < n;
-      eval_item<METRIC, kExtras>(a, v, pool, &agg, seg, &s_n, valid, valid ? s_item[threadIdx.x] : 0);
+      eval_item<METRIC, kExtras, kB>(a, v, mesh, pool, &agg, seg, &s_n, valid, valid ? s_item[threadIdx.x] : 0);
     }
   }
   __syncthreads();
@@ -896,17 +969,17 @@ __device__ inline int block_sum(int v) {
   return tot;  // valid in thread 0
 }
 
-// Re-evaluation of candidate entry e (when valid) for round `round`; every
-// lane of the wave calls it (the QEM solve pool is shared by the wave).
-// reg(c, key) registers an accept key at cluster c.
-template <int METRIC, bool kExtras, bool kCount, class Reg>
-__device__ inline void reeval_entry(const SweepArgs& a, const SweepView& v, QemPool* pool, bool valid, int64_t e,
-                                    int round, Reg&& reg, int* n_live, int* n_stale, int* n_recheck) {
-  // the candidate record in one round trip
-  const int32_t b = valid ? a.cand_tgt[e] : -1;
-  const int32_t i_e = valid ? a.cand[e] : 0;
-  const int32_t lab_e = valid ? a.cand_lab[e] : kNull;
-  const int32_t since = valid ? a.cand_since[e] : 0;
+// Re-evaluation of candidate entry e (record c, when valid) for round `round`;
+// every lane of the wave calls it (the QEM solve pool is shared by the wave).
+// reg(c, key) registers an accept key at cluster c.  Two candidates in three are
+// stale, and the rounds wait on their chain of dependent loads: what a stale
+// candidate reads of its item and cluster is read with the clusters' round tags,
+// before it is known to be stale.
+template <int METRIC, bool kExtras, bool kB, bool kCount, class Reg>
+__device__ inline void reeval_entry(const SweepArgs& a, const SweepView& v, const MeshReader<kB>& mesh, QemPool* pool,
+                                    bool valid, int64_t e, const CandRec& c, int round, Reg&& reg, int* n_live,
+                                    int* n_stale, int* n_recheck) {
+  const int32_t b = valid ? c.b : -1;
   bool live = false, stale = false, use_pool = false, recheck = false;
   int32_t i = 0, lab = kNull, target = b, m = 0;
   unsigned long long key = 0;
@@ -915,37 +988,60 @@ __device__ inline void reeval_entry(const SweepArgs& a, const SweepView& v, QemP
   uint32_t open = 0;
   int kind = kPoolNone, ntask = 0;
   if (b >= 0) {
-    i = i_e;
-    lab = lab_e;  // a live candidate has not moved
-    m = mesh_of_item(a, i);
-    const DevMesh& dm = a.meshes[m];
-    const MeshState& st = a.state[m];
+    i = c.i;
+    lab = c.lab;
+    m = mesh.of_item(i);
+    const MeshCtl mc = mesh(m);
     // a mesh past its last round of the pass registers nothing (no move); a
-    // context of one mesh has left the kernel already (past_last_round)
-    if (dm.metric == mesh_metric(METRIC) && (!a.item_mesh || round < pass_rounds(st))) {
+    // context of one mesh has left the kernel already
+    if (mc.metric == mesh_metric(METRIC) && (!kB || round < mc.rounds)) {
+      const bool qem = METRIC == 1 && mc.mode != 0;
       const int32_t ra = lab != kNull ? a.cl_round[lab] : -1, rb = a.cl_round[b];
-      stale = ra >= since || rb >= since;
-      key = accept_key(dm.seed, st.loops, round, uint32_t(i - dm.item_off));
+      int32_t nbr[kRingCache];
+      const bool is_short = load_row8(a, i, nbr);
+      const float4 p = a.xw[i];
+      const int32_t la = lab != kNull ? lab : b;
+      ShortItem t{p.x, p.y, p.z, p.w, 0, a.sizes[la], a.ring_adj[i], a.geom[la]};
+      ClusterGeom gb{0.0, 0.0, 0.0, 0.0};
+      double Ta = 0.0;
+      if (METRIC == 1) Ta = a.T[la];
+      else gb = a.geom[b];
+      stale = ra >= c.since || rb >= c.since;
+      key = accept_key(mc.seed, mc.loops, round, uint32_t(i - mc.item_off));
       live = true;
       if (stale) {
-        a.cand_since[e] = st.loops * kMatchRounds + round;
+        a.cand_since[e] = mc.loops * kMatchRounds + round;
         target = kNull;
-        use_pool = METRIC == 1 && lab != kNull && qem_mode(st);
-        if (use_pool)
-          kind = pool_screen(v, i, lab, st.connexity, nb, &s, &open, &ntask);
-        else if (lab != kNull) {  // the isotropic rule: the move itself is checked again
+        use_pool = qem && lab != kNull;
+        if (lab != kNull && is_short) {
+          t.deg = load_labels8(a, nbr, nb);
+          if (qem) {
+            if (!is_anchor(v, i, lab) && qem_screen_short(v, t, lab, mc.connexity, Ta, 1, nb, &s, &open)) {
+              kind = kPoolShort;
+              ntask = 1 + __popc(open);
+            }
+          } else {  // the isotropic rule: the move itself is checked again
+            if (METRIC == 1) gb = a.geom[b];
+            target = b;
+            recheck = true;
+            live = iso_recheck_short(v, t, lab, b, mc.connexity, nb, gb);
+          }
+        } else if (use_pool) {
+          kind = pool_screen_long(v, i, lab, mc.connexity, &s, &ntask);
+        } else if (lab != kNull) {
           target = b;
           recheck = true;
-          live = iso_recheck(v, i, lab, b, st.connexity);
-        } else  // the null-item rule
-          live = propose_item<METRIC == 1 ? 2 : METRIC>(v, i, lab, st.connexity, st.constrained, dm.level,
-                                                        dm.scales, &target);
+          live = iso_recheck(v, i, lab, b, mc.connexity);
+        } else {  // the null-item rule
+          live = propose_item<METRIC == 1 ? 2 : METRIC>(v, i, lab, mc.connexity, mc.constrained, mc.level,
+                                                        a.meshes[m].scales, &target);
+        }
       }
     }
   }
   if constexpr (METRIC == 1) {
     int32_t pt = kNull;
-    const bool r = qem_pool_choose<kExtras>(a, v, pool, kind, ntask, i, lab, m, nb, s, open, &pt);
+    const bool r = qem_pool_choose<kExtras, kB>(a, v, pool, kind, ntask, i, lab, m, nb, s, open, &pt);
     if (use_pool) {
       live = r;
       target = pt;
@@ -968,24 +1064,32 @@ __device__ inline void reeval_entry(const SweepArgs& a, const SweepView& v, QemP
 // against the state left by round r-1: it registers its round-r key with its
 // (possibly new) target or is dropped (-3).  The others keep their move, whose
 // dE depends only on the two unchanged clusters, and register it again.
+// A short list (one segment per block) registers straight at the global keys:
+// its few keys are not worth the LDS table's barriers.
 // kCount: count the registered and re-evaluated candidates (timed runs).
-template <int METRIC, bool kExtras, bool kCount>
-__global__ __launch_bounds__(kBlock) void k_reeval(SweepArgs a, int round) {
+template <int METRIC, bool kExtras, bool kB, bool kCount>
+__global__ __launch_bounds__(kBlock, METRIC == 1 ? 3 : 4) void k_reeval(SweepArgs a, int round) {
   __shared__ KeyAgg agg;
   __shared__ SegIndex si;
   __shared__ QemPool pools[METRIC == 1 ? kBlock / 64 : 1];
   const WalkCtl w = load_walk_ctl(a);
-  const bool past = past_last_round(a, round);
-  keyagg_clear(&agg);  // made visible by the barrier in round_was_empty
-  if (round_was_empty(a, round - 1) || past) return;
+  const CandRec rec = load_cand(a, int64_t(blockIdx.x) * a.cand_cap + threadIdx.x);
+  const MeshReader<kB> mesh(a);
+  const bool empty = round_was_empty(a, round - 1);
+  if (empty || (!kB && round >= mesh.one.rounds)) return;
   const SweepView v = make_view<kExtras>(a);
   QemPool* pool = &pools[METRIC == 1 ? threadIdx.x >> 6 : 0];
   int n_live = 0, n_stale = 0, n_recheck = 0;
-  walk_candidates(a, w, &si, [&](bool valid, int64_t e) {
-    reeval_entry<METRIC, kExtras, kCount>(
-        a, v, pool, valid, e, round, [&](int32_t c, unsigned long long key) { keyagg_min(&agg, c, key); },
+  if (!w.by_seg) keyagg_clear(&agg);  // made visible by the index's barrier
+  walk_candidates(a, w, &si, rec, [&](bool valid, int64_t e, const CandRec& c) {
+    reeval_entry<METRIC, kExtras, kB, kCount>(
+        a, v, mesh, pool, valid, e, c, round,
+        [&](int32_t cl, unsigned long long key) {
+          if (w.by_seg) atomicMin(&a.prio[cl], key);
+          else keyagg_min(&agg, cl, key);
+        },
         &n_live, &n_stale, &n_recheck);
-    keyagg_flush(&agg, a.prio);
+    if (!w.by_seg) keyagg_flush(&agg, a.prio);
   });
   // candidates registered and re-evaluated in this round (statistics of the
   // timed runs: the block sums cost a few barriers per round)
@@ -1043,25 +1147,22 @@ struct DeriveList {
 
 // Apply of candidate entry e (when valid) in round `round`; every lane of the
 // wave calls it.  Returns true when the candidate moved (item *moved_item).
-template <bool kSolve, bool kExtras>
-__device__ inline bool apply_entry(const SweepArgs& a, DeriveList* dl, bool valid, int64_t e, int round,
-                                   int32_t* moved_item) {
+template <bool kSolve, bool kExtras, bool kB>
+__device__ inline bool apply_entry(const SweepArgs& a, const MeshReader<kB>& mesh, DeriveList* dl, bool valid,
+                                   int64_t e, const CandRec& c, int round, int32_t* moved_item) {
   bool win = false;
   int64_t i = 0;
   int32_t lab = kNull;
-  // the candidate record in one round trip
-  const int32_t b = valid ? a.cand_tgt[e] : -1;
-  const int32_t i_e = valid ? a.cand[e] : 0;
-  const int32_t lab_e = valid ? a.cand_lab[e] : kNull;
-  int32_t mesh = 0;
+  const int32_t b = valid ? c.b : -1;
+  int32_t m = 0;
   if (b >= 0) {
-    i = i_e;
-    lab = lab_e;
-    const int m = mesh = mesh_of_item(a, i);
-    const MeshState* st = &a.state[m];
-    const int32_t L = st->loops;
+    i = c.i;
+    lab = c.lab;
+    m = mesh.of_item(i);
+    const MeshCtl mc = mesh(m);
+    const int32_t L = mc.loops;
     const DevMesh& dm = a.meshes[m];
-    const unsigned long long key = accept_key(dm.seed, L, round, uint32_t(i - dm.item_off));
+    const unsigned long long key = accept_key(mc.seed, L, round, uint32_t(i - mc.item_off));
     const unsigned long long pa = lab != kNull ? a.prio[lab] : key, pb = a.prio[b];
     win = pa == key && pb == key;
     if (win) {
@@ -1107,7 +1208,7 @@ __device__ inline bool apply_entry(const SweepArgs& a, DeriveList* dl, bool vali
       }
     }
   }
-  if (a.item_mesh) count_per_mesh(win, mesh, [&](int32_t mm) { return &a.state[mm].pass_mods; });
+  if constexpr (kB) count_per_mesh(win, m, [&](int32_t mm) { return &a.state[mm].pass_mods; });
   if constexpr (kSolve) {
     const int cnt = win ? (lab != kNull ? 2 : 1) : 0;
     const int inc = wave_prefix(cnt);
@@ -1123,8 +1224,8 @@ __device__ inline bool apply_entry(const SweepArgs& a, DeriveList* dl, bool vali
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     for (int k = __lane_id(); k < total; k += 64) {
       const int64_t c = dl->cl[k];
-      const int m = mesh_of_cluster(a, c);
-      derive_cluster<kExtras>(a, c, a.meshes[m], a.state[m].constrained, true);
+      const int mm = kB ? mesh_of_cluster(a, c) : 0;
+      derive_cluster<kExtras>(a, c, a.meshes[mm], mesh(mm).constrained, true);
     }
     wave_lds_sync();
   }
@@ -1132,23 +1233,25 @@ __device__ inline bool apply_entry(const SweepArgs& a, DeriveList* dl, bool vali
   return win;
 }
 
-template <bool kSolve, bool kExtras>
+template <bool kSolve, bool kExtras, bool kB>
 __global__ __launch_bounds__(kBlock) void k_apply(SweepArgs a, int round) {
   __shared__ int32_t s_moved;
   __shared__ SegIndex si;
   __shared__ DeriveList dlist[kSolve ? kBlock / 64 : 1];
   const int64_t mseg = int64_t(blockIdx.x) * a.cand_cap;
   const WalkCtl w = load_walk_ctl(a);
+  const CandRec rec = load_cand(a, mseg + threadIdx.x);
+  const MeshReader<kB> mesh(a);
   const int32_t moved0 = round == 0 ? 0 : a.seg_moved[blockIdx.x];
-  const bool past = past_last_round(a, round);
-  if (round > 0 && (round_was_empty(a, round - 1) || past)) return;
+  const bool empty = round > 0 && round_was_empty(a, round - 1);
+  if (empty || (!kB && round >= mesh.one.rounds)) return;
   if (threadIdx.x == 0) s_moved = moved0;
   __syncthreads();
   DeriveList* dl = &dlist[kSolve ? threadIdx.x >> 6 : 0];
   int mods = 0;
-  walk_candidates(a, w, &si, [&](bool valid, int64_t e) {
+  walk_candidates(a, w, &si, rec, [&](bool valid, int64_t e, const CandRec& c) {
     int32_t i;
-    const bool win = apply_entry<kSolve, kExtras>(a, dl, valid, e, round, &i);
+    const bool win = apply_entry<kSolve, kExtras, kB>(a, mesh, dl, valid, e, c, round, &i);
     mods += win;
     const int64_t em = seg_append(mseg, &s_moved, win);
     if (em >= 0) a.moved[em] = i;
@@ -1627,46 +1730,52 @@ hipError_t launch_scan(hipStream_t s, const SweepArgs& a, bool tiles) {
 // One evaluate block per candidate segment: block b writes segment b's count.
 // qem_unconstrained: no QEM mesh is constrained (the QEM meshes take the
 // isotropic rule, METRIC 2).
-// The kernels come in two builds: with the anchor and freeze tests (some mesh
-// has fixed or frozen clusters) and without them.
-template <bool kX>
+// The kernels come in three builds: with the anchor and freeze tests (some mesh
+// has fixed or frozen clusters), without them, and without them for a context of
+// one mesh (kB = false: no mesh lookups).
+template <bool kX, bool kB>
 void launch_eval_x(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained) {
-  if (any_iso) hipLaunchKernelGGL((k_eval<0, kX>), dim3(unsigned(a.n_seg)), dim3(kBlock), 0, s, a, 0);
-  if (any_qem && qem_unconstrained)
-    hipLaunchKernelGGL((k_eval<2, kX>), dim3(unsigned(a.n_seg)), dim3(kBlock), 0, s, a, any_iso ? 1 : 0);
-  else if (any_qem)
-    hipLaunchKernelGGL((k_eval<1, kX>), dim3(unsigned(a.n_seg)), dim3(kBlock), 0, s, a, any_iso ? 1 : 0);
+  const dim3 g(unsigned(a.n_seg)), b(kBlock);
+  if (any_iso) hipLaunchKernelGGL((k_eval<0, kX, kB>), g, b, 0, s, a, 0);
+  if (any_qem && qem_unconstrained) hipLaunchKernelGGL((k_eval<2, kX, kB>), g, b, 0, s, a, any_iso ? 1 : 0);
+  else if (any_qem) hipLaunchKernelGGL((k_eval<1, kX, kB>), g, b, 0, s, a, any_iso ? 1 : 0);
 }
 
 hipError_t launch_eval(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained) {
-  if (a.anchor || a.frozen) launch_eval_x<true>(s, a, any_iso, any_qem, qem_unconstrained);
-  else launch_eval_x<false>(s, a, any_iso, any_qem, qem_unconstrained);
+  if (a.anchor || a.frozen) launch_eval_x<true, true>(s, a, any_iso, any_qem, qem_unconstrained);
+  else if (a.item_mesh) launch_eval_x<false, true>(s, a, any_iso, any_qem, qem_unconstrained);
+  else launch_eval_x<false, false>(s, a, any_iso, any_qem, qem_unconstrained);
   return hipGetLastError();
 }
 
-template <bool kX>
+template <bool kX, bool kB>
 void launch_scan_eval_x(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained) {
   const dim3 g(unsigned(a.n_seg)), b(kBlock);
-  if (any_iso) hipLaunchKernelGGL((k_scan_eval<0, kX>), g, b, 0, s, a, 0);
-  if (any_qem && qem_unconstrained) hipLaunchKernelGGL((k_scan_eval<2, kX>), g, b, 0, s, a, any_iso ? 1 : 0);
-  else if (any_qem) hipLaunchKernelGGL((k_scan_eval<1, kX>), g, b, 0, s, a, any_iso ? 1 : 0);
+  if (any_iso) hipLaunchKernelGGL((k_scan_eval<0, kX, kB>), g, b, 0, s, a, 0);
+  if (any_qem && qem_unconstrained) hipLaunchKernelGGL((k_scan_eval<2, kX, kB>), g, b, 0, s, a, any_iso ? 1 : 0);
+  else if (any_qem) hipLaunchKernelGGL((k_scan_eval<1, kX, kB>), g, b, 0, s, a, any_iso ? 1 : 0);
 }
 
 hipError_t launch_scan_eval(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained) {
-  if (a.anchor || a.frozen) launch_scan_eval_x<true>(s, a, any_iso, any_qem, qem_unconstrained);
-  else launch_scan_eval_x<false>(s, a, any_iso, any_qem, qem_unconstrained);
+  if (a.anchor || a.frozen) launch_scan_eval_x<true, true>(s, a, any_iso, any_qem, qem_unconstrained);
+  else if (a.item_mesh) launch_scan_eval_x<false, true>(s, a, any_iso, any_qem, qem_unconstrained);
+  else launch_scan_eval_x<false, false>(s, a, any_iso, any_qem, qem_unconstrained);
   return hipGetLastError();
 }
 
 // One apply block per candidate segment (its moved segment has the same
 // index).  constrained: some mesh is constrained (derives may need a solve).
-hipError_t launch_apply(hipStream_t s, const SweepArgs& a, int round, bool constrained) {
+template <bool kX, bool kB>
+void launch_apply_x(hipStream_t s, const SweepArgs& a, int round, bool constrained) {
   const dim3 g(unsigned(a.n_seg)), b(kBlock);
-  const bool x = a.anchor || a.frozen;
-  if (constrained && x) hipLaunchKernelGGL((k_apply<true, true>), g, b, 0, s, a, round);
-  else if (constrained) hipLaunchKernelGGL((k_apply<true, false>), g, b, 0, s, a, round);
-  else if (x) hipLaunchKernelGGL((k_apply<false, true>), g, b, 0, s, a, round);
-  else hipLaunchKernelGGL((k_apply<false, false>), g, b, 0, s, a, round);
+  if (constrained) hipLaunchKernelGGL((k_apply<true, kX, kB>), g, b, 0, s, a, round);
+  else hipLaunchKernelGGL((k_apply<false, kX, kB>), g, b, 0, s, a, round);
+}
+
+hipError_t launch_apply(hipStream_t s, const SweepArgs& a, int round, bool constrained) {
+  if (a.anchor || a.frozen) launch_apply_x<true, true>(s, a, round, constrained);
+  else if (a.item_mesh) launch_apply_x<false, true>(s, a, round, constrained);
+  else launch_apply_x<false, false>(s, a, round, constrained);
   return hipGetLastError();
 }
 
@@ -1675,22 +1784,23 @@ hipError_t launch_tile_update(hipStream_t s, const SweepArgs& a) {
   return hipGetLastError();
 }
 
-template <bool kX, bool kC>
+template <bool kX, bool kB, bool kC>
 void launch_reeval_x(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained,
                      int round) {
   const dim3 g(unsigned(a.n_seg)), b(kBlock);
-  if (any_iso) hipLaunchKernelGGL((k_reeval<0, kX, kC>), g, b, 0, s, a, round);
-  if (any_qem && qem_unconstrained) hipLaunchKernelGGL((k_reeval<2, kX, kC>), g, b, 0, s, a, round);
-  else if (any_qem) hipLaunchKernelGGL((k_reeval<1, kX, kC>), g, b, 0, s, a, round);
+  if (any_iso) hipLaunchKernelGGL((k_reeval<0, kX, kB, kC>), g, b, 0, s, a, round);
+  if (any_qem && qem_unconstrained) hipLaunchKernelGGL((k_reeval<2, kX, kB, kC>), g, b, 0, s, a, round);
+  else if (any_qem) hipLaunchKernelGGL((k_reeval<1, kX, kB, kC>), g, b, 0, s, a, round);
 }
 
 hipError_t launch_reeval(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained,
                          int round) {
   const bool x = a.anchor || a.frozen, c = a.count_rounds != 0;
-  if (x && c) launch_reeval_x<true, true>(s, a, any_iso, any_qem, qem_unconstrained, round);
-  else if (x) launch_reeval_x<true, false>(s, a, any_iso, any_qem, qem_unconstrained, round);
-  else if (c) launch_reeval_x<false, true>(s, a, any_iso, any_qem, qem_unconstrained, round);
-  else launch_reeval_x<false, false>(s, a, any_iso, any_qem, qem_unconstrained, round);
+  if (x && c) launch_reeval_x<true, true, true>(s, a, any_iso, any_qem, qem_unconstrained, round);
+  else if (x) launch_reeval_x<true, true, false>(s, a, any_iso, any_qem, qem_unconstrained, round);
+  else if (c) launch_reeval_x<false, true, true>(s, a, any_iso, any_qem, qem_unconstrained, round);
+  else if (a.item_mesh) launch_reeval_x<false, true, false>(s, a, any_iso, any_qem, qem_unconstrained, round);
+  else launch_reeval_x<false, false, false>(s, a, any_iso, any_qem, qem_unconstrained, round);
   return hipGetLastError();
 }
 

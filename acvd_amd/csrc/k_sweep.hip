@@ -1233,14 +1233,93 @@ __device__ inline bool apply_entry(const SweepArgs& a, const MeshReader<kB>& mes
   return win;
 }
 
+// Apply of a short list (one segment per block) whose derives may need a solve:
+// two lanes per candidate, one for the cluster it leaves (side 0) and one for the
+// cluster it joins.  Each lane updates and derives its own cluster from registers:
+// no accumulator store is waited for and read back, and what a winner needs is
+// read with the keys that say whether it wins (a short list's losers cost little).
+// Returns true on both lanes of a candidate that moves.
+template <bool kExtras, bool kB>
+__device__ inline bool apply_pair(const SweepArgs& a, const MeshReader<kB>& mesh, bool valid, int64_t e,
+                                  const CandRec& rec, int round) {
+  const int side = threadIdx.x & 1;
+  const bool live = valid && rec.b >= 0;
+  const int32_t c = side ? rec.b : rec.lab;
+  const bool has = live && c != kNull;
+  bool ok = live;
+  int32_t m = 0, size = 0;
+  MeshCtl mc{};
+  float4 p = make_float4(0.f, 0.f, 0.f, 0.f);
+  float q[10];
+  unsigned long long ws[4], q10[10];
+  double V0[9];
+  if (live) {
+    m = mesh.of_item(rec.i);
+    mc = mesh(m);
+  }
+  if (has) {
+    const unsigned long long key = a.prio[c];
+    size = a.sizes[c];
+    p = a.xw[rec.i];
+    for (int k = 0; k < 4; ++k) ws[k] = a.acc_ws[4 * int64_t(c) + k];
+    if (mc.metric == 1) {
+      for (int k = 0; k < 10; ++k) q[k] = a.q[10 * int64_t(rec.i) + k];
+      for (int k = 0; k < 10; ++k) q10[k] = a.acc_q[10 * int64_t(c) + k];
+      for (int k = 0; k < 9; ++k) V0[k] = a.evec[9 * int64_t(c) + k];
+    }
+    ok = key == accept_key(mc.seed, mc.loops, round, uint32_t(rec.i - mc.item_off));
+  }
+  const bool other = __shfl_xor(int(ok), 1) != 0;  // every lane takes part
+  const bool win = live && ok && other;
+  if (win && side) {
+    a.labels[rec.i] = rec.b;
+    a.cand_tgt[e] = -3;
+  }
+  if (win && has) {  // exclusive owner of cluster c for this round
+    const DevMesh& dm = a.meshes[m];
+    const Scales sc = dm.scales;
+    const unsigned long long d[4] = {(unsigned long long)fix_w(p.w, sc), (unsigned long long)fix_s(p.w, p.x, sc),
+                                     (unsigned long long)fix_s(p.w, p.y, sc), (unsigned long long)fix_s(p.w, p.z, sc)};
+    for (int k = 0; k < 4; ++k) {
+      ws[k] = side ? ws[k] + d[k] : ws[k] - d[k];
+      a.acc_ws[4 * int64_t(c) + k] = ws[k];
+    }
+    a.sizes[c] = side ? size + 1 : size - 1;
+    a.stamp[c] = mc.loops;
+    a.cl_round[c] = mc.loops * kMatchRounds + round;
+    const ClusterGeom g = geom_from_fixed(int64_t(ws[0]), int64_t(ws[1]), int64_t(ws[2]), int64_t(ws[3]), sc);
+    a.geom[c] = g;
+    if (mc.metric == 1) {
+      int64_t Q[10];
+      for (int k = 0; k < 10; ++k) {
+        const unsigned long long iq = (unsigned long long)fix_q(q[k], sc);
+        q10[k] = side ? q10[k] + iq : q10[k] - iq;
+        a.acc_q[10 * int64_t(c) + k] = q10[k];
+        Q[k] = int64_t(q10[k]);
+      }
+      double T = 0.0;
+      const int32_t an = (kExtras && a.anchor) ? a.anchor[c] : -1;
+      if (an >= 0) {
+        const float4 x = a.xw[an];
+        T = anchored_T(g, AnchorPos{double(x.x), double(x.y), double(x.z), true});
+      } else if (mc.constrained) {
+        T = qem_T_from_fixed(Q, g, sc, dm.level, nullptr, V0, a.evec + 9 * int64_t(c));
+      }
+      a.T[c] = T;
+    }
+  }
+  if constexpr (kB) count_per_mesh(win && side, m, [&](int32_t mm) { return &a.state[mm].pass_mods; });
+  return win;
+}
+
 template <bool kSolve, bool kExtras, bool kB>
-__global__ __launch_bounds__(kBlock) void k_apply(SweepArgs a, int round) {
+__global__ __launch_bounds__(kBlock, kSolve ? 3 : 4) void k_apply(SweepArgs a, int round) {
   __shared__ int32_t s_moved;
   __shared__ SegIndex si;
   __shared__ DeriveList dlist[kSolve ? kBlock / 64 : 1];
   const int64_t mseg = int64_t(blockIdx.x) * a.cand_cap;
   const WalkCtl w = load_walk_ctl(a);
-  const CandRec rec = load_cand(a, mseg + threadIdx.x);
+  const CandRec rec = load_cand(a, mseg + (kSolve ? threadIdx.x >> 1 : threadIdx.x));
   const MeshReader<kB> mesh(a);
   const int32_t moved0 = round == 0 ? 0 : a.seg_moved[blockIdx.x];
   const bool empty = round > 0 && round_was_empty(a, round - 1);
@@ -1249,13 +1328,26 @@ __global__ __launch_bounds__(kBlock) void k_apply(SweepArgs a, int round) {
   __syncthreads();
   DeriveList* dl = &dlist[kSolve ? threadIdx.x >> 6 : 0];
   int mods = 0;
-  walk_candidates(a, w, &si, rec, [&](bool valid, int64_t e, const CandRec& c) {
-    int32_t i;
-    const bool win = apply_entry<kSolve, kExtras, kB>(a, mesh, dl, valid, e, c, round, &i);
-    mods += win;
-    const int64_t em = seg_append(mseg, &s_moved, win);
-    if (em >= 0) a.moved[em] = i;
-  });
+  if (kSolve && w.by_seg) {  // block-uniform
+    for (int32_t base = 0; base < w.n_own; base += kBlock / 2) {
+      const int32_t k = base + int32_t(threadIdx.x >> 1);
+      const bool valid = k < w.n_own;
+      CandRec c = rec;
+      if (base > 0 && valid) c = load_cand(a, mseg + k);
+      const bool won = apply_pair<kExtras, kB>(a, mesh, valid, mseg + k, c, round) && (threadIdx.x & 1);
+      mods += won;
+      const int64_t em = seg_append(mseg, &s_moved, won);
+      if (em >= 0) a.moved[em] = c.i;
+    }
+  } else {
+    walk_candidates(a, w, &si, rec, [&](bool valid, int64_t e, const CandRec& c) {
+      int32_t i;
+      const bool win = apply_entry<kSolve, kExtras, kB>(a, mesh, dl, valid, e, c, round, &i);
+      mods += win;
+      const int64_t em = seg_append(mseg, &s_moved, win);
+      if (em >= 0) a.moved[em] = i;
+    });
+  }
   const int tm = block_sum(mods);  // synchronises the block
   if (threadIdx.x == 0) {
     a.seg_moved[blockIdx.x] = s_moved;

@@ -24,13 +24,13 @@ constexpr int kSlices = 64;
 constexpr int kWorkSlices = 2048;
 // Upper bound of the block-owned segments (= evaluate / apply grid).
 constexpr int kMaxSeg = 2048;
-// Segments (evaluate / accept-round grid) of a large context: 4.5 blocks per
-// CU of the 256.  The round kernels fit 3 to 8 blocks per CU (VGPRs and LDS),
-// so a larger grid runs their dependent loads in a further wave of blocks.
-// QEM torus of 8.39M vertices, K = 100k, to convergence: 2048 blocks
-// 260.7 ms, 1536 245.0, 1280 243.8, 1024 245.4, 768 245.1, 512 261.1; with
-// the later kernels 1408 241.2, 1280 241.2-241.6, 1152 239.5.
-constexpr int kSweepSegs = 1152;
+// Segments (evaluate / accept-round grid) of a large context: 3 blocks per CU of
+// the 256, what the QEM kernels' registers allow, so that no block waits for
+// another to end.  To convergence at 1152 / 1024 / 768 / 512 / 384 / 256: QEM
+// torus of 8.39M vertices, K = 100k 227.6 / 227.3 / 223.6 / 236.5 / 253.6 /
+// 277.6 ms; QEM cube of 960,002 20.2 / 20.1 / 19.4 / 19.4 / 19.5 / 20.0; QEM torus
+// of 503,503 37.4 / 37.3 / 36.9 / 37.0 / 37.6 / 39.2.
+constexpr int kSweepSegs = 768;
 static_assert(kSweepSegs <= kMaxSeg, "segment index bound");
 // Candidate lists of at most this many proposals (last pass) are walked one
 // segment per block, longer ones evenly through an index of the segments.

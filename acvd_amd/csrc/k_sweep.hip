@@ -505,6 +505,34 @@ __device__ inline bool round_was_empty(const SweepArgs& a, int r) {
 // 2 QEM while unconstrained (isotropic rule, no FP64 solves compiled in).
 constexpr int mesh_metric(int kernel_metric) { return kernel_metric == 2 ? 1 : kernel_metric; }
 
+// Positions 0..n-1 of a list over the whole grid, one per thread and step (every
+// thread of the block takes every step): for (base = w.first; base < n; base +=
+// w.stride), thread position base + w.off when w.valid(base).  A list of fewer
+// positions than kSpread blocks have threads is spread evenly over those blocks
+// and their waves instead of filling the first ones: the step's time is its chain
+// of loads and, for the QEM rule, the solves of its busiest wave.  One block per CU:
+// over more of them a block's key table merges fewer keys and more blocks start.
+// To convergence, not spread / 128 / 256 / 512 / 768 / 1152 blocks: QEM torus of
+// 8.39M vertices 243.9 / 241.7 / 240.4 / 242.1 / 245.8 / 257.4 ms, of 260,533 32.9 /
+// 32.3 / 31.6 / 32.4 / 33.0 / 35.4.
+constexpr int32_t kSpread = 256;
+struct EvenWalk {
+  int32_t n, first, stride, off;
+  bool mine;
+  __device__ explicit EvenWalk(int32_t count) : n(count) {
+    const int32_t grid = int32_t(gridDim.x);
+    const int32_t blocks = grid < kSpread ? grid : kSpread;
+    const bool full = n >= blocks * kBlock;  // block-uniform
+    const int32_t per = full ? kBlock : (n + blocks - 1) / blocks;  // positions per block and step, then per wave
+    const int32_t wave = (per + kBlock / 64 - 1) / (kBlock / 64);
+    first = int32_t(blockIdx.x) * per;
+    stride = full ? grid * kBlock : n;  // a spread list takes one step
+    off = int32_t(threadIdx.x >> 6) * wave + __lane_id();
+    mine = int32_t(__lane_id()) < wave && off < per;
+  }
+  __device__ bool valid(int32_t base) const { return mine && base + off < n; }
+};
+
 // Walks the candidate list, calling f(valid, entry) for one position per
 // thread per step (every thread of the block takes part in every step).  A
 // long list (last pass's proposals above kSegWalkMax) is walked evenly by all
@@ -550,14 +578,13 @@ __device__ inline void walk_candidates(const SweepArgs& a, const WalkCtl& w, Seg
     return;
   }
   load_seg_index(a.seg_cand, a.n_seg, si);
-  const int32_t n = si->start[kMaxSeg];
-  for (int32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {
-    const int32_t k = base + int32_t(threadIdx.x);
-    const bool valid = k < n;
+  const EvenWalk ew(si->start[kMaxSeg]);
+  for (int32_t base = ew.first; base < ew.n; base += ew.stride) {
+    const bool valid = ew.valid(base);
     int64_t e = 0;
     CandRec c{-1, 0, kNull, 0};
     if (valid) {
-      e = seg_pos(si, a.cand_cap, k);
+      e = seg_pos(si, a.cand_cap, base + ew.off);
       c = load_cand(a, e);
     }
     f(valid, e, c);
@@ -823,7 +850,7 @@ __device__ inline void count_per_mesh(bool want, int32_t m, Counter&& counter) {
 // loads side by side (walked neighbour by neighbour it was three per neighbour).
 template <int METRIC, bool kExtras, bool kB>
 __device__ inline void eval_item(const SweepArgs& a, const SweepView& v, const MeshReader<kB>& mesh, QemPool* pool,
-                                 KeyAgg* agg, int64_t seg, int32_t* s_n, bool valid, int32_t i) {
+                                 KeyAgg* agg, bool direct, int64_t seg, int32_t* s_n, bool valid, int32_t i) {
   bool want = false;
   int32_t lab = kNull, target = kNull, m = 0;
   int32_t nb[kRingCache];
@@ -868,8 +895,13 @@ __device__ inline void eval_item(const SweepArgs& a, const SweepView& v, const M
   }
   if (want) {
     const unsigned long long key = accept_key(mc.seed, mc.loops, 0, uint32_t(i - mc.item_off));
-    if (lab != kNull) keyagg_min(agg, lab, key);
-    keyagg_min(agg, target, key);
+    if (direct) {
+      if (lab != kNull) atomicMin(&a.prio[lab], key);
+      atomicMin(&a.prio[target], key);
+    } else {
+      if (lab != kNull) keyagg_min(agg, lab, key);
+      keyagg_min(agg, target, key);
+    }
     a.cand_pass[i] = mc.loops;
     a.tile_prop[a.item_tile[i]] = mc.loops;
   }
@@ -881,7 +913,7 @@ __device__ inline void eval_item(const SweepArgs& a, const SweepView& v, const M
     a.cand_tgt[e] = target;
     a.cand_since[e] = mc.loops * kMatchRounds;
   }
-  keyagg_flush(agg, a.prio);
+  if (!direct) keyagg_flush(agg, a.prio);
 }
 
 // Evaluate the work list of the scan.  Block b owns segment b (capacity
@@ -901,10 +933,12 @@ __global__ __launch_bounds__(kBlock, METRIC == 1 ? 3 : 4) void k_eval(SweepArgs 
   const SweepView v = make_view<kExtras>(a);
   const int64_t seg = int64_t(blockIdx.x) * a.cand_cap;
   QemPool* pool = &pools[METRIC == 1 ? threadIdx.x >> 6 : 0];
-  for (int32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {
-    const int32_t t = base + int32_t(threadIdx.x);
-    const int32_t i = t < n ? work_entry(a, &wi, t) : 0;
-    eval_item<METRIC, kExtras, kB>(a, v, mesh, pool, &agg, seg, &s_n, t < n, i);
+  const bool direct = n <= kSegWalkMax;  // few keys are not worth the table's barriers
+  const EvenWalk ew(n);
+  for (int32_t base = ew.first; base < n; base += ew.stride) {
+    const bool valid = ew.valid(base);
+    const int32_t i = valid ? work_entry(a, &wi, base + ew.off) : 0;
+    eval_item<METRIC, kExtras, kB>(a, v, mesh, pool, &agg, direct, seg, &s_n, valid, i);
   }
   __syncthreads();
   if (threadIdx.x == 0) a.seg_cand[blockIdx.x] = s_n;
@@ -948,8 +982,11 @@ __global__ __launch_bounds__(kBlock, METRIC == 1 ? 3 : 4) void k_scan_eval(Sweep
     if (n && threadIdx.x == 0) atomicAdd(&a.work_count[blockIdx.x % kWorkSlices], n);  // items evaluated
     __syncthreads();
     if (n) {  // block-uniform
-      const bool valid = int32_t(threadIdx.x) < n;
-      eval_item<METRIC, kExtras, kB>(a, v, mesh, pool, &agg, seg, &s_n, valid, valid ? s_item[threadIdx.x] : 0);
+      // spread over the waves (walk_even)
+      const int32_t per = (n + kBlock / 64 - 1) / (kBlock / 64);
+      const int32_t off = w * per + lane;
+      const bool valid = lane < per && off < n;
+      eval_item<METRIC, kExtras, kB>(a, v, mesh, pool, &agg, false, seg, &s_n, valid, valid ? s_item[off] : 0);
     }
   }
   __syncthreads();
@@ -1059,6 +1096,11 @@ __device__ inline void reeval_entry(const SweepArgs& a, const SweepView& v, cons
   }
 }
 
+// Measured and left out: 4 waves per SIMD for the QEM kernels (128 registers):
+// 237.3 against 236.7 ms on the 8.39M-vertex torus; the item read only once it is
+// known to be stale in long lists: 238.1; a look at the global key before the
+// table's atomicMin: 255.4 (it costs what the atomic does).
+//
 // Re-evaluate (round r > 0): a live candidate (cand_tgt >= 0) whose own
 // cluster or target moved since its last evaluation is evaluated again
 // against the state left by round r-1: it registers its round-r key with its

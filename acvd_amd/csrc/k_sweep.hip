@@ -47,61 +47,139 @@ __global__ void k_zero_clusters(SweepArgs a, const int32_t* __restrict__ mask) {
   a.sizes[c] = 0;
 }
 
-// Item contributions in int64 fixed point (order-independent sums).  One
-// block per scan tile (256 items in spatial order, a few clusters): the items
-// first add into an LDS table keyed by cluster, then each table entry is
-// flushed with one global atomic per value, instead of one per item.
-static_assert(kBlock == kTileItems, "one thread per tile item");
-__global__ __launch_bounds__(kBlock) void k_accumulate(SweepArgs a, const int32_t* __restrict__ mask,
-                                                       unsigned long long* mesh_count) {
-  constexpr int kVals = 15;  // W, S[3], Q[10], count
-  __shared__ int32_t keys[kTileItems];
-  __shared__ unsigned long long vals[kTileItems * kVals];
-  __shared__ unsigned long long s_count;
-  const int32_t t = blockIdx.x;
-  const int m = a.item_mesh ? a.tile_mesh[t] : 0;
-  if (!mask[m]) return;  // whole block
-  keys[threadIdx.x] = -1;
-  for (int k = 0; k < kVals; ++k) vals[threadIdx.x * kVals + k] = 0ull;
-  if (threadIdx.x == 0) s_count = 0ull;
+template <int CTRL>
+__device__ inline unsigned long long dpp_u64(unsigned long long x) {
+  const uint32_t lo = uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(x)), CTRL, 0xf, 0xf, true));
+  const uint32_t hi = uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(x >> 32)), CTRL, 0xf, 0xf, true));
+  return (uint64_t(hi) << 32) | lo;
+}
+
+// One doubling step of the segmented sum over runs of equal clusters: lane l adds
+// lane l + D (of its 16-lane row) when rem lanes of its run follow it.
+template <int D, int V>
+__device__ inline void merge_step(unsigned long long (&v)[V], int n, int rem) {
+  const bool take = rem >= D;
+  if (__ballot(take) == 0ull) return;
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    if (k >= n) break;  // wave-uniform
+    const unsigned long long t = dpp_u64<0x100 | D>(v[k]);  // row_shl:D
+    v[k] += take ? t : 0ull;
+  }
+}
+
+// Lanes that follow in the lane's run, given the run heads of the wave.
+__device__ inline int run_left(unsigned long long heads) {
+  const int lane = __lane_id();
+  const unsigned long long after = lane == 63 ? 0ull : heads >> (lane + 1);
+  return after ? __builtin_ctzll(after) : 63 - lane;
+}
+
+// Item contributions in int64 fixed point (order-independent sums).  Each block
+// takes a contiguous range of items, 512 at a time: runs of equal clusters merge
+// in registers (at most 8 lanes), each run adds once into the block's LDS table
+// keyed by cluster, and the table goes to the global sums, consecutive threads to
+// consecutive words, when it is three quarters full and at the end.  The quadrics
+// are summed only while the mesh is constrained (nothing reads them before, and
+// the recompute of the convergence that constrains it sums them).
+// One table per 256 items, an LDS atomic per item and value and a global one per
+// cluster and table took 870 us at 8.39 M items; now 268 us (178 without quadrics;
+// a copy of the bytes read takes 100).
+constexpr int kAccBlock = 512;
+constexpr int kAccBlocks = 512;  // 2 per CU (61 KB of LDS each)
+__global__ __launch_bounds__(kAccBlock) void k_accumulate(SweepArgs a, const int32_t* __restrict__ mask,
+                                                          unsigned long long* mesh_count, int64_t chunk) {
+  constexpr int V = 15;  // W, S[3], count, Q[10]
+  constexpr int kSlots = 512, kSlotBits = 9, kFlushAt = kSlots * 3 / 4, kProbes = 32, kCheckSteps = 4;
+  __shared__ int32_t keys[kSlots];
+  __shared__ unsigned long long vals[kSlots * V];
+  __shared__ int32_t n_keys;
+  for (int k = threadIdx.x; k < kSlots; k += kAccBlock) keys[k] = -1;
+  for (int k = threadIdx.x; k < kSlots * V; k += kAccBlock) vals[k] = 0ull;
+  if (threadIdx.x == 0) n_keys = 0;
   __syncthreads();
-  const DevMesh& dm = a.meshes[m];
-  const int32_t i = a.tile_items[int64_t(t) * kTileItems + threadIdx.x];
-  const int32_t c = i >= 0 ? a.labels[i] : kNull;
-  if (c != kNull) {
-    uint32_t h = (uint32_t(c) * 2654435761u) >> 24;
-    int slot = 0;
-    for (int probe = 0; probe < kTileItems; ++probe) {  // at most 256 keys: always finds a slot
-      const int32_t old = atomicCAS(&keys[h], -1, c);
-      if (old == -1 || old == c) {
-        slot = int(h);
-        break;
-      }
-      h = (h + 1) & (kTileItems - 1);
+  auto add_global = [&](int64_t c, int k, unsigned long long x) {
+    if (k < 4) atomicAdd(&a.acc_ws[4 * c + k], x);
+    else if (k == 4) atomicAdd(&a.sizes[c], int32_t(x));
+    else atomicAdd(&a.acc_q[10 * c + k - 5], x);
+  };
+  auto flush = [&]() {  // every thread of the block; the table is complete
+    for (int k = threadIdx.x; k < kSlots * V; k += kAccBlock) {
+      const int32_t key = keys[k / V];
+      const unsigned long long x = vals[k];
+      vals[k] = 0ull;
+      if (key >= 0 && x != 0ull) add_global(key, k % V, x);
     }
-    const float4 p = a.xw[i];
+    __syncthreads();
+    for (int k = threadIdx.x; k < kSlots; k += kAccBlock) keys[k] = -1;
+    if (threadIdx.x == 0) n_keys = 0;
+    __syncthreads();
+  };
+  const int64_t begin = int64_t(blockIdx.x) * chunk, end = min(begin + chunk, a.n_items);
+  const int lane = __lane_id();
+  const int m0 = mesh_of_item(a, begin), m1 = mesh_of_item(a, end - 1);
+  int step = 0;
+  for (int m = m0; m <= m1; ++m) {
+    if (!mask[m]) continue;  // block-uniform
+    const DevMesh& dm = a.meshes[m];
     const Scales sc = dm.scales;
-    unsigned long long* v = vals + slot * kVals;
-    atomicAdd(&v[0], (unsigned long long)fix_w(p.w, sc));
-    atomicAdd(&v[1], (unsigned long long)fix_s(p.w, p.x, sc));
-    atomicAdd(&v[2], (unsigned long long)fix_s(p.w, p.y, sc));
-    atomicAdd(&v[3], (unsigned long long)fix_s(p.w, p.z, sc));
-    if (dm.metric == 1)
-      for (int k = 0; k < 10; ++k) atomicAdd(&v[4 + k], (unsigned long long)fix_q(a.q[10 * int64_t(i) + k], sc));
-    atomicAdd(&v[14], 1ull);
-    // early-stop items: those of clusters that are not frozen (:733-736)
-    if (!(a.frozen && a.frozen[c])) atomicAdd(&s_count, 1ull);
+    const bool with_q = dm.metric == 1 && a.state[m].constrained;
+    const int64_t first = max(begin, dm.item_off), last = min(end, dm.item_off + dm.n_items);
+    int counted = 0;  // items of clusters that are not frozen, per wave
+    for (int64_t base = first; base < last; base += kAccBlock) {
+      const int64_t i = base + threadIdx.x;
+      const int32_t c = i < last ? a.labels[i] : kNull;
+      unsigned long long v[V];
+#pragma unroll
+      for (int k = 0; k < V; ++k) v[k] = 0ull;
+      if (c != kNull) {
+        const float4 p = a.xw[i];
+        v[0] = (unsigned long long)fix_w(p.w, sc);
+        v[1] = (unsigned long long)fix_s(p.w, p.x, sc);
+        v[2] = (unsigned long long)fix_s(p.w, p.y, sc);
+        v[3] = (unsigned long long)fix_s(p.w, p.z, sc);
+        v[4] = 1ull;
+        if (with_q)
+          for (int k = 0; k < 10; ++k) v[5 + k] = (unsigned long long)fix_q(a.q[10 * i + k], sc);
+      }
+      counted += __popcll(__ballot(c != kNull && !(a.frozen && a.frozen[c])));
+      const int32_t prev = __builtin_amdgcn_update_dpp(-2, c, 0x111, 0xf, 0xf, false);  // row_shr:1
+      const bool head = prev != c || (lane & 7) == 0;
+      const int rem = run_left(__ballot(head));
+      const int n = with_q ? V : 5;
+      merge_step<1>(v, n, rem);
+      merge_step<2>(v, n, rem);
+      merge_step<4>(v, n, rem);
+      if (head && c != kNull) {
+        uint32_t h = (uint32_t(c) * 2654435761u) >> (32 - kSlotBits);
+        int slot = -1;
+        for (int probe = 0; probe < kProbes; ++probe) {
+          const int32_t old = atomicCAS(&keys[h], -1, c);
+          if (old == -1) atomicAdd(&n_keys, 1);
+          if (old == -1 || old == c) {
+            slot = int(h);
+            break;
+          }
+          h = (h + 1) & (kSlots - 1);
+        }
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+          if (k >= n) break;
+          if (slot >= 0) atomicAdd(&vals[slot * V + k], v[k]);
+          else if (v[k] != 0ull) add_global(c, k, v[k]);  // no free slot near by
+        }
+      }
+      if (++step % kCheckSteps == 0) {  // block-uniform
+        __syncthreads();
+        const bool full = n_keys > kFlushAt;
+        __syncthreads();
+        if (full) flush();
+      }
+    }
+    if (mesh_count && lane == 0 && counted) atomicAdd(&mesh_count[m], (unsigned long long)counted);
   }
   __syncthreads();
-  const int32_t key = keys[threadIdx.x];
-  if (key >= 0) {
-    const unsigned long long* v = vals + threadIdx.x * kVals;
-    for (int k = 0; k < 4; ++k) atomicAdd(&a.acc_ws[4 * int64_t(key) + k], v[k]);
-    if (dm.metric == 1)
-      for (int k = 0; k < 10; ++k) atomicAdd(&a.acc_q[10 * int64_t(key) + k], v[4 + k]);
-    atomicAdd(&a.sizes[key], int32_t(v[14]));
-  }
-  if (threadIdx.x == 0 && mesh_count && s_count) atomicAdd(&mesh_count[m], s_count);
+  flush();
 }
 
 // Centroid, W and (QEM, constrained) T of cluster c from its accumulators;
@@ -1599,43 +1677,115 @@ __device__ int32_t cc_find(int32_t* parent, int32_t x) {
   }
 }
 
+// f(j) for every neighbour j of item i.
+template <class F>
+__device__ inline void for_each_neighbour(const SweepArgs& a, int64_t i, F&& f) {
+  int32_t nbr[kRingCache];
+  if (load_row8(a, i, nbr)) {
+#pragma unroll
+    for (int p = 0; p < kRingCache; ++p)
+      if (nbr[p] >= 0) f(nbr[p]);
+  } else {
+    for (int32_t k = a.row_ptr[i]; k < a.row_ptr[i + 1]; ++k) f(a.col[k]);
+  }
+}
+
+// Every item starts below its smallest neighbour of the same label, so that most
+// of a component is one tree before the first compare-and-swap.
 __global__ void k_cc_init(SweepArgs a, const int32_t* __restrict__ mask, int32_t* parent, int32_t* comp_size) {
   int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= a.n_items || !mask[mesh_of_item(a, i)]) return;
-  parent[i] = int32_t(i);
+  const int32_t lab = a.labels[i];
+  int32_t low = int32_t(i);
+  if (lab != kNull)
+    for_each_neighbour(a, i, [&](int32_t j) {
+      if (j < low && a.labels[j] == lab) low = j;
+    });
+  parent[i] = low;
   comp_size[i] = 0;
 }
 
+// Every item straight below the root of its tree, so that the ends of most edges
+// show the same root at the first look.
+__global__ void k_cc_flatten(SweepArgs a, const int32_t* __restrict__ mask, int32_t* parent) {
+  int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= a.n_items || !mask[mesh_of_item(a, i)]) return;
+  int32_t r = parent[i];
+  for (int32_t p = parent[r]; p != r; p = parent[r]) r = p;
+  parent[i] = r;
+}
+
+// Joins the trees of items x and y.  A root that a stale read shows may have been
+// hooked meanwhile: the compare-and-swap then returns what it is hooked under, and
+// the walk goes on from there (ids only fall, so it ends).
+__device__ inline void cc_join(int32_t* parent, int32_t x, int32_t y) {
+  int32_t u = x, v = y;
+  while (true) {
+    u = cc_find(parent, u);
+    v = cc_find(parent, v);
+    if (u == v) return;
+    if (u > v) {
+      int32_t t = u;
+      u = v;
+      v = t;
+    }
+    // hook root v under the smaller root u
+    const int32_t old = atomicCAS(&parent[v], v, u);
+    if (old == v) return;
+    v = old;
+  }
+}
+
+// Joins the two ends of every edge inside a cluster (each edge at its larger
+// end).  The labels of a short row and then the roots of its ends are read side
+// by side; only an edge between two trees takes the walk.  8.39 M items: 1118 us
+// edge by edge from single items, 600 from the trees of k_cc_init, 397 so (and
+// k_cc_count 479 -> 65 us).
 __global__ void k_cc_hook(SweepArgs a, const int32_t* __restrict__ mask, int32_t* parent) {
   int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= a.n_items || !mask[mesh_of_item(a, i)]) return;
   const int32_t lab = a.labels[i];
   if (lab == kNull) return;
-  for (int32_t k = a.row_ptr[i]; k < a.row_ptr[i + 1]; ++k) {
-    const int32_t j = a.col[k];
-    if (j <= i || a.labels[j] != lab) continue;
-    int32_t u = int32_t(i), v = j;
-    while (true) {
-      u = cc_find(parent, u);
-      v = cc_find(parent, v);
-      if (u == v) break;
-      if (u > v) {
-        int32_t t = u;
-        u = v;
-        v = t;
-      }
-      // hook root v under the smaller root u
-      if (atomicCAS(&parent[v], v, u) == v) break;
+  int32_t nbr[kRingCache];
+  if (load_row8(a, i, nbr)) {
+    const int32_t root = parent[i];
+    int32_t r[kRingCache];
+#pragma unroll
+    for (int p = 0; p < kRingCache; ++p) r[p] = nbr[p] >= 0 && nbr[p] < i ? a.labels[nbr[p]] : kNull;
+#pragma unroll
+    for (int p = 0; p < kRingCache; ++p) r[p] = r[p] == lab ? parent[nbr[p]] : root;
+    int32_t last = root;  // the ends of a row mostly show one other root
+#pragma unroll 1
+    for (int p = 0; p < kRingCache; ++p) {
+      int32_t q = root;
+#pragma unroll
+      for (int k = 0; k < kRingCache; ++k)
+        if (k == p) q = r[k];
+      if (q == root || q == last) continue;
+      cc_join(parent, root, q);
+      last = q;
+    }
+  } else {
+    for (int32_t k = a.row_ptr[i]; k < a.row_ptr[i + 1]; ++k) {
+      const int32_t j = a.col[k];
+      if (j < i && a.labels[j] == lab) cc_join(parent, int32_t(i), j);
     }
   }
 }
 
+// Sizes of the components, one atomic per run of equal roots in a wave; the items
+// keep their root.
 __global__ void k_cc_count(SweepArgs a, const int32_t* __restrict__ mask, int32_t* parent, int32_t* comp_size) {
   int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= a.n_items || !mask[mesh_of_item(a, i)]) return;
-  if (a.labels[i] == kNull) return;
-  const int32_t r = cc_find(parent, int32_t(i));
-  atomicAdd(&comp_size[r], 1);
+  int32_t r = -1;
+  if (i < a.n_items && mask[mesh_of_item(a, i)] && a.labels[i] != kNull) {
+    r = cc_find(parent, int32_t(i));
+    parent[i] = r;
+  }
+  const int32_t prev = __shfl_up(r, 1);
+  const bool head = __lane_id() == 0 || prev != r;
+  const int len = 1 + run_left(__ballot(head));
+  if (head && r >= 0) atomicAdd(&comp_size[r], len);
 }
 
 __global__ void k_cc_best(SweepArgs a, const int32_t* __restrict__ mask, const int32_t* __restrict__ parent,
@@ -1680,10 +1830,13 @@ __global__ void k_cc_zero(SweepArgs a, const int32_t* __restrict__ mask, unsigne
 __global__ void k_cc_disc(SweepArgs a, const int32_t* __restrict__ mask, const int32_t* __restrict__ ncomp,
                           int32_t* ndisc) {
   int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (c >= a.n_clusters) return;
-  const int m = mesh_of_cluster(a, c);
-  if (!mask[m]) return;
-  if (ncomp[c] > 1) atomicAdd(&ndisc[m], 1);
+  int m = 0;
+  bool split = false;
+  if (c < a.n_clusters) {
+    m = mesh_of_cluster(a, c);
+    split = mask[m] && ncomp[c] > 1;
+  }
+  count_per_mesh(split, m, [&](int32_t mm) { return &ndisc[mm]; });
 }
 
 // ----------------------------------------------------------------- seeding
@@ -1834,7 +1987,10 @@ hipError_t launch_zero_clusters(hipStream_t s, const SweepArgs& a, const int32_t
 
 hipError_t launch_accumulate(hipStream_t s, const SweepArgs& a, const int32_t* mask, unsigned long long* mesh_count) {
   if (a.n_items == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_accumulate, dim3(unsigned(a.n_tiles)), dim3(kBlock), 0, s, a, mask, mesh_count);
+  const int64_t per = (a.n_items + kAccBlocks - 1) / kAccBlocks;
+  const int64_t chunk = (per + kAccBlock - 1) / kAccBlock * kAccBlock;
+  hipLaunchKernelGGL(k_accumulate, dim3(unsigned((a.n_items + chunk - 1) / chunk)), dim3(kAccBlock), 0, s, a, mask,
+                     mesh_count, chunk);
   return hipGetLastError();
 }
 
@@ -1956,6 +2112,7 @@ hipError_t launch_cc(hipStream_t s, const SweepArgs& a, const int32_t* mask, int
   const dim3 gi(grid_for(a.n_items)), gc(grid_for(a.n_clusters)), b(kBlock);
   hipLaunchKernelGGL(k_cc_init, gi, b, 0, s, a, mask, parent, comp_size);
   hipLaunchKernelGGL(k_cc_zero, gc, b, 0, s, a, mask, best, ncomp);
+  hipLaunchKernelGGL(k_cc_flatten, gi, b, 0, s, a, mask, parent);
   hipLaunchKernelGGL(k_cc_hook, gi, b, 0, s, a, mask, parent);
   hipLaunchKernelGGL(k_cc_count, gi, b, 0, s, a, mask, parent, comp_size);
   hipLaunchKernelGGL(k_cc_best, gi, b, 0, s, a, mask, parent, comp_size, best, ncomp);

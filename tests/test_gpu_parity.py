@@ -112,6 +112,22 @@ def test_labels_bit_exact_against_replay(gpu_ready, name):
     np.testing.assert_array_equal(ctx.cluster_sizes(0), np.bincount(lab, minlength=K)[:K])
 
 
+@pytest.mark.parametrize("metric,K", [(ISO, 40), (ISO, 4000), (QEM, 1500)])
+def test_labels_bit_exact_from_scattered_labels(gpu_ready, metric, K):
+    """From random labels: every cluster in many pieces (the statistics of more
+    clusters than a block's table holds, component trees that all need joining)."""
+    xyz, tri = meshgen.icosphere(5, 1, 0.02)
+    init = np.random.default_rng(K).integers(0, K + 1, len(xyz)).astype(np.int32)
+    ctx = run_gpu(xyz, tri, metric, K, int(metric == QEM), init)
+    rp, col = ctx.adjacency(0)
+    xw, q = ctx.items(0)
+    rlab, rst = po.replay_run(rp, col, xw, q, ctx.scales(0), K, metric, init, seed=7, unconstrained=int(metric == QEM),
+                              max_loops=200000)
+    st = ctx.stats(0)
+    assert st["loops"] == rst["loops"] and st["total_moves"] == rst["total_moves"]
+    np.testing.assert_array_equal(ctx.labels(0), rlab)
+
+
 @pytest.mark.parametrize("nu,nv,metric", [(512, 384, QEM), (512, 385, QEM), (1024, 683, ISO), (1024, 684, ISO)])
 def test_labels_bit_exact_where_the_scan_changes(gpu_ready, nu, nv, metric):
     """Either side of the sizes where the scan and the evaluate part (196,608

@@ -250,6 +250,9 @@ hipError_t launch_energy_log(hipStream_t s, const SweepArgs& a, double* e_cluste
                              double* final_e);
 hipError_t launch_clock_stamp(hipStream_t s, unsigned long long* t);
 hipError_t launch_fill_i32(hipStream_t s, int32_t* p, int64_t n, int32_t v);
+hipError_t launch_labels_in(hipStream_t s, int64_t n, int32_t K, int64_t clus_off, int32_t* labels);
+hipError_t launch_labels_out(hipStream_t s, int64_t n, int32_t K, int64_t clus_off, const int32_t* labels,
+                             int32_t* out);
 // output mesh
 hipError_t build_dual_faces(hipStream_t s, int64_t nf, const int32_t* tri, const int32_t* labels, int64_t item_off,
                             int64_t clus_off, int32_t* out_tri, int64_t* out_nf);

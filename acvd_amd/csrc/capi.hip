@@ -92,6 +92,7 @@ struct HostMesh {
 constexpr int kChunk = 16;        // passes per graph launch
 constexpr int kShortChunk = 4;    // passes per graph launch near the end of a phase
 static_assert(kPassLogCap > kChunk, "the pass log must hold a chunk of passes");
+constexpr int64_t kHostLabels = 65536;  // labels of at most so many items are renumbered on the host: a launch costs more
 constexpr int kReduceItems = 16384;  // items per block of the deterministic reductions
 constexpr int kEnergyLogRing = 2 * kChunk;  // energy log entries per mesh on the device, drained per chunk
 
@@ -1014,31 +1015,35 @@ int initial_labels(acvd_ctx* c) {
   for (auto& h : c->meshes) {
     const int32_t K = h.params.number_of_clusters;
     if (!h.init_labels.empty() || h.params.initial_sampling != 1) {
-      huge_vector<int32_t> lab(h.nv);
+      huge_vector<int32_t> lab;
+      const int32_t* src = h.init_labels.data();
       if (h.init_labels.empty() && h.params.initial_sampling >= 2) {
         // the reference's sampling types 0 (one random item per cluster) and
         // -1 (item k for cluster k)
         if (int64_t(K) > h.nv) return fail(ACVD_ERR_ARG, "more clusters than items");
+        lab.resize(h.nv);
+        src = lab.data();
         if (h.params.initial_sampling == 2) {
           reference_seed_sampling(h.nv, K, lab.data());
         } else {
           for (int64_t i = 0; i < h.nv; ++i) lab[i] = i < K ? int32_t(i) : K;
         }
-        for (int64_t i = 0; i < h.nv; ++i) lab[i] = lab[i] == K ? kNull : int32_t(lab[i] + h.clus_off);
       } else if (h.init_labels.empty()) {
-        // the reference's region growing, then local ids -> global
+        // the reference's region growing
         // the indicator of the weights: the set one, else the computed curvature
         const std::vector<double>& ind = !h.indicator.empty() ? h.indicator : h.curvature;
+        lab.resize(h.nv);
+        src = lab.data();
         if (int rc = device_reference_sampling(c, h, ind.empty() ? nullptr : ind.data(), lab.data())) return rc;
-        for (int64_t i = 0; i < h.nv; ++i) lab[i] = lab[i] == K ? kNull : int32_t(lab[i] + h.clus_off);
-      } else {
-        for (int64_t i = 0; i < h.nv; ++i) {
-          int32_t l = h.init_labels[i];
-          lab[i] = (l < 0 || l >= K) ? kNull : int32_t(l + h.clus_off);
-        }
       }
-      HIP_TRY(hipMemcpyAsync(c->d_labels.p + h.item_off, lab.data(), h.nv * sizeof(int32_t), hipMemcpyHostToDevice,
-                             s));
+      int32_t* dst = c->d_labels.p + h.item_off;
+      if (h.nv <= kHostLabels) {
+        if (lab.empty()) lab.assign(src, src + h.nv);
+        for (auto& l : lab) l = (l < 0 || l >= K) ? kNull : int32_t(l + h.clus_off);
+        src = lab.data();
+      }
+      HIP_TRY(hipMemcpyAsync(dst, src, h.nv * sizeof(int32_t), hipMemcpyHostToDevice, s));
+      if (h.nv > kHostLabels) HIP_TRY(launch_labels_in(s, h.nv, K, h.clus_off, dst));
       HIP_TRY(hipStreamSynchronize(s));
     } else {
       DBuf<uint32_t> k0, k1;
@@ -1723,9 +1728,17 @@ int acvd_get_labels(acvd_ctx* ctx, int32_t mesh_id, int32_t* labels) {
   if (!labels) return fail(ACVD_ERR_ARG, "null buffer");
   if (!ctx->built || !ctx->d_labels.p) return fail(ACVD_ERR_STATE, "no clustering computed");
   const HostMesh& h = ctx->meshes[mesh_id];
-  HIP_TRY(hipMemcpy(labels, ctx->d_labels.p + h.item_off, h.nv * sizeof(int32_t), hipMemcpyDeviceToHost));
   const int32_t K = h.params.number_of_clusters;
-  for (int64_t i = 0; i < h.nv; ++i) labels[i] = labels[i] == kNull ? K : int32_t(labels[i] - h.clus_off);
+  if (h.nv <= kHostLabels) {
+    HIP_TRY(hipMemcpy(labels, ctx->d_labels.p + h.item_off, h.nv * sizeof(int32_t), hipMemcpyDeviceToHost));
+    for (int64_t i = 0; i < h.nv; ++i) labels[i] = labels[i] == kNull ? K : int32_t(labels[i] - h.clus_off);
+    return ACVD_OK;
+  }
+  HIP_TRY(hipSetDevice(ctx->device));
+  int32_t* out = ctx->d_pending.p + h.item_off;  // scratch of the fill, free between runs
+  HIP_TRY(launch_labels_out(ctx->stream, h.nv, K, h.clus_off, ctx->d_labels.p + h.item_off, out));
+  HIP_TRY(hipMemcpyAsync(labels, out, h.nv * sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
+  HIP_TRY(hipStreamSynchronize(ctx->stream));
   return ACVD_OK;
 }
 

@@ -1967,6 +1967,22 @@ __global__ void __launch_bounds__(kLogThreads) k_log_reduce(SweepArgs a, const d
 
 __global__ void k_clock_stamp(unsigned long long* t) { *t = (unsigned long long)wall_clock64(); }
 
+// Labels between the caller's numbering (0..K-1, anything else none; K = none on
+// the way out) and the context's (global cluster ids, kNull).  A pass over device
+// memory costs 15 us at 8.39 M items; the loop over host memory, with the fresh
+// buffer it filled, took 5 ms each way.
+__global__ void k_labels_in(int64_t n, int32_t K, int32_t clus_off, int32_t* labels) {
+  int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int32_t l = labels[i];
+  labels[i] = (l < 0 || l >= K) ? kNull : l + clus_off;
+}
+__global__ void k_labels_out(int64_t n, int32_t K, int32_t clus_off, const int32_t* __restrict__ labels,
+                             int32_t* __restrict__ out) {
+  int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i < n) out[i] = labels[i] == kNull ? K : labels[i] - clus_off;
+}
+
 __global__ void k_fill_i32(int32_t* p, int64_t n, int32_t v) {
   int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -2174,6 +2190,19 @@ hipError_t launch_energy_log(hipStream_t s, const SweepArgs& a, double* e_cluste
 
 hipError_t launch_clock_stamp(hipStream_t s, unsigned long long* t) {
   hipLaunchKernelGGL(k_clock_stamp, dim3(1), dim3(1), 0, s, t);
+  return hipGetLastError();
+}
+
+hipError_t launch_labels_in(hipStream_t s, int64_t n, int32_t K, int64_t clus_off, int32_t* labels) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_labels_in, dim3(grid_for(n)), dim3(kBlock), 0, s, n, K, int32_t(clus_off), labels);
+  return hipGetLastError();
+}
+
+hipError_t launch_labels_out(hipStream_t s, int64_t n, int32_t K, int64_t clus_off, const int32_t* labels,
+                             int32_t* out) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_labels_out, dim3(grid_for(n)), dim3(kBlock), 0, s, n, K, int32_t(clus_off), labels, out);
   return hipGetLastError();
 }
 

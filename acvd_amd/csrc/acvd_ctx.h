@@ -186,6 +186,8 @@ hipError_t launch_csr_sort_unique(hipStream_t s, int64_t n, const int32_t* tptr,
                                   const int32_t* vfptr, int32_t* vfcol);
 hipError_t launch_csr_compact(hipStream_t s, int64_t n, const int32_t* tptr, const int32_t* tcol,
                               const int32_t* row_ptr, int32_t* col);
+hipError_t launch_mesh_rows(hipStream_t s, int32_t n_meshes, const DevMesh* meshes, const int32_t* row_ptr,
+                            int32_t* out);
 hipError_t exclusive_scan_i32(hipStream_t s, const int32_t* in, int32_t* out, int64_t n, void** tmp,
                               size_t* tmp_bytes);
 hipError_t launch_ring_adj(hipStream_t s, int64_t n, const int32_t* row_ptr, const int32_t* col,
@@ -253,9 +255,10 @@ hipError_t launch_fill_i32(hipStream_t s, int32_t* p, int64_t n, int32_t v);
 hipError_t launch_labels_in(hipStream_t s, int64_t n, int32_t K, int64_t clus_off, int32_t* labels);
 hipError_t launch_labels_out(hipStream_t s, int64_t n, int32_t K, int64_t clus_off, const int32_t* labels,
                              int32_t* out);
-// output mesh
+// output mesh (with a workspace of dual_faces_workspace bytes)
+hipError_t dual_faces_workspace(int64_t nf, size_t* bytes);
 hipError_t build_dual_faces(hipStream_t s, int64_t nf, const int32_t* tri, const int32_t* labels, int64_t item_off,
-                            int64_t clus_off, int32_t* out_tri, int64_t* out_nf);
+                            int64_t clus_off, int32_t* out_tri, int64_t* out_nf, void* ws, size_t ws_bytes);
 hipError_t fix_empty_cluster_points(hipStream_t s, const int32_t* sizes, int64_t clus_off, int32_t K, int32_t* first,
                                     double* pts);
 hipError_t quadric_placement(hipStream_t s, int64_t n, int64_t item_off, const int32_t* labels, int64_t clus_off,

@@ -14,12 +14,14 @@
 #include <cstdlib>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <memory>
 #include <string>
 #include <vector>
 
 #include "../../include/acvd_c.h"
 #include "acvd_ctx.h"
+#include "acvd_energy.h"
 #include "host_mesh.h"
 #include "host_sampling.h"
 #include "host_parallel.h"
@@ -46,14 +48,22 @@ template <class T>
 struct DBuf {
   T* p = nullptr;
   size_t n = 0;
+  bool own = true;  // false: a part of a slab
   DBuf() = default;
   DBuf(const DBuf&) = delete;
   DBuf& operator=(const DBuf&) = delete;
   ~DBuf() { release(); }
   void release() {
-    if (p) (void)hipFree(p);
+    if (p && own) (void)hipFree(p);
     p = nullptr;
     n = 0;
+    own = true;
+  }
+  void view(void* base, size_t offset, size_t count) {
+    release();
+    p = reinterpret_cast<T*>(static_cast<char*>(base) + offset);
+    n = count;
+    own = false;
   }
   hipError_t alloc(size_t count) {
     release();
@@ -62,6 +72,43 @@ struct DBuf {
     if (e == hipSuccess) n = count;
     else p = nullptr;
     return e;
+  }
+};
+
+// Many device arrays in one allocation: add() every array, then give out the
+// parts of the slab.  hipMalloc takes blocks of up to 1 MB from memory that is
+// mapped already (under 1 us); each larger one, and its hipFree, costs the host
+// 50-60 us, and a build of 350,000 items made 80 of each (remesh: 61.4 ms a call,
+// with slabs 47.8).  Plans of at most kSlabMin bytes keep an allocation per array
+// (remesh of 41,000 items: 7.9 ms, with slabs 8.4).
+constexpr size_t kSlabMin = size_t(32) << 20;
+struct SlabPlan {
+  size_t bytes = 0;
+  std::vector<std::function<hipError_t(void*)>> parts;  // of the slab, or (null) allocated
+  template <class T>
+  void add(DBuf<T>& b, size_t count) {
+    if (count == 0) count = 1;
+    const size_t off = bytes;
+    bytes += (count * sizeof(T) + 255) / 256 * 256;
+    parts.push_back([&b, off, count](void* base) {
+      if (!base) return b.alloc(count);
+      b.view(base, off, count);
+      return hipSuccess;
+    });
+  }
+  // gives the parts out of `slab`, which is allocated again when it is too small
+  // or (shrink: a build, whose other steps need less) more than twice the need
+  hipError_t give(DBuf<char>& slab, bool shrink = false) {
+    const bool apart = bytes <= kSlabMin && slab.n < bytes;
+    if (!apart && (slab.n < bytes || (shrink && slab.n / 2 > bytes))) {
+      const hipError_t e = slab.alloc(bytes);
+      if (e != hipSuccess) return e;
+    }
+    for (auto& f : parts) {
+      const hipError_t e = f(apart ? nullptr : slab.p);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
   }
 };
 
@@ -105,7 +152,9 @@ struct acvd_ctx {
   bool built = false;
   bool any_iso = false, any_qem = false;
   int64_t N = 0, K = 0, F = 0, E2 = 0;
-  // device arrays
+  // device memory: the arrays below are parts of d_slab (d_col apart: its size
+  // comes from the device), temporary ones of d_scratch; both go with the context
+  DBuf<char> d_slab, d_scratch;
   DBuf<DevMesh> d_meshes;
   DBuf<MeshState> d_state;
   DBuf<Ctrl> d_ctrl;
@@ -148,6 +197,7 @@ struct acvd_ctx {
   // pinned host mirrors
   Ctrl* h_ctrl = nullptr;
   MeshState* h_state = nullptr;
+  size_t h_state_n = 0;  // meshes h_state holds
   std::vector<DevMesh> h_meshes;
   void* cub_tmp = nullptr;
   size_t cub_bytes = 0;
@@ -266,8 +316,7 @@ int add_mesh(acvd_ctx* c, int64_t nv, const P* xyz, int64_t nf, const int32_t* t
   HostMesh h;
   h.nv = nv;
   h.nf = nf;
-  h.xyz.resize(3 * nv);
-  for (int64_t k = 0; k < 3 * nv; ++k) h.xyz[k] = double(xyz[k]);
+  h.xyz.assign(xyz, xyz + 3 * nv);
   h.tri.assign(tri, tri + 3 * nf);
   acvd_params_init(&h.params);
   std::memset(&h.stats, 0, sizeof(h.stats));
@@ -325,15 +374,8 @@ int build(acvd_ctx* c) {
 
   // per-mesh descriptors
   c->h_meshes.assign(M, DevMesh{});
-  std::vector<int32_t> item_mesh, clus_mesh;
-  if (M > 1) {
-    item_mesh.resize(N);
-    clus_mesh.resize(K);
-  }
-  std::vector<double> pos(3 * N), ind(N, 0.0);
-  std::vector<int32_t> tri(3 * F);
   std::vector<int32_t> tile_mesh(c->n_tiles);
-  std::vector<float> bbox(6 * M);
+  std::vector<float> bbox(6 * M, 0.0f);
   bool any_ind = false;
   // meshes whose indicator is the reference's curvature measure, computed
   // below once the adjacency exists (vtkDiscreteRemeshing::SamplingPreProcessing,
@@ -345,7 +387,13 @@ int build(acvd_ctx* c) {
     const HostMesh& h = c->meshes[m];
     curv[m] = h.indicator.empty() && h.params.curvature_indicator && h.params.gradation > 0.0;
     any_curv |= curv[m] != 0;
+    any_ind |= !h.indicator.empty();
   }
+  // Tiles follow the vertex order (contiguous items: coalesced reads, and
+  // spatially coherent when the input order is, as for grid-generated and
+  // most scanned meshes) unless ACVD_TILE_ORDER=morton asks for spatial
+  // (Morton) tiles, whose cluster sets are tighter for arbitrary orders.
+  const bool morton = morton_tiles();
   int64_t foff = 0, toff = 0;
   for (int m = 0; m < M; ++m) {
     HostMesh& h = c->meshes[m];
@@ -364,101 +412,168 @@ int build(acvd_ctx* c) {
     const int64_t nt = (h.nv + kTileItems - 1) / kTileItems;
     std::fill(tile_mesh.begin() + toff, tile_mesh.begin() + toff + nt, m);
     toff += nt;
-    {
+    if (morton) {
       double lo[3] = {h.xyz[0], h.xyz[1], h.xyz[2]}, hi[3] = {lo[0], lo[1], lo[2]};
       for (int64_t v = 0; v < h.nv; ++v)
         for (int k = 0; k < 3; ++k) {
           lo[k] = std::min(lo[k], h.xyz[3 * v + k]);
           hi[k] = std::max(hi[k], h.xyz[3 * v + k]);
         }
-      // Tiles follow the vertex order (contiguous items: coalesced reads, and
-      // spatially coherent when the input order is, as for grid-generated and
-      // most scanned meshes) unless ACVD_TILE_ORDER=morton asks for spatial
-      // (Morton) tiles, whose cluster sets are tighter for arbitrary orders.
-      const bool morton = morton_tiles();
       for (int k = 0; k < 3; ++k) {
         bbox[6 * m + k] = float(lo[k]);
-        bbox[6 * m + 3 + k] = (morton && hi[k] > lo[k]) ? float(65535.0 / (hi[k] - lo[k])) : 0.0f;
+        bbox[6 * m + 3 + k] = hi[k] > lo[k] ? float(65535.0 / (hi[k] - lo[k])) : 0.0f;
       }
     }
-    std::copy(h.xyz.begin(), h.xyz.end(), pos.begin() + 3 * h.item_off);
-    if (!h.indicator.empty()) {
-      any_ind = true;
-      std::copy(h.indicator.begin(), h.indicator.end(), ind.begin() + h.item_off);
-    }
-    for (int64_t k = 0; k < 3 * h.nf; ++k) tri[3 * foff + k] = int32_t(h.tri[k] + h.item_off);
     h.face_off = foff;
     foff += h.nf;
-    if (M > 1) {
-      std::fill(item_mesh.begin() + h.item_off, item_mesh.begin() + h.item_off + h.nv, m);
-      std::fill(clus_mesh.begin() + h.clus_off, clus_mesh.begin() + h.clus_off + d.K, m);
-    }
   }
+  // sweep geometry
+  // work slices: scan tiles are dealt round-robin to the slices
+  c->work_cap = int32_t(((int64_t(c->n_tiles) + kWorkSlices - 1) / kWorkSlices) * kTileItems);
+  // candidate segments: evaluate block b takes work positions
+  // b * kBlock + j * n_seg * kBlock (at most N of them) and proposes at most
+  // once per item; apply block b appends one moved item per candidate
+  // (once per pass)
+  c->n_seg = int32_t(sweep_grid_for(N, c->tuning.sweep_segments));
+  const int64_t steps = (N + int64_t(c->n_seg) * kBlock - 1) / (int64_t(c->n_seg) * kBlock);
+  const int64_t cap = std::max<int64_t>(1, steps) * kBlock;
+  if (cap * c->n_seg > (int64_t(1) << 31) - 1) return fail(ACVD_ERR_ARG, "too many items for one context");
+  c->cand_cap = int32_t(cap);
+  // fixed items per cluster (a change of the fixed clusters rebuilds the
+  // context, so the captured chunks never see a stale pointer)
+  c->any_fixed = false;
+  for (auto& h : c->meshes) c->any_fixed |= !h.fixed.empty();
+  c->any_frozen = false;
+  for (auto& h : c->meshes) c->any_frozen |= !h.frozen.empty();
   // allocations
-  HIP_TRY(c->d_meshes.alloc(M));
-  HIP_TRY(c->d_state.alloc(M));
-  HIP_TRY(c->d_ctrl.alloc(1));
-  HIP_TRY(c->d_mask_all.alloc(M));
-  HIP_TRY(c->d_mask.alloc(M));
-  HIP_TRY(c->d_ndisc.alloc(M));
-  HIP_TRY(c->d_mesh_count.alloc(M));
-  if (M > 1) {
-    HIP_TRY(c->d_item_mesh.alloc(N));
-    HIP_TRY(c->d_clus_mesh.alloc(K));
-    HIP_TRY(hipMemcpyAsync(c->d_item_mesh.p, item_mesh.data(), N * sizeof(int32_t), hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemcpyAsync(c->d_clus_mesh.p, clus_mesh.data(), K * sizeof(int32_t), hipMemcpyHostToDevice, s));
+  {
+    const size_t n = size_t(N), k = size_t(K), f3 = 3 * size_t(F), nt = size_t(c->n_tiles);
+    const size_t nc = size_t(c->cand_cap) * size_t(c->n_seg);
+    SlabPlan p;
+    p.add(c->d_meshes, M);
+    p.add(c->d_state, M);
+    p.add(c->d_ctrl, 1);
+    p.add(c->d_mask_all, M);
+    p.add(c->d_mask, M);
+    p.add(c->d_ndisc, M);
+    p.add(c->d_mesh_count, M);
+    if (M > 1) {
+      p.add(c->d_item_mesh, n);
+      p.add(c->d_clus_mesh, k);
+    }
+    p.add(c->d_tri, f3);
+    p.add(c->d_pos, 3 * n);
+    p.add(c->d_vfptr, n + 1);
+    p.add(c->d_vfcol, f3);
+    p.add(c->d_row_ptr, n + 1);
+    p.add(c->d_row8, 2 * n);
+    p.add(c->d_ring_adj, n);
+    p.add(c->d_xw, n);
+    p.add(c->d_q, 10 * n);  // vertex quadrics of every mesh
+    p.add(c->d_tile_items, nt * kTileItems);
+    p.add(c->d_item_tile, n);
+    p.add(c->d_tile_mesh, nt);
+    p.add(c->d_tile_cnt, nt);
+    p.add(c->d_tile_set, nt * kTileSet);
+    p.add(c->d_tile_prop, nt);
+    p.add(c->d_labels, n);
+    p.add(c->d_sizes, k);
+    p.add(c->d_stamp, k);
+    p.add(c->d_cand_pass, n);
+    p.add(c->d_pending, n);
+    p.add(c->d_acc_ws, 4 * k);
+    if (c->any_qem) {
+      p.add(c->d_acc_q, 10 * k);
+      p.add(c->d_T, k);
+      p.add(c->d_evec, 9 * k);
+    }
+    p.add(c->d_prio, k);
+    p.add(c->d_geom, k);
+    if (c->any_fixed) p.add(c->d_anchor, k);
+    if (c->any_frozen) p.add(c->d_frozen, k);
+    p.add(c->d_cl_round, k);
+    p.add(c->d_work, size_t(c->work_cap) * kWorkSlices);
+    p.add(c->d_work_count, kWorkSlices);
+    p.add(c->d_cand, nc);
+    p.add(c->d_cand_tgt, nc);
+    p.add(c->d_cand_lab, nc);
+    p.add(c->d_cand_since, nc);
+    p.add(c->d_moved, nc);
+    p.add(c->d_seg_cand, c->n_seg);
+    p.add(c->d_seg_moved, c->n_seg);
+    p.add(c->d_parent, n);
+    p.add(c->d_comp_size, n);
+    p.add(c->d_ncomp, k);
+    p.add(c->d_best, k);
+    HIP_TRY(p.give(c->d_slab, true));
   }
+  // temporary arrays
+  std::vector<int2> tab;  // blocks of the deterministic reductions
+  for (auto& h : c->meshes)
+    for (int64_t b = h.item_off; b < h.item_off + h.nv; b += kReduceItems)
+      tab.push_back(make_int2(int32_t(b), int32_t(std::min<int64_t>(b + kReduceItems, h.item_off + h.nv))));
+  DBuf<double> d_ind, d_raw, d_part;
+  DBuf<int32_t> counts, tptr, tcol, d_adj_off;
+  DBuf<int2> d_tab;
+  DBuf<float> d_bbox;
+  {
+    SlabPlan p;
+    if (any_ind || any_curv) p.add(d_ind, N);
+    p.add(d_raw, N);
+    p.add(d_part, 4 * tab.size() + M);
+    p.add(counts, 5 * size_t(N) + 3);  // degrees, face degrees, fill counts (2), unique degrees
+    p.add(tptr, N + 1);
+    p.add(tcol, 6 * size_t(F));
+    p.add(d_adj_off, M + 1);
+    p.add(d_tab, tab.size());
+    p.add(d_bbox, 6 * M);
+    HIP_TRY(p.give(c->d_scratch, true));
+  }
+  // uploads (the copies from pageable memory return once the source is read)
   HIP_TRY(hipMemcpyAsync(c->d_meshes.p, c->h_meshes.data(), M * sizeof(DevMesh), hipMemcpyHostToDevice, s));
-  std::vector<int32_t> ones(M, 1);
-  HIP_TRY(hipMemcpyAsync(c->d_mask_all.p, ones.data(), M * sizeof(int32_t), hipMemcpyHostToDevice, s));
-  HIP_TRY(c->d_tri.alloc(3 * F));
-  HIP_TRY(hipMemcpyAsync(c->d_tri.p, tri.data(), 3 * F * sizeof(int32_t), hipMemcpyHostToDevice, s));
-  DBuf<double> d_ind, d_raw;
+  HIP_TRY(launch_fill_i32(s, c->d_mask_all.p, M, 1));
   DBuf<double>& d_pos = c->d_pos;
-  HIP_TRY(d_pos.alloc(3 * N));
-  HIP_TRY(hipMemcpyAsync(d_pos.p, pos.data(), 3 * N * sizeof(double), hipMemcpyHostToDevice, s));
-  if (any_ind || any_curv) {
-    HIP_TRY(d_ind.alloc(N));
-    HIP_TRY(hipMemcpyAsync(d_ind.p, ind.data(), N * sizeof(double), hipMemcpyHostToDevice, s));
+  for (int m = 0; m < M; ++m) {
+    const HostMesh& h = c->meshes[m];
+    int32_t* tri = c->d_tri.p + 3 * h.face_off;
+    HIP_TRY(hipMemcpyAsync(tri, h.tri.data(), 3 * h.nf * sizeof(int32_t), hipMemcpyHostToDevice, s));
+    HIP_TRY(energy_offset_tri(s, 3 * h.nf, int32_t(h.item_off), tri));
+    HIP_TRY(hipMemcpyAsync(d_pos.p + 3 * h.item_off, h.xyz.data(), 3 * h.nv * sizeof(double), hipMemcpyHostToDevice,
+                           s));
+    if (!h.indicator.empty())
+      HIP_TRY(hipMemcpyAsync(d_ind.p + h.item_off, h.indicator.data(), h.nv * sizeof(double), hipMemcpyHostToDevice,
+                             s));
+    if (M > 1) {
+      HIP_TRY(launch_fill_i32(s, c->d_item_mesh.p + h.item_off, h.nv, m));
+      HIP_TRY(launch_fill_i32(s, c->d_clus_mesh.p + h.clus_off, h.params.number_of_clusters, m));
+    }
   }
   // ---- CSR
   {
-    DBuf<int32_t> deg2, vfdeg, tptr, tfill, vffill, tcol, deg;
     DBuf<int32_t>& vfptr = c->d_vfptr;
     DBuf<int32_t>& vfcol = c->d_vfcol;
-    HIP_TRY(deg2.alloc(N + 1));
-    HIP_TRY(vfdeg.alloc(N + 1));
-    HIP_TRY(tptr.alloc(N + 1));
-    HIP_TRY(vfptr.alloc(N + 1));
-    HIP_TRY(tfill.alloc(N));
-    HIP_TRY(vffill.alloc(N));
-    HIP_TRY(hipMemsetAsync(deg2.p, 0, (N + 1) * sizeof(int32_t), s));
-    HIP_TRY(hipMemsetAsync(vfdeg.p, 0, (N + 1) * sizeof(int32_t), s));
-    HIP_TRY(hipMemsetAsync(tfill.p, 0, N * sizeof(int32_t), s));
-    HIP_TRY(hipMemsetAsync(vffill.p, 0, N * sizeof(int32_t), s));
-    HIP_TRY(launch_csr_count(s, F, c->d_tri.p, deg2.p, vfdeg.p));
-    HIP_TRY(exclusive_scan_i32(s, deg2.p, tptr.p, N + 1, &c->cub_tmp, &c->cub_bytes));
-    HIP_TRY(exclusive_scan_i32(s, vfdeg.p, vfptr.p, N + 1, &c->cub_tmp, &c->cub_bytes));
-    int32_t tot[2] = {0, 0};
-    HIP_TRY(hipMemcpyAsync(&tot[0], tptr.p + N, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(&tot[1], vfptr.p + N, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    int32_t *deg2 = counts.p, *vfdeg = deg2 + N + 1, *deg = vfdeg + N + 1, *tfill = deg + N + 1, *vffill = tfill + N;
+    HIP_TRY(hipMemsetAsync(counts.p, 0, counts.n * sizeof(int32_t), s));
+    HIP_TRY(launch_csr_count(s, F, c->d_tri.p, deg2, vfdeg));
+    HIP_TRY(exclusive_scan_i32(s, deg2, tptr.p, N + 1, &c->cub_tmp, &c->cub_bytes));
+    HIP_TRY(exclusive_scan_i32(s, vfdeg, vfptr.p, N + 1, &c->cub_tmp, &c->cub_bytes));
+    HIP_TRY(launch_csr_fill(s, F, c->d_tri.p, tptr.p, tfill, tcol.p, vfptr.p, vffill, vfcol.p));
+    HIP_TRY(launch_csr_sort_unique(s, N, tptr.p, tcol.p, deg, vfptr.p, vfcol.p));
+    HIP_TRY(exclusive_scan_i32(s, deg, c->d_row_ptr.p, N + 1, &c->cub_tmp, &c->cub_bytes));
+    // the rows of each mesh: row_ptr at the mesh boundaries
+    std::vector<int32_t> bound(M + 1);
+    if (M > 1) HIP_TRY(launch_mesh_rows(s, M, c->d_meshes.p, c->d_row_ptr.p, d_adj_off.p));
+    const int32_t* rows = M > 1 ? d_adj_off.p : c->d_row_ptr.p + N;
+    HIP_TRY(hipMemcpyAsync(M > 1 ? bound.data() : bound.data() + 1, rows, (M > 1 ? M + 1 : 1) * sizeof(int32_t),
+                           hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
-    HIP_TRY(tcol.alloc(tot[0]));
-    HIP_TRY(vfcol.alloc(tot[1]));
-    HIP_TRY(launch_csr_fill(s, F, c->d_tri.p, tptr.p, tfill.p, tcol.p, vfptr.p, vffill.p, vfcol.p));
-    HIP_TRY(deg.alloc(N + 1));
-    HIP_TRY(hipMemsetAsync(deg.p, 0, (N + 1) * sizeof(int32_t), s));
-    HIP_TRY(launch_csr_sort_unique(s, N, tptr.p, tcol.p, deg.p, vfptr.p, vfcol.p));
-    HIP_TRY(c->d_row_ptr.alloc(N + 1));
-    HIP_TRY(exclusive_scan_i32(s, deg.p, c->d_row_ptr.p, N + 1, &c->cub_tmp, &c->cub_bytes));
-    int32_t e2 = 0;
-    HIP_TRY(hipMemcpyAsync(&e2, c->d_row_ptr.p + N, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    c->E2 = e2;
-    HIP_TRY(c->d_col.alloc(e2));
+    for (int m = 0; m < M; ++m) {
+      c->meshes[m].adj_off = bound[m];
+      c->meshes[m].n_adj = int64_t(bound[m + 1]) - bound[m];
+    }
+    c->E2 = bound[M];
+    if (c->d_col.n < size_t(c->E2) || c->d_col.n / 2 > size_t(c->E2)) HIP_TRY(c->d_col.alloc(size_t(c->E2)));
     HIP_TRY(launch_csr_compact(s, N, tptr.p, tcol.p, c->d_row_ptr.p, c->d_col.p));
-    HIP_TRY(c->d_ring_adj.alloc(N));
-    HIP_TRY(c->d_row8.alloc(2 * N));
     HIP_TRY(launch_ring_adj(s, N, c->d_row_ptr.p, c->d_col.p, c->d_ring_adj.p, c->d_row8.p));
     // ---- curvature indicators (before the weights that use them)
     for (int m = 0; m < M; ++m) {
@@ -473,41 +588,24 @@ int build(acvd_ctx* c) {
     }
     if (any_curv) HIP_TRY(hipStreamSynchronize(s));
     // ---- items
-    HIP_TRY(c->d_xw.alloc(N));
-    HIP_TRY(c->d_q.alloc(10 * N));  // vertex quadrics of every mesh
-    HIP_TRY(d_raw.alloc(N));
     SweepArgs a = c->args();
     HIP_TRY(launch_item_build(s, a, d_pos.p, c->d_tri.p, vfptr.p, vfcol.p, (any_ind || any_curv) ? d_ind.p : nullptr,
                               d_raw.p, c->d_xw.p, c->d_q.p));
   }
-  // ---- scan tiles in spatial order
+  // ---- scan tiles
   {
     const int64_t nt = c->n_tiles;
-    HIP_TRY(c->d_tile_items.alloc(nt * kTileItems));
-    HIP_TRY(c->d_item_tile.alloc(N));
-    HIP_TRY(c->d_tile_mesh.alloc(nt));
-    HIP_TRY(c->d_tile_cnt.alloc(nt));
-    HIP_TRY(c->d_tile_set.alloc(nt * kTileSet));
-    HIP_TRY(c->d_tile_prop.alloc(nt));
     // no cluster id equals the fill value (free set slots, see k_tile_sets)
     HIP_TRY(launch_fill_i32(s, c->d_tile_set.p, nt * kTileSet, -2));
     HIP_TRY(hipMemcpyAsync(c->d_tile_mesh.p, tile_mesh.data(), nt * sizeof(int32_t), hipMemcpyHostToDevice, s));
-    DBuf<float> d_bbox;
-    HIP_TRY(d_bbox.alloc(6 * M));
-    HIP_TRY(hipMemcpyAsync(d_bbox.p, bbox.data(), 6 * M * sizeof(float), hipMemcpyHostToDevice, s));
+    if (morton)
+      HIP_TRY(hipMemcpyAsync(d_bbox.p, bbox.data(), 6 * M * sizeof(float), hipMemcpyHostToDevice, s));
     SweepArgs a = c->args();
-    HIP_TRY(launch_tile_order(s, a, d_bbox.p, c->d_tile_items.p, c->d_item_tile.p, &c->cub_tmp, &c->cub_bytes));
+    HIP_TRY(launch_tile_order(s, a, morton ? d_bbox.p : nullptr, c->d_tile_items.p, c->d_item_tile.p, &c->cub_tmp,
+                              &c->cub_bytes));
   }
   // ---- deterministic reductions: clamp then scales
   {
-    std::vector<int2> tab;
-    for (auto& h : c->meshes)
-      for (int64_t b = h.item_off; b < h.item_off + h.nv; b += kReduceItems)
-        tab.push_back(make_int2(int32_t(b), int32_t(std::min<int64_t>(b + kReduceItems, h.item_off + h.nv))));
-    DBuf<int2> d_tab;
-    DBuf<double> d_part;
-    HIP_TRY(d_tab.alloc(tab.size()));
-    HIP_TRY(d_part.alloc(4 * tab.size() + M));
     HIP_TRY(hipMemcpyAsync(d_tab.p, tab.data(), tab.size() * sizeof(int2), hipMemcpyHostToDevice, s));
     SweepArgs a = c->args();
     HIP_TRY(launch_seg_reduce(s, int(tab.size()), d_tab.p, a, d_raw.p, 0, d_part.p));
@@ -518,56 +616,7 @@ int build(acvd_ctx* c) {
     HIP_TRY(hipStreamSynchronize(s));
   }
   // ---- sweep state
-  HIP_TRY(c->d_labels.alloc(N));
-  HIP_TRY(c->d_sizes.alloc(K));
-  HIP_TRY(c->d_stamp.alloc(K));
-  HIP_TRY(c->d_cand_pass.alloc(N));
-  HIP_TRY(c->d_pending.alloc(N));
-  HIP_TRY(c->d_acc_ws.alloc(4 * K));
-  if (c->any_qem) {
-    HIP_TRY(c->d_acc_q.alloc(10 * K));
-    HIP_TRY(c->d_T.alloc(K));
-    HIP_TRY(c->d_evec.alloc(9 * K));
-  }
-  HIP_TRY(c->d_prio.alloc(K));
-  HIP_TRY(c->d_geom.alloc(K));
-  // fixed items per cluster (a change of the fixed clusters rebuilds the
-  // context, so the captured chunks never see a stale pointer)
-  c->any_fixed = false;
-  for (auto& h : c->meshes) c->any_fixed |= !h.fixed.empty();
-  if (c->any_fixed) HIP_TRY(c->d_anchor.alloc(K));
-  c->any_frozen = false;
-  for (auto& h : c->meshes) c->any_frozen |= !h.frozen.empty();
-  if (c->any_frozen) HIP_TRY(c->d_frozen.alloc(K));
-  HIP_TRY(c->d_cl_round.alloc(K));
-  {
-    // work slices: scan tiles are dealt round-robin to the slices
-    c->work_cap = int32_t(((int64_t(c->n_tiles) + kWorkSlices - 1) / kWorkSlices) * kTileItems);
-    HIP_TRY(c->d_work.alloc(size_t(c->work_cap) * kWorkSlices));
-    HIP_TRY(c->d_work_count.alloc(kWorkSlices));
-    HIP_TRY(hipMemsetAsync(c->d_work_count.p, 0, kWorkSlices * sizeof(int32_t), s));
-    // candidate segments: evaluate block b takes work positions
-    // b * kBlock + j * n_seg * kBlock (at most N of them) and proposes at most
-    // once per item; apply block b appends one moved item per candidate
-    // (once per pass)
-    c->n_seg = int32_t(sweep_grid_for(N, c->tuning.sweep_segments));
-    const int64_t steps = (N + int64_t(c->n_seg) * kBlock - 1) / (int64_t(c->n_seg) * kBlock);
-    const int64_t cap = std::max<int64_t>(1, steps) * kBlock;
-    if (cap * c->n_seg > (int64_t(1) << 31) - 1) return fail(ACVD_ERR_ARG, "too many items for one context");
-    c->cand_cap = int32_t(cap);
-    const size_t nc = size_t(c->cand_cap) * size_t(c->n_seg);
-    HIP_TRY(c->d_cand.alloc(nc));
-    HIP_TRY(c->d_cand_tgt.alloc(nc));
-    HIP_TRY(c->d_cand_lab.alloc(nc));
-    HIP_TRY(c->d_cand_since.alloc(nc));
-    HIP_TRY(c->d_moved.alloc(nc));
-    HIP_TRY(c->d_seg_cand.alloc(c->n_seg));
-    HIP_TRY(c->d_seg_moved.alloc(c->n_seg));
-  }
-  HIP_TRY(c->d_parent.alloc(N));
-  HIP_TRY(c->d_comp_size.alloc(N));
-  HIP_TRY(c->d_ncomp.alloc(K));
-  HIP_TRY(c->d_best.alloc(K));
+  HIP_TRY(hipMemsetAsync(c->d_work_count.p, 0, kWorkSlices * sizeof(int32_t), s));
   HIP_TRY(hipMemsetAsync(c->d_ctrl.p, 0, sizeof(Ctrl), s));
   HIP_TRY(hipEventRecord(e1, s));
   HIP_TRY(hipEventSynchronize(e1));
@@ -576,18 +625,6 @@ int build(acvd_ctx* c) {
   c->build_ms = ms;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  for (auto& h : c->meshes) {
-    h.n_adj = 0;
-  }
-  // per-mesh adjacency sizes (row_ptr at mesh boundaries)
-  {
-    std::vector<int32_t> rp(N + 1);
-    HIP_TRY(hipMemcpy(rp.data(), c->d_row_ptr.p, (N + 1) * sizeof(int32_t), hipMemcpyDeviceToHost));
-    for (auto& h : c->meshes) {
-      h.adj_off = rp[h.item_off];
-      h.n_adj = int64_t(rp[h.item_off + h.nv]) - h.adj_off;
-    }
-  }
   c->built = true;
   return ACVD_OK;
 }
@@ -932,8 +969,8 @@ int minimize_energy(acvd_ctx* c) {
       near_end = false;
       stop_props = early_stop_props();
       HIP_TRY(launch_fill_i32(s, c->d_tile_cnt.p, c->n_tiles, kTileSet + 1));
+      // (h_state is written again only by a copy behind this one in the stream)
       HIP_TRY(hipMemcpyAsync(c->d_state.p, c->h_state, M * sizeof(MeshState), hipMemcpyHostToDevice, s));
-      HIP_TRY(hipStreamSynchronize(s));
       bool any = false;
       for (int m = 0; m < M; ++m) any |= c->h_state[m].phase == kPhaseSweep;
       if (!any) break;
@@ -981,10 +1018,12 @@ int device_reference_sampling(acvd_ctx* c, const HostMesh& h, const double* ind,
   } join{shuffler};
   DBuf<int32_t> ring, len, key;
   DBuf<double> area;
-  HIP_TRY(ring.alloc(size_t(c->E2)));
-  HIP_TRY(len.alloc(size_t(nv)));
-  HIP_TRY(key.alloc(c->d_vfcol.n));
-  HIP_TRY(area.alloc(size_t(nv)));
+  SlabPlan plan;
+  plan.add(ring, size_t(c->E2));
+  plan.add(len, size_t(nv));
+  plan.add(key, c->d_vfcol.n);
+  plan.add(area, size_t(nv));
+  HIP_TRY(plan.give(c->d_scratch));
   HIP_TRY(launch_sample_topology(s, h.item_off, nv, c->d_pos.p, c->d_tri.p, c->d_vfptr.p, c->d_vfcol.p,
                                  c->d_row_ptr.p, ring.p, len.p, key.p, area.p));
   huge_vector<int32_t> h_ring(static_cast<size_t>(h.n_adj)), h_len(static_cast<size_t>(nv)),
@@ -1237,15 +1276,17 @@ int acvd_subdivide_input(acvd_ctx* ctx, int32_t mesh_id, int64_t min_vertices, i
     if (n3 + 1 >= int64_t(INT32_MAX)) return fail(ACVD_ERR_LIMIT, "subdivision: more than 2^31 half-edges");
     DBuf<unsigned long long> k0, k1;
     DBuf<int32_t> v0, v1, flag, num, face_edge, active, fpos;
-    HIP_TRY(k0.alloc(size_t(n3)));
-    HIP_TRY(k1.alloc(size_t(n3)));
-    HIP_TRY(v0.alloc(size_t(n3)));
-    HIP_TRY(v1.alloc(size_t(n3)));
-    HIP_TRY(flag.alloc(size_t(n3 + 1)));
-    HIP_TRY(num.alloc(size_t(n3 + 1)));
-    HIP_TRY(face_edge.alloc(size_t(n3)));
-    HIP_TRY(active.alloc(size_t(nf + 1)));
-    HIP_TRY(fpos.alloc(size_t(nf + 1)));
+    SlabPlan plan;
+    plan.add(k0, size_t(n3));
+    plan.add(k1, size_t(n3));
+    plan.add(v0, size_t(n3));
+    plan.add(v1, size_t(n3));
+    plan.add(flag, size_t(n3 + 1));
+    plan.add(num, size_t(n3 + 1));
+    plan.add(face_edge, size_t(n3));
+    plan.add(active, size_t(nf + 1));
+    plan.add(fpos, size_t(nf + 1));
+    HIP_TRY(plan.give(ctx->d_scratch));
     HIP_TRY(hipMemsetAsync(flag.p + n3, 0, sizeof(int32_t), s));
     HIP_TRY(hipMemsetAsync(active.p + nf, 0, sizeof(int32_t), s));
     HIP_TRY(launch_sub_keys(s, nf, nv, tri.p, k0.p, v0.p, face_edge.p, active.p));
@@ -1366,10 +1407,14 @@ int acvd_process_clustering(acvd_ctx* ctx) {
   rc = upload_anchors(ctx);
   if (rc) return rc;
   const int M = int(ctx->meshes.size());
-  // (re)allocate the pinned state mirror for M meshes
-  if (ctx->h_state) (void)hipHostFree(ctx->h_state);
-  ctx->h_state = nullptr;
-  HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&ctx->h_state), M * sizeof(MeshState), hipHostMallocDefault));
+  // the pinned state mirror holds M meshes
+  if (ctx->h_state_n < size_t(M)) {
+    if (ctx->h_state) (void)hipHostFree(ctx->h_state);
+    ctx->h_state = nullptr;
+    ctx->h_state_n = 0;
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&ctx->h_state), M * sizeof(MeshState), hipHostMallocDefault));
+    ctx->h_state_n = size_t(M);
+  }
   for (auto& h : ctx->meshes)
     if (h.params.console_output) std::printf("Clustering......\n");
   rc = initial_labels(ctx);
@@ -1467,22 +1512,27 @@ int acvd_build_output(acvd_ctx* ctx, int32_t mesh_id, int32_t quadrics_level) {
   const int32_t K = h.params.number_of_clusters;
   DBuf<double> pts;
   DBuf<int32_t> first, otri;
-  HIP_TRY(pts.alloc(3 * size_t(K)));
-  HIP_TRY(first.alloc(1));
-  HIP_TRY(otri.alloc(3 * size_t(h.nf)));
+  DBuf<unsigned long long> acc;
+  DBuf<char> ws;
+  size_t ws_bytes = 0;
+  HIP_TRY(dual_faces_workspace(h.nf, &ws_bytes));
+  SlabPlan plan;
+  plan.add(pts, 3 * size_t(K));
+  plan.add(first, 1);
+  plan.add(otri, 3 * size_t(h.nf));
+  if (quadrics_level > 0) plan.add(acc, 10 * size_t(K));
+  plan.add(ws, ws_bytes);
+  HIP_TRY(plan.give(ctx->d_scratch));
   HIP_TRY(launch_cluster_points(s, ctx->args(), mesh_id, pts.p));
   HIP_TRY(launch_fill_i32(s, first.p, 1, K));
   HIP_TRY(fix_empty_cluster_points(s, ctx->d_sizes.p, h.clus_off, K, first.p, pts.p));
   if (quadrics_level > 0) {
-    DBuf<unsigned long long> acc;
-    HIP_TRY(acc.alloc(10 * size_t(K)));
     HIP_TRY(quadric_placement(s, h.nv, h.item_off, ctx->d_labels.p, h.clus_off, K, ctx->d_q.p,
                               ctx->h_meshes[mesh_id].scales.sq, acc.p, quadrics_level, pts.p));
-    HIP_TRY(hipStreamSynchronize(s));
   }
   int64_t nf_out = 0;
   HIP_TRY(build_dual_faces(s, h.nf, ctx->d_tri.p + 3 * h.face_off, ctx->d_labels.p, h.item_off, h.clus_off, otri.p,
-                           &nf_out));
+                           &nf_out, ws.p, ws_bytes));
   h.out_xyz.resize(3 * size_t(K));
   h.out_tri.resize(3 * size_t(nf_out));
   HIP_TRY(hipMemcpyAsync(h.out_xyz.data(), pts.p, 3 * size_t(K) * sizeof(double), hipMemcpyDeviceToHost, s));
@@ -1854,7 +1904,6 @@ int acvd_get_scales(acvd_ctx* ctx, int32_t mesh_id, double* scales3) {
 }  // extern "C"
 
 // ====================================================== fixed-assignment energy
-#include "acvd_energy.h"
 
 struct acvd_energy {
   int device = 0;

@@ -253,6 +253,21 @@ __global__ void k_ring_adj(int64_t n, const int32_t* __restrict__ row_ptr, const
 
 }  // namespace
 
+// out[m] = row_ptr at the first item of mesh m, out[M] at the end of the last.
+__global__ void k_mesh_rows(int32_t n_meshes, const DevMesh* __restrict__ meshes, const int32_t* __restrict__ row_ptr,
+                            int32_t* out) {
+  const int32_t m = int32_t(blockIdx.x) * kBlock + threadIdx.x;
+  if (m >= n_meshes) return;
+  out[m] = row_ptr[meshes[m].item_off];
+  if (m == n_meshes - 1) out[n_meshes] = row_ptr[meshes[m].item_off + meshes[m].n_items];
+}
+
+hipError_t launch_mesh_rows(hipStream_t s, int32_t n_meshes, const DevMesh* meshes, const int32_t* row_ptr,
+                            int32_t* out) {
+  hipLaunchKernelGGL(k_mesh_rows, dim3(grid_for(n_meshes)), dim3(kBlock), 0, s, n_meshes, meshes, row_ptr, out);
+  return hipGetLastError();
+}
+
 hipError_t launch_csr_count(hipStream_t s, int64_t nf, const int32_t* tri, int32_t* deg2, int32_t* vfdeg) {
   if (nf == 0) return hipSuccess;
   hipLaunchKernelGGL(k_csr_count, dim3(grid_for(nf)), dim3(kBlock), 0, s, nf, tri, deg2, vfdeg);
@@ -659,6 +674,16 @@ __device__ inline uint64_t spread3(uint32_t v) {
   return x;
 }
 
+// Tiles in vertex order: the tile slots of each mesh's items in turn.
+__global__ void k_tile_linear(SweepArgs a, int32_t* tile_items, int32_t* item_tile) {
+  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= a.n_items) return;
+  const DevMesh& dm = a.meshes[a.item_mesh ? a.item_mesh[i] : 0];
+  const int64_t local = i - dm.item_off, t = dm.tile_off + local / kTileItems;
+  tile_items[t * kTileItems + local % kTileItems] = int32_t(i);
+  item_tile[i] = int32_t(t);
+}
+
 // key = mesh << 48 | Morton code of the position quantised to 16 bits per
 // axis inside the mesh's bounding box (bbox: lo[3], scale[3] per mesh)
 __global__ void k_morton_keys(SweepArgs a, const float* __restrict__ bbox, unsigned long long* keys, int32_t* vals) {
@@ -702,6 +727,12 @@ __global__ void k_fill_tiles(int64_t n, int32_t* p) {
 hipError_t launch_tile_order(hipStream_t s, const SweepArgs& a, const float* bbox, int32_t* tile_items,
                              int32_t* item_tile, void** tmp, size_t* tmp_bytes) {
   const int64_t n = a.n_items;
+  if (!bbox) {  // vertex order: nothing to sort
+    const int64_t slots = int64_t(a.n_tiles) * kTileItems;
+    hipLaunchKernelGGL(k_fill_tiles, dim3(grid_for(slots)), dim3(kBlock), 0, s, slots, tile_items);
+    hipLaunchKernelGGL(k_tile_linear, dim3(grid_for(n)), dim3(kBlock), 0, s, a, tile_items, item_tile);
+    return hipGetLastError();
+  }
   unsigned long long *k0 = nullptr, *k1 = nullptr;
   int32_t *v0 = nullptr, *v1 = nullptr;
   hipError_t e = hipSuccess;

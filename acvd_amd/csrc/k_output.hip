@@ -115,47 +115,74 @@ __global__ void k_place(int32_t K, const unsigned long long* __restrict__ acc, d
 
 }  // namespace
 
+// Parts of the workspace of build_dual_faces.
+struct DualWorkspace {
+  unsigned long long *k0, *k1;
+  int32_t *f0, *f1, *flag, *pos;
+  void* tmp;
+  size_t tmp_bytes, total;
+};
+
+static hipError_t dual_layout(int64_t nf, char* base, DualWorkspace* w) {
+  size_t off = 0;
+  auto part = [&](size_t bytes) {
+    char* p = base ? base + off : nullptr;
+    off += (bytes + 255) / 256 * 256;
+    return p;
+  };
+  w->k0 = reinterpret_cast<unsigned long long*>(part(nf * sizeof(unsigned long long)));
+  w->k1 = reinterpret_cast<unsigned long long*>(part(nf * sizeof(unsigned long long)));
+  w->f0 = reinterpret_cast<int32_t*>(part(nf * sizeof(int32_t)));
+  w->f1 = reinterpret_cast<int32_t*>(part(nf * sizeof(int32_t)));
+  w->flag = reinterpret_cast<int32_t*>(part((nf + 1) * sizeof(int32_t)));
+  w->pos = reinterpret_cast<int32_t*>(part((nf + 1) * sizeof(int32_t)));
+  size_t sort = 0, scan = 0;
+  hipError_t e = hipcub::DeviceRadixSort::SortPairs(nullptr, sort, w->k0, w->k1, w->f0, w->f1, int(nf), 0, 64);
+  if (e != hipSuccess) return e;
+  e = hipcub::DeviceScan::ExclusiveSum(nullptr, scan, w->flag, w->pos, int(nf + 1));
+  if (e != hipSuccess) return e;
+  w->tmp_bytes = sort > scan ? sort : scan;
+  w->tmp = part(w->tmp_bytes);
+  w->total = off;
+  return hipSuccess;
+}
+
+hipError_t dual_faces_workspace(int64_t nf, size_t* bytes) {
+  DualWorkspace w;
+  const hipError_t e = dual_layout(nf, nullptr, &w);
+  *bytes = w.total;
+  return e;
+}
+
 // Builds the output triangles of one mesh (faces tri[0..nf) with global
 // vertex ids, global labels).  out_tri must hold 3*nf entries; *out_nf receives the
-// count.  Temporary device memory is allocated here.
+// count.  ws: device memory of dual_faces_workspace(nf) bytes.
 hipError_t build_dual_faces(hipStream_t s, int64_t nf, const int32_t* tri, const int32_t* labels, int64_t item_off,
-                            int64_t clus_off, int32_t* out_tri, int64_t* out_nf) {
+                            int64_t clus_off, int32_t* out_tri, int64_t* out_nf, void* ws, size_t ws_bytes) {
   *out_nf = 0;
   if (nf == 0) return hipSuccess;
-  unsigned long long *k0 = nullptr, *k1 = nullptr;
-  int32_t *f0 = nullptr, *f1 = nullptr, *flag = nullptr, *pos = nullptr;
-  void* tmp = nullptr;
-  size_t tb = 0, tb2 = 0;
-  hipError_t e = hipSuccess;
-  auto cleanup = [&]() {
-    (void)hipFree(k0); (void)hipFree(k1); (void)hipFree(f0); (void)hipFree(f1);
-    (void)hipFree(flag); (void)hipFree(pos); (void)hipFree(tmp);
-  };
-#define ACVD_OUT_TRY(x) do { e = (x); if (e != hipSuccess) { cleanup(); return e; } } while (0)
-  ACVD_OUT_TRY(hipMalloc(&k0, nf * sizeof(unsigned long long)));
-  ACVD_OUT_TRY(hipMalloc(&k1, nf * sizeof(unsigned long long)));
-  ACVD_OUT_TRY(hipMalloc(&f0, nf * sizeof(int32_t)));
-  ACVD_OUT_TRY(hipMalloc(&f1, nf * sizeof(int32_t)));
-  ACVD_OUT_TRY(hipMalloc(&flag, (nf + 1) * sizeof(int32_t)));
-  ACVD_OUT_TRY(hipMalloc(&pos, (nf + 1) * sizeof(int32_t)));
-  hipLaunchKernelGGL(k_dual_keys, dim3(grid_for(nf)), dim3(kBlock), 0, s, nf, tri, labels, item_off, clus_off, k0, f0);
+  DualWorkspace w;
+  hipError_t e = dual_layout(nf, static_cast<char*>(ws), &w);
+  if (e != hipSuccess) return e;
+  if (w.total > ws_bytes) return hipErrorInvalidValue;
+#define ACVD_OUT_TRY(x) do { e = (x); if (e != hipSuccess) return e; } while (0)
+  hipLaunchKernelGGL(k_dual_keys, dim3(grid_for(nf)), dim3(kBlock), 0, s, nf, tri, labels, item_off, clus_off, w.k0,
+                     w.f0);
   ACVD_OUT_TRY(hipGetLastError());
-  ACVD_OUT_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, k0, k1, f0, f1, int(nf), 0, 64, s));
-  ACVD_OUT_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, tb2, flag, pos, int(nf + 1), s));
-  ACVD_OUT_TRY(hipMalloc(&tmp, tb > tb2 ? tb : tb2));
-  ACVD_OUT_TRY(hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, f0, f1, int(nf), 0, 64, s));
-  ACVD_OUT_TRY(hipMemsetAsync(flag, 0, (nf + 1) * sizeof(int32_t), s));
-  hipLaunchKernelGGL(k_dual_heads, dim3(grid_for(nf)), dim3(kBlock), 0, s, nf, k1, f1, flag);
+  size_t tb = w.tmp_bytes;
+  ACVD_OUT_TRY(hipcub::DeviceRadixSort::SortPairs(w.tmp, tb, w.k0, w.k1, w.f0, w.f1, int(nf), 0, 64, s));
+  ACVD_OUT_TRY(hipMemsetAsync(w.flag, 0, (nf + 1) * sizeof(int32_t), s));
+  hipLaunchKernelGGL(k_dual_heads, dim3(grid_for(nf)), dim3(kBlock), 0, s, nf, w.k1, w.f1, w.flag);
   ACVD_OUT_TRY(hipGetLastError());
-  ACVD_OUT_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, tb2, flag, pos, int(nf + 1), s));
-  hipLaunchKernelGGL(k_dual_emit, dim3(grid_for(nf)), dim3(kBlock), 0, s, nf, tri, labels, item_off, clus_off, flag,
-                     pos, out_tri);
+  tb = w.tmp_bytes;
+  ACVD_OUT_TRY(hipcub::DeviceScan::ExclusiveSum(w.tmp, tb, w.flag, w.pos, int(nf + 1), s));
+  hipLaunchKernelGGL(k_dual_emit, dim3(grid_for(nf)), dim3(kBlock), 0, s, nf, tri, labels, item_off, clus_off, w.flag,
+                     w.pos, out_tri);
   ACVD_OUT_TRY(hipGetLastError());
   int32_t cnt = 0;
-  ACVD_OUT_TRY(hipMemcpyAsync(&cnt, pos + nf, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+  ACVD_OUT_TRY(hipMemcpyAsync(&cnt, w.pos + nf, sizeof(int32_t), hipMemcpyDeviceToHost, s));
   ACVD_OUT_TRY(hipStreamSynchronize(s));
   *out_nf = cnt;
-  cleanup();
 #undef ACVD_OUT_TRY
   return hipSuccess;
 }

@@ -1027,14 +1027,15 @@ __global__ __launch_bounds__(kBlock, METRIC == 1 ? 3 : 4) void k_eval(SweepArgs 
 // evaluate in LDS and evaluates them.  The work list, its index of slice starts
 // and a launch go; what they give, an even share of the work items for every
 // block, counts only where the blocks have more than a step or two of them.
+// The keys go straight to the clusters: the LDS table's clearing, flush and
+// barriers cost more than its merging saves here (2,562 items to convergence 1.23
+// / 1.16 ms, 163,842 7.87 / 7.83).
 template <int METRIC, bool kExtras, bool kB>
 __global__ __launch_bounds__(kBlock, METRIC == 1 ? 3 : 4) void k_scan_eval(SweepArgs a, int append) {
-  __shared__ KeyAgg agg;
   __shared__ QemPool pools[METRIC == 1 ? kBlock / 64 : 1];
   __shared__ int32_t s_n, s_cnt[kBlock / 64], s_item[kBlock];
   const MeshReader<kB> mesh(a);
   if (threadIdx.x == 0) s_n = append ? a.seg_cand[blockIdx.x] : 0;
-  keyagg_clear(&agg);
   const SweepView v = make_view<kExtras>(a);
   const int64_t seg = int64_t(blockIdx.x) * a.cand_cap;
   QemPool* pool = &pools[METRIC == 1 ? threadIdx.x >> 6 : 0];
@@ -1064,7 +1065,7 @@ __global__ __launch_bounds__(kBlock, METRIC == 1 ? 3 : 4) void k_scan_eval(Sweep
       const int32_t per = (n + kBlock / 64 - 1) / (kBlock / 64);
       const int32_t off = w * per + lane;
       const bool valid = lane < per && off < n;
-      eval_item<METRIC, kExtras, kB>(a, v, mesh, pool, &agg, false, seg, &s_n, valid, valid ? s_item[off] : 0);
+      eval_item<METRIC, kExtras, kB>(a, v, mesh, pool, nullptr, true, seg, &s_n, valid, valid ? s_item[off] : 0);
     }
   }
   __syncthreads();
@@ -1506,24 +1507,45 @@ __global__ __launch_bounds__(kBlock) void k_tile_update(SweepArgs a) {
 }
 
 // ---------------------------------------------------------------- controller
-__global__ void k_controller(SweepArgs a) {
+// One block after every pass: the pass's counts, then each sweeping mesh's phase
+// logic.  Bound by its dependent loads (7 us of every pass, whatever its work):
+// the state and the control words are read with the counters, and a context of
+// one mesh is stepped from registers (5.1 -> 3.7 us on an icosphere of 2,562).
+__global__ __launch_bounds__(kBlock) void k_controller(SweepArgs a) {
   __shared__ int any_sweep, any_clean;
+  __shared__ int s_part[2][kBlock / 64], s_round_mods[kMatchRounds], s_count[3];
+  __shared__ int s_flags;   // phase flags of mesh 0 during this pass
+  __shared__ int s_rounds;  // most accept rounds a sweeping mesh ran this pass
+  static_assert(kSlices == 64, "one wave sums the slice counters");
+  Ctrl* ctrl = a.ctrl;
+  MeshState s0{};
+  unsigned long long c_eval = 0, c_prop = 0, c_acc = 0, c_accq = 0, c_pass = 0, c_rounds = 0, c_walked = 0;
   if (threadIdx.x == 0) {
+    s0 = a.state[0];
+    c_eval = ctrl->evaluated;
+    c_prop = ctrl->proposed;
+    c_acc = ctrl->accepted;
+    c_accq = ctrl->accepted_constrained;
+    c_pass = ctrl->passes;
+    c_rounds = ctrl->rounds;
+    c_walked = ctrl->walked;
     any_sweep = 0;
     any_clean = 0;
+    s_rounds = 1;
+    s_count[0] = s_count[1] = s_count[2] = 0;
   }
-  __syncthreads();
-  __shared__ int s_work, s_props, s_mods, s_round_mods[kMatchRounds];
-  __shared__ int s_part[2][kBlock / 64];
-  static_assert(kSlices == 64, "one wave sums the slice counters");
   {  // items evaluated and proposals of the pass: sums over the work slices
      // (cleared for the next scan) and the candidate segments
     int w = 0, p = 0;
-    for (int k = threadIdx.x; k < kWorkSlices; k += blockDim.x) {
-      w += a.work_count[k];
-      a.work_count[k] = 0;
+    int wv[kWorkSlices / kBlock];
+#pragma unroll
+    for (int k = 0; k < kWorkSlices / kBlock; ++k) wv[k] = a.work_count[k * kBlock + threadIdx.x];
+    for (int k = threadIdx.x; k < a.n_seg; k += kBlock) p += a.seg_cand[k];
+#pragma unroll
+    for (int k = 0; k < kWorkSlices / kBlock; ++k) {
+      w += wv[k];
+      if (wv[k]) a.work_count[k * kBlock + threadIdx.x] = 0;
     }
-    for (int k = threadIdx.x; k < a.n_seg; k += blockDim.x) p += a.seg_cand[k];
     for (int off = 32; off > 0; off >>= 1) {
       w += __shfl_xor(w, off);
       p += __shfl_xor(p, off);
@@ -1533,59 +1555,50 @@ __global__ void k_controller(SweepArgs a) {
       s_part[1][threadIdx.x >> 6] = p;
     }
   }
-  __shared__ int s_live, s_stale, s_recheck;
-  if (threadIdx.x < 64) {  // lane k reads slice k of the move counters, wave sums
-    int dr[kMatchRounds];
-    int lv = 0, st = 0, rc = 0;
-    for (int r = 0; r < kMatchRounds; ++r) {
-      dr[r] = a.ctrl->mods[r][threadIdx.x];
-      lv += a.ctrl->live[r][threadIdx.x];
-      st += a.ctrl->stale[r][threadIdx.x];
-      rc += a.ctrl->recheck[r][threadIdx.x];
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-      for (int r = 0; r < kMatchRounds; ++r) dr[r] += __shfl_xor(dr[r], off);
-      lv += __shfl_xor(lv, off);
-      st += __shfl_xor(st, off);
-      rc += __shfl_xor(rc, off);
-    }
-    if (threadIdx.x == 0) {
-      int d = 0;
-      for (int r = 0; r < kMatchRounds; ++r) {
-        s_round_mods[r] = dr[r];
-        d += dr[r];
-      }
-      s_mods = d;
-      s_live = lv;
-      s_stale = st;
-      s_recheck = rc;
+  // wave k sums the move counters of rounds k, k + 4, ... (lane l reads slice l)
+  {
+    constexpr int kPer = kMatchRounds / (kBlock / 64);
+    static_assert(kMatchRounds % (kBlock / 64) == 0, "rounds per wave");
+    const int w = threadIdx.x >> 6, lane = __lane_id();
+    int dr[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) dr[k] = ctrl->mods[w + k * (kBlock / 64)][lane];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      if (dr[k]) ctrl->mods[w + k * (kBlock / 64)][lane] = 0;
+      for (int off = 32; off > 0; off >>= 1) dr[k] += __shfl_xor(dr[k], off);
+      if (lane == 0) s_round_mods[w + k * (kBlock / 64)] = dr[k];
     }
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int w = 0, p = 0;
-    for (int k = 0; k < kBlock / 64; ++k) {
-      w += s_part[0][k];
-      p += s_part[1][k];
+  if (a.count_rounds) {  // timed runs: the registered, re-evaluated and re-checked candidates
+    int v[3] = {0, 0, 0};
+    for (int k = threadIdx.x; k < kMatchRounds * kSlices; k += kBlock) {
+      v[0] += ctrl->live[0][k];
+      v[1] += ctrl->stale[0][k];
+      v[2] += ctrl->recheck[0][k];
+      ctrl->live[0][k] = 0;
+      ctrl->stale[0][k] = 0;
+      ctrl->recheck[0][k] = 0;
     }
-    s_work = w;
-    s_props = p;
+    for (int j = 0; j < 3; ++j)
+      if (v[j]) atomicAdd(&s_count[j], v[j]);
   }
-  __syncthreads();
-  bool ran = false;
-  __shared__ int s_flags;  // phase flags of mesh 0 during this pass
-  __shared__ int s_rounds; // most accept rounds a sweeping mesh ran this pass
-  if (threadIdx.x == 0) s_rounds = 1;
-  __syncthreads();
-  for (int m = threadIdx.x; m < a.n_meshes; m += blockDim.x) {
-    MeshState s = a.state[m];
+  int work = 0, props = 0, mods = 0;
+  for (int k = 0; k < kBlock / 64; ++k) {
+    work += s_part[0][k];
+    props += s_part[1][k];
+  }
+  for (int r = 0; r < kMatchRounds; ++r) mods += s_round_mods[r];
+  for (int m = threadIdx.x; m < a.n_meshes; m += kBlock) {
+    MeshState s = m == 0 ? s0 : a.state[m];
     if (m == 0) s_flags = (s.constrained ? 1 : 0) | (s.connexity ? 2 : 0);
     if (s.phase == kPhaseSweep) {
       atomicMax(&s_rounds, pass_rounds(s));
-      ran = true;
+      atomicOr(&any_sweep, 2);
       if (!a.item_mesh) {  // one mesh: the sliced counters are its own
-        s.pass_props = s_props;
-        s.pass_mods = s_mods;
+        s.pass_props = props;
+        s.pass_mods = mods;
       }
       controller_step(s);
       a.state[m] = s;
@@ -1593,47 +1606,38 @@ __global__ void k_controller(SweepArgs a) {
     if (s.phase == kPhaseSweep) atomicOr(&any_sweep, 1);
     if (s.phase == kPhaseNeedClean) atomicOr(&any_clean, 1);
   }
-  if (ran) atomicOr(&any_sweep, 2);
   __syncthreads();
-  if (threadIdx.x < kSlices)
-    for (int r = 0; r < kMatchRounds; ++r) {
-      a.ctrl->mods[r][threadIdx.x] = 0;
-      a.ctrl->live[r][threadIdx.x] = 0;
-      a.ctrl->stale[r][threadIdx.x] = 0;
-      a.ctrl->recheck[r][threadIdx.x] = 0;
-    }
-  if (threadIdx.x == 0 && (any_sweep & 2)) {
-    const unsigned long long pass = a.ctrl->passes;
-    int32_t* e = a.ctrl->pass_log[pass % kPassLogCap];
-    e[0] = int32_t(pass);
-    e[1] = s_work;
-    e[2] = s_props;
-    e[3] = s_mods;
+  if (threadIdx.x != 0) return;
+  const bool ran = any_sweep & 2;
+  ctrl->evaluated = c_eval + (unsigned long long)work;
+  ctrl->proposed = c_prop + (unsigned long long)props;
+  ctrl->accepted = c_acc + (unsigned long long)mods;
+  if (s_flags & 1) ctrl->accepted_constrained = c_accq + (unsigned long long)mods;
+  if (ran) {
+    int32_t* e = ctrl->pass_log[c_pass % kPassLogCap];
+    e[0] = int32_t(c_pass);
+    e[1] = work;
+    e[2] = props;
+    e[3] = mods;
     for (int r = 0; r < kMatchRounds; ++r) e[4 + r] = s_round_mods[r];
     e[4 + kMatchRounds] = s_flags;
-  }
-  if (threadIdx.x == 0) {
-    a.ctrl->evaluated += (unsigned long long)s_work;
-    a.ctrl->proposed += (unsigned long long)s_props;
-    a.ctrl->accepted += (unsigned long long)s_mods;
-    if (s_flags & 1) a.ctrl->accepted_constrained += (unsigned long long)s_mods;
     // accept rounds that walked the candidate list: round 0, and each later
     // round whose predecessor applied a move (a round after one without moves
     // exits at once); the re-evaluate kernels walked the list in all but one
-    if (any_sweep & 2) {
-      int walked = 1;
-      while (walked < s_rounds && s_round_mods[walked - 1] > 0) ++walked;
-      a.ctrl->rounds += (unsigned long long)walked;
-      a.ctrl->walked += (unsigned long long)s_props * (unsigned long long)(2 * walked - 1);
-      a.ctrl->reeval_live += (unsigned long long)s_live;
-      a.ctrl->reevaluated += (unsigned long long)s_stale;
-      a.ctrl->rechecked += (unsigned long long)s_recheck;
+    int walked = 1;
+    while (walked < s_rounds && s_round_mods[walked - 1] > 0) ++walked;
+    ctrl->rounds = c_rounds + (unsigned long long)walked;
+    ctrl->walked = c_walked + (unsigned long long)props * (unsigned long long)(2 * walked - 1);
+    if (a.count_rounds) {
+      ctrl->reeval_live += (unsigned long long)s_count[0];
+      ctrl->reevaluated += (unsigned long long)s_count[1];
+      ctrl->rechecked += (unsigned long long)s_count[2];
     }
-    a.ctrl->any_sweep = any_sweep & 1;
-    a.ctrl->seg_walk = s_props <= kSegWalkMax ? 1 : 0;
-    a.ctrl->any_need_clean = any_clean;
-    if (any_sweep & 2) a.ctrl->passes += 1;
+    ctrl->passes = c_pass + 1;
   }
+  ctrl->any_sweep = any_sweep & 1;
+  ctrl->seg_walk = props <= kSegWalkMax ? 1 : 0;
+  ctrl->any_need_clean = any_clean;
 }
 
 // ---------------------------------------------------------------------- fill

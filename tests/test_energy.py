@@ -253,6 +253,32 @@ def test_gpu_energy_rings_match_oracle(gpu_ready, metric, shape):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,K", [(1, 1), (63, 5), (1025, 40), (4096, 1024), (4096, 1025), (4097, 1024)])
+def test_gpu_iso_energy_at_the_small_path(gpu_ready, n, K):
+    """Either side of the sizes that one block takes, against the closed form in
+    FP64 (sums of at most 4,097 terms in another order: 1e-12; gradients in FP32)."""
+    import torch
+    from acvd_amd.energy import ClusterEnergy
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((n, 3)).astype(np.float32)
+    w = rng.uniform(0.5, 2.0, n).astype(np.float32)
+    lab = np.sort(rng.integers(0, K + 1, n)).astype(np.int32)  # runs, empty clusters, unlabelled items
+    ce = ClusterEnergy(0)
+    ce.add_mesh(n, [[0, 0, 0]], K, ISO)
+    tx, tw, tl = gpu_inputs(x, w, lab, K)
+    e = ce.forward_raw(tx, tw, tl)
+    dx, dw = ce.backward_raw(tx, tw, tl, torch.full((1,), 2.0, dtype=torch.float64, device=tx.device))
+    x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    W = np.bincount(lab, weights=w64, minlength=K + 1)
+    c = np.stack([np.bincount(lab, weights=w64 * x64[:, k], minlength=K + 1) for k in range(3)], 1)
+    c /= np.where(W > 0, W, 1)[:, None]
+    d = np.where((lab < K)[:, None], x64 - c[lab], 0.0)
+    np.testing.assert_allclose(e.item(), (w64 * (d ** 2).sum(1)).sum(), rtol=1e-12, atol=1e-30)
+    np.testing.assert_allclose(dx.cpu().numpy(), 4.0 * w64[:, None] * d, rtol=1e-6, atol=1e-12)
+    np.testing.assert_allclose(dw.cpu().numpy(), 2.0 * (d ** 2).sum(1), rtol=1e-6, atol=1e-12)
+
+
+@pytest.mark.gpu
 def test_gpu_energy_errors(gpu_ready):
     import torch
     from acvd_amd.energy import ClusterEnergy

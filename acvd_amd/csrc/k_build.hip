@@ -386,13 +386,67 @@ __device__ inline void for_each_star2_face(const int32_t* rp, const int32_t* col
   }
 }
 
-__global__ void k_curvature(int64_t off, int64_t n, const double* __restrict__ pos, const int32_t* __restrict__ tri,
+// The vertices within two edges of v, in the order for_each_star2_face visits them,
+// in a column of LDS (one per thread).  Whether a vertex lies within two edges is
+// then a look through some 20 ids instead of a binary search in each neighbour's
+// row, which was most of the kernel's time (352,603 vertices 3450 -> 1610 us).  A star of
+// more than kStarCap vertices does not fit and takes the searches.
+constexpr int kCurvBlock = 64;
+constexpr int kStarCap = 48;
+struct Star2 {
+  int32_t* ids;
+  int n;
+  bool fits;
+  __device__ bool has(int32_t w) const {
+    bool found = false;
+    for (int k = 0; k < n; ++k) found = found || ids[kCurvBlock * k] == w;
+    return found;
+  }
+  __device__ void push(int32_t u) {
+    if (n < kStarCap) ids[kCurvBlock * n++] = u;
+    else fits = false;
+  }
+  __device__ Star2(int32_t* column, const int32_t* rp, const int32_t* col, int32_t v) : ids(column), n(0), fits(true) {
+    push(v);
+    for (int32_t k = rp[v]; k < rp[v + 1]; ++k) push(col[k]);
+    for (int32_t k = rp[v]; k < rp[v + 1] && fits; ++k)
+      for (int32_t t = rp[col[k]]; t < rp[col[k] + 1] && fits; ++t)
+        if (!has(col[t])) push(col[t]);
+  }
+  // for_each_star2_face over the list: the same faces in the same order
+  template <class F>
+  __device__ void for_each_face(const int32_t* vfptr, const int32_t* vfcol, const int32_t* tri, F&& f) const {
+    for (int k = 0; k < n; ++k) {
+      const int32_t u = ids[kCurvBlock * k];
+      for (int32_t t = vfptr[u]; t < vfptr[u + 1]; ++t) {
+        const int32_t face = vfcol[t];
+        bool first = true;
+        for (int c = 0; c < 3; ++c) {
+          const int32_t w = tri[3 * int64_t(face) + c];
+          if (w < u && has(w)) {
+            first = false;
+            break;
+          }
+        }
+        if (first) f(face);
+      }
+    }
+  }
+};
+
+__global__ __launch_bounds__(kCurvBlock) void k_curvature(int64_t off, int64_t n, const double* __restrict__ pos, const int32_t* __restrict__ tri,
                             const int32_t* __restrict__ rp, const int32_t* __restrict__ col,
                             const int32_t* __restrict__ vfptr, const int32_t* __restrict__ vfcol,
                             double* __restrict__ out) {
   const int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (idx >= n) return;
   const int32_t v = int32_t(off + idx);
+  __shared__ int32_t s_star[kStarCap * kCurvBlock];
+  const Star2 star(s_star + threadIdx.x, rp, col, v);
+  auto for_each = [&](auto&& f) {
+    if (star.fits) star.for_each_face(vfptr, vfcol, tri, f);
+    else for_each_star2_face(rp, col, vfptr, vfcol, tri, v, f);
+  };
   // face data: area (Common/vtkSurface.cxx:1280-1283), unit normal, barycentre
   auto face = [&](int32_t f, double* area, double* nrm, double* bary) {
     const int32_t i0 = tri[3 * int64_t(f)], i1 = tri[3 * int64_t(f) + 1], i2 = tri[3 * int64_t(f) + 2];
@@ -420,7 +474,7 @@ __global__ void k_curvature(int64_t off, int64_t n, const double* __restrict__ p
   };
   double sa = 0.0, org[3] = {0, 0, 0}, f0[3] = {0, 0, 0};
   int cnt = 0;
-  for_each_star2_face(rp, col, vfptr, vfcol, tri, v, [&](int32_t f) {
+  for_each([&](int32_t f) {
     double ar, nr[3], bc[3];
     face(f, &ar, nr, bc);
     sa += ar;
@@ -457,7 +511,7 @@ __global__ void k_curvature(int64_t off, int64_t n, const double* __restrict__ p
         r[i] = 0.0;
         for (int j = 0; j < 6; ++j) M[i][j] = 0.0;
       }
-      for_each_star2_face(rp, col, vfptr, vfcol, tri, v, [&](int32_t f) {
+      for_each([&](int32_t f) {
         double ar, nr[3], bc[3];
         face(f, &ar, nr, bc);
         double d[3] = {bc[0] - org[0], bc[1] - org[1], bc[2] - org[2]};
@@ -624,7 +678,7 @@ hipError_t launch_curvature(hipStream_t s, int64_t off, int64_t n, const double*
                             const int32_t* row_ptr, const int32_t* col, const int32_t* vfptr, const int32_t* vfcol,
                             double* out) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_curvature, dim3(grid_for(n)), dim3(kBlock), 0, s, off, n, pos, tri, row_ptr, col, vfptr,
+  hipLaunchKernelGGL(k_curvature, dim3(unsigned((n + kCurvBlock - 1) / kCurvBlock)), dim3(kCurvBlock), 0, s, off, n, pos, tri, row_ptr, col, vfptr,
                      vfcol, out);
   return hipGetLastError();
 }

@@ -30,6 +30,8 @@ def meshes():
         "torus": meshgen.torus(128, 64, 3),
         "cube": meshgen.cube(40, 2, 1e-4),
         "split-ico": centroid_split(*meshgen.icosphere(3, 9, 0.02)),
+        # two-rings of more vertices than the kernel lists
+        "split-split-ico": centroid_split(*centroid_split(*meshgen.icosphere(2, 9, 0.02))),
         "open-grid": grid(40, 30, lambda u, v: np.stack([u * 0.05, v * 0.05, 0.3 * np.sin(u * 0.2) * np.cos(v * 0.15)], 1)),
         "open-cylinder": (P, T),
     }

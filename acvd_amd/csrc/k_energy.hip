@@ -715,12 +715,15 @@ __device__ inline PlaneAdjoint no_adjoint() {
 // Per vertex: dE/dx (3) and dE/dw.  QEM: the faces around the vertex v, each as
 // (v, v + u, v + s), feed the clusters of their three vertices.  The adjoints of
 // the vertex's cluster and of the first two others its ring meets are read
-// before the faces are visited (a third one, rare, in a second walk): read face
-// by face, behind the labels, they were most of this kernel's waits.  Consecutive
-// blocks run on one XCD, whose L2 then holds the rows a block shares with its
-// neighbours (HBM reads 1.27 -> 0.87 GB).  Bound by the f64 work (950
+// before the faces are visited: read face by face, behind the labels, they were
+// most of this kernel's waits.  A wave with a ring of more clusters visits the
+// faces again for the next two (against reading them face by face: labels of a
+// graded clustering of 4 x 1 M vertices 296 -> 257 us, 12 vertices a cluster
+// 306 -> 266, 42 a cluster 708 -> 715).  Consecutive blocks run on one XCD, whose
+// L2 then holds the rows a block shares with its neighbours (HBM reads 1.27 ->
+// 0.87 GB).  Bound by the f64 work (950
 // instructions per 64 vertices, half of the time) and by gather latency at 3
-// waves per SIMD (158 registers; held to 128 the spills cost more: 1359 us;
+// waves per SIMD (168 registers; held to 128 the spills cost more: 1359 us;
 // a loop over the faces that keeps one position in flight: 831 us).
 // 16.8 M QEM vertices 2050 -> 765 us, 1 M isotropic ones 10.5 -> 8.6 us.
 template <bool kQem>
@@ -761,41 +764,26 @@ __global__ __launch_bounds__(kEBlock) void ke_item_grad(EnergyArgs a, const doub
       }
     }
     if (qem && active) {
-      // clusters of the ring: code 0 the vertex's own, 1 and 2 the first two
-      // others, 3 none or a further one (more = true)
-      int32_t c1 = -1, c2 = -1;
-      uint32_t code = 0;
+      // clusters of the ring's first entries: bit k of own_bits the vertex's own, of
+      // todo another one whose part is still to be taken
       const bool is_long = e[0] == kRingLong;
-      bool more = is_long || (slots > kRingChunk && e[kRingChunk - 1] != kRingEnd);
-      {
-        int32_t l[kRingChunk];
+      const bool more = is_long || (slots > kRingChunk && e[kRingChunk - 1] != kRingEnd);
+      int32_t cl[kRingChunk];
+      uint32_t own_bits = 0, todo = 0;
 #pragma unroll
-        for (int k = 0; k < kRingChunk; ++k) {
-          if (k >= slots) break;  // wave-uniform
-          if (e[k] == kRingEnd || is_long) e[k] = int32_t(uint32_t(i) | 0x80000000u);  // no face
-          l[k] = a.labels[e[k] & kRingId];
-        }
-#pragma unroll
-        for (int k = 0; k < kRingChunk; ++k) {
-          if (k >= slots) break;
-          const int32_t cj = cluster_of(em, l[k]);
-          uint32_t t = 3;
-          if (cj == c) t = c >= 0 ? 0 : 3;
-          else if (cj >= 0) {
-            if (c1 < 0) c1 = cj;
-            if (cj == c1) t = 1;
-            else {
-              if (c2 < 0) c2 = cj;
-              if (cj == c2) t = 2;
-              else more = true;
-            }
-          }
-          code |= t << (2 * k);
-        }
+      for (int k = 0; k < kRingChunk; ++k) {
+        if (k >= slots) break;  // wave-uniform
+        if (e[k] == kRingEnd || is_long) e[k] = int32_t(uint32_t(i) | 0x80000000u);  // no face
+        cl[k] = a.labels[e[k] & kRingId];
       }
-      const PlaneAdjoint A0 = c >= 0 ? plane_adjoint(a.adj + kAdjStride * int64_t(c), x) : no_adjoint();
-      const PlaneAdjoint A1 = c1 >= 0 ? plane_adjoint(a.adj + kAdjStride * int64_t(c1), x) : no_adjoint();
-      const PlaneAdjoint A2 = c2 >= 0 ? plane_adjoint(a.adj + kAdjStride * int64_t(c2), x) : no_adjoint();
+#pragma unroll
+      for (int k = 0; k < kRingChunk; ++k) {
+        if (k >= slots) break;
+        cl[k] = cluster_of(em, cl[k]);
+        if (cl[k] >= 0) (cl[k] == c ? own_bits : todo) |= 1u << k;
+      }
+      PlaneAdjoint A0 = c >= 0 ? plane_adjoint(a.adj + kAdjStride * int64_t(c), x) : no_adjoint();
+      double own = c >= 0 ? 1.0 : 0.0;
       // the face (v, v + u, v + s) with adjoint F: n = u x s; u receives s x dn,
       // s receives dn x u, and v minus both (dn x (u - s)) and minus (g . n) n
       auto pull = [&](const PlaneAdjoint& F, const Vec3& u, const Vec3& s) {
@@ -809,51 +797,59 @@ __global__ __launch_bounds__(kEBlock) void ke_item_grad(EnergyArgs a, const doub
         gx[2] -= __builtin_fma(gn, n.z, __builtin_fma(n0, t.y, -(n1 * t.x)));
       };
       Vec3 u{0.0, 0.0, 0.0};
-      const double own = c >= 0 ? 1.0 : 0.0;
+      while (true) {
+        int32_t c1 = -1, c2 = -1;
+        uint32_t bits1 = 0, bits2 = 0;
 #pragma unroll
-      for (int k = 0; k < kRingChunk; ++k) {
-        if (k >= slots) break;
-        const Vec3 s = sub(ring_point(a, e[k]), x);
-        if (k > 0 && e[k] >= 0) {
-          const uint32_t tu = code >> (2 * (k - 1)) & 3u, ts = code >> (2 * k) & 3u;
-          const double w0 = own + (tu == 0 ? 1.0 : 0.0) + (ts == 0 ? 1.0 : 0.0);
-          const double w1 = (tu == 1 ? 1.0 : 0.0) + (ts == 1 ? 1.0 : 0.0);
-          const double w2 = (tu == 2 ? 1.0 : 0.0) + (ts == 2 ? 1.0 : 0.0);
-          PlaneAdjoint F;
-          for (int j = 0; j < 6; ++j) F.m[j] = __builtin_fma(w2, A2.m[j], __builtin_fma(w1, A1.m[j], w0 * A0.m[j]));
-          for (int j = 0; j < 3; ++j) F.g[j] = __builtin_fma(w2, A2.g[j], __builtin_fma(w1, A1.g[j], w0 * A0.g[j]));
-          pull(F, u, s);
+        for (int k = 0; k < kRingChunk; ++k) {
+          if (k >= slots) break;
+          if (!(todo >> k & 1u)) continue;
+          if (c1 < 0) c1 = cl[k];
+          if (cl[k] == c1) bits1 |= 1u << k;
+          else {
+            if (c2 < 0) c2 = cl[k];
+            if (cl[k] == c2) bits2 |= 1u << k;
+          }
         }
-        u = s;
+        todo &= ~(bits1 | bits2);
+        const PlaneAdjoint A1 = c1 >= 0 ? plane_adjoint(a.adj + kAdjStride * int64_t(c1), x) : no_adjoint();
+        const PlaneAdjoint A2 = c2 >= 0 ? plane_adjoint(a.adj + kAdjStride * int64_t(c2), x) : no_adjoint();
+#pragma unroll
+        for (int k = 0; k < kRingChunk; ++k) {
+          if (k >= slots) break;
+          const Vec3 s = sub(ring_point(a, e[k]), x);
+          if (k > 0 && e[k] >= 0) {
+            const double w0 = own + ((own_bits >> (k - 1) & 1u) ? 1.0 : 0.0) + ((own_bits >> k & 1u) ? 1.0 : 0.0);
+            const double w1 = ((bits1 >> (k - 1) & 1u) ? 1.0 : 0.0) + ((bits1 >> k & 1u) ? 1.0 : 0.0);
+            const double w2 = ((bits2 >> (k - 1) & 1u) ? 1.0 : 0.0) + ((bits2 >> k & 1u) ? 1.0 : 0.0);
+            PlaneAdjoint F;
+            for (int j = 0; j < 6; ++j)
+              F.m[j] = __builtin_fma(w2, A2.m[j], __builtin_fma(w1, A1.m[j], w0 * A0.m[j]));
+            for (int j = 0; j < 3; ++j)
+              F.g[j] = __builtin_fma(w2, A2.g[j], __builtin_fma(w1, A1.g[j], w0 * A0.g[j]));
+            pull(F, u, s);
+          }
+          u = s;
+        }
+        if (__ballot(todo != 0) == 0ull) break;
+        // rings of more clusters: the faces again for the next two, the own part done
+        A0 = no_adjoint();
+        own = 0.0;
+        own_bits = 0;
       }
-      if (more) {
-        // faces past the first entries in full; of the others the part of the
-        // clusters the codes leave out
-        auto tag = [&](int32_t j) { return cluster_of(em, a.labels[j]); };
+      if (more) {  // faces past the first entries, in full
         auto pull_of = [&](int32_t cj, const Vec3& r, const Vec3& s) {
           if (cj >= 0) pull(plane_adjoint(a.adj + kAdjStride * int64_t(cj), x), r, s);
         };
-        int32_t cu = -1;
-        u = Vec3{0.0, 0.0, 0.0};
-        if (!is_long)
-          for (int k = 0; k < kRingChunk; ++k) {
-            const int32_t ek = k < slots ? a.ring[int64_t(a.ring_slot[i >> 6] + k) * 64 + (i & 63)] : kRingEnd;
-            if (ek == kRingEnd) break;
-            const Vec3 s = sub(ring_point(a, ek), x);
-            const int32_t cs = tag(ek & kRingId);
-            if (ek >= 0) {
-              if (cu != c && cu != c1 && cu != c2) pull_of(cu, u, s);
-              if (cs != c && cs != c1 && cs != c2) pull_of(cs, u, s);
-            }
-            u = s;
-            cu = cs;
-          }
-        walk_rest(a, i, x, is_long ? kRingLong : 0, kRingChunk, u, cu, tag,
-                  [&](const Vec3& r, int32_t cr, const Vec3& s, int32_t cs) {
-                    pull_of(c, r, s);
-                    pull_of(cr, r, s);
-                    pull_of(cs, r, s);
-                  });
+        const int32_t cu = is_long ? -1 : cl[kRingChunk - 1];
+        walk_rest(
+            a, i, x, is_long ? kRingLong : 0, kRingChunk, u, cu,
+            [&](int32_t j) { return cluster_of(em, a.labels[j]); },
+            [&](const Vec3& r, int32_t cr, const Vec3& s, int32_t cs) {
+              pull_of(c, r, s);
+              pull_of(cr, r, s);
+              pull_of(cs, r, s);
+            });
       }
     }
     if (active) {

@@ -35,8 +35,8 @@ static_assert(kSweepSegs <= kMaxSeg, "segment index bound");
 // Candidate lists of at most this many proposals (last pass) are walked one
 // segment per block, longer ones evenly through an index of the segments.
 constexpr int kSegWalkMax = 16384;
-// Scan tiles: groups of kTileItems items of one mesh in spatial (Morton)
-// order.  Each tile keeps a superset of the clusters its items and their
+// Scan tiles: groups of kTileItems items of one mesh in vertex order (Morton
+// order on request).  Each tile keeps a superset of the clusters its items and their
 // neighbours belong to; a tile none of whose clusters changed in the last
 // pass (and none of whose proposals lost) has no item to evaluate and is
 // skipped after reading that set.

@@ -89,9 +89,10 @@ typedef struct acvd_params {
  * nearest knob is vtkThreadedClustering's PoolingRatio / mesh slices,
  * DiscreteRemeshing/vtkThreadedClustering.h:58-74, 891-987).  None of the
  * knobs changes the labels; they trade launches, occupancy and host syncs:
- *   sweep_segments      evaluate / accept-round grid (blocks) cap, 1..2048 (default 1152)
+ *   sweep_segments      evaluate / accept-round grid (blocks) cap, 1..2048 (default 768)
  *   tile_on_divisor     the scan's tile sets are kept once a pass moves at most K / divisor
- *                       items, 1..1024 (default 16)
+ *                       items, 1..1024 (default 16); contexts of at most 700,000
+ *                       items keep none
  *   chunk_passes        passes per captured graph launch, 1..16 (default 16)
  *   short_chunk_passes  passes per launch near the end of a phase, 1..chunk_passes (default 4) */
 typedef struct acvd_tuning {

@@ -93,7 +93,7 @@ EXPORTS = [
     "acvd_get_energy_log", "acvd_force_manifold",
     "acvd_set_frozen_clusters", "acvd_vertex_manifold", "acvd_force_manifold_step", "acvd_fix_mesh_boundaries",
     "acvd_mesh_boundary_fix", "acvd_reference_seed_sampling", "acvd_set_tuning", "acvd_get_tuning", "acvd_autotune",
-    "acvd_energy_forward_cvt_noalloc",
+    "acvd_energy_forward_cvt_noalloc", "acvd_set_path_limits", "acvd_get_path_passes",
 ]
 
 _lib = None
@@ -168,6 +168,8 @@ def lib():
     L.acvd_reference_seed_sampling.argtypes = [i64, i32, P]
     L.acvd_set_tuning.argtypes = [P, ctypes.POINTER(Tuning)]
     L.acvd_get_tuning.argtypes = [P, ctypes.POINTER(Tuning)]
+    L.acvd_set_path_limits.argtypes = [P, i64, i64]
+    L.acvd_get_path_passes.argtypes = [P, ctypes.POINTER(i64)]
     L.acvd_autotune.argtypes = [P, i32, ctypes.POINTER(Tuning), ctypes.POINTER(ctypes.c_double)]
     L.acvd_mesh_boundary_fix.argtypes = [i64, P, i64, P, P, i32, ctypes.POINTER(i64), ctypes.POINTER(i64), P, P]
     L.acvd_vertex_manifold.argtypes = [i64, i64, P, P]

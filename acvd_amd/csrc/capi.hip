@@ -180,6 +180,11 @@ struct acvd_ctx {
   int32_t work_cap = 0, n_seg = 0, cand_cap = 0;
   // launch-shape knobs (acvd_set_tuning); none changes the labels
   acvd_tuning tuning = {kSweepSegs, kTileOnDivisor, kChunk, kShortChunk};
+  // item counts up to which the fused scan runs and above which tile sets are
+  // kept (acvd_set_path_limits), and the passes the last run launched per path
+  int64_t fused_items = kFusedItems, tile_min_items = kTileMinItems;
+  enum Path { kPathFused = 0, kPathList = 1, kPathTiles = 2, kPaths = 3 };
+  int64_t path_passes[kPaths] = {};
   // scan tiles
   int32_t n_tiles = 0;
   DBuf<int32_t> d_tile_items, d_item_tile, d_tile_mesh, d_tile_cnt, d_tile_set, d_tile_prop;
@@ -657,7 +662,7 @@ int recompute_statistics(acvd_ctx* c, const int32_t* mask, int set_stamp, unsign
 int enqueue_chunk(acvd_ctx* c, bool qem_unc, bool tiles, int n_pass, int n_rounds) {
   hipStream_t s = c->stream;
   SweepArgs a = c->args();
-  const bool fused = !tiles && c->N <= kFusedItems;
+  const bool fused = !tiles && c->N <= c->fused_items;
   for (int p = 0; p < n_pass; ++p) {
     if (fused) {
       HIP_TRY(launch_scan_eval(s, a, c->any_iso, c->any_qem, qem_unc));
@@ -682,7 +687,7 @@ int enqueue_chunk(acvd_ctx* c, bool qem_unc, bool tiles, int n_pass, int n_round
 int run_chunk_timed(acvd_ctx* c, bool qem_unc, bool tiles, int n_pass, int n_rounds) {
   hipStream_t s = c->stream;
   SweepArgs a = c->args();
-  const bool fused = !tiles && c->N <= kFusedItems;
+  const bool fused = !tiles && c->N <= c->fused_items;
   std::vector<hipEvent_t> ev(5 * n_pass);
   for (auto& e : ev) HIP_TRY(hipEventCreate(&e));
   for (int p = 0; p < n_pass; ++p) {
@@ -730,6 +735,8 @@ int run_chunk(acvd_ctx* c, bool use_graph, bool qem_unc, bool tiles, bool short_
   hipStream_t s = c->stream;
   const int n_pass = short_chunk ? c->tuning.short_chunk_passes : c->tuning.chunk_passes;
   const int n_rounds = chunk_rounds(c);
+  c->path_passes[tiles ? acvd_ctx::kPathTiles : c->N <= c->fused_items ? acvd_ctx::kPathFused : acvd_ctx::kPathList] +=
+      n_pass;
   if (c->timing) return run_chunk_timed(c, qem_unc, tiles, n_pass, n_rounds);
   if (use_graph) {
     const int k = int(qem_unc) + 2 * int(tiles) + 4 * int(short_chunk) + 8 * (n_rounds - 1);
@@ -914,6 +921,7 @@ int minimize_energy(acvd_ctx* c) {
     c->kernel_ms[k] = 0.0;
     c->kernel_launches[k] = 0;
   }
+  for (auto& n : c->path_passes) n = 0;
   std::vector<int32_t> mask(M), ndisc(M);
   int64_t guard = 0;
   // per-loop console output (SetConsoleOutput(2), vtkUniformClustering.h:751-758)
@@ -984,7 +992,7 @@ int minimize_energy(acvd_ctx* c) {
       near_end = 2 * int64_t(c->h_ctrl->pass_log[(c->h_ctrl->passes - 1) % kPassLogCap][2]) <= 3 * stop_props;
     // tile sets on once the last pass moved at most K / kTileOnDivisor items:
     // most tiles then hold no changed cluster and the scan skips them
-    if (!tiles && c->N > kTileMinItems && c->h_ctrl->passes > 0 &&
+    if (!tiles && c->N > c->tile_min_items && c->h_ctrl->passes > 0 &&
         int64_t(c->h_ctrl->pass_log[(c->h_ctrl->passes - 1) % kPassLogCap][3]) * c->tuning.tile_on_divisor <= c->K) {
       HIP_TRY(launch_tile_sets(s, a, nullptr));
       tiles = true;
@@ -1562,6 +1570,21 @@ int acvd_get_tuning(acvd_ctx* ctx, acvd_tuning* t) {
   if (int rc = check_ctx(ctx)) return rc;
   if (!t) return fail(ACVD_ERR_ARG, "null tuning");
   *t = ctx->tuning;
+  return ACVD_OK;
+}
+
+int acvd_set_path_limits(acvd_ctx* ctx, int64_t fused_items, int64_t tile_min_items) {
+  if (int rc = check_ctx(ctx)) return rc;
+  ctx->fused_items = fused_items < 0 ? kFusedItems : fused_items;
+  ctx->tile_min_items = tile_min_items < 0 ? kTileMinItems : tile_min_items;
+  ctx->drop_graphs();
+  return ACVD_OK;
+}
+
+int acvd_get_path_passes(const acvd_ctx* ctx, int64_t* passes) {
+  if (int rc = check_ctx(ctx)) return rc;
+  if (!passes) return fail(ACVD_ERR_ARG, "null buffer");
+  for (int k = 0; k < acvd_ctx::kPaths; ++k) passes[k] = ctx->path_passes[k];
   return ACVD_OK;
 }
 

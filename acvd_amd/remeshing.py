@@ -216,6 +216,18 @@ class Context:
         check(N.lib().acvd_get_tuning(self._h, ctypes.byref(t)))
         return {k: getattr(t, k) for k, _ in t._fields_}
 
+    def set_path_limits(self, fused_items=-1, tile_min_items=-1):
+        """Item counts at which the kernels of a pass change
+        (acvd_set_path_limits; negative: the default)."""
+        check(N.lib().acvd_set_path_limits(self._h, int(fused_items), int(tile_min_items)))
+
+    def path_passes(self):
+        """Passes the last run launched fused, with scan and evaluate apart, and
+        apart with tile sets (acvd_get_path_passes)."""
+        n = (ctypes.c_int64 * 3)()
+        check(N.lib().acvd_get_path_passes(self._h, n))
+        return {"fused": n[0], "list": n[1], "tiles": n[2]}
+
     def autotune(self, repeats=2):
         """acvd_autotune: (best launch shape, device ms per clustering); the
         shape stays set."""

@@ -326,6 +326,15 @@ int acvd_build(acvd_ctx* ctx);
 int acvd_set_tuning(acvd_ctx* ctx, const acvd_tuning* t);
 int acvd_get_tuning(acvd_ctx* ctx, acvd_tuning* t);
 int acvd_autotune(acvd_ctx* ctx, int32_t repeats, acvd_tuning* best, double* best_ms);
+/* The kernels of a pass depend on the context's items: at most fused_items
+ * (default 196,608) scan and evaluate in one kernel, more than tile_min_items
+ * (default 700,000) keep tile sets once few items move.  These calls set the
+ * two limits (negative: the default) and report which kernels the last run
+ * took, so that a test can drive every path on a small mesh; the labels depend
+ * on neither.  passes[3]: passes launched with the fused kernel, with scan and
+ * evaluate apart, and apart with tile sets. */
+int acvd_set_path_limits(acvd_ctx* ctx, int64_t fused_items, int64_t tile_min_items);
+int acvd_get_path_passes(const acvd_ctx* ctx, int64_t* passes);
 
 /* ---- ForceManifold (Remesh with SetForceManifold(1)) ------------------------
  * acvd_force_manifold: the restart loop of vtkDiscreteRemeshing::Remesh

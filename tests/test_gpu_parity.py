@@ -142,6 +142,8 @@ def test_labels_bit_exact_where_the_scan_changes(gpu_ready, nu, nv, metric):
                               max_loops=200000)
     st = ctx.stats(0)
     print(nu * nv, st["loops"], st["total_moves"], flush=True)
+    ran = {k for k, n in ctx.path_passes().items() if n > 0}
+    assert ran == ({"fused"} if nu * nv <= 196608 else {"list"} if nu * nv <= 700000 else {"list", "tiles"}), ran
     assert st["loops"] == rst["loops"] and st["total_moves"] == rst["total_moves"]
     np.testing.assert_array_equal(ctx.labels(0), rlab)
 

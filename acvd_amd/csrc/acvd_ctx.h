@@ -35,6 +35,15 @@ static_assert(kSweepSegs <= kMaxSeg, "segment index bound");
 // Candidate lists of at most this many proposals (last pass) are walked one
 // segment per block, longer ones evenly through an index of the segments.
 constexpr int kSegWalkMax = 16384;
+// A pass is crowded when it proposes more than this many moves per cluster of
+// some mesh.  Short lists and small contexts register their accept keys straight
+// at the clusters; atomics on one address take their turns, so the chunk of
+// passes after a crowded one merges the keys of a block in its LDS table first.  To
+// convergence, isotropic, direct always / crowded from 32 / 16 / 8 / 4 / 1 per
+// cluster: torus of 256,000 vertices into 50 clusters 1355 / 778 / 768 / 765 /
+// 765 / 764 ms, icosphere of 163,842 into 300 79.3 / 73.7 / 70.9 / 70.3 / 70.3 /
+// 70.5, of 40,962 into 500 12.33 / 12.27 / 12.30 / 12.20 / 12.29 / 12.36.
+constexpr int32_t kCrowdedProps = 8;
 // Scan tiles: groups of kTileItems items of one mesh in vertex order (Morton
 // order on request).  Each tile keeps a superset of the clusters its items and their
 // neighbours belong to; a tile none of whose clusters changed in the last
@@ -101,6 +110,7 @@ struct Ctrl {
   int32_t any_need_clean;
   int32_t fill_changed;
   int32_t seg_walk;  // candidate walk of the next pass: 1 segment per block, 0 dense
+  int32_t crowded;   // the last pass was crowded (kCrowdedProps)
   int32_t mods[kMatchRounds][kSlices];  // applied moves of this pass, per accept round
   int32_t live[kMatchRounds][kSlices];  // candidates registered by the re-evaluate of round r
   int32_t stale[kMatchRounds][kSlices]; // candidates re-evaluated in round r
@@ -136,6 +146,7 @@ struct SweepArgs {
   const unsigned long long* ring_adj;  // ring adjacency per item (ring_adjacency of acvd_math.h)
   const int32_t* anchor;     // per cluster: global id of its fixed item or -1; null when no mesh has any
   const int32_t* frozen;     // per cluster: nonzero when frozen (ForceManifold restarts); null when none is
+  int32_t crowded;           // accept keys go through the blocks' tables (kCrowdedProps)
   int32_t count_rounds;      // count the live and re-evaluated candidates of each round (timed runs)
   const float4* xw;          // position + weight
   const float* q;            // 10 floats per item (QEM meshes), may be null

@@ -209,7 +209,7 @@ struct acvd_ctx {
   // pass-chunk graphs by (QEM meshes unconstrained, tile sets maintained,
   // short chunk): index qem_unc + 2 * tiles + 4 * short
   // captured chunks by (QEM unconstrained, tile sets on, short, rounds - 1)
-  static constexpr int kChunkKinds = 8 * kMatchRounds;
+  static constexpr int kChunkKinds = 16 * kMatchRounds;
   hipGraphExec_t chunk_exec[kChunkKinds] = {};
   hipGraph_t chunk_graph[kChunkKinds] = {};
   double build_ms = 0.0, converge_ms = 0.0;
@@ -659,9 +659,10 @@ int recompute_statistics(acvd_ctx* c, const int32_t* mask, int set_stamp, unsign
   return ACVD_OK;
 }
 
-int enqueue_chunk(acvd_ctx* c, bool qem_unc, bool tiles, int n_pass, int n_rounds) {
+int enqueue_chunk(acvd_ctx* c, bool qem_unc, bool tiles, bool crowded, int n_pass, int n_rounds) {
   hipStream_t s = c->stream;
   SweepArgs a = c->args();
+  a.crowded = crowded ? 1 : 0;
   const bool fused = !tiles && c->N <= c->fused_items;
   for (int p = 0; p < n_pass; ++p) {
     if (fused) {
@@ -684,9 +685,10 @@ int enqueue_chunk(acvd_ctx* c, bool qem_unc, bool tiles, int n_pass, int n_round
 }
 
 // Passes launched one by one with events around each kernel.
-int run_chunk_timed(acvd_ctx* c, bool qem_unc, bool tiles, int n_pass, int n_rounds) {
+int run_chunk_timed(acvd_ctx* c, bool qem_unc, bool tiles, bool crowded, int n_pass, int n_rounds) {
   hipStream_t s = c->stream;
   SweepArgs a = c->args();
+  a.crowded = crowded ? 1 : 0;
   const bool fused = !tiles && c->N <= c->fused_items;
   std::vector<hipEvent_t> ev(5 * n_pass);
   for (auto& e : ev) HIP_TRY(hipEventCreate(&e));
@@ -731,18 +733,18 @@ int chunk_rounds(const acvd_ctx* c) {
   return r;
 }
 
-int run_chunk(acvd_ctx* c, bool use_graph, bool qem_unc, bool tiles, bool short_chunk) {
+int run_chunk(acvd_ctx* c, bool use_graph, bool qem_unc, bool tiles, bool short_chunk, bool crowded) {
   hipStream_t s = c->stream;
   const int n_pass = short_chunk ? c->tuning.short_chunk_passes : c->tuning.chunk_passes;
   const int n_rounds = chunk_rounds(c);
   c->path_passes[tiles ? acvd_ctx::kPathTiles : c->N <= c->fused_items ? acvd_ctx::kPathFused : acvd_ctx::kPathList] +=
       n_pass;
-  if (c->timing) return run_chunk_timed(c, qem_unc, tiles, n_pass, n_rounds);
+  if (c->timing) return run_chunk_timed(c, qem_unc, tiles, crowded, n_pass, n_rounds);
   if (use_graph) {
-    const int k = int(qem_unc) + 2 * int(tiles) + 4 * int(short_chunk) + 8 * (n_rounds - 1);
+    const int k = int(qem_unc) + 2 * int(tiles) + 4 * int(short_chunk) + 8 * int(crowded) + 16 * (n_rounds - 1);
     if (!c->chunk_exec[k]) {
       HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-      int rc = enqueue_chunk(c, qem_unc, tiles, n_pass, n_rounds);
+      int rc = enqueue_chunk(c, qem_unc, tiles, crowded, n_pass, n_rounds);
       hipGraph_t g = nullptr;
       hipError_t ec = hipStreamEndCapture(s, &g);
       if (rc != ACVD_OK) return rc;
@@ -753,7 +755,7 @@ int run_chunk(acvd_ctx* c, bool use_graph, bool qem_unc, bool tiles, bool short_
     HIP_TRY(hipGraphLaunch(c->chunk_exec[k], s));
     return ACVD_OK;
   }
-  return enqueue_chunk(c, qem_unc, tiles, n_pass, n_rounds);
+  return enqueue_chunk(c, qem_unc, tiles, crowded, n_pass, n_rounds);
 }
 
 // True when no QEM mesh of the context is constrained (the state flips only
@@ -940,11 +942,13 @@ int minimize_energy(acvd_ctx* c) {
   };
   int64_t stop_props = early_stop_props();
   bool near_end = false;  // short chunks: the phase is about to end
+  bool crowded = false;   // the last chunk ended with a crowded pass
   while (true) {
-    int rc2 = run_chunk(c, use_graph, qem_unconstrained(c), tiles, near_end);
+    int rc2 = run_chunk(c, use_graph, qem_unconstrained(c), tiles, near_end, crowded);
     if (rc2) return rc2;
     HIP_TRY(hipMemcpyAsync(c->h_ctrl, c->d_ctrl.p, sizeof(Ctrl), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
+    crowded = c->h_ctrl->crowded != 0;
     rc = drain_energy_log(c);
     if (rc) return rc;
     if (loop_output) print_pass_log(*c->h_ctrl, &printed);

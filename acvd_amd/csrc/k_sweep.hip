@@ -1011,7 +1011,7 @@ __global__ __launch_bounds__(kBlock, METRIC == 1 ? 3 : 4) void k_eval(SweepArgs 
   const SweepView v = make_view<kExtras>(a);
   const int64_t seg = int64_t(blockIdx.x) * a.cand_cap;
   QemPool* pool = &pools[METRIC == 1 ? threadIdx.x >> 6 : 0];
-  const bool direct = n <= kSegWalkMax;  // few keys are not worth the table's barriers
+  const bool direct = n <= kSegWalkMax && !a.crowded;  // few keys apart are not worth the table's barriers
   const EvenWalk ew(n);
   for (int32_t base = ew.first; base < n; base += ew.stride) {
     const bool valid = ew.valid(base);
@@ -1027,14 +1027,16 @@ __global__ __launch_bounds__(kBlock, METRIC == 1 ? 3 : 4) void k_eval(SweepArgs 
 // evaluate in LDS and evaluates them.  The work list, its index of slice starts
 // and a launch go; what they give, an even share of the work items for every
 // block, counts only where the blocks have more than a step or two of them.
-// The keys go straight to the clusters: the LDS table's clearing, flush and
-// barriers cost more than its merging saves here (2,562 items to convergence 1.23
-// / 1.16 ms, 163,842 7.87 / 7.83).
-template <int METRIC, bool kExtras, bool kB>
+// The keys go straight to the clusters (kTable: a crowded chunk): the LDS table's
+// clearing, flush and barriers cost more than its merging saves here (2,562 items
+// into 170 clusters to convergence 1.23 / 1.16 ms, 163,842 into 10,900 7.87 / 7.83).
+template <int METRIC, bool kExtras, bool kB, bool kTable>
 __global__ __launch_bounds__(kBlock, METRIC == 1 ? 3 : 4) void k_scan_eval(SweepArgs a, int append) {
+  __shared__ KeyAgg agg;  // kTable
   __shared__ QemPool pools[METRIC == 1 ? kBlock / 64 : 1];
   __shared__ int32_t s_n, s_cnt[kBlock / 64], s_item[kBlock];
   const MeshReader<kB> mesh(a);
+  if (kTable) keyagg_clear(&agg);  // made visible by the barriers of the first step
   if (threadIdx.x == 0) s_n = append ? a.seg_cand[blockIdx.x] : 0;
   const SweepView v = make_view<kExtras>(a);
   const int64_t seg = int64_t(blockIdx.x) * a.cand_cap;
@@ -1065,7 +1067,8 @@ __global__ __launch_bounds__(kBlock, METRIC == 1 ? 3 : 4) void k_scan_eval(Sweep
       const int32_t per = (n + kBlock / 64 - 1) / (kBlock / 64);
       const int32_t off = w * per + lane;
       const bool valid = lane < per && off < n;
-      eval_item<METRIC, kExtras, kB>(a, v, mesh, pool, nullptr, true, seg, &s_n, valid, valid ? s_item[off] : 0);
+      eval_item<METRIC, kExtras, kB>(a, v, mesh, pool, kTable ? &agg : nullptr, !kTable, seg, &s_n, valid,
+                                     valid ? s_item[off] : 0);
     }
   }
   __syncthreads();
@@ -1185,10 +1188,10 @@ __device__ inline void reeval_entry(const SweepArgs& a, const SweepView& v, cons
 // against the state left by round r-1: it registers its round-r key with its
 // (possibly new) target or is dropped (-3).  The others keep their move, whose
 // dE depends only on the two unchanged clusters, and register it again.
-// A short list (one segment per block) registers straight at the global keys:
-// its few keys are not worth the LDS table's barriers.
+// A short list (one segment per block) registers straight at the global keys
+// (kTable, a crowded chunk: not): its few keys are not worth the LDS table's barriers.
 // kCount: count the registered and re-evaluated candidates (timed runs).
-template <int METRIC, bool kExtras, bool kB, bool kCount>
+template <int METRIC, bool kExtras, bool kB, bool kCount, bool kTable>
 __global__ __launch_bounds__(kBlock, METRIC == 1 ? 3 : 4) void k_reeval(SweepArgs a, int round) {
   __shared__ KeyAgg agg;
   __shared__ SegIndex si;
@@ -1201,16 +1204,17 @@ __global__ __launch_bounds__(kBlock, METRIC == 1 ? 3 : 4) void k_reeval(SweepArg
   const SweepView v = make_view<kExtras>(a);
   QemPool* pool = &pools[METRIC == 1 ? threadIdx.x >> 6 : 0];
   int n_live = 0, n_stale = 0, n_recheck = 0;
-  if (!w.by_seg) keyagg_clear(&agg);  // made visible by the index's barrier
+  if (kTable || !w.by_seg) keyagg_clear(&agg);  // made visible by the index's barrier
+  if (kTable && w.by_seg) __syncthreads();      // (without an index by this one)
   walk_candidates(a, w, &si, rec, [&](bool valid, int64_t e, const CandRec& c) {
     reeval_entry<METRIC, kExtras, kB, kCount>(
         a, v, mesh, pool, valid, e, c, round,
         [&](int32_t cl, unsigned long long key) {
-          if (w.by_seg) atomicMin(&a.prio[cl], key);
+          if (!kTable && w.by_seg) atomicMin(&a.prio[cl], key);
           else keyagg_min(&agg, cl, key);
         },
         &n_live, &n_stale, &n_recheck);
-    if (!w.by_seg) keyagg_flush(&agg, a.prio);
+    if (kTable || !w.by_seg) keyagg_flush(&agg, a.prio);
   });
   // candidates registered and re-evaluated in this round (statistics of the
   // timed runs: the block sums cost a few barriers per round)
@@ -1600,6 +1604,7 @@ __global__ __launch_bounds__(kBlock) void k_controller(SweepArgs a) {
         s.pass_props = props;
         s.pass_mods = mods;
       }
+      if (s.pass_props > kCrowdedProps * (a.item_mesh ? int64_t(a.meshes[m].K) : a.n_clusters)) atomicOr(&any_sweep, 4);
       controller_step(s);
       a.state[m] = s;
     }
@@ -1637,6 +1642,7 @@ __global__ __launch_bounds__(kBlock) void k_controller(SweepArgs a) {
   }
   ctrl->any_sweep = any_sweep & 1;
   ctrl->seg_walk = props <= kSegWalkMax ? 1 : 0;
+  ctrl->crowded = any_sweep & 4 ? 1 : 0;
   ctrl->any_need_clean = any_clean;
 }
 
@@ -2058,12 +2064,17 @@ hipError_t launch_eval(hipStream_t s, const SweepArgs& a, bool any_iso, bool any
   return hipGetLastError();
 }
 
+template <bool kX, bool kB, bool kT>
+void launch_scan_eval_t(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained) {
+  const dim3 g(unsigned(a.n_seg)), b(kBlock);
+  if (any_iso) hipLaunchKernelGGL((k_scan_eval<0, kX, kB, kT>), g, b, 0, s, a, 0);
+  if (any_qem && qem_unconstrained) hipLaunchKernelGGL((k_scan_eval<2, kX, kB, kT>), g, b, 0, s, a, any_iso ? 1 : 0);
+  else if (any_qem) hipLaunchKernelGGL((k_scan_eval<1, kX, kB, kT>), g, b, 0, s, a, any_iso ? 1 : 0);
+}
 template <bool kX, bool kB>
 void launch_scan_eval_x(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained) {
-  const dim3 g(unsigned(a.n_seg)), b(kBlock);
-  if (any_iso) hipLaunchKernelGGL((k_scan_eval<0, kX, kB>), g, b, 0, s, a, 0);
-  if (any_qem && qem_unconstrained) hipLaunchKernelGGL((k_scan_eval<2, kX, kB>), g, b, 0, s, a, any_iso ? 1 : 0);
-  else if (any_qem) hipLaunchKernelGGL((k_scan_eval<1, kX, kB>), g, b, 0, s, a, any_iso ? 1 : 0);
+  if (a.crowded) launch_scan_eval_t<kX, kB, true>(s, a, any_iso, any_qem, qem_unconstrained);
+  else launch_scan_eval_t<kX, kB, false>(s, a, any_iso, any_qem, qem_unconstrained);
 }
 
 hipError_t launch_scan_eval(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained) {
@@ -2094,13 +2105,19 @@ hipError_t launch_tile_update(hipStream_t s, const SweepArgs& a) {
   return hipGetLastError();
 }
 
+template <bool kX, bool kB, bool kC, bool kT>
+void launch_reeval_t(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained,
+                     int round) {
+  const dim3 g(unsigned(a.n_seg)), b(kBlock);
+  if (any_iso) hipLaunchKernelGGL((k_reeval<0, kX, kB, kC, kT>), g, b, 0, s, a, round);
+  if (any_qem && qem_unconstrained) hipLaunchKernelGGL((k_reeval<2, kX, kB, kC, kT>), g, b, 0, s, a, round);
+  else if (any_qem) hipLaunchKernelGGL((k_reeval<1, kX, kB, kC, kT>), g, b, 0, s, a, round);
+}
 template <bool kX, bool kB, bool kC>
 void launch_reeval_x(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained,
                      int round) {
-  const dim3 g(unsigned(a.n_seg)), b(kBlock);
-  if (any_iso) hipLaunchKernelGGL((k_reeval<0, kX, kB, kC>), g, b, 0, s, a, round);
-  if (any_qem && qem_unconstrained) hipLaunchKernelGGL((k_reeval<2, kX, kB, kC>), g, b, 0, s, a, round);
-  else if (any_qem) hipLaunchKernelGGL((k_reeval<1, kX, kB, kC>), g, b, 0, s, a, round);
+  if (a.crowded) launch_reeval_t<kX, kB, kC, true>(s, a, any_iso, any_qem, qem_unconstrained, round);
+  else launch_reeval_t<kX, kB, kC, false>(s, a, any_iso, any_qem, qem_unconstrained, round);
 }
 
 hipError_t launch_reeval(hipStream_t s, const SweepArgs& a, bool any_iso, bool any_qem, bool qem_unconstrained,

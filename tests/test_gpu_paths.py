@@ -58,11 +58,12 @@ def fixed_items(n_items, n, seed):
 @pytest.mark.parametrize("metric,unc,kind", [(ISO, 0, "plain"), (QEM, 1, "plain"), (QEM, 0, "plain"),
                                              (QEM, 1, "long rows"), (ISO, 0, "long rows"), (QEM, 1, "fixed"),
                                              (QEM, 0, "fixed"), (ISO, 0, "fixed"), (QEM, 0, "frozen"),
-                                             (ISO, 0, "frozen")])
+                                             (ISO, 0, "frozen"), (ISO, 0, "few clusters"),
+                                             (QEM, 1, "few clusters")])
 def test_one_mesh_on_every_path(gpu_ready, path, metric, unc, kind):
     print(path, metric, unc, kind, flush=True)
     xyz, tri = centroid_split(*meshgen.icosphere(4, 9, 0.02)) if kind == "long rows" else meshgen.icosphere(5, 4, 0.03)
-    K = 400
+    K = 20 if kind == "few clusters" else 400  # 20: many proposals meet at a cluster
     ctx = acvd_amd.Context()
     ctx.set_input(xyz, tri)
     ctx.set_params(0, number_of_clusters=K, metric=metric, unconstrained_initialization=unc, seed=5)
@@ -91,7 +92,8 @@ def test_one_mesh_on_every_path(gpu_ready, path, metric, unc, kind):
 def test_batch_on_every_path(gpu_ready, path, anchored):
     print(path, anchored, flush=True)
     specs = [(meshgen.icosphere(4, 6, 0.03), QEM, 170, 1), (meshgen.star_icosphere(4, 7), ISO, 170, 0),
-             (meshgen.cube(20, 14, 1e-4), QEM, 160, 0), (meshgen.icosphere(3, 8, 0.02), ISO, 40, 0)]
+             (meshgen.cube(20, 14, 1e-4), QEM, 160, 0), (meshgen.icosphere(3, 8, 0.02), ISO, 40, 0),
+             (meshgen.icosphere(4, 9, 0.02), ISO, 6, 0)]  # the last with many proposals per cluster
     ctx = acvd_amd.Context()
     want = []
     for k, ((xyz, tri), metric, K, unc) in enumerate(specs):

@@ -51,9 +51,27 @@ inline unsigned egrid(int64_t n) { return unsigned((n + kEBlock - 1) / kEBlock);
 
 __device__ inline int mesh_of(const EnergyArgs& a, int64_t i) { return a.item_mesh ? a.item_mesh[i] : 0; }
 
+// What the kernels over items use of a mesh: uniform over the block, or (kMany)
+// each lane's own.
+struct ItemMesh {
+  int32_t off, K;  // clusters
+  bool qem;
+};
+
+__device__ inline ItemMesh item_mesh(const EnergyMesh& em) {
+  return ItemMesh{int32_t(em.clus_off), em.K, em.metric == 1};
+}
+
 // global cluster of an item labelled l, or -1
-__device__ inline int32_t cluster_of(const EnergyMesh& em, int32_t l) {
-  return (l < 0 || l >= em.K) ? -1 : int32_t(em.clus_off) + l;
+__device__ inline int32_t cluster_of(const ItemMesh& im, int32_t l) {
+  return (l < 0 || l >= im.K) ? -1 : im.off + l;
+}
+
+// Lanes that follow in the lane's run, given the run heads of the wave.
+__device__ inline int run_left(unsigned long long heads) {
+  const int lane = threadIdx.x & 63;
+  const unsigned long long after = lane == 63 ? 0ull : heads >> (lane + 1);
+  return after ? __builtin_ctzll(after) : 63 - lane;
 }
 
 struct Vec3 {
@@ -357,7 +375,7 @@ __device__ inline void merge_step(double (&v)[V], int rem) {
 // work (580 instructions a step of 64 items, 60 % of the time) and the gathers'
 // latency at 4 waves per SIMD: 16.8 M QEM vertices 2328 -> 372 us (a copy of the
 // bytes takes 168 us), 1 M isotropic ones 45.7 -> 16.7 us.
-template <bool kQem>
+template <bool kQem, bool kMany>
 __global__ __launch_bounds__(kAccBlock) void ke_accumulate(EnergyArgs a, int64_t chunk) {
   constexpr int V = kQem ? 13 : 4;  // W, S[3], Q[9]
   constexpr int kSlots = kQem ? 512 : 1024;
@@ -388,23 +406,30 @@ __global__ __launch_bounds__(kAccBlock) void ke_accumulate(EnergyArgs a, int64_t
     if (threadIdx.x == 0) n_keys = 0;
     __syncthreads();
   };
-  const int m0 = mesh_of(a, begin), m1 = mesh_of(a, end - 1);
+  const int m0 = kMany ? 0 : mesh_of(a, begin), m1 = kMany ? 0 : mesh_of(a, end - 1);
   int step = 0;
   for (int m = m0; m <= m1; ++m) {
     const EnergyMesh em = a.meshes[m];
-    const int64_t first = max(begin, em.item_off), last = min(end, em.item_off + em.n_items);
-    const bool qem = kQem && em.metric == 1;  // block-uniform
+    const int64_t first = kMany ? begin : max(begin, em.item_off);
+    const int64_t last = kMany ? end : min(end, em.item_off + em.n_items);
+    ItemMesh im = item_mesh(em);
+    const bool rings = kQem && (kMany || im.qem);  // block-uniform
     // steps stay aligned to the chunk (and so to the ring groups)
     const int64_t base0 = begin + (first - begin) / kAccBlock * kAccBlock;
     int32_t e[kRingChunk];
-    int32_t slots = 0, lab = -1;
-    // the ring entries and labels of a step are read during the step before it
-    if (qem && base0 < last) slots = load_ring(a, base0 + threadIdx.x, e);
-    if (base0 + int64_t(threadIdx.x) >= first && base0 + int64_t(threadIdx.x) < last) lab = a.labels[base0 + threadIdx.x];
+    int32_t slots = 0, lab = -1, mi = 0;
+    // the ring entries, labels and (kMany) meshes of a step are read during the step before it
+    if (rings && base0 < last) slots = load_ring(a, base0 + threadIdx.x, e);
+    if (base0 + int64_t(threadIdx.x) >= first && base0 + int64_t(threadIdx.x) < last) {
+      lab = a.labels[base0 + threadIdx.x];
+      if (kMany) mi = a.item_mesh[base0 + threadIdx.x];
+    }
     for (int64_t base = base0; base < last; base += kAccBlock) {
       const int64_t i = base + threadIdx.x;
       const bool active = i >= first && i < last;
-      const int32_t c = active ? cluster_of(em, lab) : -1;
+      if (kMany) im = item_mesh(a.meshes[mi]);
+      const int32_t c = active ? cluster_of(im, lab) : -1;
+      const bool qem = kQem && im.qem;
       double v[V];
 #pragma unroll
       for (int k = 0; k < V; ++k) v[k] = 0.0;
@@ -430,8 +455,9 @@ __global__ __launch_bounds__(kAccBlock) void ke_accumulate(EnergyArgs a, int64_t
         v[3] = w * x.z;
       }
       if (base + kAccBlock < last) {
-        if (qem) slots = load_ring(a, i + kAccBlock, e);
+        if (rings) slots = load_ring(a, i + kAccBlock, e);
         lab = i + kAccBlock < last ? a.labels[i + kAccBlock] : -1;
+        if (kMany && i + kAccBlock < last) mi = a.item_mesh[i + kAccBlock];
       }
       if constexpr (kQem) {
         if (qem && c >= 0) {
@@ -463,9 +489,7 @@ __global__ __launch_bounds__(kAccBlock) void ke_accumulate(EnergyArgs a, int64_t
       // runs of equal clusters
       const int32_t prev = __builtin_amdgcn_update_dpp(-2, c, 0x111, 0xf, 0xf, false);  // row_shr:1
       const bool head = prev != c || (lane & (kRun - 1)) == 0;
-      const unsigned long long heads = __ballot(head);
-      const unsigned long long after = lane == 63 ? 0ull : heads >> (lane + 1);
-      const int rem = after ? __builtin_ctzll(after) : 63 - lane;
+      const int rem = run_left(__ballot(head));
       static_assert(kRun == 8, "three doubling steps");
       merge_step<1>(v, rem);
       merge_step<2>(v, rem);
@@ -588,33 +612,85 @@ __global__ __launch_bounds__(64) void ke_points(EnergyArgs a) {
 // their sums to the mesh's energy: one atomic per block and mesh (atomics on one
 // address take 12.7 ns each; with one per 256 items they were this kernel's
 // time: 1 M vertices 52 -> 8 us, 16 x 1 M 694 -> 92 us, 3.6 TB/s).
+template <bool kMany>
 __global__ __launch_bounds__(kAccBlock) void ke_energy(EnergyArgs a, int64_t chunk, double* energy) {
-  __shared__ double red[kAccBlock / 64];
+  constexpr int kWaves = kAccBlock / 64;
+  __shared__ double red[kWaves];
   const int64_t begin = int64_t(blockIdx.x) * chunk;
   const int64_t end = min(begin + chunk, a.n_items);
-  const int m0 = mesh_of(a, begin), m1 = mesh_of(a, end - 1);
-  for (int m = m0; m <= m1; ++m) {
-    const EnergyMesh em = a.meshes[m];
-    const int64_t first = max(begin, em.item_off), last = min(end, em.item_off + em.n_items);
+  auto term = [&](const ItemMesh& im, int64_t i) {
+    const int32_t c = cluster_of(im, a.labels[i]);
+    const Vec3 x = load_point(a.xyz, i);
+    const double w = double(a.w[i]);
+    if (c < 0) return 0.0;
+    const double* q = a.pts + 4 * int64_t(c);
+    const double dx = x.x - q[0], dy = x.y - q[1], dz = x.z - q[2];
+    return w * (dx * dx + dy * dy + dz * dz);
+  };
+  if constexpr (kMany) {
+    // A wave adds up the items of one mesh while its lanes lie in it (cur), and
+    // else the runs of its lanes in each mesh.
+    __shared__ int32_t mesh[kWaves];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     double e = 0.0;
-#pragma unroll 4
-    for (int64_t i = first + threadIdx.x; i < last; i += kAccBlock) {
-      const int32_t c = cluster_of(em, a.labels[i]);
-      const Vec3 x = load_point(a.xyz, i);
-      const double w = double(a.w[i]);
-      if (c >= 0) {
-        const double* q = a.pts + 4 * int64_t(c);
-        const double dx = x.x - q[0], dy = x.y - q[1], dz = x.z - q[2];
-        e += w * (dx * dx + dy * dy + dz * dz);
+    int32_t cur = -1;
+    auto wave_sum = [&]() {
+      for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off);
+    };
+    for (int64_t base = begin; base < end; base += kAccBlock) {
+      const int64_t i = base + threadIdx.x;
+      const int32_t m = i < end ? a.item_mesh[i] : -1;
+      double t = m >= 0 ? term(item_mesh(a.meshes[m]), i) : 0.0;
+      const int32_t m0 = __builtin_amdgcn_readfirstlane(m);
+      if (__ballot(m != m0) == 0ull) {
+        if (m0 != cur) {
+          wave_sum();
+          if (lane == 0 && cur >= 0) atomicAdd(&energy[cur], e);
+          e = 0.0;
+          cur = m0;
+        }
+        e += t;
+      } else {
+        const int32_t prev = __shfl_up(m, 1);
+        const bool head = lane == 0 || prev != m;
+        const int rem = run_left(__ballot(head));
+        for (int off = 1; off < 64; off <<= 1) {
+          const double u = __shfl_down(t, off);
+          if (rem >= off) t += u;
+        }
+        if (head && m >= 0) atomicAdd(&energy[m], t);
       }
     }
-    for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off);
-    __syncthreads();  // red of the previous mesh has been read
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = e;
+    wave_sum();
+    if (lane == 0) {
+      red[wave] = e;
+      mesh[wave] = cur;
+    }
     __syncthreads();
-    if (threadIdx.x == 0) {
-      for (int k = 1; k < kAccBlock / 64; ++k) e += red[k];
-      atomicAdd(&energy[m], e);
+    if (threadIdx.x == 0)  // one atomic for neighbouring waves of one mesh
+      for (int k = 0; k < kWaves;) {
+        const int32_t m = mesh[k];
+        double sum = 0.0;
+        for (; k < kWaves && mesh[k] == m; ++k) sum += red[k];
+        if (m >= 0) atomicAdd(&energy[m], sum);
+      }
+  } else {
+    const int m0 = mesh_of(a, begin), m1 = mesh_of(a, end - 1);
+    for (int m = m0; m <= m1; ++m) {
+      const EnergyMesh em = a.meshes[m];
+      const ItemMesh im = item_mesh(em);
+      const int64_t first = max(begin, em.item_off), last = min(end, em.item_off + em.n_items);
+      double e = 0.0;
+#pragma unroll 4
+      for (int64_t i = first + threadIdx.x; i < last; i += kAccBlock) e += term(im, i);
+      for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off);
+      __syncthreads();  // red of the previous mesh has been read
+      if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = e;
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        for (int k = 1; k < kWaves; ++k) e += red[k];
+        atomicAdd(&energy[m], e);
+      }
     }
   }
 }
@@ -629,7 +705,7 @@ constexpr int64_t kSmallClusters = 1024;
 __global__ __launch_bounds__(kSmallBlock) void ke_forward_small(EnergyArgs a, double* energy) {
   __shared__ double acc[kSmallClusters * 4];
   __shared__ double red[kSmallBlock / 64];
-  const EnergyMesh em = a.meshes[0];
+  const ItemMesh em = item_mesh(a.meshes[0]);
   const int lane = threadIdx.x & 63;
   for (int k = threadIdx.x; k < em.K * 4; k += kSmallBlock) acc[k] = 0.0;
   __syncthreads();
@@ -646,9 +722,7 @@ __global__ __launch_bounds__(kSmallBlock) void ke_forward_small(EnergyArgs a, do
     }
     const int32_t prev = __builtin_amdgcn_update_dpp(-2, c, 0x111, 0xf, 0xf, false);  // row_shr:1
     const bool head = prev != c || (lane & 7) == 0;
-    const unsigned long long heads = __ballot(head);
-    const unsigned long long after = lane == 63 ? 0ull : heads >> (lane + 1);
-    const int rem = after ? __builtin_ctzll(after) : 63 - lane;
+    const int rem = run_left(__ballot(head));
     merge_step<1>(v, rem);
     merge_step<2>(v, rem);
     merge_step<4>(v, rem);
@@ -726,7 +800,7 @@ __device__ inline PlaneAdjoint no_adjoint() {
 // waves per SIMD (168 registers; held to 128 the spills cost more: 1359 us;
 // a loop over the faces that keeps one position in flight: 831 us).
 // 16.8 M QEM vertices 2050 -> 765 us, 1 M isotropic ones 10.5 -> 8.6 us.
-template <bool kQem>
+template <bool kQem, bool kMany>
 __global__ __launch_bounds__(kEBlock) void ke_item_grad(EnergyArgs a, const double* __restrict__ gE,
                                                         float* __restrict__ dxyz, float* __restrict__ dw) {
   constexpr int kXcd = 8;
@@ -743,14 +817,15 @@ __global__ __launch_bounds__(kEBlock) void ke_item_grad(EnergyArgs a, const doub
   int32_t e[kRingChunk];
   int32_t slots = 0;
   if constexpr (kQem) slots = load_ring(a, i, e);
-  const int m0 = mesh_of(a, begin), m1 = mesh_of(a, end - 1);
+  const int m0 = kMany ? 0 : mesh_of(a, begin), m1 = kMany ? 0 : mesh_of(a, end - 1);
   for (int m = m0; m <= m1; ++m) {
-    const EnergyMesh em = a.meshes[m];
-    const bool active = i < end && i >= em.item_off && i < em.item_off + em.n_items;
-    const double g = gE[m];
+    const EnergyMesh& mesh = a.meshes[kMany ? a.item_mesh[ic] : m];
+    const ItemMesh em = item_mesh(mesh);
+    const bool active = i < end && (kMany || (i >= mesh.item_off && i < mesh.item_off + mesh.n_items));
+    const double g = gE[kMany ? a.item_mesh[ic] : m];
     double gx[3] = {0, 0, 0}, gw = 0.0;
     const int32_t c = active ? cluster_of(em, lab) : -1;
-    const bool qem = kQem && em.metric == 1;  // block-uniform
+    const bool qem = kQem && em.qem;  // block-uniform unless kMany
     if (c >= 0) {
       const double w = double(wf);
       const double* q = a.pts + 4 * int64_t(c);
@@ -882,15 +957,16 @@ hipError_t energy_forward(hipStream_t s, const EnergyArgs& a, double* energy, in
   if (a.n_items > 0) {
     const int64_t chunk = item_chunk(a.n_items, kAccMaxBlocks);
     const dim3 grid(unsigned((a.n_items + chunk - 1) / chunk));
-    if (a.adj) hipLaunchKernelGGL(ke_accumulate<true>, grid, dim3(kAccBlock), 0, s, a, chunk);
-    else hipLaunchKernelGGL(ke_accumulate<false>, grid, dim3(kAccBlock), 0, s, a, chunk);
+    const auto k = a.adj ? (a.many ? ke_accumulate<true, true> : ke_accumulate<true, false>)
+                         : (a.many ? ke_accumulate<false, true> : ke_accumulate<false, false>);
+    hipLaunchKernelGGL(k, grid, dim3(kAccBlock), 0, s, a, chunk);
   }
   if (a.n_clusters > 0)
     hipLaunchKernelGGL(ke_points, dim3(unsigned((a.n_clusters + 63) / 64)), dim3(64), 0, s, a);
   if (a.n_items > 0) {
     const int64_t chunk = item_chunk(a.n_items, 512);
-    hipLaunchKernelGGL(ke_energy, dim3(unsigned((a.n_items + chunk - 1) / chunk)), dim3(kAccBlock), 0, s, a, chunk,
-                       energy);
+    hipLaunchKernelGGL(a.many ? ke_energy<true> : ke_energy<false>, dim3(unsigned((a.n_items + chunk - 1) / chunk)),
+                       dim3(kAccBlock), 0, s, a, chunk, energy);
   }
   return hipGetLastError();
 }
@@ -988,10 +1064,11 @@ hipError_t energy_forward_cvt_noalloc(hipStream_t s, int64_t n, int32_t K, const
 }
 
 hipError_t energy_backward(hipStream_t s, const EnergyArgs& a, const double* grad_energy, float* dxyz, float* dw) {
-  if (a.n_items > 0 && a.adj)
-    hipLaunchKernelGGL(ke_item_grad<true>, dim3(egrid(a.n_items)), dim3(kEBlock), 0, s, a, grad_energy, dxyz, dw);
-  else if (a.n_items > 0)
-    hipLaunchKernelGGL(ke_item_grad<false>, dim3(egrid(a.n_items)), dim3(kEBlock), 0, s, a, grad_energy, dxyz, dw);
+  if (a.n_items > 0) {
+    const auto k = a.adj ? (a.many ? ke_item_grad<true, true> : ke_item_grad<true, false>)
+                         : (a.many ? ke_item_grad<false, true> : ke_item_grad<false, false>);
+    hipLaunchKernelGGL(k, dim3(egrid(a.n_items)), dim3(kEBlock), 0, s, a, grad_energy, dxyz, dw);
+  }
   return hipGetLastError();
 }
 

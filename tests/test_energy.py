@@ -253,6 +253,55 @@ def test_gpu_energy_rings_match_oracle(gpu_ready, metric, shape):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("large", [False, True])
+def test_gpu_energy_of_many_small_meshes(gpu_ready, large):
+    """Meshes of 3 to 700 vertices, isotropic and QEM in turn, several to a wave and
+    some over a few blocks; with `large` one of 150,000 vertices among them (blocks of
+    several steps).  The small ones against the oracle, the large one against itself
+    alone.  Tolerances: FP64 sums in another order (1e-9), gradients in FP32 (1e-5 of
+    the largest component, as above; 1e-6 against itself)."""
+    import torch
+    from acvd_amd.energy import ClusterEnergy
+    rng = np.random.default_rng(11)
+    shapes = [ring_problem(f"hub{n}") for n in (3, 10, 62, 63, 64, 254, 510, 698)] + [ring_problem("grid")]
+    shapes.append((np.asarray([[0, 0, 0], [1, 0, 0], [0, 1, 0.5]], np.float64), np.ones(3), np.asarray([[0, 1, 2]], np.int32),
+                   np.asarray([0, 0, 1], np.int32), 2))
+    order = rng.integers(0, len(shapes), 120)
+    meshes = [(shapes[k], QEM if rng.random() < 0.5 else ISO) for k in order]
+    if large:
+        xyz, tri = meshgen.torus(500, 300, 4)
+        x = np.asarray(xyz, np.float32).astype(np.float64)
+        meshes.insert(60, ((x, rng.uniform(0.5, 2.0, len(x)), np.asarray(tri, np.int32),
+                            (np.arange(len(x)) // 40).astype(np.int32), len(x) // 40), QEM))
+    ce = ClusterEnergy(0)
+    for (x, _, tri, _, K), metric in meshes:
+        ce.add_mesh(len(x), tri, K, metric, 2)
+    parts = [gpu_inputs(x, w, lab, K) for (x, w, _, lab, K), _ in meshes]
+    tx, tw, tl = (torch.cat(t).contiguous() for t in zip(*parts))
+    e = ce.forward_raw(tx, tw, tl).cpu().numpy()
+    g = torch.arange(1, len(meshes) + 1, dtype=torch.float64, device=tx.device)
+    dx, dw = (t.cpu().numpy() for t in ce.backward_raw(tx, tw, tl, g))
+    off = 0
+    for j, ((x, w, tri, lab, K), metric) in enumerate(meshes):
+        s = slice(off, off + len(x))
+        off += len(x)
+        if len(x) > 10000:
+            alone = ClusterEnergy(0)
+            alone.add_mesh(len(x), tri, K, metric, 2)
+            e_ref = alone.forward_raw(*parts[j]).item()
+            d = np.concatenate([t.cpu().numpy().reshape(-1) for t in alone.backward_raw(*parts[j], g[j:j + 1])]) / (j + 1)
+            tol = 1e-6
+        else:
+            ref = po.EnergyRef(len(x), tri, np.where(lab < K, lab, K), K, metric, 2)
+            w = w.astype(np.float32).astype(np.float64)
+            e_ref, d = ref.total(x, w), ref.derivatives(x, w, np.arange(4 * len(x)))
+            tol = 1e-5
+        assert np.isclose(e[j], e_ref, rtol=1e-9, atol=1e-30), (j, len(x), metric, e[j], e_ref)
+        got = np.concatenate([dx[s].reshape(-1), dw[s]]).astype(np.float64) / (j + 1)
+        assert np.abs(got - d).max() <= tol * np.abs(d).max() + 1e-30, (j, len(x), metric)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,K", [(1, 1), (63, 5), (1025, 40), (4096, 1024), (4096, 1025), (4097, 1024)])
 def test_gpu_iso_energy_at_the_small_path(gpu_ready, n, K):
     """Either side of the sizes that one block takes, against the closed form in

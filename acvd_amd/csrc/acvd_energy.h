@@ -26,7 +26,6 @@ struct EnergyArgs {
   const EnergyMesh* meshes;
   const int32_t* item_mesh;  // null for one mesh
   const int32_t* clus_mesh;  // null for one mesh
-  int32_t many;              // meshes are looked up per item (kManyMeshes; needs item_mesh)
   const int32_t* tri;        // 3 global vertex ids per face (contexts with QEM meshes; else null)
   const int32_t* vfptr;      // vertex -> incident faces, one entry per corner
   const int32_t* vfcol;
@@ -46,19 +45,6 @@ struct EnergyArgs {
                              // dE/dQ[9], (dE/dc)/W [3]; centroid [3]
 };
 
-// The kernels over items take the meshes that meet in a block one after the
-// other, a mesh's numbers in scalar registers.  Where many small ones meet
-// (`many`) every lane reads its own item's mesh instead: more than kManyMeshes in
-// a window of kManyItems items, or meshes that share windows and have fewer than
-// kManyMean items in the mean.  Forward and backward, one after the other / by
-// lane: 33,333 QEM meshes of 12 vertices 720 / 112 us, 3,125 of 128 115 / 78, 64 of
-// 4,095 54 / 46, 64 of 16,383 120 / 114, 16 of 262,143 343 / 351; isotropic 388 /
-// 112, 51 / 35, 28.7 / 28.9, 35.6 / 35.5, 81 / 88; one QEM mesh of 1,048,576
-// followed by 5,000 of 12 1,550 / 124.
-constexpr int64_t kManyItems = 256;
-constexpr int kManyMeshes = 3;
-constexpr int64_t kManyMean = 16384;
-
 constexpr int kAdjStride = 16;
 // Ring entries: a neighbour id; with the sign bit set the first id of a chain;
 // kRingEnd past the end; kRingLong (first entry alone) for a vertex of more than
@@ -66,7 +52,7 @@ constexpr int kAdjStride = 16;
 constexpr int32_t kRingEnd = -1;
 constexpr int32_t kRingLong = -2;
 constexpr int32_t kRingId = 0x7fffffff;
-constexpr int kRingFaces = 16;
+constexpr int kRingFaces = 32;
 constexpr int kRingChunk = 8;  // ids read at once
 
 // Device build of the vertex -> face rows and rings.

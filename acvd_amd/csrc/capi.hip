@@ -1947,7 +1947,6 @@ struct acvd_energy {
   DBuf<double> d_acc, d_pts, d_adj;
   bool have_forward = false;
   bool any_qem = false;
-  bool many = false;  // EnergyArgs::many
   EnergyArgs args() const {
     EnergyArgs a{};
     a.n_items = N;
@@ -1962,7 +1961,6 @@ struct acvd_energy {
       a.ring_slot = d_topo.p + 6 * F + N + 1;
       a.ring = d_ring.p;
     }
-    a.many = many ? 1 : 0;
     a.acc_stride = any_qem ? 13 : 4;
     a.acc = d_acc.p;
     a.pts = d_pts.p;
@@ -1993,13 +1991,9 @@ int energy_build(acvd_energy* e) {
     clus_mesh.resize(K);
   }
   e->any_qem = false;
-  int64_t io = 0, co = 0, fo = 0, window = -1;
-  int in_window = 0, most = 1;  // meshes in the window that the last one started in, and in any
+  int64_t io = 0, co = 0, fo = 0;
   for (int m = 0; m < M; ++m) {
     const auto& h = e->meshes[m];
-    in_window = io / kManyItems == window ? in_window + 1 : 1 + (io % kManyItems != 0);
-    window = io / kManyItems;
-    most = std::max(most, in_window);
     hm[m] = EnergyMesh{io, h.nv, co, fo, h.K, h.metric, h.level, 0};
     e->any_qem |= h.metric == ACVD_METRIC_QEM;
     if (M > 1) {
@@ -2010,7 +2004,6 @@ int energy_build(acvd_energy* e) {
     co += h.K;
     fo += h.nf;
   }
-  e->many = most > kManyMeshes || (most > 1 && N < kManyMean * M);
   HIP_TRY(e->d_meshes.alloc(M));
   HIP_TRY(hipMemcpy(e->d_meshes.p, hm.data(), M * sizeof(EnergyMesh), hipMemcpyHostToDevice));
   if (M > 1) {

@@ -51,8 +51,11 @@ inline unsigned egrid(int64_t n) { return unsigned((n + kEBlock - 1) / kEBlock);
 
 __device__ inline int mesh_of(const EnergyArgs& a, int64_t i) { return a.item_mesh ? a.item_mesh[i] : 0; }
 
-// What the kernels over items use of a mesh: uniform over the block, or (kMany)
-// each lane's own.
+// What the kernels over items use of a mesh.  A block whose items lie in one mesh
+// reads it once; in another each lane reads its own item's (its meshes taken one
+// after the other, a pass of the block each, batches of small meshes took several
+// times as long: forward and backward of 33,333 QEM meshes of 12 vertices 720 us,
+// by lane 112, 3,125 of 128 115 / 78, 64 of 4,095 54 / 46).
 struct ItemMesh {
   int32_t off, K;  // clusters
   bool qem;
@@ -98,9 +101,9 @@ __device__ inline Vec3 ring_point(const EnergyArgs& a, int32_t e) {
   return load_point(a.xyz, int64_t(e & kRingId));
 }
 
-// The first kRingChunk ring entries of item i (64 consecutive items per wave:
-// i = 64 g + lane), loaded together; returns the group's slots.
-__device__ inline int32_t load_ring(const EnergyArgs& a, int64_t i, int32_t e[kRingChunk]) {
+// kRingChunk ring entries of item i from entry `from` on (64 consecutive items per
+// wave: i = 64 g + lane), loaded together; returns the group's slots.
+__device__ inline int32_t load_ring(const EnergyArgs& a, int64_t i, int from, int32_t e[kRingChunk]) {
   const int64_t g = __builtin_amdgcn_readfirstlane(int32_t(i >> 6));
   const int lane = threadIdx.x & 63;
 #pragma unroll
@@ -109,38 +112,29 @@ __device__ inline int32_t load_ring(const EnergyArgs& a, int64_t i, int32_t e[kR
   const int32_t s0 = a.ring_slot[g], n = a.ring_slot[g + 1] - s0;  // scalar loads
 #pragma unroll
   for (int k = 0; k < kRingChunk; ++k)
-    if (k < n) e[k] = a.ring[int64_t(s0 + k) * 64 + lane];
+    if (from + k < n) e[k] = a.ring[int64_t(s0 + from + k) * 64 + lane];
   return n;
 }
 
-// Faces around item i past its first `from` ring entries (u: the previous ring
-// vertex less the item's position, cu: its tag), and those of a vertex with more
-// faces than a ring holds: the paths of rare vertices, an entry at a time.
-// tag(id) labels a ring vertex; face(u, cu, s, cs) takes a face.
-template <class Tag, class Face>
-__device__ inline void walk_rest(const EnergyArgs& a, int64_t i, const Vec3& x, int32_t first, int from, Vec3 u,
-                                 int32_t cu, Tag&& tag, Face&& face) {
-  if (first == kRingLong) {
-    for (int32_t k = a.vfptr[i]; k < a.vfptr[i + 1]; ++k) {
-      const int64_t f = a.vfcol[k];
-      // the corner of this entry: a face listed more than once for the vertex
-      // (a degenerate face, whose normal is zero) takes its first corner
-      int j = 0;
-      while (j < 2 && a.tri[3 * f + j] != int32_t(i)) ++j;
-      const int32_t v1 = a.tri[3 * f + (j + 1) % 3], v2 = a.tri[3 * f + (j + 2) % 3];
-      face(sub(load_point(a.xyz, v1), x), tag(v1), sub(load_point(a.xyz, v2), x), tag(v2));
+// The faces of a vertex with more faces than a ring holds, from its vertex -> face
+// row: visit(n, v1, v2) takes kFaceBatch of them at a time, n real ones in the
+// face's orientation behind the vertex.  A face listed more than once for the
+// vertex (a degenerate one, whose normal is zero) takes its first corner.
+constexpr int kFaceBatch = 4;
+template <class Visit>
+__device__ inline void walk_faces(const EnergyArgs& a, int64_t i, Visit&& visit) {
+  const int32_t begin = a.vfptr[i], end = a.vfptr[i + 1];
+  for (int32_t base = begin; base < end; base += kFaceBatch) {
+    int32_t v1[kFaceBatch], v2[kFaceBatch];
+#pragma unroll
+    for (int k = 0; k < kFaceBatch; ++k) {
+      const int64_t f = a.vfcol[min(base + k, end - 1)];
+      const int32_t t0 = a.tri[3 * f], t1 = a.tri[3 * f + 1], t2 = a.tri[3 * f + 2];
+      const int j = t0 == int32_t(i) ? 0 : t1 == int32_t(i) ? 1 : 2;
+      v1[k] = j == 0 ? t1 : j == 1 ? t2 : t0;
+      v2[k] = j == 0 ? t2 : j == 1 ? t0 : t1;
     }
-    return;
-  }
-  const int32_t s0 = a.ring_slot[i >> 6], s1 = a.ring_slot[(i >> 6) + 1];
-  for (int32_t s = s0 + from; s < s1; ++s) {
-    const int32_t e = a.ring[int64_t(s) * 64 + (i & 63)];
-    if (e == kRingEnd) break;
-    const Vec3 t = sub(ring_point(a, e), x);
-    const int32_t ct = tag(e & kRingId);
-    if (e >= 0) face(u, cu, t, ct);
-    u = t;
-    cu = ct;
+    visit(min(end - base, kFaceBatch), v1, v2);
   }
 }
 
@@ -375,7 +369,7 @@ __device__ inline void merge_step(double (&v)[V], int rem) {
 // work (580 instructions a step of 64 items, 60 % of the time) and the gathers'
 // latency at 4 waves per SIMD: 16.8 M QEM vertices 2328 -> 372 us (a copy of the
 // bytes takes 168 us), 1 M isotropic ones 45.7 -> 16.7 us.
-template <bool kQem, bool kMany>
+template <bool kQem>
 __global__ __launch_bounds__(kAccBlock) void ke_accumulate(EnergyArgs a, int64_t chunk) {
   constexpr int V = kQem ? 13 : 4;  // W, S[3], Q[9]
   constexpr int kSlots = kQem ? 512 : 1024;
@@ -406,121 +400,141 @@ __global__ __launch_bounds__(kAccBlock) void ke_accumulate(EnergyArgs a, int64_t
     if (threadIdx.x == 0) n_keys = 0;
     __syncthreads();
   };
-  const int m0 = kMany ? 0 : mesh_of(a, begin), m1 = kMany ? 0 : mesh_of(a, end - 1);
+  const int m0 = mesh_of(a, begin);
+  const bool one = m0 == mesh_of(a, end - 1);  // block-uniform
+  ItemMesh im = item_mesh(a.meshes[m0]);
+  const bool rings = kQem && (!one || im.qem);
+  int32_t e[kRingChunk];
+  int32_t slots = 0, lab = -1, mi = m0;
+  // the ring entries, labels and meshes of a step are read during the step before it
+  if (rings) slots = load_ring(a, begin + threadIdx.x, 0, e);
+  if (begin + int64_t(threadIdx.x) < end) {
+    lab = a.labels[begin + threadIdx.x];
+    if (!one) mi = a.item_mesh[begin + threadIdx.x];
+  }
+  if (!one) im = item_mesh(a.meshes[mi]);
   int step = 0;
-  for (int m = m0; m <= m1; ++m) {
-    const EnergyMesh em = a.meshes[m];
-    const int64_t first = kMany ? begin : max(begin, em.item_off);
-    const int64_t last = kMany ? end : min(end, em.item_off + em.n_items);
-    ItemMesh im = item_mesh(em);
-    const bool rings = kQem && (kMany || im.qem);  // block-uniform
-    // steps stay aligned to the chunk (and so to the ring groups)
-    const int64_t base0 = begin + (first - begin) / kAccBlock * kAccBlock;
-    int32_t e[kRingChunk];
-    int32_t slots = 0, lab = -1, mi = 0;
-    // the ring entries, labels and (kMany) meshes of a step are read during the step before it
-    if (rings && base0 < last) slots = load_ring(a, base0 + threadIdx.x, e);
-    if (base0 + int64_t(threadIdx.x) >= first && base0 + int64_t(threadIdx.x) < last) {
-      lab = a.labels[base0 + threadIdx.x];
-      if (kMany) mi = a.item_mesh[base0 + threadIdx.x];
-    }
-    for (int64_t base = base0; base < last; base += kAccBlock) {
-      const int64_t i = base + threadIdx.x;
-      const bool active = i >= first && i < last;
-      if (kMany) im = item_mesh(a.meshes[mi]);
-      const int32_t c = active ? cluster_of(im, lab) : -1;
-      const bool qem = kQem && im.qem;
-      double v[V];
+  for (int64_t base = begin; base < end; base += kAccBlock) {
+    const int64_t i = base + threadIdx.x;
+    const int32_t c = i < end ? cluster_of(im, lab) : -1;
+    const bool qem = kQem && im.qem;
+    double v[V];
 #pragma unroll
-      for (int k = 0; k < V; ++k) v[k] = 0.0;
-      Vec3 x{0.0, 0.0, 0.0};
-      RingPoint q[kRingChunk];
-      const int32_t e0 = e[0], cur_slots = slots;
-      uint32_t faces = 0;  // entries that close a face
+    for (int k = 0; k < V; ++k) v[k] = 0.0;
+    Vec3 x{0.0, 0.0, 0.0};
+    RingPoint q[kRingChunk];
+    const int32_t e0 = e[0], cur_slots = slots;
+    uint32_t faces = 0;  // entries that close a face
+    if (qem && c >= 0) {
+#pragma unroll
+      for (int k = 0; k < kRingChunk; ++k) {
+        const int64_t j = (e[k] == kRingEnd || e0 == kRingLong) ? i : int64_t(e[k] & kRingId);
+        q[k] = RingPoint{a.xyz[3 * j], a.xyz[3 * j + 1], a.xyz[3 * j + 2]};
+        if (e[k] >= 0) faces |= 1u << k;
+      }
+    }
+    const bool more = qem && c >= 0 && (e0 == kRingLong || (cur_slots > kRingChunk && e[kRingChunk - 1] != kRingEnd));
+    if (c >= 0) {
+      const double w = double(a.w[i]);
+      x = load_point(a.xyz, i);
+      v[0] = w;
+      v[1] = w * x.x;
+      v[2] = w * x.y;
+      v[3] = w * x.z;
+    }
+    if (base + kAccBlock < end) {
+      if (rings) slots = load_ring(a, i + kAccBlock, 0, e);
+      lab = i + kAccBlock < end ? a.labels[i + kAccBlock] : -1;
+      if (!one && i + kAccBlock < end) mi = a.item_mesh[i + kAccBlock];
+    }
+    if constexpr (kQem) {
       if (qem && c >= 0) {
+        auto add = [&](const Vec3& n) {
+          v[4] = __builtin_fma(n.x, n.x, v[4]);
+          v[5] = __builtin_fma(n.x, n.y, v[5]);
+          v[6] = __builtin_fma(n.x, n.z, v[6]);
+          v[8] = __builtin_fma(n.y, n.y, v[8]);
+          v[9] = __builtin_fma(n.y, n.z, v[9]);
+          v[11] = __builtin_fma(n.z, n.z, v[11]);
+        };
+        Vec3 u{0.0, 0.0, 0.0};
 #pragma unroll
         for (int k = 0; k < kRingChunk; ++k) {
-          const int64_t j = (e[k] == kRingEnd || e0 == kRingLong) ? i : int64_t(e[k] & kRingId);
-          q[k] = RingPoint{a.xyz[3 * j], a.xyz[3 * j + 1], a.xyz[3 * j + 2]};
-          if (e[k] >= 0) faces |= 1u << k;
+          const Vec3 t = sub(Vec3{double(q[k].x), double(q[k].y), double(q[k].z)}, x);
+          if (faces >> k & 1u) add(cross(u, t));
+          u = t;
         }
-      }
-      const bool more = qem && c >= 0 && (e0 == kRingLong || (cur_slots > kRingChunk && e[kRingChunk - 1] != kRingEnd));
-      if (c >= 0) {
-        const double w = double(a.w[i]);
-        x = load_point(a.xyz, i);
-        v[0] = w;
-        v[1] = w * x.x;
-        v[2] = w * x.y;
-        v[3] = w * x.z;
-      }
-      if (base + kAccBlock < last) {
-        if (rings) slots = load_ring(a, i + kAccBlock, e);
-        lab = i + kAccBlock < last ? a.labels[i + kAccBlock] : -1;
-        if (kMany && i + kAccBlock < last) mi = a.item_mesh[i + kAccBlock];
-      }
-      if constexpr (kQem) {
-        if (qem && c >= 0) {
-          auto add = [&](const Vec3& n) {
-            v[4] = __builtin_fma(n.x, n.x, v[4]);
-            v[5] = __builtin_fma(n.x, n.y, v[5]);
-            v[6] = __builtin_fma(n.x, n.z, v[6]);
-            v[8] = __builtin_fma(n.y, n.y, v[8]);
-            v[9] = __builtin_fma(n.y, n.z, v[9]);
-            v[11] = __builtin_fma(n.z, n.z, v[11]);
-          };
-          Vec3 u{0.0, 0.0, 0.0};
+        if (more && e0 != kRingLong) {
+          int32_t f[kRingChunk];
+          for (int from = kRingChunk; from < cur_slots; from += kRingChunk) {
+            load_ring(a, i, from, f);
+            if (f[0] == kRingEnd) break;
 #pragma unroll
-          for (int k = 0; k < kRingChunk; ++k) {
-            const Vec3 t = sub(Vec3{double(q[k].x), double(q[k].y), double(q[k].z)}, x);
-            if (faces >> k & 1u) add(cross(u, t));
-            u = t;
+            for (int k = 0; k < kRingChunk; ++k) {
+              const int64_t j = f[k] == kRingEnd ? i : int64_t(f[k] & kRingId);
+              q[k] = RingPoint{a.xyz[3 * j], a.xyz[3 * j + 1], a.xyz[3 * j + 2]};
+            }
+#pragma unroll
+            for (int k = 0; k < kRingChunk; ++k) {
+              const Vec3 t = sub(Vec3{double(q[k].x), double(q[k].y), double(q[k].z)}, x);
+              if (f[k] >= 0) add(cross(u, t));
+              u = t;
+            }
           }
-          if (more)
-            walk_rest(
-                a, i, x, e0, kRingChunk, u, 0, [](int32_t) { return 0; },
-                [&](const Vec3& r, int32_t, const Vec3& t, int32_t) { add(cross(r, t)); });
-          // every plane passes through the vertex (d = -n . x): sum n d = -(sum n n^T) x
-          v[7] = -(v[4] * x.x + v[5] * x.y + v[6] * x.z);
-          v[10] = -(v[5] * x.x + v[8] * x.y + v[9] * x.z);
-          v[12] = -(v[6] * x.x + v[9] * x.y + v[11] * x.z);
-        }
-      }
-      // runs of equal clusters
-      const int32_t prev = __builtin_amdgcn_update_dpp(-2, c, 0x111, 0xf, 0xf, false);  // row_shr:1
-      const bool head = prev != c || (lane & (kRun - 1)) == 0;
-      const int rem = run_left(__ballot(head));
-      static_assert(kRun == 8, "three doubling steps");
-      merge_step<1>(v, rem);
-      merge_step<2>(v, rem);
-      merge_step<4>(v, rem);
-      if (head && c >= 0) {
-        uint32_t h = (uint32_t(c) * 2654435761u) >> (32 - kSlotBits);
-        int slot = -1;
-        for (int probe = 0; probe < kProbes; ++probe) {
-          const int32_t old = atomicCAS(&keys[h], -1, c);
-          if (old == -1) atomicAdd(&n_keys, 1);
-          if (old == -1 || old == c) {
-            slot = int(h);
-            break;
-          }
-          h = (h + 1) & (kSlots - 1);
-        }
-        if (slot >= 0) {
+        } else if (more) {
+          walk_faces(a, i, [&](int n, const int32_t* v1, const int32_t* v2) {
+            Vec3 r[kFaceBatch], t[kFaceBatch];
 #pragma unroll
-          for (int k = 0; k < V; ++k) atomicAdd(&vals[slot * V + k], v[k]);
-        } else {  // no free slot near by: straight to the global sums
+            for (int k = 0; k < kFaceBatch; ++k) {
+              r[k] = sub(load_point(a.xyz, v1[k]), x);
+              t[k] = sub(load_point(a.xyz, v2[k]), x);
+            }
 #pragma unroll
-          for (int k = 0; k < V; ++k)
-            if (v[k] != 0.0) atomicAdd(&a.acc[int64_t(c) * a.acc_stride + k], v[k]);
+            for (int k = 0; k < kFaceBatch; ++k)
+              if (k < n) add(cross(r[k], t[k]));
+          });
         }
+        // every plane passes through the vertex (d = -n . x): sum n d = -(sum n n^T) x
+        v[7] = -(v[4] * x.x + v[5] * x.y + v[6] * x.z);
+        v[10] = -(v[5] * x.x + v[8] * x.y + v[9] * x.z);
+        v[12] = -(v[6] * x.x + v[9] * x.y + v[11] * x.z);
       }
-      if (++step % kCheckSteps == 0) {  // block-uniform
-        __syncthreads();
-        const bool full = n_keys > kFlushAt;
-        __syncthreads();
-        if (full) flush();
+    }
+    if (!one) im = item_mesh(a.meshes[mi]);  // of the next step
+    // runs of equal clusters
+    const int32_t prev = __builtin_amdgcn_update_dpp(-2, c, 0x111, 0xf, 0xf, false);  // row_shr:1
+    const bool head = prev != c || (lane & (kRun - 1)) == 0;
+    const int rem = run_left(__ballot(head));
+    static_assert(kRun == 8, "three doubling steps");
+    merge_step<1>(v, rem);
+    merge_step<2>(v, rem);
+    merge_step<4>(v, rem);
+    if (head && c >= 0) {
+      uint32_t h = (uint32_t(c) * 2654435761u) >> (32 - kSlotBits);
+      int slot = -1;
+      for (int probe = 0; probe < kProbes; ++probe) {
+        const int32_t old = atomicCAS(&keys[h], -1, c);
+        if (old == -1) atomicAdd(&n_keys, 1);
+        if (old == -1 || old == c) {
+          slot = int(h);
+          break;
+        }
+        h = (h + 1) & (kSlots - 1);
       }
+      if (slot >= 0) {
+#pragma unroll
+        for (int k = 0; k < V; ++k) atomicAdd(&vals[slot * V + k], v[k]);
+      } else {  // no free slot near by: straight to the global sums
+#pragma unroll
+        for (int k = 0; k < V; ++k)
+          if (v[k] != 0.0) atomicAdd(&a.acc[int64_t(c) * a.acc_stride + k], v[k]);
+      }
+    }
+    if (++step % kCheckSteps == 0) {  // block-uniform
+      __syncthreads();
+      const bool full = n_keys > kFlushAt;
+      __syncthreads();
+      if (full) flush();
     }
   }
   __syncthreads();
@@ -612,87 +626,90 @@ __global__ __launch_bounds__(64) void ke_points(EnergyArgs a) {
 // their sums to the mesh's energy: one atomic per block and mesh (atomics on one
 // address take 12.7 ns each; with one per 256 items they were this kernel's
 // time: 1 M vertices 52 -> 8 us, 16 x 1 M 694 -> 92 us, 3.6 TB/s).
-template <bool kMany>
 __global__ __launch_bounds__(kAccBlock) void ke_energy(EnergyArgs a, int64_t chunk, double* energy) {
   constexpr int kWaves = kAccBlock / 64;
+  constexpr int kLoopMeshes = 3;  // a block of so few meshes takes them one after the other
   __shared__ double red[kWaves];
+  __shared__ int32_t mesh[kWaves];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t begin = int64_t(blockIdx.x) * chunk;
   const int64_t end = min(begin + chunk, a.n_items);
   auto term = [&](const ItemMesh& im, int64_t i) {
     const int32_t c = cluster_of(im, a.labels[i]);
     const Vec3 x = load_point(a.xyz, i);
     const double w = double(a.w[i]);
-    if (c < 0) return 0.0;
-    const double* q = a.pts + 4 * int64_t(c);
-    const double dx = x.x - q[0], dy = x.y - q[1], dz = x.z - q[2];
-    return w * (dx * dx + dy * dy + dz * dz);
+    double t = 0.0;
+    if (c >= 0) {
+      const double* q = a.pts + 4 * int64_t(c);
+      const double dx = x.x - q[0], dy = x.y - q[1], dz = x.z - q[2];
+      t = w * (dx * dx + dy * dy + dz * dz);
+    }
+    return t;
   };
-  if constexpr (kMany) {
-    // A wave adds up the items of one mesh while its lanes lie in it (cur), and
-    // else the runs of its lanes in each mesh.
-    __shared__ int32_t mesh[kWaves];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    double e = 0.0;
-    int32_t cur = -1;
-    auto wave_sum = [&]() {
-      for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off);
-    };
-    for (int64_t base = begin; base < end; base += kAccBlock) {
-      const int64_t i = base + threadIdx.x;
-      const int32_t m = i < end ? a.item_mesh[i] : -1;
-      double t = m >= 0 ? term(item_mesh(a.meshes[m]), i) : 0.0;
-      const int32_t m0 = __builtin_amdgcn_readfirstlane(m);
-      if (__ballot(m != m0) == 0ull) {
-        if (m0 != cur) {
-          wave_sum();
-          if (lane == 0 && cur >= 0) atomicAdd(&energy[cur], e);
-          e = 0.0;
-          cur = m0;
-        }
-        e += t;
-      } else {
-        const int32_t prev = __shfl_up(m, 1);
-        const bool head = lane == 0 || prev != m;
-        const int rem = run_left(__ballot(head));
-        for (int off = 1; off < 64; off <<= 1) {
-          const double u = __shfl_down(t, off);
-          if (rem >= off) t += u;
-        }
-        if (head && m >= 0) atomicAdd(&energy[m], t);
-      }
-    }
-    wave_sum();
-    if (lane == 0) {
-      red[wave] = e;
-      mesh[wave] = cur;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0)  // one atomic for neighbouring waves of one mesh
-      for (int k = 0; k < kWaves;) {
-        const int32_t m = mesh[k];
-        double sum = 0.0;
-        for (; k < kWaves && mesh[k] == m; ++k) sum += red[k];
-        if (m >= 0) atomicAdd(&energy[m], sum);
-      }
-  } else {
-    const int m0 = mesh_of(a, begin), m1 = mesh_of(a, end - 1);
+  double e = 0.0;
+  auto wave_sum = [&]() {
+    for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off);
+  };
+  const int m0 = mesh_of(a, begin), m1 = mesh_of(a, end - 1);
+  if (m1 - m0 < kLoopMeshes) {  // block-uniform
     for (int m = m0; m <= m1; ++m) {
       const EnergyMesh em = a.meshes[m];
       const ItemMesh im = item_mesh(em);
-      const int64_t first = max(begin, em.item_off), last = min(end, em.item_off + em.n_items);
-      double e = 0.0;
+      const int64_t last = min(end, em.item_off + em.n_items);
+      e = 0.0;
 #pragma unroll 4
-      for (int64_t i = first + threadIdx.x; i < last; i += kAccBlock) e += term(im, i);
-      for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off);
+      for (int64_t i = max(begin, em.item_off) + threadIdx.x; i < last; i += kAccBlock) e += term(im, i);
+      wave_sum();
       __syncthreads();  // red of the previous mesh has been read
-      if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = e;
+      if (lane == 0) red[wave] = e;
       __syncthreads();
       if (threadIdx.x == 0) {
         for (int k = 1; k < kWaves; ++k) e += red[k];
         atomicAdd(&energy[m], e);
       }
     }
+    return;
   }
+  // a wave adds up the items of one mesh (cur) while its lanes lie in it, and else
+  // the runs of its lanes in each mesh
+  int32_t cur = -1;
+  for (int64_t base = begin; base < end; base += kAccBlock) {
+    const int64_t i = base + threadIdx.x;
+    const int32_t m = i < end ? a.item_mesh[i] : -1;
+    double t = m >= 0 ? term(item_mesh(a.meshes[m]), i) : 0.0;
+    const int32_t first = __builtin_amdgcn_readfirstlane(m);
+    if (__ballot(m != first) == 0ull) {
+      if (first != cur) {
+        wave_sum();
+        if (lane == 0 && cur >= 0) atomicAdd(&energy[cur], e);
+        e = 0.0;
+        cur = first;
+      }
+      e += t;
+    } else {
+      const int32_t prev = __shfl_up(m, 1);
+      const bool head = lane == 0 || prev != m;
+      const int rem = run_left(__ballot(head));
+      for (int off = 1; off < 64; off <<= 1) {
+        const double u = __shfl_down(t, off);
+        if (rem >= off) t += u;
+      }
+      if (head && m >= 0) atomicAdd(&energy[m], t);
+    }
+  }
+  wave_sum();
+  if (lane == 0) {
+    red[wave] = e;
+    mesh[wave] = cur;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int k = 0; k < kWaves;) {  // one atomic for neighbouring waves of one mesh
+      const int32_t m = mesh[k];
+      double sum = 0.0;
+      for (; k < kWaves && mesh[k] == m; ++k) sum += red[k];
+      if (m >= 0) atomicAdd(&energy[m], sum);
+    }
 }
 
 // The whole forward of one small isotropic mesh in one block: sums, points and
@@ -793,14 +810,17 @@ __device__ inline PlaneAdjoint no_adjoint() {
 // most of this kernel's waits.  A wave with a ring of more clusters visits the
 // faces again for the next two (against reading them face by face: labels of a
 // graded clustering of 4 x 1 M vertices 296 -> 257 us, 12 vertices a cluster
-// 306 -> 266, 42 a cluster 708 -> 715).  Consecutive blocks run on one XCD, whose
+// 306 -> 266, 42 a cluster 708 -> 715).  A ring of more than eight entries takes
+// them eight at a time, faces past 32 come four at a time from the vertex's row (one
+// by one behind its loads, and from the row past 16: a sphere of 368,642 vertices of
+// valence 3 to 24, labels of a clustering, 303 us, so 95; the forward 232, 101).  Consecutive blocks run on one XCD, whose
 // L2 then holds the rows a block shares with its neighbours (HBM reads 1.27 ->
 // 0.87 GB).  Bound by the f64 work (950
 // instructions per 64 vertices, half of the time) and by gather latency at 3
 // waves per SIMD (168 registers; held to 128 the spills cost more: 1359 us;
 // a loop over the faces that keeps one position in flight: 831 us).
 // 16.8 M QEM vertices 2050 -> 765 us, 1 M isotropic ones 10.5 -> 8.6 us.
-template <bool kQem, bool kMany>
+template <bool kQem>
 __global__ __launch_bounds__(kEBlock) void ke_item_grad(EnergyArgs a, const double* __restrict__ gE,
                                                         float* __restrict__ dxyz, float* __restrict__ dw) {
   constexpr int kXcd = 8;
@@ -816,16 +836,15 @@ __global__ __launch_bounds__(kEBlock) void ke_item_grad(EnergyArgs a, const doub
   const Vec3 x = load_point(a.xyz, ic);
   int32_t e[kRingChunk];
   int32_t slots = 0;
-  if constexpr (kQem) slots = load_ring(a, i, e);
-  const int m0 = kMany ? 0 : mesh_of(a, begin), m1 = kMany ? 0 : mesh_of(a, end - 1);
-  for (int m = m0; m <= m1; ++m) {
-    const EnergyMesh& mesh = a.meshes[kMany ? a.item_mesh[ic] : m];
-    const ItemMesh em = item_mesh(mesh);
-    const bool active = i < end && (kMany || (i >= mesh.item_off && i < mesh.item_off + mesh.n_items));
-    const double g = gE[kMany ? a.item_mesh[ic] : m];
+  if constexpr (kQem) slots = load_ring(a, i, 0, e);
+  const int m0 = mesh_of(a, begin);
+  const bool one = m0 == mesh_of(a, end - 1);  // block-uniform
+  // (a build of it with the mesh in scalar registers and one without)
+  auto grad = [&](const ItemMesh& em, double g) {
+    const bool active = i < end;
     double gx[3] = {0, 0, 0}, gw = 0.0;
     const int32_t c = active ? cluster_of(em, lab) : -1;
-    const bool qem = kQem && em.qem;  // block-uniform unless kMany
+    const bool qem = kQem && em.qem;
     if (c >= 0) {
       const double w = double(wf);
       const double* q = a.pts + 4 * int64_t(c);
@@ -839,26 +858,6 @@ __global__ __launch_bounds__(kEBlock) void ke_item_grad(EnergyArgs a, const doub
       }
     }
     if (qem && active) {
-      // clusters of the ring's first entries: bit k of own_bits the vertex's own, of
-      // todo another one whose part is still to be taken
-      const bool is_long = e[0] == kRingLong;
-      const bool more = is_long || (slots > kRingChunk && e[kRingChunk - 1] != kRingEnd);
-      int32_t cl[kRingChunk];
-      uint32_t own_bits = 0, todo = 0;
-#pragma unroll
-      for (int k = 0; k < kRingChunk; ++k) {
-        if (k >= slots) break;  // wave-uniform
-        if (e[k] == kRingEnd || is_long) e[k] = int32_t(uint32_t(i) | 0x80000000u);  // no face
-        cl[k] = a.labels[e[k] & kRingId];
-      }
-#pragma unroll
-      for (int k = 0; k < kRingChunk; ++k) {
-        if (k >= slots) break;
-        cl[k] = cluster_of(em, cl[k]);
-        if (cl[k] >= 0) (cl[k] == c ? own_bits : todo) |= 1u << k;
-      }
-      PlaneAdjoint A0 = c >= 0 ? plane_adjoint(a.adj + kAdjStride * int64_t(c), x) : no_adjoint();
-      double own = c >= 0 ? 1.0 : 0.0;
       // the face (v, v + u, v + s) with adjoint F: n = u x s; u receives s x dn,
       // s receives dn x u, and v minus both (dn x (u - s)) and minus (g . n) n
       auto pull = [&](const PlaneAdjoint& F, const Vec3& u, const Vec3& s) {
@@ -871,66 +870,110 @@ __global__ __launch_bounds__(kEBlock) void ke_item_grad(EnergyArgs a, const doub
         gx[1] -= __builtin_fma(gn, n.y, __builtin_fma(n2, t.x, -(n0 * t.z)));
         gx[2] -= __builtin_fma(gn, n.z, __builtin_fma(n0, t.y, -(n1 * t.x)));
       };
-      Vec3 u{0.0, 0.0, 0.0};
-      while (true) {
-        int32_t c1 = -1, c2 = -1;
-        uint32_t bits1 = 0, bits2 = 0;
+      auto adjoint_of = [&](int32_t cl) {
+        return cl >= 0 ? plane_adjoint(a.adj + kAdjStride * int64_t(cl), x) : no_adjoint();
+      };
+      const bool is_long = e[0] == kRingLong;
+      // kRingChunk entries at a time; a further chunk starts at the last entry of the
+      // one before, whose face with the next entry it takes
+      for (int from = 0;;) {
+        // clusters of the entries: bit k of own_bits the vertex's own, of todo another
+        // one whose part is still to be taken
+        const bool more = !is_long && slots - from > kRingChunk && e[kRingChunk - 1] != kRingEnd;
+        int32_t cl[kRingChunk];
+        uint32_t own_bits = 0, todo = 0;
 #pragma unroll
         for (int k = 0; k < kRingChunk; ++k) {
-          if (k >= slots) break;
-          if (!(todo >> k & 1u)) continue;
-          if (c1 < 0) c1 = cl[k];
-          if (cl[k] == c1) bits1 |= 1u << k;
-          else {
-            if (c2 < 0) c2 = cl[k];
-            if (cl[k] == c2) bits2 |= 1u << k;
-          }
+          if (k >= slots - from) break;  // wave-uniform
+          if (e[k] == kRingEnd || is_long) e[k] = int32_t(uint32_t(i) | 0x80000000u);  // no face
+          cl[k] = a.labels[e[k] & kRingId];
         }
-        todo &= ~(bits1 | bits2);
-        const PlaneAdjoint A1 = c1 >= 0 ? plane_adjoint(a.adj + kAdjStride * int64_t(c1), x) : no_adjoint();
-        const PlaneAdjoint A2 = c2 >= 0 ? plane_adjoint(a.adj + kAdjStride * int64_t(c2), x) : no_adjoint();
 #pragma unroll
         for (int k = 0; k < kRingChunk; ++k) {
-          if (k >= slots) break;
-          const Vec3 s = sub(ring_point(a, e[k]), x);
-          if (k > 0 && e[k] >= 0) {
-            const double w0 = own + ((own_bits >> (k - 1) & 1u) ? 1.0 : 0.0) + ((own_bits >> k & 1u) ? 1.0 : 0.0);
-            const double w1 = ((bits1 >> (k - 1) & 1u) ? 1.0 : 0.0) + ((bits1 >> k & 1u) ? 1.0 : 0.0);
-            const double w2 = ((bits2 >> (k - 1) & 1u) ? 1.0 : 0.0) + ((bits2 >> k & 1u) ? 1.0 : 0.0);
-            PlaneAdjoint F;
-            for (int j = 0; j < 6; ++j)
-              F.m[j] = __builtin_fma(w2, A2.m[j], __builtin_fma(w1, A1.m[j], w0 * A0.m[j]));
-            for (int j = 0; j < 3; ++j)
-              F.g[j] = __builtin_fma(w2, A2.g[j], __builtin_fma(w1, A1.g[j], w0 * A0.g[j]));
-            pull(F, u, s);
-          }
-          u = s;
+          if (k >= slots - from) break;
+          cl[k] = cluster_of(em, cl[k]);
+          if (cl[k] >= 0) (cl[k] == c ? own_bits : todo) |= 1u << k;
         }
-        if (__ballot(todo != 0) == 0ull) break;
-        // rings of more clusters: the faces again for the next two, the own part done
-        A0 = no_adjoint();
-        own = 0.0;
-        own_bits = 0;
+        PlaneAdjoint A0 = adjoint_of(c);
+        double own = c >= 0 ? 1.0 : 0.0;
+        Vec3 u{0.0, 0.0, 0.0};
+        while (true) {
+          int32_t c1 = -1, c2 = -1;
+          uint32_t bits1 = 0, bits2 = 0;
+#pragma unroll
+          for (int k = 0; k < kRingChunk; ++k) {
+            if (k >= slots - from) break;
+            if (!(todo >> k & 1u)) continue;
+            if (c1 < 0) c1 = cl[k];
+            if (cl[k] == c1) bits1 |= 1u << k;
+            else {
+              if (c2 < 0) c2 = cl[k];
+              if (cl[k] == c2) bits2 |= 1u << k;
+            }
+          }
+          todo &= ~(bits1 | bits2);
+          const PlaneAdjoint A1 = adjoint_of(c1), A2 = adjoint_of(c2);
+#pragma unroll
+          for (int k = 0; k < kRingChunk; ++k) {
+            if (k >= slots - from) break;
+            const Vec3 s = sub(ring_point(a, e[k]), x);
+            if (k > 0 && e[k] >= 0) {
+              const double w0 = own + ((own_bits >> (k - 1) & 1u) ? 1.0 : 0.0) + ((own_bits >> k & 1u) ? 1.0 : 0.0);
+              const double w1 = ((bits1 >> (k - 1) & 1u) ? 1.0 : 0.0) + ((bits1 >> k & 1u) ? 1.0 : 0.0);
+              const double w2 = ((bits2 >> (k - 1) & 1u) ? 1.0 : 0.0) + ((bits2 >> k & 1u) ? 1.0 : 0.0);
+              PlaneAdjoint F;
+              for (int j = 0; j < 6; ++j)
+                F.m[j] = __builtin_fma(w2, A2.m[j], __builtin_fma(w1, A1.m[j], w0 * A0.m[j]));
+              for (int j = 0; j < 3; ++j)
+                F.g[j] = __builtin_fma(w2, A2.g[j], __builtin_fma(w1, A1.g[j], w0 * A0.g[j]));
+              pull(F, u, s);
+            }
+            u = s;
+          }
+          if (__ballot(todo != 0) == 0ull) break;
+          // rings of more clusters: the faces again for the next two, the own part done
+          A0 = no_adjoint();
+          own = 0.0;
+          own_bits = 0;
+        }
+        if (!more) break;
+        from += kRingChunk - 1;
+        load_ring(a, i, from, e);
       }
-      if (more) {  // faces past the first entries, in full
-        auto pull_of = [&](int32_t cj, const Vec3& r, const Vec3& s) {
-          if (cj >= 0) pull(plane_adjoint(a.adj + kAdjStride * int64_t(cj), x), r, s);
-        };
-        const int32_t cu = is_long ? -1 : cl[kRingChunk - 1];
-        walk_rest(
-            a, i, x, is_long ? kRingLong : 0, kRingChunk, u, cu,
-            [&](int32_t j) { return cluster_of(em, a.labels[j]); },
-            [&](const Vec3& r, int32_t cr, const Vec3& s, int32_t cs) {
-              pull_of(c, r, s);
-              pull_of(cr, r, s);
-              pull_of(cs, r, s);
-            });
+      if (is_long) {
+        const PlaneAdjoint A0 = adjoint_of(c);
+        walk_faces(a, i, [&](int n, const int32_t* v1, const int32_t* v2) {
+          Vec3 r[kFaceBatch], t[kFaceBatch];
+          int32_t c1[kFaceBatch], c2[kFaceBatch];
+#pragma unroll
+          for (int k = 0; k < kFaceBatch; ++k) {
+            r[k] = sub(load_point(a.xyz, v1[k]), x);
+            t[k] = sub(load_point(a.xyz, v2[k]), x);
+            c1[k] = a.labels[v1[k]];
+            c2[k] = a.labels[v2[k]];
+          }
+#pragma unroll
+          for (int k = 0; k < kFaceBatch; ++k) {
+            if (k >= n) break;
+            const PlaneAdjoint A1 = adjoint_of(cluster_of(em, c1[k])), A2 = adjoint_of(cluster_of(em, c2[k]));
+            PlaneAdjoint F;
+            for (int j = 0; j < 6; ++j) F.m[j] = A0.m[j] + A1.m[j] + A2.m[j];
+            for (int j = 0; j < 3; ++j) F.g[j] = A0.g[j] + A1.g[j] + A2.g[j];
+            pull(F, r[k], t[k]);
+          }
+        });
       }
     }
     if (active) {
       for (int k = 0; k < 3; ++k) dxyz[3 * i + k] = float(g * gx[k]);
       dw[i] = float(g * gw);
     }
+  };
+  if (one) {
+    grad(item_mesh(a.meshes[m0]), gE[m0]);
+  } else {
+    const int32_t m = a.item_mesh[ic];
+    grad(item_mesh(a.meshes[m]), gE[m]);
   }
 }
 
@@ -957,16 +1000,15 @@ hipError_t energy_forward(hipStream_t s, const EnergyArgs& a, double* energy, in
   if (a.n_items > 0) {
     const int64_t chunk = item_chunk(a.n_items, kAccMaxBlocks);
     const dim3 grid(unsigned((a.n_items + chunk - 1) / chunk));
-    const auto k = a.adj ? (a.many ? ke_accumulate<true, true> : ke_accumulate<true, false>)
-                         : (a.many ? ke_accumulate<false, true> : ke_accumulate<false, false>);
+    const auto k = a.adj ? ke_accumulate<true> : ke_accumulate<false>;
     hipLaunchKernelGGL(k, grid, dim3(kAccBlock), 0, s, a, chunk);
   }
   if (a.n_clusters > 0)
     hipLaunchKernelGGL(ke_points, dim3(unsigned((a.n_clusters + 63) / 64)), dim3(64), 0, s, a);
   if (a.n_items > 0) {
     const int64_t chunk = item_chunk(a.n_items, 512);
-    hipLaunchKernelGGL(a.many ? ke_energy<true> : ke_energy<false>, dim3(unsigned((a.n_items + chunk - 1) / chunk)),
-                       dim3(kAccBlock), 0, s, a, chunk, energy);
+    hipLaunchKernelGGL(ke_energy, dim3(unsigned((a.n_items + chunk - 1) / chunk)), dim3(kAccBlock), 0, s, a, chunk,
+                       energy);
   }
   return hipGetLastError();
 }
@@ -1065,8 +1107,7 @@ hipError_t energy_forward_cvt_noalloc(hipStream_t s, int64_t n, int32_t K, const
 
 hipError_t energy_backward(hipStream_t s, const EnergyArgs& a, const double* grad_energy, float* dxyz, float* dw) {
   if (a.n_items > 0) {
-    const auto k = a.adj ? (a.many ? ke_item_grad<true, true> : ke_item_grad<true, false>)
-                         : (a.many ? ke_item_grad<false, true> : ke_item_grad<false, false>);
+    const auto k = a.adj ? ke_item_grad<true> : ke_item_grad<false>;
     hipLaunchKernelGGL(k, dim3(egrid(a.n_items)), dim3(kEBlock), 0, s, a, grad_energy, dxyz, dw);
   }
   return hipGetLastError();

@@ -224,7 +224,8 @@ def ring_problem(shape):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("shape", ["hub9", "hub16", "hub17", "hub70", "grid", "bowtie", "scattered4", "scattered5"])
+@pytest.mark.parametrize("shape", ["hub9", "hub16", "hub17", "hub70", "grid", "bowtie", "scattered4", "scattered5"] +
+                         [f"hub{n}" for n in (7, 8, 14, 15, 21, 22, 31, 32, 33, 37)])  # a ring's chunks; rows past a ring
 @pytest.mark.parametrize("metric", [ISO, QEM])
 def test_gpu_energy_rings_match_oracle(gpu_ready, metric, shape):
     """Against the oracle on meshes with every form of ring, alone and behind

@@ -30,8 +30,8 @@ struct EnergyArgs {
   const int32_t* vfptr;      // vertex -> incident faces, one entry per corner
   const int32_t* vfcol;
   // rings (faces around each QEM vertex as chains of neighbour ids): group g of
-  // 64 items holds slots [ring_slot[g], ring_slot[g + 1]) of 64 ids
-  const int32_t* ring_slot;
+  // 64 items holds ring_slot[g].y slots of 64 ids from slot ring_slot[g].x on
+  const int2* ring_slot;
   const int32_t* ring;
   // inputs of one call
   const float* xyz;          // 3 per item
@@ -61,7 +61,9 @@ hipError_t energy_vf_count(hipStream_t s, int64_t n3, const int32_t* tri, int32_
 hipError_t energy_vf_fill(hipStream_t s, int64_t n, int64_t n3, const int32_t* tri, const int32_t* vfptr,
                           int32_t* fill, int32_t* vfcol);
 hipError_t energy_ring_slots(hipStream_t s, const EnergyArgs& a, int32_t* slots);
-hipError_t energy_ring_fill(hipStream_t s, const EnergyArgs& a, const int32_t* slot, int32_t* ring);
+// start: first slot of each group; null: those in ring_slot[g].x
+hipError_t energy_ring_fill(hipStream_t s, const EnergyArgs& a, const int32_t* start, int2* ring_slot, int32_t* ring);
+hipError_t energy_set_mesh(hipStream_t s, const EnergyMesh& m, EnergyMesh* dst);
 
 hipError_t energy_forward(hipStream_t s, const EnergyArgs& a, double* energy, int n_meshes);
 // Largest cluster count of energy_forward_cvt_noalloc (its static scratch).

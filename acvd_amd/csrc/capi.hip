@@ -140,6 +140,9 @@ constexpr int kChunk = 16;        // passes per graph launch
 constexpr int kShortChunk = 4;    // passes per graph launch near the end of a phase
 static_assert(kPassLogCap > kChunk, "the pass log must hold a chunk of passes");
 constexpr int64_t kHostLabels = 65536;  // labels of at most so many items are renumbered on the host: a launch costs more
+// Meshes of at most so many faces are uploaded together by way of a host array: a
+// copy costs more (first energy of 64 QEM meshes of 1,024 vertices 1,777 -> 552 us).
+constexpr int64_t kStageFaces = 16384;
 constexpr int kReduceItems = 16384;  // items per block of the deterministic reductions
 constexpr int kEnergyLogRing = 2 * kChunk;  // energy log entries per mesh on the device, drained per chunk
 
@@ -1947,6 +1950,7 @@ struct acvd_energy {
   DBuf<double> d_acc, d_pts, d_adj;
   bool have_forward = false;
   bool any_qem = false;
+  size_t ring_slot_at() const { return (6 * size_t(F) + size_t(N) + 2) / 2 * 2; }  // in d_topo, a multiple of 8 bytes
   EnergyArgs args() const {
     EnergyArgs a{};
     a.n_items = N;
@@ -1958,7 +1962,7 @@ struct acvd_energy {
       a.tri = d_topo.p;
       a.vfptr = d_topo.p + 3 * F;
       a.vfcol = d_topo.p + 3 * F + N + 1;
-      a.ring_slot = d_topo.p + 6 * F + N + 1;
+      a.ring_slot = reinterpret_cast<const int2*>(d_topo.p + ring_slot_at());
       a.ring = d_ring.p;
     }
     a.acc_stride = any_qem ? 13 : 4;
@@ -1970,6 +1974,90 @@ struct acvd_energy {
 };
 
 namespace {
+
+// Vertex -> face rows and rings of a small context: the rows, and room for any
+// ring of a row's length, on the host, in one upload.  The launches, scans and
+// waits of the device build cost more than the loops up to kHostRowItems (first
+// forward, host / device: 2,500 QEM vertices 103 / 178 us, 7,000 128 / 171, 10,240
+// 162 / 174, 40,000 211 / 206).
+constexpr int64_t kHostRowItems = 16384;
+int energy_rows_host(acvd_energy* e, const std::vector<EnergyMesh>& hm, hipStream_t s) {
+  const int64_t N = e->N, F = e->F, G = (N + 63) / 64;
+  std::vector<int32_t> topo(e->d_topo.n, 0);
+  int32_t *tri = topo.data(), *vfptr = tri + 3 * F, *vfcol = vfptr + N + 1, *slot = tri + e->ring_slot_at();
+  for (size_t m = 0; m < hm.size(); ++m) {
+    const std::vector<int32_t>& t = e->meshes[m].tri;
+    for (size_t k = 0; k < t.size(); ++k) tri[3 * hm[m].face_off + k] = t[k] + int32_t(hm[m].item_off);
+  }
+  for (int64_t k = 0; k < 3 * F; ++k) vfptr[tri[k] + 1]++;
+  for (int64_t v = 0; v < N; ++v) vfptr[v + 1] += vfptr[v];
+  std::vector<int32_t> next(vfptr, vfptr + N);
+  for (int64_t f = 0; f < F; ++f)
+    for (int j = 0; j < 3; ++j) vfcol[next[tri[3 * f + j]]++] = int32_t(f);
+  int32_t slots = 0;
+  for (int64_t g = 0; g < G; ++g) {
+    int32_t most = 0;
+    for (int64_t v = 64 * g; v < std::min(N, 64 * g + 64); ++v) {
+      const int32_t faces = vfptr[v + 1] - vfptr[v];
+      most = std::max(most, faces > kRingFaces ? 1 : 2 * faces);  // (a ring of n faces: at most n chains)
+    }
+    slot[2 * g] = slots;
+    slots += most;
+  }
+  HIP_TRY(hipMemcpy(e->d_topo.p, topo.data(), topo.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+  HIP_TRY(e->d_ring.alloc(64 * size_t(slots)));
+  HIP_TRY(energy_ring_fill(s, e->args(), nullptr, reinterpret_cast<int2*>(e->d_topo.p + e->ring_slot_at()),
+                           e->d_ring.p));
+  return ACVD_OK;
+}
+
+int energy_rows_device(acvd_energy* e, const std::vector<EnergyMesh>& hm, hipStream_t s) {
+  const int64_t N = e->N, F = e->F, G = (N + 63) / 64;
+  const int M = int(hm.size());
+  int32_t* tri = e->d_topo.p;
+  int32_t* vfptr = tri + 3 * F;
+  int32_t* vfcol = vfptr + N + 1;
+  // faces: small meshes by way of one host array a run of them, large ones as they are
+  std::vector<int32_t> stage;
+  for (int m = 0; m < M;) {
+    if (M == 1 || e->meshes[m].nf > kStageFaces) {
+      const auto& h = e->meshes[m];
+      int32_t* t = tri + 3 * hm[m].face_off;
+      HIP_TRY(hipMemcpy(t, h.tri.data(), 3 * h.nf * sizeof(int32_t), hipMemcpyHostToDevice));
+      HIP_TRY(energy_offset_tri(s, 3 * h.nf, int32_t(hm[m].item_off), t));
+      ++m;
+      continue;
+    }
+    const int first = m;
+    stage.clear();
+    for (; m < M && e->meshes[m].nf <= kStageFaces; ++m)
+      for (int32_t v : e->meshes[m].tri) stage.push_back(v + int32_t(hm[m].item_off));
+    HIP_TRY(hipMemcpy(tri + 3 * hm[first].face_off, stage.data(), stage.size() * sizeof(int32_t),
+                      hipMemcpyHostToDevice));
+  }
+  DBuf<int32_t> tmp;  // face counts, fill counts, ring slots and their starts
+  struct Tmp {  // scan workspace
+    void* p = nullptr;
+    size_t n = 0;
+    ~Tmp() {
+      if (p) (void)hipFree(p);
+    }
+  } scan;
+  HIP_TRY(tmp.alloc((N + 1) + N + 2 * (G + 1)));
+  int32_t *deg = tmp.p, *fill = deg + N + 1, *slots = fill + N, *start = slots + G + 1;
+  HIP_TRY(hipMemsetAsync(tmp.p, 0, tmp.n * sizeof(int32_t), s));
+  HIP_TRY(energy_vf_count(s, 3 * F, tri, deg));
+  HIP_TRY(exclusive_scan_i32(s, deg, vfptr, N + 1, &scan.p, &scan.n));
+  HIP_TRY(energy_vf_fill(s, N, 3 * F, tri, vfptr, fill, vfcol));
+  HIP_TRY(energy_ring_slots(s, e->args(), slots));
+  HIP_TRY(exclusive_scan_i32(s, slots, start, G + 1, &scan.p, &scan.n));
+  int32_t total = 0;
+  HIP_TRY(hipMemcpy(&total, start + G, sizeof(int32_t), hipMemcpyDeviceToHost));
+  HIP_TRY(e->d_ring.alloc(64 * size_t(total)));
+  HIP_TRY(energy_ring_fill(s, e->args(), start, reinterpret_cast<int2*>(e->d_topo.p + e->ring_slot_at()),
+                           e->d_ring.p));
+  return ACVD_OK;
+}
 
 int energy_build(acvd_energy* e) {
   if (e->built) return ACVD_OK;
@@ -2004,8 +2092,10 @@ int energy_build(acvd_energy* e) {
     co += h.K;
     fo += h.nf;
   }
+  const hipStream_t s = nullptr;  // the default stream, as the copies
   HIP_TRY(e->d_meshes.alloc(M));
-  HIP_TRY(hipMemcpy(e->d_meshes.p, hm.data(), M * sizeof(EnergyMesh), hipMemcpyHostToDevice));
+  if (M == 1) HIP_TRY(energy_set_mesh(s, hm[0], e->d_meshes.p));
+  else HIP_TRY(hipMemcpy(e->d_meshes.p, hm.data(), M * sizeof(EnergyMesh), hipMemcpyHostToDevice));
   if (M > 1) {
     HIP_TRY(e->d_item_mesh.alloc(N));
     HIP_TRY(e->d_clus_mesh.alloc(K));
@@ -2021,42 +2111,12 @@ int energy_build(acvd_energy* e) {
   e->K = K;
   e->F = F;
   if (e->any_qem) {  // the isotropic energy needs no faces
-    const hipStream_t s = nullptr;  // as the copies above: the default stream
-    const int64_t G = (N + 63) / 64;
     HIP_TRY(e->d_adj.alloc(kAdjStride * K));
-    HIP_TRY(e->d_topo.alloc(6 * F + (N + 1) + (G + 1)));
-    int32_t* tri = e->d_topo.p;
-    int32_t* vfptr = tri + 3 * F;
-    int32_t* vfcol = vfptr + N + 1;
-    int32_t* ring_slot = vfcol + 3 * F;
-    DBuf<int32_t> tmp;  // face counts, fill counts, ring slots
-    struct Tmp {  // scan workspace
-      void* p = nullptr;
-      size_t n = 0;
-      ~Tmp() {
-        if (p) (void)hipFree(p);
-      }
-    } scan;
-    HIP_TRY(tmp.alloc((N + 1) + N + (G + 1)));
-    int32_t *deg = tmp.p, *fill = deg + N + 1, *slots = fill + N;
-    HIP_TRY(hipMemsetAsync(tmp.p, 0, tmp.n * sizeof(int32_t), s));
-    for (int m = 0; m < M; ++m) {
-      const auto& h = e->meshes[m];
-      int32_t* t = tri + 3 * hm[m].face_off;
-      HIP_TRY(hipMemcpy(t, h.tri.data(), 3 * h.nf * sizeof(int32_t), hipMemcpyHostToDevice));
-      HIP_TRY(energy_offset_tri(s, 3 * h.nf, int32_t(hm[m].item_off), t));
-    }
-    HIP_TRY(energy_vf_count(s, 3 * F, tri, deg));
-    HIP_TRY(exclusive_scan_i32(s, deg, vfptr, N + 1, &scan.p, &scan.n));
-    HIP_TRY(energy_vf_fill(s, N, 3 * F, tri, vfptr, fill, vfcol));
-    HIP_TRY(energy_ring_slots(s, e->args(), slots));
-    HIP_TRY(exclusive_scan_i32(s, slots, ring_slot, G + 1, &scan.p, &scan.n));
-    int32_t total = 0;
-    HIP_TRY(hipMemcpy(&total, ring_slot + G, sizeof(int32_t), hipMemcpyDeviceToHost));
-    HIP_TRY(e->d_ring.alloc(64 * size_t(total)));
-    HIP_TRY(energy_ring_fill(s, e->args(), ring_slot, e->d_ring.p));
-    HIP_TRY(hipStreamSynchronize(s));  // a caller's stream need not wait for the default one
+    HIP_TRY(e->d_topo.alloc(e->ring_slot_at() + 2 * size_t((N + 63) / 64)));
+    const bool small = N <= kHostRowItems && F <= 4 * kHostRowItems;
+    if (int rc = small ? energy_rows_host(e, hm, s) : energy_rows_device(e, hm, s)) return rc;
   }
+  HIP_TRY(hipStreamSynchronize(s));  // a caller's stream need not wait for the default one
   e->built = true;
   return ACVD_OK;
 }

@@ -109,7 +109,8 @@ __device__ inline int32_t load_ring(const EnergyArgs& a, int64_t i, int from, in
 #pragma unroll
   for (int k = 0; k < kRingChunk; ++k) e[k] = kRingEnd;
   if (64 * g >= a.n_items) return 0;  // a wave past the last group
-  const int32_t s0 = a.ring_slot[g], n = a.ring_slot[g + 1] - s0;  // scalar loads
+  const int2 slot = a.ring_slot[g];  // a scalar load
+  const int32_t s0 = slot.x, n = slot.y;
 #pragma unroll
   for (int k = 0; k < kRingChunk; ++k)
     if (from + k < n) e[k] = a.ring[int64_t(s0 + from + k) * 64 + lane];
@@ -209,6 +210,8 @@ __device__ inline void kept_set(const double lam[3], int level, bool keep[3]) {
 __device__ inline double dot3(const double* a, const double* b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; }
 
 // ---------------------------------------------------------------- ring build
+__global__ void ke_set_mesh(EnergyMesh m, EnergyMesh* dst) { *dst = m; }
+
 __global__ void ke_offset_tri(int64_t n, int32_t off, int32_t* tri) {
   const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (k < n) tri[k] += off;
@@ -227,13 +230,9 @@ __global__ void ke_vf_fill(int64_t n3, const int32_t* __restrict__ tri, const in
   vfcol[vfptr[v] + atomicAdd(&fill[v], 1)] = int32_t(k / 3);
 }
 
-// Sorts the vertex -> face rows by face id (heap sort: a row of any length in
+// Sorts a vertex -> face row by face id (heap sort: a row of any length in
 // n log n steps), so that a ring does not depend on the order of the atomics.
-__global__ void ke_vf_sort(int64_t n, const int32_t* __restrict__ vfptr, int32_t* vfcol) {
-  const int64_t v = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (v >= n) return;
-  int32_t* r = vfcol + vfptr[v];
-  const int32_t len = vfptr[v + 1] - vfptr[v];
+__device__ inline void sort_row(int32_t* r, int32_t len) {
   if (len <= 32) {
     for (int32_t i = 1; i < len; ++i) {
       const int32_t x = r[i];
@@ -260,6 +259,11 @@ __global__ void ke_vf_sort(int64_t n, const int32_t* __restrict__ vfptr, int32_t
     }
     r[p] = x;
   }
+}
+
+__global__ void ke_vf_sort(int64_t n, const int32_t* __restrict__ vfptr, int32_t* vfcol) {
+  const int64_t v = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (v < n) sort_row(vfcol + vfptr[v], vfptr[v + 1] - vfptr[v]);
 }
 
 // Ring of vertex v (at most kRingFaces faces): the links a -> b of its faces
@@ -301,32 +305,33 @@ __device__ int ring_chains(const EnergyArgs& a, int64_t v, Emit&& emit) {
   return n;
 }
 
+// Entries of the ring of vertex v (0 past the end and outside QEM meshes).
+template <class Emit>
+__device__ inline int ring_of(const EnergyArgs& a, int64_t v, Emit&& emit) {
+  if (v >= a.n_items || a.meshes[mesh_of(a, v)].metric != 1) return 0;
+  if (a.vfptr[v + 1] - a.vfptr[v] <= kRingFaces) return ring_chains(a, v, emit);
+  emit(0, kRingLong);
+  return 1;
+}
+
+__device__ inline int wave_max(int n) {
+  for (int off = 32; off > 0; off >>= 1) n = max(n, __shfl_xor(n, off));
+  return n;
+}
+
 // Slots of each group of 64 vertices: the longest ring of its QEM vertices.
 __global__ __launch_bounds__(64) void ke_ring_slots(EnergyArgs a, int32_t* slots) {
-  const int64_t v = int64_t(blockIdx.x) * 64 + threadIdx.x;
-  int n = 0;
-  if (v < a.n_items && a.meshes[mesh_of(a, v)].metric == 1) {
-    if (a.vfptr[v + 1] - a.vfptr[v] > kRingFaces) n = 1;
-    else n = ring_chains(a, v, [](int, int32_t) {});
-  }
-  for (int off = 32; off > 0; off >>= 1) n = max(n, __shfl_xor(n, off));
+  const int n = wave_max(ring_of(a, int64_t(blockIdx.x) * 64 + threadIdx.x, [](int, int32_t) {}));
   if (threadIdx.x == 0) slots[blockIdx.x] = n;
 }
 
-__global__ __launch_bounds__(64) void ke_ring_fill(EnergyArgs a, const int32_t* __restrict__ slot, int32_t* ring) {
-  const int64_t v = int64_t(blockIdx.x) * 64 + threadIdx.x;
-  const int32_t s0 = slot[blockIdx.x], s1 = slot[blockIdx.x + 1];
+__global__ __launch_bounds__(64) void ke_ring_fill(EnergyArgs a, const int32_t* start, int2* ring_slot, int32_t* ring) {
+  const int32_t s0 = start ? start[blockIdx.x] : ring_slot[blockIdx.x].x;
   int32_t* r = ring + int64_t(s0) * 64 + threadIdx.x;
-  int n = 0;
-  if (v < a.n_items && a.meshes[mesh_of(a, v)].metric == 1) {
-    if (a.vfptr[v + 1] - a.vfptr[v] > kRingFaces) {
-      r[0] = kRingLong;
-      n = 1;
-    } else {
-      n = ring_chains(a, v, [&](int k, int32_t e) { r[int64_t(k) * 64] = e; });
-    }
-  }
-  for (; n < s1 - s0; ++n) r[int64_t(n) * 64] = kRingEnd;
+  int n = ring_of(a, int64_t(blockIdx.x) * 64 + threadIdx.x, [&](int k, int32_t e) { r[int64_t(k) * 64] = e; });
+  const int most = wave_max(n);
+  for (; n < most; ++n) r[int64_t(n) * 64] = kRingEnd;
+  if (threadIdx.x == 0) ring_slot[blockIdx.x] = make_int2(s0, most);
 }
 
 // ------------------------------------------------------------------ forward
@@ -1038,8 +1043,13 @@ hipError_t energy_ring_slots(hipStream_t s, const EnergyArgs& a, int32_t* slots)
   return hipGetLastError();
 }
 
-hipError_t energy_ring_fill(hipStream_t s, const EnergyArgs& a, const int32_t* slot, int32_t* ring) {
-  hipLaunchKernelGGL(ke_ring_fill, dim3(unsigned((a.n_items + 63) / 64)), dim3(64), 0, s, a, slot, ring);
+hipError_t energy_ring_fill(hipStream_t s, const EnergyArgs& a, const int32_t* start, int2* ring_slot, int32_t* ring) {
+  hipLaunchKernelGGL(ke_ring_fill, dim3(unsigned((a.n_items + 63) / 64)), dim3(64), 0, s, a, start, ring_slot, ring);
+  return hipGetLastError();
+}
+
+hipError_t energy_set_mesh(hipStream_t s, const EnergyMesh& m, EnergyMesh* dst) {
+  hipLaunchKernelGGL(ke_set_mesh, dim3(1), dim3(1), 0, s, m, dst);
   return hipGetLastError();
 }
 
@@ -1079,8 +1089,6 @@ hipError_t noalloc_scratch(unsigned char** out) {
   return hipSuccess;
 }
 
-__global__ void ke_set_mesh(EnergyMesh m, EnergyMesh* dst) { *dst = m; }
-
 }  // namespace
 
 hipError_t energy_forward_cvt_noalloc(hipStream_t s, int64_t n, int32_t K, const float* xyz, const float* w,
@@ -1101,8 +1109,8 @@ hipError_t energy_forward_cvt_noalloc(hipStream_t s, int64_t n, int32_t K, const
   a.acc_stride = 4;
   a.pts = acc + size_t(kNoAllocMaxClusters) * 4;
   // the descriptor is written by a kernel (no host copy: the call may be captured)
-  hipLaunchKernelGGL(ke_set_mesh, dim3(1), dim3(1), 0, s, EnergyMesh{0, n, 0, 0, K, 0, 0, 0}, mesh);
-  return energy_forward(s, a, energy, 1);
+  err = energy_set_mesh(s, EnergyMesh{0, n, 0, 0, K, 0, 0, 0}, mesh);
+  return err != hipSuccess ? err : energy_forward(s, a, energy, 1);
 }
 
 hipError_t energy_backward(hipStream_t s, const EnergyArgs& a, const double* grad_energy, float* dxyz, float* dw) {

@@ -228,8 +228,9 @@ def ring_problem(shape):
                          [f"hub{n}" for n in (7, 8, 14, 15, 21, 22, 31, 32, 33, 37)])  # a ring's chunks; rows past a ring
 @pytest.mark.parametrize("metric", [ISO, QEM])
 def test_gpu_energy_rings_match_oracle(gpu_ready, metric, shape):
-    """Against the oracle on meshes with every form of ring, alone and behind
-    another mesh of 37 vertices (rings and blocks not aligned to the mesh).
+    """Against the oracle on meshes with every form of ring, alone, behind
+    another mesh of 37 vertices (rings and blocks not aligned to the mesh) and
+    behind one of 17,600 too (rows built on the device).
     Tolerances: the energy sums FP64 terms in another order (1e-9), the gradients
     are rounded to FP32 (1e-5 of the largest component, as above)."""
     import torch
@@ -238,8 +239,11 @@ def test_gpu_energy_rings_match_oracle(gpu_ready, metric, shape):
     ref = po.EnergyRef(len(x), tri, np.where(lab < K, lab, K), K, metric, 2)
     e_ref, d = ref.total(x, w), ref.derivatives(x, w, np.arange(4 * len(x)))
     pad = ring_problem("hub35")
-    for lead in (False, True):
-        meshes = ([(pad, QEM)] if lead else []) + [((x, w, tri, lab, K), metric)]
+    xyz_t, tri_t = meshgen.torus(160, 110, 2)  # past the contexts whose rows the host builds
+    torus = (np.asarray(xyz_t, np.float64), np.ones(17600), np.asarray(tri_t, np.int32),
+             (np.arange(17600) // 50).astype(np.int32), 352)
+    for lead in ([], [(pad, QEM)], [(torus, QEM), (pad, QEM)]):
+        meshes = lead + [((x, w, tri, lab, K), metric)]
         ce = ClusterEnergy(0)
         for (mx, _, mt, _, mk), mm in meshes:
             ce.add_mesh(len(mx), mt, mk, mm, 2)

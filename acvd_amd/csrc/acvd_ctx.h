@@ -197,6 +197,9 @@ hipError_t launch_csr_sort_unique(hipStream_t s, int64_t n, const int32_t* tptr,
                                   const int32_t* vfptr, int32_t* vfcol);
 hipError_t launch_csr_compact(hipStream_t s, int64_t n, const int32_t* tptr, const int32_t* tcol,
                               const int32_t* row_ptr, int32_t* col);
+// The mesh of every item and cluster.
+hipError_t launch_mesh_ids(hipStream_t s, int32_t n_meshes, const DevMesh* meshes, int64_t n_items, int32_t* item_mesh,
+                           int64_t n_clusters, int32_t* clus_mesh);
 hipError_t launch_mesh_rows(hipStream_t s, int32_t n_meshes, const DevMesh* meshes, const int32_t* row_ptr,
                             int32_t* out);
 hipError_t exclusive_scan_i32(hipStream_t s, const int32_t* in, int32_t* out, int64_t n, void** tmp,

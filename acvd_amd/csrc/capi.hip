@@ -541,21 +541,51 @@ int build(acvd_ctx* c) {
   HIP_TRY(hipMemcpyAsync(c->d_meshes.p, c->h_meshes.data(), M * sizeof(DevMesh), hipMemcpyHostToDevice, s));
   HIP_TRY(launch_fill_i32(s, c->d_mask_all.p, M, 1));
   DBuf<double>& d_pos = c->d_pos;
-  for (int m = 0; m < M; ++m) {
+  // Meshes of a run of small ones go up together by way of host arrays (held until
+  // the build has ended), large ones as they are.  A copy, offset or fill for each
+  // of 8,000 meshes of 42 vertices took 115 ms of a first call of 317.
+  std::vector<int32_t> tri_stage;
+  std::vector<double> pos_stage, ind_stage;
+  auto staged = [&](int m) { return M > 1 && c->meshes[m].nf <= kStageFaces && c->meshes[m].nv <= kStageFaces; };
+  {
+    size_t v = 0, f = 0;
+    for (int m = 0; m < M; ++m)
+      if (staged(m)) {
+        v += size_t(c->meshes[m].nv);
+        f += size_t(c->meshes[m].nf);
+      }
+    tri_stage.reserve(3 * f);
+    pos_stage.reserve(3 * v);
+    if (any_ind) ind_stage.reserve(v);
+  }
+  for (int m = 0; m < M;) {
     const HostMesh& h = c->meshes[m];
     int32_t* tri = c->d_tri.p + 3 * h.face_off;
-    HIP_TRY(hipMemcpyAsync(tri, h.tri.data(), 3 * h.nf * sizeof(int32_t), hipMemcpyHostToDevice, s));
-    HIP_TRY(energy_offset_tri(s, 3 * h.nf, int32_t(h.item_off), tri));
-    HIP_TRY(hipMemcpyAsync(d_pos.p + 3 * h.item_off, h.xyz.data(), 3 * h.nv * sizeof(double), hipMemcpyHostToDevice,
-                           s));
-    if (!h.indicator.empty())
-      HIP_TRY(hipMemcpyAsync(d_ind.p + h.item_off, h.indicator.data(), h.nv * sizeof(double), hipMemcpyHostToDevice,
-                             s));
-    if (M > 1) {
-      HIP_TRY(launch_fill_i32(s, c->d_item_mesh.p + h.item_off, h.nv, m));
-      HIP_TRY(launch_fill_i32(s, c->d_clus_mesh.p + h.clus_off, h.params.number_of_clusters, m));
+    double *pos = d_pos.p + 3 * h.item_off, *ind = any_ind ? d_ind.p + h.item_off : nullptr;
+    if (!staged(m)) {
+      HIP_TRY(hipMemcpyAsync(tri, h.tri.data(), 3 * h.nf * sizeof(int32_t), hipMemcpyHostToDevice, s));
+      HIP_TRY(energy_offset_tri(s, 3 * h.nf, int32_t(h.item_off), tri));
+      HIP_TRY(hipMemcpyAsync(pos, h.xyz.data(), 3 * h.nv * sizeof(double), hipMemcpyHostToDevice, s));
+      if (!h.indicator.empty())
+        HIP_TRY(hipMemcpyAsync(ind, h.indicator.data(), h.nv * sizeof(double), hipMemcpyHostToDevice, s));
+      ++m;
+      continue;
     }
+    const size_t t0 = tri_stage.size(), p0 = pos_stage.size(), i0 = ind_stage.size();
+    for (; m < M && staged(m); ++m) {
+      const HostMesh& g = c->meshes[m];
+      for (int32_t v : g.tri) tri_stage.push_back(v + int32_t(g.item_off));
+      pos_stage.insert(pos_stage.end(), g.xyz.begin(), g.xyz.end());
+      if (!any_ind) continue;
+      if (g.indicator.empty()) ind_stage.resize(ind_stage.size() + size_t(g.nv), 0.0);
+      else ind_stage.insert(ind_stage.end(), g.indicator.begin(), g.indicator.end());
+    }
+    HIP_TRY(hipMemcpyAsync(tri, &tri_stage[t0], (tri_stage.size() - t0) * sizeof(int32_t), hipMemcpyHostToDevice, s));
+    HIP_TRY(hipMemcpyAsync(pos, &pos_stage[p0], (pos_stage.size() - p0) * sizeof(double), hipMemcpyHostToDevice, s));
+    if (any_ind)
+      HIP_TRY(hipMemcpyAsync(ind, &ind_stage[i0], (ind_stage.size() - i0) * sizeof(double), hipMemcpyHostToDevice, s));
   }
+  if (M > 1) HIP_TRY(launch_mesh_ids(s, M, c->d_meshes.p, N, c->d_item_mesh.p, K, c->d_clus_mesh.p));
   // ---- CSR
   {
     DBuf<int32_t>& vfptr = c->d_vfptr;

@@ -262,6 +262,32 @@ __global__ void k_mesh_rows(int32_t n_meshes, const DevMesh* __restrict__ meshes
   if (m == n_meshes - 1) out[n_meshes] = row_ptr[meshes[m].item_off + meshes[m].n_items];
 }
 
+// Mesh of item i (i < n_items) and of cluster i (i < n_clusters), by bisection.
+__global__ void k_mesh_ids(int32_t n_meshes, const DevMesh* __restrict__ meshes, int64_t n_items, int32_t* item_mesh,
+                           int64_t n_clusters, int32_t* clus_mesh) {
+  const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+  int32_t a = 0, b = 0;  // last mesh whose first item (cluster) is at most i
+  for (int32_t lo = 0, hi = n_meshes; hi - lo > 1;) {
+    const int32_t mid = (lo + hi) >> 1;
+    if (meshes[mid].item_off <= i) lo = a = mid;
+    else hi = mid;
+  }
+  for (int32_t lo = 0, hi = n_meshes; hi - lo > 1;) {
+    const int32_t mid = (lo + hi) >> 1;
+    if (meshes[mid].clus_off <= i) lo = b = mid;
+    else hi = mid;
+  }
+  if (i < n_items) item_mesh[i] = a;
+  if (i < n_clusters) clus_mesh[i] = b;
+}
+
+hipError_t launch_mesh_ids(hipStream_t s, int32_t n_meshes, const DevMesh* meshes, int64_t n_items, int32_t* item_mesh,
+                           int64_t n_clusters, int32_t* clus_mesh) {
+  hipLaunchKernelGGL(k_mesh_ids, dim3(grid_for(n_items > n_clusters ? n_items : n_clusters)), dim3(kBlock), 0, s,
+                     n_meshes, meshes, n_items, item_mesh, n_clusters, clus_mesh);
+  return hipGetLastError();
+}
+
 hipError_t launch_mesh_rows(hipStream_t s, int32_t n_meshes, const DevMesh* meshes, const int32_t* row_ptr,
                             int32_t* out) {
   hipLaunchKernelGGL(k_mesh_rows, dim3(grid_for(n_meshes)), dim3(kBlock), 0, s, n_meshes, meshes, row_ptr, out);

@@ -135,3 +135,34 @@ def test_shapes_on_every_path(gpu_ready, path):
         if ref is None:
             ref, _ = replay(ctx, 0, K, QEM, init, 1, 1)
         np.testing.assert_array_equal(ctx.labels(0), ref)
+
+
+def test_build_of_small_and_large_meshes(gpu_ready):
+    """A batch whose small meshes go to the device together, around two large ones, some
+    with an indicator: items, adjacency and labels of every mesh as alone."""
+    specs = [(meshgen.icosphere(2, 1, 0.02), ISO, False), (meshgen.icosphere(3, 2, 0.02), QEM, True),
+             (meshgen.icosphere(6, 3, 0.02), QEM, True), (meshgen.cube(60, 4, 1e-4), ISO, False),
+             (meshgen.icosphere(1, 5, 0.02), QEM, False), (meshgen.torus(33, 17, 6), ISO, True),
+             (meshgen.cube(12, 7, 1e-4), QEM, True)]
+
+    def add(ctx, k):
+        (xyz, tri), metric, graded = specs[k]
+        mid = ctx.add_input(xyz, tri)
+        ctx.set_params(mid, number_of_clusters=len(xyz) // 15, metric=metric, unconstrained_initialization=metric,
+                       seed=k, gradation=1.0 if graded else 0.0)
+        if graded:
+            ctx.set_indicator(mid, 1.0 + np.random.default_rng(k).random(len(xyz)))
+        ctx.set_initial_labels(mid, meshgen.seed_labels(len(xyz), len(xyz) // 15, 3))
+
+    ctx = acvd_amd.Context()
+    for k in range(len(specs)):
+        add(ctx, k)
+    ctx.process()
+    for k in range(len(specs)):
+        alone = acvd_amd.Context()
+        add(alone, k)
+        alone.process()
+        for got, want in zip((*ctx.items(k), *ctx.adjacency(k), ctx.scales(k), ctx.labels(k)),
+                             (*alone.items(0), *alone.adjacency(0), alone.scales(0), alone.labels(0))):
+            np.testing.assert_array_equal(got, want, err_msg=f"mesh {k}")
+        alone.close()

@@ -166,3 +166,21 @@ def test_build_of_small_and_large_meshes(gpu_ready):
                              (*alone.items(0), *alone.adjacency(0), alone.scales(0), alone.labels(0))):
             np.testing.assert_array_equal(got, want, err_msg=f"mesh {k}")
         alone.close()
+
+
+def test_build_memory_is_given_back(gpu_ready):
+    """A context of 2,097,152 items holds its arrays (258 bytes an item with 50 items
+    a cluster, summed from the build's plan; 5 % for rounding) and at most 64 MiB of the
+    temporaries of its build, sampling and output (88 bytes an item)."""
+    import torch
+    xyz, tri = meshgen.torus(2048, 1024, 5)
+    torch.zeros(1, device="cuda")
+    free = torch.cuda.mem_get_info()[0]
+    ctx = acvd_amd.Context()
+    ctx.set_input(np.asarray(xyz, np.float32), tri)
+    ctx.set_params(0, number_of_clusters=len(xyz) // 50, metric=QEM, unconstrained_initialization=1)
+    ctx.process()
+    ctx.output(0, 1)
+    held = free - torch.cuda.mem_get_info()[0]
+    print(f"{held / len(xyz):.1f} bytes an item", flush=True)
+    assert held <= 1.05 * 258 * len(xyz) + (64 << 20)

@@ -85,6 +85,7 @@ constexpr size_t kSlabMin = size_t(32) << 20;
 struct SlabPlan {
   size_t bytes = 0;
   std::vector<std::function<hipError_t(void*)>> parts;  // of the slab, or (null) allocated
+  std::vector<std::function<void()>> releases;
   template <class T>
   void add(DBuf<T>& b, size_t count) {
     if (count == 0) count = 1;
@@ -95,20 +96,28 @@ struct SlabPlan {
       b.view(base, off, count);
       return hipSuccess;
     });
+    releases.push_back([&b] { b.release(); });
   }
-  // gives the parts out of `slab`, which is allocated again when it is too small
-  // or (shrink: a build, whose other steps need less) more than twice the need
-  hipError_t give(DBuf<char>& slab, bool shrink = false) {
-    const bool apart = bytes <= kSlabMin && slab.n < bytes;
-    if (!apart && (slab.n < bytes || (shrink && slab.n / 2 > bytes))) {
+  // gives the parts out of `slab`, which is allocated again when it is too small or
+  // more than twice the need
+  hipError_t give(DBuf<char>& slab) {
+    const bool whole = bytes > kSlabMin;
+    if (whole && (slab.n < bytes || slab.n / 2 > bytes)) {
       const hipError_t e = slab.alloc(bytes);
       if (e != hipSuccess) return e;
     }
     for (auto& f : parts) {
-      const hipError_t e = f(apart ? nullptr : slab.p);
+      const hipError_t e = f(whole ? slab.p : nullptr);
       if (e != hipSuccess) return e;
     }
     return hipSuccess;
+  }
+  // no array of the plan points into the slab any more
+  void release() {
+    for (auto& f : releases) f();
+    bytes = 0;
+    parts.clear();
+    releases.clear();
   }
 };
 
@@ -159,6 +168,7 @@ struct acvd_ctx {
   // comes from the device), temporary ones of d_scratch (Scratch); both go with
   // the context
   DBuf<char> d_slab, d_scratch;
+  SlabPlan arrays;  // of d_slab, as last built
   DBuf<DevMesh> d_meshes;
   DBuf<MeshState> d_state;
   DBuf<Ctrl> d_ctrl;
@@ -467,7 +477,9 @@ int build(acvd_ctx* c) {
   {
     const size_t n = size_t(N), k = size_t(K), f3 = 3 * size_t(F), nt = size_t(c->n_tiles);
     const size_t nc = size_t(c->cand_cap) * size_t(c->n_seg);
-    SlabPlan p;
+    // (arrays that this build leaves out hold nothing of the last one)
+    SlabPlan& p = c->arrays;
+    p.release();
     p.add(c->d_meshes, M);
     p.add(c->d_state, M);
     p.add(c->d_ctrl, 1);
@@ -523,7 +535,8 @@ int build(acvd_ctx* c) {
     p.add(c->d_comp_size, n);
     p.add(c->d_ncomp, k);
     p.add(c->d_best, k);
-    HIP_TRY(p.give(c->d_slab, true));
+    if (p.bytes <= kSlabMin) c->d_slab.release();
+    HIP_TRY(p.give(c->d_slab));
   }
   // temporary arrays
   std::vector<int2> tab;  // blocks of the deterministic reductions

@@ -184,3 +184,44 @@ def test_build_memory_is_given_back(gpu_ready):
     held = free - torch.cuda.mem_get_info()[0]
     print(f"{held / len(xyz):.1f} bytes an item", flush=True)
     assert held <= 1.05 * 258 * len(xyz) + (64 << 20)
+
+
+def test_a_context_built_again(gpu_ready):
+    """One context of more than 32 MB of arrays (one allocation) taken through other
+    meshes, metrics, flags and shapes, larger and smaller: labels as from a new one."""
+    big = meshgen.torus(500, 400, 3)
+    small = meshgen.icosphere(4, 2, 0.02)
+    larger = meshgen.torus(700, 430, 4)
+
+    def setup(ctx, meshes, metric, fixed=False, frozen=False):
+        for k, (xyz, tri) in enumerate(meshes):
+            mid = 0
+            if k == 0:
+                ctx.set_input(xyz, tri)
+            else:
+                mid = ctx.add_input(xyz, tri)
+            K = len(xyz) // 40
+            ctx.set_params(mid, number_of_clusters=K, metric=metric, unconstrained_initialization=metric, seed=9,
+                           max_number_of_loops=12)
+            if fixed:
+                ctx.set_fixed_clusters(mid, fixed_items(len(xyz), 9, 1))
+            ctx.set_initial_labels(mid, meshgen.seed_labels(len(xyz), K, 3))
+            if frozen:
+                ctx.set_frozen_clusters(mid, (np.arange(K) % 3 == 0).astype(np.int32))
+        ctx.process()
+        return [ctx.labels(k) for k in range(len(meshes))]
+
+    steps = [dict(meshes=[big], metric=QEM, fixed=True), dict(meshes=[big], metric=ISO),
+             dict(meshes=[big, small], metric=QEM), dict(meshes=[larger], metric=QEM, frozen=True),
+             dict(meshes=[small], metric=ISO), dict(meshes=[small, big], metric=ISO, fixed=True),
+             dict(meshes=[larger], metric=QEM)]
+    ctx = acvd_amd.Context()
+    for k, step in enumerate(steps):
+        print(k, step["metric"], [len(m[0]) for m in step["meshes"]], flush=True)
+        if k % 2:
+            ctx.set_tuning(sweep_segments=512 + k)
+        got = setup(ctx, **step)
+        fresh = acvd_amd.Context()
+        for a, b in zip(got, setup(fresh, **step)):
+            np.testing.assert_array_equal(a, b, err_msg=f"step {k}")
+        fresh.close()

@@ -770,7 +770,7 @@ int run_chunk_timed(acvd_ctx* c, bool qem_unc, bool tiles, bool crowded, int n_p
   }
   HIP_TRY(hipStreamSynchronize(s));
   for (int p = 0; p < n_pass; ++p)
-    for (int k = 0; k < 4; ++k) {
+    for (int k = fused ? 1 : 0; k < 4; ++k) {  // fused: no scan of its own
       float ms = 0;
       HIP_TRY(hipEventElapsedTime(&ms, ev[5 * p + k], ev[5 * p + k + 1]));
       c->kernel_ms[k] += ms;

@@ -120,7 +120,8 @@ typedef struct acvd_stats {
   int64_t n_adjacency;      /* CSR entries of this mesh (2E) */
   /* per-kernel device time when timing is on (acvd_set_timing), context-wide:
    * [0] scan, [1] evaluate, [2] accept rounds (apply, re-evaluate, apply ...),
-   * [3] controller; launches count one per pass for [2] */
+   * [3] controller; launches count one per pass for [2].  Passes that scan and
+   * evaluate in one kernel (acvd_set_path_limits) count in [1] alone */
   double kernel_ms[4];
   int64_t kernel_launches[4];
   /* accept-round work, context-wide, all passes (the re-registered,

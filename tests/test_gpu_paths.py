@@ -225,3 +225,22 @@ def test_a_context_built_again(gpu_ready):
         for a, b in zip(got, setup(fresh, **step)):
             np.testing.assert_array_equal(a, b, err_msg=f"step {k}")
         fresh.close()
+
+
+@pytest.mark.parametrize("path", list(PATHS))
+def test_timed_runs_count_the_kernels_that_ran(gpu_ready, path):
+    xyz, tri = meshgen.icosphere(5, 4, 0.03)
+    ctx = acvd_amd.Context()
+    ctx.set_input(xyz, tri)
+    ctx.set_params(0, number_of_clusters=400, metric=QEM, unconstrained_initialization=1, seed=5)
+    ctx.set_initial_labels(0, meshgen.seed_labels(len(xyz), 400, 3))
+    set_path(ctx, path)
+    ctx.process()
+    lab = ctx.labels(0)
+    ctx.set_timing(True)
+    ctx.process()
+    np.testing.assert_array_equal(ctx.labels(0), lab)
+    n, ms, passes = ctx.stats(0)["kernel_launches"], ctx.stats(0)["kernel_ms"], ctx.path_passes()
+    assert n[0] == passes["list"] + passes["tiles"]
+    assert n[1] == n[2] == n[3] == sum(passes.values())
+    assert all((a > 0) == (b > 0) for a, b in zip(n, ms)), (n, ms)

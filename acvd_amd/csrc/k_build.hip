@@ -460,10 +460,13 @@ struct Star2 {
   }
 };
 
-__global__ __launch_bounds__(kCurvBlock) void k_curvature(int64_t off, int64_t n, const double* __restrict__ pos, const int32_t* __restrict__ tri,
-                            const int32_t* __restrict__ rp, const int32_t* __restrict__ col,
-                            const int32_t* __restrict__ vfptr, const int32_t* __restrict__ vfcol,
-                            double* __restrict__ out) {
+__global__ __launch_bounds__(kCurvBlock) void k_curvature(int64_t off, int64_t n, const double* __restrict__ pos,
+                                                          const int32_t* __restrict__ tri,
+                                                          const int32_t* __restrict__ rp,
+                                                          const int32_t* __restrict__ col,
+                                                          const int32_t* __restrict__ vfptr,
+                                                          const int32_t* __restrict__ vfcol,
+                                                          double* __restrict__ out) {
   const int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (idx >= n) return;
   const int32_t v = int32_t(off + idx);
@@ -704,8 +707,8 @@ hipError_t launch_curvature(hipStream_t s, int64_t off, int64_t n, const double*
                             const int32_t* row_ptr, const int32_t* col, const int32_t* vfptr, const int32_t* vfcol,
                             double* out) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_curvature, dim3(unsigned((n + kCurvBlock - 1) / kCurvBlock)), dim3(kCurvBlock), 0, s, off, n, pos, tri, row_ptr, col, vfptr,
-                     vfcol, out);
+  hipLaunchKernelGGL(k_curvature, dim3(unsigned((n + kCurvBlock - 1) / kCurvBlock)), dim3(kCurvBlock), 0, s, off, n,
+                     pos, tri, row_ptr, col, vfptr, vfcol, out);
   return hipGetLastError();
 }
 

@@ -798,7 +798,7 @@ __device__ inline void pool_post_long(const SweepView& v, QemPool* pool, int64_t
     int32_t c = ~lab;
     if (j > 0) {
       k = qem_next_open(v, lab, s, 1, k);
-      c = k < s.r1 ? v.labels[v.col[k]] : ~lab;  // the state is frozen: the count of pool_screen holds
+      c = k < s.r1 ? v.labels[v.col[k]] : ~lab;  // the state is frozen: the count of pool_screen_long holds
     }
     pool->cl[first + j - j0] = c;
     pool->owner[first + j - j0] = uint8_t(__lane_id());
@@ -806,7 +806,7 @@ __device__ inline void pool_post_long(const SweepView& v, QemPool* pool, int64_t
 }
 
 // Every lane of the wave calls it.  An owner (kind != kPoolNone, from
-// pool_screen, mesh m) receives its item's move as qem_propose_short_row /
+// its screen, mesh m) receives its item's move as qem_propose_short_row /
 // the generic QEM rule would return it.  Short-row owners post all their
 // solves first (a wave posts at most kPoolTasks of them), so that the lanes
 // keep only the choice state across the solve steps; long-row owners post
@@ -1063,7 +1063,7 @@ __global__ __launch_bounds__(kBlock, METRIC == 1 ? 3 : 4) void k_scan_eval(Sweep
     if (n && threadIdx.x == 0) atomicAdd(&a.work_count[blockIdx.x % kWorkSlices], n);  // items evaluated
     __syncthreads();
     if (n) {  // block-uniform
-      // spread over the waves (walk_even)
+      // spread over the waves (EvenWalk)
       const int32_t per = (n + kBlock / 64 - 1) / (kBlock / 64);
       const int32_t off = w * per + lane;
       const bool valid = lane < per && off < n;

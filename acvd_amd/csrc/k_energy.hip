@@ -372,7 +372,7 @@ __device__ inline void merge_step(double (&v)[V], int rem) {
 // times, 34 M f64 atomics for 16.8 M QEM vertices and most of the kernel's time;
 // kept over a block's range it flushes each 1 to 2 times.  Now bound by the f64
 // work (580 instructions a step of 64 items, 60 % of the time) and the gathers'
-// latency at 4 waves per SIMD: 16.8 M QEM vertices 2328 -> 372 us (a copy of the
+// latency at 4 waves per SIMD: 16.8 M QEM vertices 2328 -> 377 us (a copy of the
 // bytes takes 168 us), 1 M isotropic ones 45.7 -> 16.7 us.
 template <bool kQem>
 __global__ __launch_bounds__(kAccBlock) void ke_accumulate(EnergyArgs a, int64_t chunk) {
@@ -823,11 +823,11 @@ __device__ inline PlaneAdjoint no_adjoint() {
 // by one behind its loads, and from the row past 16: a sphere of 368,642 vertices of
 // valence 3 to 24, labels of a clustering, 303 us, so 95; the forward 232, 101).  Consecutive blocks run on one XCD, whose
 // L2 then holds the rows a block shares with its neighbours (HBM reads 1.27 ->
-// 0.87 GB).  Bound by the f64 work (950
+// 0.89 GB).  Bound by the f64 work (980
 // instructions per 64 vertices, half of the time) and by gather latency at 3
 // waves per SIMD (168 registers; held to 128 the spills cost more: 1359 us;
 // a loop over the faces that keeps one position in flight: 831 us).
-// 16.8 M QEM vertices 2050 -> 765 us, 1 M isotropic ones 10.5 -> 8.6 us.
+// 16.8 M QEM vertices 2050 -> 752 us, 1 M isotropic ones 10.5 -> 8.6 us.
 template <bool kQem>
 __global__ __launch_bounds__(kEBlock) void ke_item_grad(EnergyArgs a, const double* __restrict__ gE,
                                                         float* __restrict__ dxyz, float* __restrict__ dw) {
